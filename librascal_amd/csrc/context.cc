@@ -1049,8 +1049,9 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     blks.push_back(gap_block<T>(c, s, X, sparse_values<T>(c)));
     blks.back().D = D;
     wt_off.push_back(wt_total);
-    // blocks start on 8-element (16-byte) boundaries
-    wt_total += (blks.back().n_rows * blks.back().n_cols + 7) / 8 * 8;
+    // (mixed: rows padded to whole 32-column steps)
+    wt_total += blks.back().n_rows *
+                (std::is_same<T, float>::value ? gap_mixed_wt_stride(blks.back().n_cols) : blks.back().n_cols);
     if (blks.back().n_rows > 0 && blks.back().n_cols == 0) rows_without_points = true;
   }
   T* G = nullptr;
@@ -1955,7 +1956,7 @@ int rgpu_set_sparse_points(rgpu_context* ctx, int zeta, int64_t n_sparse, const 
     c.M = n_sparse;
     c.have_weights = weights != nullptr;
     // (the mixed path's packed operands; a sparsified layout is FP64 only)
-    if (!c.sparsified()) prepare_mixed_sparse(c.mixed_sparse, T, n_sparse, S, c.rd.N, c.rd.L1, c.stream);
+    if (!c.sparsified()) prepare_mixed_sparse(c.mixed_sparse, dT, n_sparse, S, c.rd.N, c.rd.L1, c.sp_off, c.stream);
     c.have_sparse = true;
   });
 }

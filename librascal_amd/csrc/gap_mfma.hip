@@ -14,16 +14,20 @@
 // Tiling: 256 threads (4 wavefronts, 2 x 2), block tile 128 x 128, K step 32;
 // each wavefront owns 64 x 64 = 2 x 2 MFMA tiles.  Two LDS stages (one
 // barrier per K step), the next K step's global loads issued before the
-// MFMAs of the current one.  Where every row is 16-byte aligned and K is a
-// multiple of 32 (the packed layout guarantees both), the loads go straight
-// to LDS (global_load_lds_dwordx4) in a swizzled layout; otherwise they pass
-// through registers with a guarded K tail.  All species blocks of one
+// MFMAs of the current one.  Every operand row is 16-byte aligned and every
+// K a multiple of 32: the packed feature rows are padded to that, and so are
+// the sparse points of each species in the force product (W~ rows and T^T
+// columns carry zero pads up to the next multiple of 32).  So the loads
+// always go straight to LDS (global_load_lds_dwordx4) in a swizzled layout.
+// Unpadded W~ went through a second, register-staged kernel with a guarded K
+// tail: a whole prediction of 1331 centres against 2 x 1000 sparse points
+// (n_max 10, l_max 8) took 572 us with it and takes 369 us with the pads.
+// All species blocks of one
 // product go in one grouped launch, dealt to the XCDs so that a row panel
 // stays in one L2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstring>
 
 #include "common.hh"
 #include "gap_mfma.hh"
@@ -56,14 +60,14 @@ struct Problem {
   const int* c_rows;           // output row ids (centre indices)
   int64_t tile0;               // first linear tile of this problem
   int tiles_m, tiles_n;        // tiles along M and N
-  int fast;                    // K % 32 == 0 and every row 16-byte aligned
   // kernel epilogue
   const double* norm2;
   const double* alpha;         // offset to the block's first sparse point
   double* epart;               // energy partials [tiles_n][ldp], by centre
   int64_t ldp;
-  unsigned short* wth;         // [M][N] W~ split (may be null)
+  unsigned short* wth;         // [M][ldw] W~ split (may be null), columns N .. ldw zero
   unsigned short* wtl;
+  int64_t ldw;
   // force epilogue
   float* G;
   int64_t ldg;
@@ -92,25 +96,6 @@ __device__ __forceinline__ T pow_int(T v, int n) {
   } while (u);
   return r;
 }
-
-// 32-row block rb, 16-wide K chunk c, lane l (row l%32, K 8*(l/32) .. +8):
-// fragment slot in an LDS stage, XOR-swizzled by 4 c + 2 (l / 32) inside
-// aligned groups of 8 so the K-coalesced stores and the fragment reads hit
-// distinct banks
-__device__ __forceinline__ int frag_slot(int rb, int c, int l) {
-  return (rb * (BK / 16) + c) * 64 + (l ^ (4 * c + 2 * (l >> 5)));
-}
-
-constexpr int FR = (BM / 32) * (BK / 16) * 64;  // fragments per operand per LDS stage
-
-// LDS of one workgroup: two stages of the four operand planes
-struct GemmLds {
-  bf16x8 Ah[2][FR];
-  bf16x8 Al[2][FR];
-  bf16x8 Bh[2][FR];
-  bf16x8 Bl[2][FR];
-  double esum[2][BM];
-};
 
 // Epilogue of a TBM x 128 block tile whose wavefronts form (TBM / 64) x 2
 // and own 64 x 64 = 2 x 2 MFMA tiles each; esum: LDS [2][TBM]
@@ -144,7 +129,10 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const int64_t c = c0 + wn * 64 + j * 32 + fr;
-          if (c >= P.N) continue;
+          if (c >= P.N) {
+            if (P.wth && c < P.ldw) P.wth[r * P.ldw + c] = P.wtl[r * P.ldw + c] = 0;
+            continue;
+          }
           const float k = float(double(acc[i][j][e]) * inv);
           const double a = P.alpha[c];
           rowsum[i][e] += a * double(pow_int(k, ps.zeta));
@@ -152,8 +140,8 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
             const float g = ps.zeta > 1 ? float(ps.zeta) * pow_int(k, ps.zeta - 1) : 1.f;
             const float v = float(a) * g;
             const __bf16 h = (__bf16)v;
-            P.wth[r * P.N + c] = bf16_bits(h);
-            P.wtl[r * P.N + c] = bf16_bits((__bf16)(v - (float)h));
+            P.wth[r * P.ldw + c] = bf16_bits(h);
+            P.wtl[r * P.ldw + c] = bf16_bits((__bf16)(v - (float)h));
           }
         }
       }
@@ -196,137 +184,6 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
   }
 }
 
-template <int EPI, bool FAST>
-__device__ __forceinline__ void gemm_tile(const ProblemSet& ps, const Problem& P, int64_t r0, int64_t c0,
-                                          GemmLds& sm) {
-  auto& sAh = sm.Ah;
-  auto& sAl = sm.Al;
-  auto& sBh = sm.Bh;
-  auto& sBl = sm.Bl;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // Global loads are coalesced along K: four lanes read the 32 K values
-  // (64 B per plane) of one row, rows rs + 64 j (j < 2).  Rows past the
-  // matrix edge repeat its last row (their results are never stored).
-  const int rs = tid >> 2, kq = tid & 3;
-  const unsigned short *Ah[2], *Al[2], *Bh[2], *Bl[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    int64_t ra = r0 + rs + 64 * j;
-    ra = ra < P.M ? ra : P.M - 1;
-    if (P.a_rows) ra = P.a_rows[ra];
-    Ah[j] = P.Ahi + ra * P.lda;
-    Al[j] = P.Alo + ra * P.lda;
-    int64_t rb = c0 + rs + 64 * j;
-    rb = rb < P.N ? rb : P.N - 1;
-    Bh[j] = P.Bhi + rb * P.ldb;
-    Bl[j] = P.Blo + rb * P.ldb;
-  }
-  const int sc = kq >> 1, shalf = kq & 1;
-  int fs[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int r = rs + 64 * j;
-    fs[j] = frag_slot(r >> 5, sc, (r & 31) + 32 * shalf);
-  }
-
-  // two register stages: the global loads of K step kt + 2 are issued while
-  // step kt computes, and stored to LDS at the end of step kt + 1
-  uint4 rah[2][2], ral[2][2], rbh[2][2], rbl[2][2];
-  auto load8 = [&](const unsigned short* p, int64_t k) -> uint4 {
-    if (FAST) return *reinterpret_cast<const uint4*>(p + k);
-    unsigned short t[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) t[q] = (k + q < P.K) ? p[k + q] : (unsigned short)0;
-    uint4 v;
-    memcpy(&v, t, 16);
-    return v;
-  };
-  auto gload = [&](int rs_, int64_t k0) {
-    const int64_t k = k0 + 8 * kq;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      rah[rs_][j] = load8(Ah[j], k);
-      ral[rs_][j] = load8(Al[j], k);
-      rbh[rs_][j] = load8(Bh[j], k);
-      rbl[rs_][j] = load8(Bl[j], k);
-    }
-  };
-  auto lstore = [&](int rs_, int st) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      sAh[st][fs[j]] = __builtin_bit_cast(bf16x8, rah[rs_][j]);
-      sAl[st][fs[j]] = __builtin_bit_cast(bf16x8, ral[rs_][j]);
-      sBh[st][fs[j]] = __builtin_bit_cast(bf16x8, rbh[rs_][j]);
-      sBl[st][fs[j]] = __builtin_bit_cast(bf16x8, rbl[rs_][j]);
-    }
-  };
-
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-  auto compute = [&](int st) {
-#pragma unroll
-    for (int c = 0; c < BK / 16; ++c) {
-      bf16x8 ah[2], al[2], bh[2], bl[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int f = frag_slot(wm * 2 + i, c, lane);
-        ah[i] = sAh[st][f];
-        al[i] = sAl[st][f];
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int f = frag_slot(wn * 2 + j, c, lane);
-        bh[j] = sBh[st][f];
-        bl[j] = sBl[st][f];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
-        }
-    }
-  };
-
-  const int64_t nk = (P.K + BK - 1) / BK;
-  // K step of a prefetch, clamped to the last one: the loads and LDS stores
-  // are issued unconditionally (the surplus ones at the end are never read),
-  // which keeps the wait before each LDS store at the loads it consumes
-  // rather than at every load in flight
-  auto step = [&](int64_t kt) { return (kt < nk ? kt : nk - 1) * BK; };
-  gload(0, 0);
-  gload(1, step(1));
-  lstore(0, 0);
-  __syncthreads();
-  // K steps in pairs so that the register stage indices are constants;
-  // step kt reads LDS stage kt & 1 and register stage kt & 1 is refilled
-  for (int64_t kt = 0; kt < nk; kt += 2) {
-    gload(0, step(kt + 2));
-    compute(0);
-    // the other LDS stage was last read before the previous barrier
-    lstore(1, 1);
-    __syncthreads();
-    if (kt + 1 >= nk) break;
-    gload(1, step(kt + 3));
-    compute(1);
-    lstore(0, 0);
-    __syncthreads();
-  }
-
-  gemm_epilogue<EPI, BM>(ps, P, r0, c0, acc, sm.esum);
-}
-
 // s_waitcnt vmcnt(N), the other counters left alone (gfx9 encoding)
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
@@ -356,7 +213,7 @@ struct DmaLds {
 };
 
 // TBM x 128 block tile, TBM / 32 wavefronts, NS LDS stages with NS - 1 K
-// steps in flight; requires the fast layout (K % 32 == 0, aligned rows)
+// steps in flight; K % 32 == 0 and 16-byte aligned rows
 template <int EPI, int TBM, int NS>
 __device__ __forceinline__ void gemm_tile_dma(const ProblemSet& ps, const Problem& P, int64_t r0,
                                               int64_t c0, DmaLds<TBM, NS>& sm) {
@@ -483,20 +340,7 @@ __device__ __forceinline__ bool tile_of(const ProblemSet& ps, int* pi_out, int64
   return true;
 }
 
-template <int EPI>  // 0: GAP kernel epilogue, 1: store rows of G
-__global__ __launch_bounds__(NT, 2) void bf16x3_gemm(ProblemSet ps) {
-  int pi;
-  int64_t tm, tn;
-  if (!tile_of(ps, &pi, &tm, &tn)) return;
-  const Problem& P = ps.p[pi];
-  __shared__ __align__(16) GemmLds sm;
-  if (P.fast)
-    gemm_tile<EPI, true>(ps, P, tm * BM, tn * BN, sm);
-  else
-    gemm_tile<EPI, false>(ps, P, tm * BM, tn * BN, sm);
-}
-
-// every problem of the set in the fast layout
+// EPI 0: GAP kernel epilogue, 1: store rows of G
 template <int EPI, int TBM, int NS>
 __global__ __launch_bounds__(TBM * 2, 512 / (TBM * 2)) void bf16x3_gemm_dma(ProblemSet ps) {
   int pi;
@@ -507,24 +351,48 @@ __global__ __launch_bounds__(TBM * 2, 512 / (TBM * 2)) void bf16x3_gemm_dma(Prob
   gemm_tile_dma<EPI, TBM, NS>(ps, P, tm * TBM, tn * BN, sm);
 }
 
-unsigned short bf16_rne_host(float x) {
-  unsigned u;
-  std::memcpy(&u, &x, 4);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
-float bf16_to_float_host(unsigned short h) {
-  unsigned u = unsigned(h) << 16;
-  float f;
-  std::memcpy(&f, &u, 4);
-  return f;
-}
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
-void finish_problem(Problem& P) {
-  P.fast = (P.K % BK == 0) && (P.lda % 8 == 0) && (P.ldb % 8 == 0) && aligned16(P.Ahi) &&
-           aligned16(P.Alo) && aligned16(P.Bhi) && aligned16(P.Blo);
+// Packed BF16 planes of the sparse points in both orientations: 32 points x
+// 64 packed columns per workgroup, the values formed once (src: the one or
+// two full-layout columns of a packed column, equal for a plain copy, -1 for
+// a pad) and turned through LDS, so that both layouts are stored along their
+// rows.  Memory bound; setting 4096 points of 14400 columns took 975 ms with
+// the host loop it replaced and takes 178 ms, host copies of the values.
+constexpr int kPrepM = 32, kPrepD = 64;
+__global__ __launch_bounds__(NT) void split_sparse_kernel(const double* __restrict__ T, int64_t M, int64_t D,
+                                                          int64_t Dq, const int2* __restrict__ src,
+                                                          const int64_t* __restrict__ col, int64_t Mp,
+                                                          unsigned short* __restrict__ t_hi,
+                                                          unsigned short* __restrict__ t_lo,
+                                                          unsigned short* __restrict__ tt_hi,
+                                                          unsigned short* __restrict__ tt_lo) {
+  __shared__ unsigned short th[kPrepD][kPrepM + 2], tl[kPrepD][kPrepM + 2];
+  const int64_t d0 = int64_t(blockIdx.x) * kPrepD, m0 = int64_t(blockIdx.y) * kPrepM;
+  const int dx = threadIdx.x & (kPrepD - 1), my = threadIdx.x / kPrepD;
+  const int64_t d = d0 + dx;
+  const int2 sc = d < Dq ? src[d] : make_int2(-1, -1);
+  for (int k = my; k < kPrepM; k += NT / kPrepD) {
+    const int64_t m = m0 + k;
+    if (d >= Dq || m >= M) continue;
+    const double* row = T + m * D;
+    double v = 0.0;
+    if (sc.x >= 0) v = sc.x == sc.y ? row[sc.x] : (row[sc.x] + row[sc.y]) * 0.70710678118654752440;
+    const float x = float(v);
+    const __bf16 h = (__bf16)x;
+    const unsigned short hb = bf16_bits(h), lb = bf16_bits((__bf16)(x - (float)h));
+    t_hi[m * Dq + d] = hb;
+    t_lo[m * Dq + d] = lb;
+    th[dx][k] = hb;
+    tl[dx][k] = lb;
+  }
+  __syncthreads();
+  const int mx = threadIdx.x & (kPrepM - 1), dy = threadIdx.x / kPrepM;
+  const int64_t m = m0 + mx;
+  const int64_t c = m < M ? col[m] : -1;
+  if (c < 0) return;
+  for (int k = dy; k < kPrepD && d0 + k < Dq; k += NT / kPrepM) {
+    tt_hi[(d0 + k) * Mp + c] = th[k][mx];
+    tt_lo[(d0 + k) * Mp + c] = tl[k][mx];
+  }
 }
 
 // tile counts and first tiles of the set's problems for block rows bm
@@ -540,83 +408,90 @@ int64_t layout_tiles(ProblemSet& ps, int bm) {
   return tiles;
 }
 
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
 template <int EPI>
 void launch_set(ProblemSet& ps, hipStream_t stream) {
   if (ps.n == 0) return;
-  bool fast = true;
-  for (int i = 0; i < ps.n; ++i) fast = fast && ps.p[i].fast;
-  auto go = [&](auto kernel, int bm, int threads) {
-    ps.total_tiles = layout_tiles(ps, bm);
-    if (ps.total_tiles == 0) return;
-    const unsigned grid = unsigned((ps.total_tiles + 7) / 8 * 8);  // whole rounds over the 8 XCDs
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, stream, ps);
-    RGPU_LAUNCH_CHECK();
-  };
-  // 128 x 128 tiles either way; two stages of direct-to-LDS loads measured
-  // faster than three (with 256-row tiles) and than the register-staged loop
-  if (fast)
-    go(bf16x3_gemm_dma<EPI, BM, 2>, BM, NT);
-  else
-    go(bf16x3_gemm<EPI>, BM, NT);
+  for (int i = 0; i < ps.n; ++i) {
+    const Problem& P = ps.p[i];
+    if (P.K % BK != 0 || P.lda % 8 != 0 || P.ldb % 8 != 0 || !aligned16(P.Ahi) || !aligned16(P.Alo) ||
+        !aligned16(P.Bhi) || !aligned16(P.Blo))
+      throw InvalidArgument("internal: unaligned operands of the mixed GAP product");
+  }
+  ps.total_tiles = layout_tiles(ps, BM);
+  if (ps.total_tiles == 0) return;
+  const unsigned grid = unsigned((ps.total_tiles + 7) / 8 * 8);  // whole rounds over the 8 XCDs
+  // 128 x 128 tiles; two stages of direct-to-LDS loads measured faster than
+  // three (with 256-row tiles)
+  hipLaunchKernelGGL((bf16x3_gemm_dma<EPI, BM, 2>), dim3(grid), dim3(NT), 0, stream, ps);
+  RGPU_LAUNCH_CHECK();
 }
 
 }  // namespace
 
 bool mfma_available() { return true; }
 
-void prepare_mixed_sparse(MixedSparse& ms, const std::vector<double>& T, int64_t M, int S, int N,
-                          int L1, hipStream_t stream) {
+void prepare_mixed_sparse(MixedSparse& ms, const double* T, int64_t M, int S, int N, int L1,
+                          const std::vector<int64_t>& sp_off, hipStream_t stream) {
   // rows of T in the packed layout (packing.hh); a sparse point's diagonal
   // blocks need not be symmetric: (t[n1][n2] + t[n2][n1]) / sqrt 2 keeps
   // every product with a symmetric feature row exact
   const int K = S * (S + 1) / 2, KB = N * N * L1, KD = packed_diag_block(N, L1);
   const int64_t D = int64_t(K) * KB;
   const int64_t Dq = packed_row_stride(S, N, L1);  // zero pad columns
-  ms.M = M;
   ms.D = Dq;
-  const size_t n = size_t(M * Dq);
-  std::vector<unsigned short> hi(std::max<size_t>(n, 1)), lo(std::max<size_t>(n, 1)),
-      thi(std::max<size_t>(n, 1)), tlo(std::max<size_t>(n, 1));
-  std::vector<double> row(size_t(std::max<int64_t>(Dq, 1)), 0.0);
-  for (int64_t m = 0; m < M; ++m) {
-    const double* src = T.data() + m * D;
-    for (int k = 0; k < K; ++k) {
-      int a, b;
-      key_pair(k, S, &a, &b);
-      const double* sk = src + int64_t(k) * KB;
-      double* dk = row.data() + packed_key_offset(a, b, S, N, L1);
-      if (a < b) {
-        std::copy(sk, sk + KB, dk);
-      } else {
-        for (int o = 0; o < KD; ++o) {
-          const int t = o / L1, l = o - t * L1;
-          int n1, n2;
-          packed_pair(t, N, &n1, &n2);
-          dk[o] = n1 < n2 ? (sk[(n1 * N + n2) * L1 + l] + sk[(n2 * N + n1) * L1 + l]) * 0.70710678118654752440
-                          : sk[(n1 * N + n1) * L1 + l];
-        }
-      }
-    }
-    for (int64_t d = 0; d < Dq; ++d) {
-      const float x = float(row[size_t(d)]);
-      const unsigned short h = bf16_rne_host(x);
-      const unsigned short l = bf16_rne_host(x - bf16_to_float_host(h));
-      hi[size_t(m * Dq + d)] = h;
-      lo[size_t(m * Dq + d)] = l;
-      thi[size_t(d * M + m)] = h;
-      tlo[size_t(d * M + m)] = l;
+  std::vector<int2> src(size_t(std::max<int64_t>(Dq, 1)), make_int2(-1, -1));
+  for (int k = 0; k < K; ++k) {
+    int a, b;
+    key_pair(k, S, &a, &b);
+    int2* dk = src.data() + packed_key_offset(a, b, S, N, L1);
+    const int k0 = k * KB;
+    for (int o = 0; o < (a < b ? KB : KD); ++o) {
+      int n1 = 0, n2 = 0;
+      const int l = o % L1;
+      if (a == b) packed_pair(o / L1, N, &n1, &n2);
+      dk[o] = a < b ? make_int2(k0 + o, k0 + o)
+                    : make_int2(k0 + (n1 * N + n2) * L1 + l, k0 + (n2 * N + n1) * L1 + l);
     }
   }
-  auto up = [&](DeviceBuffer<unsigned short>& b, const std::vector<unsigned short>& v) {
-    unsigned short* p = b.reserve(v.size());
-    RGPU_HIP(hipMemcpyAsync(p, v.data(), v.size() * 2, hipMemcpyHostToDevice, stream));
-  };
-  up(ms.t_hi, hi);
-  up(ms.t_lo, lo);
-  up(ms.tt_hi, thi);
-  up(ms.tt_lo, tlo);
-  RGPU_HIP(hipStreamSynchronize(stream));
+  // columns of the force operand: the points of each batch species from a
+  // multiple of 32 on, zero pads between (points of other species have none)
+  ms.col.assign(size_t(S), 0);
+  std::vector<int64_t> col(size_t(std::max<int64_t>(M, 1)), -1);
+  ms.Mp = 0;
+  for (int s = 0; s < S; ++s) {
+    ms.col[size_t(s)] = ms.Mp;
+    for (int64_t m = sp_off[size_t(s)]; m < sp_off[size_t(s) + 1]; ++m)
+      col[size_t(m)] = ms.Mp + (m - sp_off[size_t(s)]);
+    ms.Mp += gap_mixed_wt_stride(sp_off[size_t(s) + 1] - sp_off[size_t(s)]);
+  }
+  const size_t n = size_t(std::max<int64_t>(M * Dq, 1)), nt = size_t(std::max<int64_t>(ms.Mp * Dq, 1));
+  unsigned short *th = ms.t_hi.reserve(n), *tl = ms.t_lo.reserve(n);
+  unsigned short *tth = ms.tt_hi.reserve(nt), *ttl = ms.tt_lo.reserve(nt);
+  RGPU_HIP(hipMemsetAsync(tth, 0, nt * 2, stream));
+  RGPU_HIP(hipMemsetAsync(ttl, 0, nt * 2, stream));
+  if (M > 0 && Dq > 0) {
+    DeviceBuffer<int2> d_src;
+    DeviceBuffer<int64_t> d_col;
+    int2* ds = d_src.reserve(src.size());
+    int64_t* dc = d_col.reserve(col.size());
+    RGPU_HIP(hipMemcpyAsync(ds, src.data(), sizeof(int2) * src.size(), hipMemcpyHostToDevice, stream));
+    RGPU_HIP(hipMemcpyAsync(dc, col.data(), sizeof(int64_t) * col.size(), hipMemcpyHostToDevice, stream));
+    // column blocks along x: at most 65535 blocks of points along y at a time
+    for (int64_t m0 = 0; m0 < M; m0 += int64_t(65535) * kPrepM) {
+      const int64_t mm = std::min<int64_t>(M - m0, int64_t(65535) * kPrepM);
+      hipLaunchKernelGGL(split_sparse_kernel,
+                         dim3(unsigned((Dq + kPrepD - 1) / kPrepD), unsigned((mm + kPrepM - 1) / kPrepM)),
+                         dim3(NT), 0, stream, T + m0 * D, mm, D, Dq, ds, dc + m0, ms.Mp, th + m0 * Dq,
+                         tl + m0 * Dq, tth, ttl);
+      RGPU_LAUNCH_CHECK();
+    }
+    RGPU_HIP(hipStreamSynchronize(stream));  // before the maps are freed
+  }
 }
+
+int64_t gap_mixed_wt_stride(int64_t n_cols) { return (n_cols + BK - 1) / BK * BK; }
 
 int gap_mixed_energy_tiles(int64_t n_cols) { return int((n_cols + BN - 1) / BN); }
 
@@ -649,7 +524,7 @@ void run_gap_mixed_kernel(const GapBlock<float>* blks, int n_blocks, const Mixed
       P.ldp = ld;
       P.wth = wts ? wts[b].hi : nullptr;
       P.wtl = wts ? wts[b].lo : nullptr;
-      finish_problem(P);
+      P.ldw = gap_mixed_wt_stride(blk.n_cols);
       ps.normalize = blk.normalize;
       ps.zeta = blk.zeta;
       et.rows[et.n] = blk.row_idx;
@@ -671,18 +546,17 @@ void run_gap_mixed_force(const GapBlock<float>* blks, int n_blocks, const MixedS
       Problem& P = ps.p[ps.n++];
       P.M = blk.n_rows;
       P.N = blk.D;
-      P.K = blk.n_cols;
+      P.K = gap_mixed_wt_stride(blk.n_cols);  // zero pads on both operands
       P.Ahi = wts[b].hi;
       P.Alo = wts[b].lo;
-      P.lda = blk.n_cols;
+      P.lda = P.K;
       P.a_rows = nullptr;
-      P.Bhi = ms.tt_hi.get() + blk.col0;
-      P.Blo = ms.tt_lo.get() + blk.col0;
-      P.ldb = ms.M;
+      P.Bhi = ms.tt_hi.get() + ms.col[size_t(b)];
+      P.Blo = ms.tt_lo.get() + ms.col[size_t(b)];
+      P.ldb = ms.Mp;
       P.c_rows = blk.row_idx;
       P.G = G;
       P.ldg = blk.D;
-      finish_problem(P);
     }
     launch_set<1>(ps, stream);
   }
