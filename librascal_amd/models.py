@@ -150,6 +150,7 @@ def _set_model(rep, sparse_points, zeta, weights):
     old = rep._sparse_token
     if (old is not None and old[0] is sparse_points and old[1:] == token[1:]):
         return
+    rep._sparse_token = None  # nothing to go by if the upload fails
     ctx.set_sparse_points(zeta, sparse_points.numbers, sparse_points.values_for(species),
                           None if weights is None else np.asarray(weights, np.float64).ravel())
     rep._sparse_token = token

@@ -64,6 +64,8 @@ class _SphericalBase:
         # the batch whose structures are loaded in the context (an AtomsList,
         # or a species tuple for an empty batch that only fixes the layout)
         self._loaded = None
+        # the model the context holds and the species list it was loaded for
+        # (the context drops it when a batch with another list is set)
         self._sparse_token = None
 
     @property
@@ -83,20 +85,28 @@ class _SphericalBase:
         """Make atoms_list the batch held by the context (recomputing its
         representation if another batch was loaded since)."""
         if self._loaded is not atoms_list:
+            self._keep_model(atoms_list.species)
             atoms_list._upload(self)
             self._context.compute()
             self._loaded = atoms_list
+
+    def _keep_model(self, species):
+        """Before a batch with this species list is set: the context keeps its
+        sparse points, weights and zeta for the same list and drops them for
+        another (a batch of 24 cells took 21 ms with the model uploaded again
+        for each batch)."""
+        if self._sparse_token is not None and self._sparse_token[2] != tuple(species):
             self._sparse_token = None
 
     def _load_species(self, species):
         """Empty batch with the given species list (feature layout only)."""
         sp = tuple(sorted(set(int(z) for z in species)))
         if self._loaded != sp:
+            self._keep_model(sp)
             self._context.set_structures(np.zeros(1, np.int64), np.zeros((0, 3)),
                                          np.zeros(0, np.int32), np.zeros((0, 9)),
                                          np.zeros((0, 3), np.int32), list(sp))
             self._loaded = sp
-            self._sparse_token = None
 
     def get_name(self):
         return json.dumps(self.hypers, sort_keys=True)

@@ -11,6 +11,8 @@ import pytest
 
 from conftest import soap_hypers
 from librascal_amd import _capi
+from librascal_amd.models import KRR, Kernel, SparsePoints
+from librascal_amd.representations import SphericalInvariants
 from librascal_amd.synthetic import pack, periodic_box
 
 pytestmark = pytest.mark.gpu
@@ -49,3 +51,36 @@ def test_mixed_products_at_uneven_sparse_counts(m1, m8):
     em, gm, _ = ctx.gap_predict()
     assert abs(em[0] - e[0]) <= 1e-4 * abs(e[0])
     assert np.sqrt(np.mean((gm - g) ** 2)) <= 1e-4 * np.sqrt(np.mean(g ** 2))
+
+
+def test_model_kept_across_batches():
+    """A loaded model stays in the context while batches share the species
+    list, and is loaded again after a batch (or an empty layout batch) with
+    another list or another model: every prediction equals a fresh
+    calculator's bit for bit."""
+    def calculator():
+        return SphericalInvariants(interaction_cutoff=3.5, cutoff_smooth_width=0.5, max_radial=4,
+                                   max_angular=3, gaussian_sigma_type="Constant")
+
+    a = periodic_box(40, 0.05, (1, 8), d_min=1.0, seed=61)
+    b = periodic_box(51, 0.05, (1, 8), d_min=1.0, seed=62)
+    other = periodic_box(30, 0.05, (1, 6), d_min=1.0, seed=63)
+    def model(rep, seed, species=(1, 8)):
+        r = np.random.default_rng(seed)
+        D = rep.get_num_coefficients(len(species))
+        pts = SparsePoints.from_arrays(rep, species, np.repeat(species, 5), r.normal(size=(5 * len(species), D)))
+        ker = Kernel(rep, name="GAP", kernel_type="Sparse", target_type="Structure", zeta=2)
+        return KRR(r.normal(size=5 * len(species)), ker, pts, {z: 0.0 for z in (1, 6, 8)})
+
+    rep = calculator()
+    m1, m2, m3 = model(rep, 1), model(rep, 2), model(rep, 3, (1, 6))
+    for m, seed, sp, frames in ((m1, 1, (1, 8), a), (m1, 1, (1, 8), b), (m3, 3, (1, 6), other),
+                                (m1, 1, (1, 8), a), (m2, 2, (1, 8), b), (m1, 1, (1, 8), b)):
+        got = m.predict_energy_forces_stress(rep.transform(frames))
+        fresh = calculator()
+        want = model(fresh, seed, sp).predict_energy_forces_stress(fresh.transform(frames))
+        for x, y in zip(got, want):
+            assert np.array_equal(x, y)
+    # a batch of another list set in between without a prediction
+    rep.transform(other)
+    m1.predict(rep.transform(a))
