@@ -23,6 +23,7 @@
 #include "radial.hh"
 #include "scan.hh"
 #include "soap_kernels.hh"
+#include "sym_kernels.hh"
 
 namespace rgpu {
 
@@ -87,9 +88,12 @@ struct Context {
 
   // representation
   bool have_rep = false;
-  DeviceBuffer<double> c64, p64;
-  DeviceBuffer<double> ps64;         // selected invariants [n_atoms][n_sel] (un-normalised)
-  DeviceBuffer<double> gfull;        // dL/dX scattered into the full layout
+  // FP64 invariants as symmetric packed rows (sym_kernels.hh), and in the
+  // full layout where something needs that (sparsified: S^T ps64)
+  DeviceBuffer<double> c64, p64, pfull;
+  DeviceBuffer<double> ps64;         // selected invariants [n_atoms][ldx64()] (un-normalised)
+  DeviceBuffer<double> gfull, gsym;  // dL/dX scattered into the full layout, and packed
+  DeviceBuffer<double> dc64, xdot;   // dL/dc of the FP64 adjoint, X . dL/dX
   DeviceBuffer<double> dcp, dcs;     // stored expansion derivatives (gradient export)
   DeviceBuffer<float> adj_work;      // dL/dc between the adjoint's two kernels (adj_kind 3)
   // deterministic force sum: the adjoint's pair and centre forces, and the
@@ -127,7 +131,8 @@ struct Context {
   std::vector<int64_t> sp_order;  // sorted position -> given position
   std::vector<int64_t> sp_off;    // per species index s: [sp_off[s], sp_off[s+1])
   bool have_weights = false;
-  DeviceBuffer<double> T64, alpha;
+  DeviceBuffer<double> T64, alpha;  // T64 [M][ldx64()]: rows as the FP64 features'
+  DeviceBuffer<double> T64f;        // full layout [M][D] (K_NM gradient rows)
   DeviceBuffer<float> T32;
   MixedSparse mixed_sparse;
 
@@ -159,7 +164,7 @@ struct Context {
   bool use_graphs = false;
   hipStream_t own_stream = nullptr;  // created for capture when no stream was given
   hipGraphExec_t rep_exec = nullptr;
-  std::array<uintptr_t, 29> rep_sig{};
+  std::array<uintptr_t, 30> rep_sig{};
   int64_t graph_captures = 0, graph_launches = 0;
   void drop_graph() {
     if (rep_exec) (void)hipGraphExecDestroy(rep_exec);
@@ -231,6 +236,12 @@ struct Context {
     return int64_t(S) * N * L1 * L1;
   }
   bool sparsified() const { return hp.kind == SoapHypers::kPowerSpectrum && hp.sparsified; }
+  // row stride of the FP64 features and sparse points the GAP products
+  // contract: symmetric packed rows, or the selected coefficients
+  int64_t ldx64() const {
+    return sparsified() ? gap_f64_k_stride(D())
+                        : sym_row_stride(int(species.size()), hp.max_radial, hp.max_angular + 1);
+  }
   // row stride of the packed invariants of the mixed path (PowerSpectrum):
   // the packed columns rounded up to 32, pad columns zero
   int64_t Dp() const {
@@ -638,17 +649,6 @@ template <>
 DeviceBuffer<float>& cbuf<float>(Context& c) {
   return c.c32;
 }
-template <class T>
-DeviceBuffer<T>& pbuf(Context& c);
-template <>
-DeviceBuffer<double>& pbuf<double>(Context& c) {
-  return c.p64;
-}
-template <>
-DeviceBuffer<float>& pbuf<float>(Context& c) {
-  return c.p32;
-}
-
 void check_half_list(const Context& c);
 
 template <class T>
@@ -666,16 +666,21 @@ void compute_rep(Context& c) {
   unsigned long long* km = c.keymask.reserve(size_t(std::max<int64_t>(n, 1)));
   double* fc = c.pair_fc.reserve(size_t(std::max<int64_t>(cap, 1)));
   double* dfc = c.pair_dfc.reserve(size_t(std::max<int64_t>(cap, 1)));
-  // FP64 keeps the invariants in FP64; the mixed path stores them as the
-  // BF16 hi/lo operand planes of the matrix-core GEMMs
-  T* pp = ps && !split ? pbuf<T>(c).reserve(size_t(std::max<int64_t>(n * D, 1))) : nullptr;
+  // FP64 keeps the invariants in FP64 (symmetric packed rows); the mixed
+  // path stores them as the BF16 hi/lo operand planes of the matrix-core GEMMs
+  double* pp = nullptr;
+  double* pf = nullptr;  // the full layout of the fused launch and of a selection
+  if (ps && !split) {
+    pp = c.p64.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
+    if (c.sparsified() || c.tile().fused == 1) pf = c.pfull.reserve(size_t(std::max<int64_t>(n * D, 1)));
+  }
   const int64_t Dp = c.Dp();
   unsigned short* ph = ps && split ? c.p_hi.reserve(size_t(std::max<int64_t>(n * Dp, 1))) : nullptr;
   unsigned short* pl = ps && split ? c.p_lo.reserve(size_t(std::max<int64_t>(n * Dp, 1))) : nullptr;
   double* n2 = ps ? c.norm2.reserve(size_t(std::max<int64_t>(n, 1))) : nullptr;
   // sparsified: the selected coefficients and their norms (p keeps S^T xs)
   double* xs = split || !c.sparsified() ? nullptr
-                                        : c.ps64.reserve(size_t(std::max<int64_t>(n * c.D(), 1)));
+                                        : c.ps64.reserve(size_t(std::max<int64_t>(n * c.ldx64(), 1)));
   c.p32_valid = false;
   const int64_t* n_pairs_dev = c.pl.centre_off.get() + n;
   // the half list's buffers are sized for the full list, before any capture
@@ -704,7 +709,8 @@ void compute_rep(Context& c) {
   auto cutoff_and_expansion = [&] {
     launch_pair_cutoff(c.rd, n_pairs_dev, cap, c.pl.pair_dist.get(), fc, dfc, c.stream);
     if (fused)
-      launch_expansion_ps<T>(c.rd, S, pair_view(c), cc, km, pp, ph, pl, n2, c.stream, c.tile());
+      launch_expansion_ps<T>(c.rd, S, pair_view(c), cc, km, reinterpret_cast<T*>(pf), ph, pl, n2, c.stream,
+                             c.tile());
     else if (!hl.rows && c.tile().fwd_lds == 1)
       launch_expansion_ps<T>(c.rd, S, pair_view(c), cc, km, nullptr, nullptr, nullptr, nullptr,
                              c.stream, c.tile());
@@ -715,20 +721,19 @@ void compute_rep(Context& c) {
   };
   auto invariants = [&] {
     if (!ps) return;
-    if (fused) {
-      // (the invariants came with the expansion: the selection only)
-      if constexpr (!split)
-        if (xs) launch_sparsify(n, D, c.D(), c.selection(), pp, xs, n2, c.stream);
-      return;
-    }
     if constexpr (split) {
-      launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, c.tile());
+      if (!fused) launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, c.tile());
     } else {
-      launch_power_spectrum<T>(c.rd, S, n, cc, pp, n2, c.stream, c.tile());
-      if (xs) launch_sparsify(n, D, c.D(), c.selection(), pp, xs, n2, c.stream);
+      if (!fused) launch_sym_power(S, c.rd.N, c.rd.L1, n, cc, pp, n2, c.stream);
+      if (xs) {
+        if (!fused) launch_sym_unpack(S, c.rd.N, c.rd.L1, n, pp, nullptr, nullptr, false, pf, c.stream);
+        launch_sparsify(n, D, c.D(), c.ldx64(), c.selection(), pf, xs, n2, c.stream);
+      }
+      if (fused || xs)
+        launch_sym_pack(S, c.rd.N, c.rd.L1, n, pf, nullptr, pp, c.stream);
     }
   };
-  std::array<uintptr_t, 29> sig{};
+  std::array<uintptr_t, 30> sig{};
   bool replay = c.use_graphs && !c.timing && n > 0;
   if (replay) {
     sig = {
@@ -739,7 +744,8 @@ void compute_rep(Context& c) {
         uintptr_t(c.d_species_of.get()), uintptr_t(c.tile().pb_fwd), uintptr_t(c.tile().kc),
         uintptr_t(c.d_sel_col.get()), uintptr_t(c.tile().half_nl), uintptr_t(hl.src),
         uintptr_t(hl.rows), uintptr_t(c.tile().fused), uintptr_t(c.tile().fwd_lds),
-        uintptr_t(c.tile().fwd_group), uintptr_t(c.d_sel_inv_off.get()), uintptr_t(c.d_sel_inv_k.get())};
+        uintptr_t(c.tile().fwd_group), uintptr_t(c.d_sel_inv_off.get()), uintptr_t(c.d_sel_inv_k.get()),
+        uintptr_t(pf)};
     // (instantiating a graph allocates: the allocation-free path launches
     // the stage eagerly instead of capturing it)
     if ((!c.rep_exec || sig != c.rep_sig) && g_no_alloc) replay = false;
@@ -884,7 +890,7 @@ GapBlock<T> gap_block(Context& c, int s, const T* X, const T* Tm) {
   b.Tm = Tm;
   b.alpha = c.have_weights ? c.alpha.get() : nullptr;
   b.zeta = c.zeta;
-  b.D = c.D();
+  b.D = std::is_same<T, double>::value ? c.ldx64() : c.D();
   return b;
 }
 
@@ -908,35 +914,50 @@ template <>
 DeviceBuffer<float>& Gbuf<float>(Context& c) {
   return c.G32;
 }
-// Backward from G (device, [n][D] in precision T) to grad/virial (device).
-// xg (may be null): X_i . G_i per centre, times xg_scale.
-// (FP64, sparsified: G holds the selected columns and is scattered into the
-// full layout first)
-template <class T>
-void backward_device(Context& c, const T* G, double* grad, double* cvir, const double* xg = nullptr,
-                     double xg_scale = 1.0) {
+// Backward from G (device, rows as the GAP products write them in precision
+// T) to grad/virial (device).  Mixed: packed dL/dX, xg: X_i . G_i per centre,
+// times xg_scale (may be null).
+void backward_device(Context& c, const float* G, double* grad, double* cvir, const double* xg, double xg_scale) {
   const int S = int(c.species.size());
   StageTimer t(c, RGPU_STAGE_BACKWARD);
   ReverseLists rl;
   const PairView pv = backward_view(c, &rl);
-  if constexpr (std::is_same<T, double>::value) {
-    if (c.sparsified()) {
-      double* gf = c.gfull.reserve(size_t(std::max<int64_t>(c.n_atoms * c.D_full(), 1)));
-      launch_scatter_columns(c.n_atoms, c.D(), c.selection(), G, c.D_full(), gf, c.stream);
-      G = gf;
-    }
-  }
-  if constexpr (std::is_same<T, float>::value) {
-    float* work = nullptr;
-    if (c.tile().adj_kind == 3)
-      work = c.adj_work.reserve(size_t(std::max<int64_t>(c.n_atoms * S * c.rd.N * c.rd.LL, 1)));
-    launch_backward_split(c.rd, S, pv, c.c32.get(), c.p_hi.get(), c.p_lo.get(), c.norm2.get(),
-                          c.hp.normalize, xg, xg_scale, G, cvir, c.stream, c.tile(), work);
-  } else {
-    launch_backward<T>(c.rd, S, pv, cbuf<T>(c).get(), pbuf<T>(c).get(), c.norm2.get(),
-                       c.hp.normalize, xg, xg_scale, G, cvir, c.stream, c.tile());
-  }
+  float* work = nullptr;
+  if (c.tile().adj_kind == 3)
+    work = c.adj_work.reserve(size_t(std::max<int64_t>(c.n_atoms * S * c.rd.N * c.rd.LL, 1)));
+  launch_backward_split(c.rd, S, pv, c.c32.get(), c.p_hi.get(), c.p_lo.get(), c.norm2.get(), c.hp.normalize, xg,
+                        xg_scale, G, cvir, c.stream, c.tile(), work);
   launch_force_gather(pv, rl, grad, c.stream);
+}
+// FP64: G in symmetric packed rows of dL/dp, or (full) dL/dX in the full
+// layout, xg = X_i . dL/dX_i (null: summed here)
+void backward_device(Context& c, const double* G, bool full, const double* xg, double* grad, double* cvir) {
+  const int S = int(c.species.size()), N = c.rd.N, L1 = c.rd.L1;
+  StageTimer t(c, RGPU_STAGE_BACKWARD);
+  ReverseLists rl;
+  const PairView pv = backward_view(c, &rl);
+  double* dc = c.dc64.reserve(size_t(std::max<int64_t>(c.n_atoms * S * N * c.rd.LL, 1)));
+  if (full)
+    launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), c.hp.normalize ? c.p64.get() : nullptr, c.norm2.get(),
+                             xg, G, c.gsym, dc, c.stream);
+  else
+    launch_sym_contract(S, N, L1, c.n_atoms, c.c64.get(), G, dc, c.stream);
+  launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
+  launch_force_gather(pv, rl, grad, c.stream);
+}
+// selected columns of dL/dX (or dL/dp, rows ld apart) into the full layout
+const double* scatter_selected(Context& c, const double* G, int64_t ld) {
+  double* gf = c.gfull.reserve(size_t(std::max<int64_t>(c.n_atoms * c.D_full(), 1)));
+  launch_scatter_columns(c.n_atoms, ld, c.selection(), G, c.D_full(), gf, c.stream);
+  return gf;
+}
+// the FP64 invariants in the full layout (a selection keeps them: S^T xs)
+const double* full_invariants(Context& c) {
+  if (c.sparsified()) return c.pfull.get();
+  double* pf = c.pfull.reserve(size_t(std::max<int64_t>(c.n_atoms * c.D_full(), 1)));
+  launch_sym_unpack(int(c.species.size()), c.rd.N, c.rd.L1, c.n_atoms, c.p64.get(), nullptr, nullptr, false, pf,
+                    c.stream);
+  return pf;
 }
 
 // FP32 invariants of the mixed path in the full layout (for export and
@@ -980,6 +1001,17 @@ bool is_device_memory(const void* p) {
     return false;
   }
   return a.type == hipMemoryTypeDevice || a.type == hipMemoryTypeManaged;
+}
+
+// memory of the current device, which kernels read and write in place
+bool is_own_device_memory(const void* p) {
+  hipPointerAttribute_t a{};
+  int dev = 0;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && hipGetDevice(&dev) == hipSuccess && a.device == dev;
 }
 
 void emit_outputs(Context& c, const double* e_centre, double* energy, double* grad_d,
@@ -1033,7 +1065,7 @@ template <class T>
 void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_stress) {
   const int S = int(c.species.size());
   // the mixed path works on the packed invariants
-  const int64_t n = c.n_atoms, D = std::is_same<T, float>::value ? c.Dp() : c.D();
+  const int64_t n = c.n_atoms, D = std::is_same<T, float>::value ? c.Dp() : c.ldx64();
   const bool want_grad = gradient || neg_stress;
   if (want_grad) require_unmasked(c);
   double* ec = c.e_centre.reserve(size_t(std::max<int64_t>(n, 1)));
@@ -1049,9 +1081,9 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     blks.push_back(gap_block<T>(c, s, X, sparse_values<T>(c)));
     blks.back().D = D;
     wt_off.push_back(wt_total);
-    // (mixed: rows padded to whole 32-column steps)
-    wt_total += blks.back().n_rows *
-                (std::is_same<T, float>::value ? gap_mixed_wt_stride(blks.back().n_cols) : blks.back().n_cols);
+    // (rows padded to whole K steps of the force product)
+    wt_total += blks.back().n_rows * (std::is_same<T, float>::value ? gap_mixed_wt_stride(blks.back().n_cols)
+                                                                    : gap_f64_k_stride(blks.back().n_cols));
     if (blks.back().n_rows > 0 && blks.back().n_cols == 0) rows_without_points = true;
   }
   T* G = nullptr;
@@ -1088,7 +1120,8 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     }
     if (want_grad) {
       StageTimer t(c, RGPU_STAGE_GAP_FORCE);
-      run_gap_f64_force(blks.data(), S, wts.data(), G, c.stream);
+      // the GAP energy is homogeneous of degree zeta in X, so X_i . dL/dX_i = zeta E_i
+      run_gap_f64_force(blks.data(), S, wts.data(), ec, double(c.zeta), G, c.stream);
     }
   }
   double *gd = nullptr, *cv = nullptr;
@@ -1097,7 +1130,17 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     cv = c.cvir.reserve(size_t(std::max<int64_t>(6 * n, 1)));
     // (the force gather writes every atom's gradient)
     // the GAP energy is homogeneous of degree zeta in X, so X_i . G_i = zeta E_i
-    backward_device<T>(c, G, gd, cv, ec, double(c.zeta));
+    if constexpr (std::is_same<T, double>::value) {
+      // (dL/dp already: a selection's is scattered into the full layout and packed)
+      if (c.sparsified()) {
+        double* gs = c.gsym.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
+        launch_sym_pack(S, c.rd.N, c.rd.L1, n, scatter_selected(c, G, c.ldx64()), nullptr, gs, c.stream);
+        G = gs;
+      }
+      backward_device(c, G, false, nullptr, gd, cv);
+    } else {
+      backward_device(c, G, gd, cv, ec, double(c.zeta));
+    }
   }
   emit_outputs(c, ec, energy, gd, cv, gradient, neg_stress);
 }
@@ -1109,7 +1152,7 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
 template <class T>
 void gap_energy_noalloc_t(Context& c, double* ec, double* part, double* energy) {
   const int S = int(c.species.size());
-  const int64_t n = c.n_atoms, D = std::is_same<T, float>::value ? c.Dp() : c.D();
+  const int64_t n = c.n_atoms, D = std::is_same<T, float>::value ? c.Dp() : c.ldx64();
   launch_fill(ec, n, 0.0, c.stream);
   const T* X = nullptr;
   if constexpr (std::is_same<T, double>::value) X = invariants_of<double>(c);
@@ -1138,12 +1181,12 @@ void gap_knm_t(Context& c, int target, double* knm) {
   double* k = target == 0 ? c.out64.reserve(size_t(std::max<int64_t>(rows * c.M, 1))) : ka;
   RGPU_HIP(hipMemsetAsync(ka, 0, sizeof(double) * n * c.M, c.stream));
   const T* X = invariants_of<T>(c);
-  for (int s = 0; s < S; ++s) {
-    GapBlock<T> blk = gap_block<T>(c, s, X, sparse_values<T>(c));
-    blk.alpha = nullptr;
-    if (blk.n_rows == 0 || blk.n_cols == 0) continue;
-    launch_gap_kernel<T>(blk, c.M, nullptr, nullptr, ka, c.stream);
-  }
+  std::vector<GapBlock<T>> blks;
+  for (int s = 0; s < S; ++s) blks.push_back(gap_block<T>(c, s, X, sparse_values<T>(c)));
+  if constexpr (std::is_same<T, double>::value)
+    run_gap_f64_rows(blks.data(), S, ka, c.M, c.stream);
+  else
+    for (const GapBlock<T>& blk : blks) launch_gap_knm<T>(blk, c.M, ka, c.stream);
   if (target == 0) launch_rows_segment_sum(ka, c.M, c.d_atom_off.get(), c.n_struct, k, c.stream);
   // columns back to the order the sparse points were given; Atom rows of
   // the centres only
@@ -1300,22 +1343,21 @@ void autotune_t(Context& c) {
   if (ps) {
     const int K = S * (S + 1) / 2;
     constexpr bool split = std::is_same<T, float>::value;
-    T* pp = split ? nullptr : pbuf<T>(c).get();
+    double* pp = split ? nullptr : c.p64.get();
     unsigned short* ph = c.p_hi.get();
     unsigned short* pl = c.p_lo.get();
     double* n2 = c.norm2.get();
     float best = 1e30f;
-    int pick = 0;
-    for (int kc = 1; kc <= std::min(K, 12); ++kc) {
+    // (the FP64 invariants are formed by key blocks in the fused launch only,
+    // one at a time)
+    int pick = split ? 0 : 1;
+    for (int kc = 1; split && kc <= std::min(K, 12); ++kc) {
       SoapTiles cand = t;
       cand.kc = kc;
       float ms;
       try {
         ms = time_ms([&] {
-          if constexpr (split)
-            launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, cand);
-          else
-            launch_power_spectrum<T>(c.rd, S, n, cc, pp, n2, c.stream, cand);
+          if constexpr (split) launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, cand);
         });
       } catch (const InvalidArgument&) {
         continue;
@@ -1333,19 +1375,22 @@ void autotune_t(Context& c) {
         if constexpr (split)
           launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, sep);
         else
-          launch_power_spectrum<T>(c.rd, S, n, cc, pp, n2, c.stream, sep);
+          launch_sym_power(S, c.rd.N, c.rd.L1, n, cc, pp, n2, c.stream);
       });
       float ms_fu = 1e30f;
+      T* pf = split ? nullptr : reinterpret_cast<T*>(c.pfull.reserve(size_t(n * c.D_full())));
       try {
         ms_fu = time_ms([&] {
-          launch_expansion_ps<T>(c.rd, S, pv, cc, km, pp, ph, pl, n2, c.stream, fu);
+          launch_expansion_ps<T>(c.rd, S, pv, cc, km, pf, ph, pl, n2, c.stream, fu);
+          if constexpr (!split)
+            launch_sym_pack(S, c.rd.N, c.rd.L1, n, pf, nullptr, pp, c.stream);
         });
       } catch (const InvalidArgument&) {
       }
       t.fused = ms_fu < ms_sep ? 1 : 0;
     }
     // adjoint on a zero dL/dX (its time does not depend on the values)
-    const int64_t D = std::max(c.D(), c.Dp());
+    const int64_t D = split ? c.Dp() : sym_row_stride(S, c.rd.N, c.rd.L1);
     DeviceBuffer<T> G;
     DeviceBuffer<double> cv;
     T* g = G.reserve(size_t(n * D));
@@ -1353,17 +1398,19 @@ void autotune_t(Context& c) {
     double* cvir = cv.reserve(size_t(6 * n));
     ReverseLists rl;
     const PairView bpv = backward_view(c, &rl);
-    float* work = split ? c.adj_work.reserve(size_t(std::max<int64_t>(n * S * c.rd.N * c.rd.LL, 1)))
-                        : nullptr;
+    const size_t E = size_t(std::max<int64_t>(n * S * c.rd.N * c.rd.LL, 1));
+    float* work = split ? c.adj_work.reserve(E) : nullptr;
+    double* dc = split ? nullptr : c.dc64.reserve(E);
     auto time_adjoint = [&](const SoapTiles& cand) {
       try {
         return time_ms([&] {
           if constexpr (split)
             launch_backward_split(c.rd, S, bpv, cc, ph, pl, n2, c.hp.normalize, nullptr, 1.0, g,
                                   cvir, c.stream, cand, cand.adj_kind == 3 ? work : nullptr);
-          else
-            launch_backward<T>(c.rd, S, bpv, cc, pp, n2, c.hp.normalize, nullptr, 1.0, g, cvir,
-                               c.stream, cand);
+          else {
+            launch_sym_contract(S, c.rd.N, c.rd.L1, n, cc, g, dc, c.stream);
+            launch_adjoint_pairs(c.rd, S, bpv, dc, cvir, c.stream, cand);
+          }
         });
       } catch (const InvalidArgument&) {
         return 1e30f;  // needs more LDS than the device provides
@@ -1415,7 +1462,7 @@ void autotune_t(Context& c) {
     // most that fit; adj_kind 3 has a kernel of its own for it)
     best = 1e30f;
     pick = 0;
-    if (t.adj_kind != 3)
+    if (!split || t.adj_kind != 3)
       for (int pb : {0, 2, 4, 6, 8, 12, 16, 24, 32}) {
         SoapTiles cand = t;
         cand.pb_adj = pb;
@@ -1832,9 +1879,11 @@ int rgpu_get_features(rgpu_context* ctx, double* features, double* inv_norms) {
     const int64_t* rows = c.masked ? c.d_centre_idx.get() : nullptr;
     if (features && nc) {
       double* o = c.out64.reserve(size_t(nc * D));
-      if (c.precision == RGPU_FP64)
-        launch_normalise<double>(nc, D, invariants_of<double>(c), c.norm2.get(), c.hp.normalize, o,
-                                 c.stream, rows);
+      if (c.precision == RGPU_FP64 && c.sparsified())
+        launch_normalise<double>(nc, D, c.ps64.get(), c.norm2.get(), c.hp.normalize, o, c.stream, rows, c.ldx64());
+      else if (c.precision == RGPU_FP64)
+        launch_sym_unpack(int(c.species.size()), c.rd.N, c.rd.L1, nc, c.p64.get(), rows, c.norm2.get(),
+                          c.hp.normalize, o, c.stream);
       else
         launch_normalise<float>(nc, D, ensure_p32(c), c.norm2.get(), c.hp.normalize, o, c.stream,
                                 rows);
@@ -1873,8 +1922,15 @@ int rgpu_get_features_gradient(rgpu_context* ctx, double* out) {
     double* dcs = c.dcs.reserve(size_t(std::max<int64_t>(n * 3 * S * B, 1)));
     launch_pair_gradients(c.rd, S, pair_view(c), dcp, dcs, c.stream);
     double* o = is_device_memory(out) ? out : c.tmp64.reserve(size_t(3 * np * D));
+    // un-normalised invariants of the output columns, rows D apart
+    const double* sel = nullptr;
+    if (c.sparsified()) {
+      double* t = c.gfull.reserve(size_t(n * D));
+      launch_normalise<double>(n, D, c.ps64.get(), nullptr, false, t, c.stream, nullptr, c.ldx64());
+      sel = t;
+    }
     launch_feature_gradient_rows(c.rd.N, c.rd.L1, S, pair_view(c), np, c.c64.get(),
-                                 invariants_of<double>(c), c.norm2.get(), c.hp.normalize, dcp, dcs,
+                                 sel ? sel : full_invariants(c), c.norm2.get(), c.hp.normalize, dcp, dcs,
                                  D, c.sparsified() ? c.d_sel_col.get() : nullptr, o, c.stream);
     if (o != out)
       RGPU_HIP(hipMemcpyAsync(out, o, sizeof(double) * 3 * np * D, hipMemcpyDeviceToHost, c.stream));
@@ -1893,15 +1949,28 @@ int rgpu_features_backward(rgpu_context* ctx, const double* dL_dX, double* dL_dr
     const int64_t D = c.D(), n = c.n_atoms;
     double* gd = c.grad.reserve(size_t(std::max<int64_t>(3 * n, 1)));
     double* cv = c.cvir.reserve(size_t(std::max<int64_t>(6 * n, 1)));
-    double* g64 = c.tmp64.reserve(size_t(std::max<int64_t>(n * D, 1)));
-    RGPU_HIP(hipMemcpyAsync(g64, dL_dX, sizeof(double) * n * D, hipMemcpyDefault, c.stream));
+    const double* g64 = dL_dX;
+    if (!is_own_device_memory(dL_dX)) {
+      double* t = c.tmp64.reserve(size_t(std::max<int64_t>(n * D, 1)));
+      RGPU_HIP(hipMemcpyAsync(t, dL_dX, sizeof(double) * n * D, hipMemcpyDefault, c.stream));
+      g64 = t;
+    }
     if (c.precision == RGPU_FP64) {
-      backward_device<double>(c, g64, gd, cv);
+      const double* dot = nullptr;
+      if (c.sparsified()) {
+        g64 = scatter_selected(c, g64, D);
+        if (c.hp.normalize) {
+          double* d = c.xdot.reserve(size_t(std::max<int64_t>(n, 1)));
+          launch_row_dot(n, c.D_full(), c.pfull.get(), g64, c.norm2.get(), d, c.stream);
+          dot = d;
+        }
+      }
+      backward_device(c, g64, true, dot, gd, cv);
     } else {
       // dL/dX in the packed layout of the mixed path
       float* g32 = c.G32.reserve(size_t(std::max<int64_t>(n * c.Dp(), 1)));
       launch_pack_gradient(int(c.species.size()), c.rd.N, c.rd.L1, n, g64, g32, c.stream);
-      backward_device<float>(c, g32, gd, cv);
+      backward_device(c, g32, gd, cv, nullptr, 1.0);
     }
     emit_outputs(c, nullptr, nullptr, gd, cv, dL_dr, neg_stress);
   });
@@ -1940,23 +2009,38 @@ int rgpu_set_sparse_points(rgpu_context* ctx, int zeta, int64_t n_sparse, const 
       if (sidx[order[m]] < S) c.sp_off[sidx[order[m]] + 1]++;
     }
     for (int s = 0; s < S; ++s) c.sp_off[s + 1] += c.sp_off[s];
-    std::vector<double> T(size_t(n_sparse * D)), a(size_t(std::max<int64_t>(n_sparse, 1)), 0.0);
-    for (int64_t m = 0; m < n_sparse; ++m) {
-      std::copy(values + order[m] * D, values + (order[m] + 1) * D, T.begin() + m * D);
-      if (weights) a[m] = weights[order[m]];
+    std::vector<double> a(size_t(std::max<int64_t>(n_sparse, 1)), 0.0);
+    if (weights)
+      for (int64_t m = 0; m < n_sparse; ++m) a[size_t(m)] = weights[order[size_t(m)]];
+    // the values as given, then every layout the kernels read from them in
+    // sorted row order
+    const int64_t ldx = c.ldx64(), n1 = std::max<int64_t>(n_sparse, 1);
+    DeviceBuffer<double> raw;
+    DeviceBuffer<int64_t> d_order;
+    double* dr = raw.reserve(size_t(n1 * D));
+    int64_t* dord = d_order.reserve(size_t(n1));
+    double* dT = c.T64.reserve(size_t(n1 * ldx));
+    double* dTf = c.T64f.reserve(size_t(n1 * D));
+    float* dT32 = c.T32.reserve(size_t(n1 * D));
+    if (n_sparse > 0) {
+      RGPU_HIP(hipMemcpyAsync(dr, values, sizeof(double) * size_t(n_sparse * D), hipMemcpyHostToDevice, c.stream));
+      RGPU_HIP(hipMemcpyAsync(dord, order.data(), sizeof(int64_t) * size_t(n_sparse), hipMemcpyHostToDevice,
+                              c.stream));
+      launch_gather_rows<double>(n_sparse, D, D, dr, dord, dTf, c.stream);
+      launch_gather_rows<float>(n_sparse, D, D, dr, dord, dT32, c.stream);
+      if (c.sparsified())
+        launch_gather_rows<double>(n_sparse, D, ldx, dr, dord, dT, c.stream);
+      else
+        launch_sym_pack(S, c.rd.N, c.rd.L1, n_sparse, dr, dord, dT, c.stream);
+      RGPU_HIP(hipStreamSynchronize(c.stream));
     }
-    double* dT = c.T64.reserve(std::max<size_t>(T.size(), 1));
-    if (!T.empty()) RGPU_HIP(hipMemcpy(dT, T.data(), sizeof(double) * T.size(), hipMemcpyHostToDevice));
-    std::vector<float> Tf(T.begin(), T.end());
-    float* dTf = c.T32.reserve(std::max<size_t>(Tf.size(), 1));
-    if (!Tf.empty()) RGPU_HIP(hipMemcpy(dTf, Tf.data(), sizeof(float) * Tf.size(), hipMemcpyHostToDevice));
     double* da = c.alpha.reserve(a.size());
     RGPU_HIP(hipMemcpy(da, a.data(), sizeof(double) * a.size(), hipMemcpyHostToDevice));
     c.zeta = zeta;
     c.M = n_sparse;
     c.have_weights = weights != nullptr;
     // (the mixed path's packed operands; a sparsified layout is FP64 only)
-    if (!c.sparsified()) prepare_mixed_sparse(c.mixed_sparse, dT, n_sparse, S, c.rd.N, c.rd.L1, c.sp_off, c.stream);
+    if (!c.sparsified()) prepare_mixed_sparse(c.mixed_sparse, dTf, n_sparse, S, c.rd.N, c.rd.L1, c.sp_off, c.stream);
     c.have_sparse = true;
   });
 }
@@ -1976,14 +2060,20 @@ int rgpu_gram_f64(int64_t rows, int64_t cols, const double* A, double* out) {
     DeviceBuffer<int> dI;
     std::vector<int> iota(static_cast<size_t>(cols));
     for (int64_t k = 0; k < cols; ++k) iota[size_t(k)] = int(k);
-    const size_t na = size_t(rows) * size_t(cols);
-    double* a = dA.reserve(na);
-    double* at = dAt.reserve(na);
+    const int64_t lda = (cols + 1) / 2 * 2;  // 16-byte rows
+    double* a = dA.reserve(size_t(rows) * size_t(lda));
+    double* at = dAt.reserve(size_t(cols) * size_t(gap_f64_k_stride(rows)));
     double* cm = dC.reserve(nc);
     int* io = dI.reserve(iota.size());
-    RGPU_HIP(hipMemcpy(a, A, sizeof(double) * na, hipMemcpyHostToDevice));
+    if (lda == cols) {
+      RGPU_HIP(hipMemcpy(a, A, sizeof(double) * size_t(rows) * size_t(cols), hipMemcpyHostToDevice));
+    } else {
+      RGPU_HIP(hipMemset(a, 0, sizeof(double) * size_t(rows) * size_t(lda)));
+      RGPU_HIP(hipMemcpy2D(a, sizeof(double) * size_t(lda), A, sizeof(double) * size_t(cols),
+                           sizeof(double) * size_t(cols), size_t(rows), hipMemcpyHostToDevice));
+    }
     RGPU_HIP(hipMemcpy(io, iota.data(), sizeof(int) * iota.size(), hipMemcpyHostToDevice));
-    run_gram_f64(rows, cols, a, at, io, cm, nullptr);
+    run_gram_f64(rows, cols, a, lda, at, io, cm, nullptr);
     RGPU_HIP(hipMemcpy(out, cm, sizeof(double) * nc, hipMemcpyDeviceToHost));
   });
 }
@@ -1993,7 +2083,7 @@ int rgpu_gap_kmm(rgpu_context* ctx, double* kmm) {
     if (!ctx || !kmm) throw InvalidArgument("null argument");
     Context& c = ctx->c;
     if (!c.have_sparse) throw InvalidArgument(kNoSparse);
-    const int64_t M = c.M, D = c.D();
+    const int64_t M = c.M;
     std::vector<int> iota(static_cast<size_t>(std::max<int64_t>(M, 1)));
     for (int64_t m = 0; m < M; ++m) iota[size_t(m)] = int(m);
     int* rows = c.d_sp_rows.reserve(iota.size());
@@ -2001,23 +2091,21 @@ int rgpu_gap_kmm(rgpu_context* ctx, double* kmm) {
     double* k = c.tmp64.reserve(size_t(std::max<int64_t>(M * M, 1)));
     RGPU_HIP(hipMemsetAsync(k, 0, sizeof(double) * M * M, c.stream));
     // one block per run of equal species (sparse points are species-sorted)
+    std::vector<GapBlock<double>> blks;
     for (int64_t m0 = 0; m0 < M;) {
       int64_t m1 = m0 + 1;
       while (m1 < M && c.sp_species[size_t(m1)] == c.sp_species[size_t(m0)]) ++m1;
-      GapBlock<double> b;
+      GapBlock<double> b{};
       b.n_rows = b.n_cols = m1 - m0;
       b.row_idx = rows + m0;
       b.col0 = m0;
-      b.X = c.T64.get();
-      b.norm2 = nullptr;
-      b.normalize = 0;
-      b.Tm = c.T64.get();
-      b.alpha = nullptr;
+      b.X = b.Tm = c.T64.get();
       b.zeta = c.zeta;
-      b.D = D;
-      launch_gap_kernel<double>(b, M, nullptr, nullptr, k, c.stream);
+      b.D = c.ldx64();
+      blks.push_back(b);
       m0 = m1;
     }
+    run_gap_f64_rows(blks.data(), int(blks.size()), k, M, c.stream);
     std::vector<double> h(static_cast<size_t>(M * M)), o(h.size());
     RGPU_HIP(hipMemcpyAsync(h.data(), k, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c.stream));
     RGPU_HIP(hipStreamSynchronize(c.stream));
@@ -2047,13 +2135,13 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
     // d[i][m] = X_i . T_m for the centre's species (the K_NM of zeta 1)
     double* d = c.tmp64.reserve(size_t(std::max<int64_t>(n * M, 1)));
     RGPU_HIP(hipMemsetAsync(d, 0, sizeof(double) * n * M, c.stream));
+    std::vector<GapBlock<double>> blks;
     for (int s = 0; s < S; ++s) {
-      GapBlock<double> blk = gap_block<double>(c, s, invariants_of<double>(c), c.T64.get());
-      blk.alpha = nullptr;
-      blk.zeta = 1;
-      if (blk.n_rows == 0 || blk.n_cols == 0) continue;
-      launch_gap_kernel<double>(blk, M, nullptr, nullptr, d, c.stream);
+      blks.push_back(gap_block<double>(c, s, invariants_of<double>(c), c.T64.get()));
+      blks.back().zeta = 1;
     }
+    run_gap_f64_rows(blks.data(), S, d, M, c.stream);
+    const double* pf = full_invariants(c);
     double* gs = c.knm_scale.reserve(size_t(std::max<int64_t>(n, 1)));
     double* gd = c.grad.reserve(size_t(std::max<int64_t>(3 * n, 1)));
     double* cv = c.cvir.reserve(size_t(std::max<int64_t>(6 * n, 1)));
@@ -2068,12 +2156,12 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
     for (int s = 0; s < S; ++s)
       for (int64_t m = c.sp_off[s]; m < c.sp_off[s + 1]; ++m) {
         launch_knm_gradient_scale(n, d + m, M, c.d_species_of.get(), s, c.zeta, gs, c.stream);
-        const double* row = c.T64.get() + m * D;
+        const double* row = c.T64f.get() + m * D;
         if (grow) {
           launch_scatter_columns(1, D, c.selection(), row, c.D_full(), grow, c.stream);
           row = grow;
         }
-        launch_backward_rank1(c.rd, S, bpv, c.c64.get(), c.p64.get(), c.norm2.get(),
+        launch_backward_rank1(c.rd, S, bpv, c.c64.get(), pf, c.norm2.get(),
                               c.hp.normalize, row, gs, cv, c.stream, c.tile());
         launch_force_gather(bpv, rl, gd, c.stream);
         const int64_t col = c.sp_order[size_t(m)];

@@ -1,7 +1,6 @@
-// Sparse GAP kernel on the GPU: K = (X T^T)^zeta per species block, energy,
-// the weighted kernel gradient W~ = alpha zeta (X T^T)^(zeta-1) and the force
-// contraction T~ = W~ T (models/sparse_kernels.hh:104-190,
-// models/sparse_kernel_predict.hh:70-181).
+// Sparse GAP kernel on the GPU: K = (X T^T)^zeta per species block
+// (models/sparse_kernels.hh:104-190, models/sparse_kernel_predict.hh:70-181;
+// the products of a prediction are in gap_mfma.hh and gap_f64.hh).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -18,7 +17,7 @@ struct GapBlock {
   const int* row_idx;     // [n_rows] centre indices
   int64_t n_cols;         // sparse points of this species
   int64_t col0;           // first sparse point (global, species-sorted order)
-  const T* X;             // [n_centres][D] un-normalised power spectrum
+  const T* X;             // [n_centres][D] un-normalised power spectrum (rows D apart)
   const double* norm2;    // [n_centres]
   int normalize;
   const T* Tm;            // [M][D] sparse points (species-sorted)
@@ -27,11 +26,10 @@ struct GapBlock {
   int64_t D;
 };
 
-// GEMM1 + epilogue.  Any of energy (per centre, +=), wt ([n_rows][n_cols]),
-// knm_atom ([n_centres][M], written) may be null.
+// K_NM rows knm_atom[row_idx[r]][col0 + m] = (X_r . T_m)^zeta of one block
+// (rows of M columns), full-layout features
 template <class T>
-void launch_gap_kernel(const GapBlock<T>& blk, int64_t M, double* energy, T* wt, double* knm_atom,
-                       hipStream_t stream);
+void launch_gap_knm(const GapBlock<T>& blk, int64_t M, double* knm_atom, hipStream_t stream);
 
 // out[s][:] = sum over rows a in [seg_off[s], seg_off[s+1]) of in[a][:]
 // (rows of w doubles, summed in row order; out written)
@@ -52,9 +50,5 @@ struct EnergyTiles {
 };
 void launch_energy_tiles(const EnergyTiles& et, const double* part, int64_t ld, double* energy,
                          hipStream_t stream);
-
-// GEMM2: G[row_idx[r]][:] = sum_m wt[r][m] Tm[col0+m][:]
-template <class T>
-void launch_gap_force_contraction(const GapBlock<T>& blk, const T* wt, T* G, hipStream_t stream);
 
 }  // namespace rgpu

@@ -123,10 +123,11 @@ void launch_power_spectrum_split(const RadialDev& rad, int S, int64_t n_centres,
                                  hipStream_t stream, const SoapTiles& tiles = SoapTiles());
 
 // Normalised copy X = p / |p| (or X = p), FP64 output for export: n rows,
-// row r from row rows[r] of p (rows null: row r).
+// row r from row rows[r] of p (rows null: row r), p's rows ld values apart
+// (0: D).
 template <class T>
 void launch_normalise(int64_t n, int64_t D, const T* p, const double* norm2, bool normalize,
-                      double* out, hipStream_t stream, const int64_t* rows = nullptr);
+                      double* out, hipStream_t stream, const int64_t* rows = nullptr, int64_t ld = 0);
 
 // Stored expansion derivatives (FP64) for the feature-gradient export:
 // dcp[p][3][N][(L+1)^2] per pair (the self slot unused) and the centre
@@ -152,29 +153,31 @@ struct SelectionMap {
   const int64_t* inv_off = nullptr;
   const int64_t* inv_k = nullptr;
 };
-// xs[i][k] = p[i][col[k]], norm2[i] = |xs_i|^2, then p[i] = S^T xs_i (the
-// selected coefficients, zero elsewhere)
-void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, const SelectionMap& sel, double* p, double* xs,
+// xs[i][k] = p[i][col[k]] (rows lds apart, zero pad), norm2[i] = |xs_i|^2,
+// then p[i] = S^T xs_i (the selected coefficients, zero elsewhere)
+void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, int64_t lds, const SelectionMap& sel, double* p, double* xs,
                      double* norm2, hipStream_t stream);
-// dst[i][:D] = S^T src[i][:Dsel] (repeated selections summed in ascending
+// dst[i][:D] = S^T src[i][:Dsel], src rows lds apart (repeated selections summed in ascending
 // selection order)
-void launch_scatter_columns(int64_t n, int64_t Dsel, const SelectionMap& sel, const double* src, int64_t D,
+void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t D,
                             double* dst, hipStream_t stream);
 
-// Adjoint (FP64): given G = dL/dX per centre (X the exported features), write
-// the pair and centre forces of dL/dr (pv.pair_force, pv.centre_force;
-// launch_force_gather sums them per atom) and per-centre virials
-// centre_virial[n_centres][6] (sum over the centre's pairs of r_ji (x)
-// dL/dr_j, Voigt xx,yy,zz,yz,xz,xy, not divided by the volume).  xg, when
-// not null, holds X_i . G_i per centre (times xg_scale); otherwise it is
-// reduced from p and G.
-template <class T>
-void launch_backward(const RadialDev& rad, int S, const PairView& pv, const T* c, const T* p,
-                     const double* norm2, bool normalize, const double* xg, double xg_scale,
-                     const T* G, double* centre_virial, hipStream_t stream,
-                     const SoapTiles& tiles = SoapTiles());
+// Pair phase of the FP64 adjoint: from dL/dc [n][S][(L+1)^2][N] of each
+// centre, the pair and centre forces of dL/dr (pv.pair_force,
+// pv.centre_force; launch_force_gather sums them per atom) and the per-centre
+// virials centre_virial[n_centres][6] (sum over the centre's pairs of r_ji (x)
+// dL/dr_j, Voigt xx,yy,zz,yz,xz,xy, not divided by the volume).
+void launch_adjoint_pairs(const RadialDev& rad, int S, const PairView& pv, const double* dc,
+                          double* centre_virial, hipStream_t stream, const SoapTiles& tiles = SoapTiles());
+// dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values
+void launch_row_dot(int64_t n, int64_t D, const double* a, const double* b, const double* norm2, double* dot,
+                    hipStream_t stream);
+// dst row r (ldd values, zero past D) = src row rows[r] (D values)
+template <class To>
+void launch_gather_rows(int64_t n, int64_t D, int64_t ldd, const double* src, const int64_t* rows, To* dst,
+                        hipStream_t stream);
 
-// launch_backward<double> for a rank-one dL/dX: G_i = Gscale[i] * Grow
+// FP64 adjoint (full layout) for a rank-one dL/dX: G_i = Gscale[i] * Grow
 // (Grow [D], one sparse point's features; centres with a zero scale are
 // skipped and get a zero virial).  Used for the K_NM gradient rows.
 void launch_backward_rank1(const RadialDev& rad, int S, const PairView& pv, const double* c,

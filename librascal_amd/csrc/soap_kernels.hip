@@ -957,7 +957,7 @@ __global__ __launch_bounds__(kThreads, 4) void expansion_ps_kernel(
 }
 
 template <class T>
-__global__ void normalise_kernel(int64_t n, int64_t D, const T* __restrict__ p,
+__global__ void normalise_kernel(int64_t n, int64_t D, int64_t ld, const T* __restrict__ p,
                                  const double* __restrict__ norm2, int normalize,
                                  const int64_t* __restrict__ rows, double* __restrict__ out) {
   const int64_t total = n * D;
@@ -965,7 +965,7 @@ __global__ void normalise_kernel(int64_t n, int64_t D, const T* __restrict__ p,
        e += int64_t(gridDim.x) * blockDim.x) {
     const int64_t r = e / D;
     const int64_t i = rows ? rows[r] : r;
-    double v = double(p[i * D + (e - r * D)]);
+    double v = double(p[i * ld + (e - r * D)]);
     if (normalize) {
       const double nr = sqrt(norm2[i]);
       if (nr > 0) v /= nr;
@@ -1287,6 +1287,50 @@ __global__ __launch_bounds__(kThreads) void adjoint_kernel(
 
   // per-pair contraction; the batch reuses the region after dL/dc
   adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, dc, region, i, centre_virial);
+}
+
+// Pair phase alone, dL/dc [S][LL][N] of each centre from memory (dcg).
+template <class T, bool DIRECT>
+__global__ __launch_bounds__(kThreads) void adjoint_pairs_kernel(RadialDev rad, int S, int PB, PairView pv,
+                                                                 const T* __restrict__ dcg,
+                                                                 double* __restrict__ centre_virial) {
+  const int64_t i = blockIdx.x;
+  const int E = S * rad.N * rad.LL;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  T* yc = reinterpret_cast<T*>(smem_raw);
+  T* dc = reinterpret_cast<T*>(smem_raw + ylm_table_bytes<T>(rad.L1));
+  unsigned char* region = reinterpret_cast<unsigned char*>(dc) + align_up(sizeof(T) * E, 64);
+  load_ylm_table<T>(rad, yc);
+  for (int e = threadIdx.x; e < E; e += kThreads) dc[e] = dcg[i * int64_t(E) + e];
+  adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, dc, region, i, centre_virial);
+}
+
+// dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values
+__global__ __launch_bounds__(kThreads) void row_dot_kernel(int64_t D, const double* __restrict__ a,
+                                                           const double* __restrict__ b,
+                                                           const double* __restrict__ norm2,
+                                                           double* __restrict__ dot) {
+  const int64_t i = blockIdx.x;
+  __shared__ double red[kWaves];
+  double d = 0;
+  for (int64_t o = threadIdx.x; o < D; o += kThreads) d += a[i * D + o] * b[i * D + o];
+  for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0;
+    for (int w = 0; w < kWaves; ++w) t += red[w];
+    dot[i] = norm2[i] > 0 ? t / sqrt(norm2[i]) : 0.0;
+  }
+}
+
+// dst row r (ldd >= D values, zero pad) = src row rows[r] (D values)
+template <class To>
+__global__ __launch_bounds__(kThreads) void gather_rows_kernel(int64_t D, int64_t ldd, const double* __restrict__ src,
+                                                               const int64_t* __restrict__ rows,
+                                                               To* __restrict__ dst) {
+  const int64_t r = blockIdx.x, s = rows[r];
+  for (int64_t o = threadIdx.x; o < ldd; o += kThreads) dst[r * ldd + o] = o < D ? To(src[s * D + o]) : To(0);
 }
 
 // Adjoint of the mixed path: dL/dX (G) and p in the packed layout (p as its
@@ -3081,7 +3125,7 @@ __global__ __launch_bounds__(kThreads) void feature_gradient_rows_kernel(
 // for the selection matrix S (the selected coefficients, summed over
 // repeated selections, zero elsewhere): with it and |xs_i| the adjoint's
 // normalisation term is the one of the selected features.
-__global__ __launch_bounds__(kThreads) void sparsify_kernel(int64_t D, int64_t Dsel,
+__global__ __launch_bounds__(kThreads) void sparsify_kernel(int64_t D, int64_t Dsel, int64_t lds,
                                                             const int64_t* __restrict__ col,
                                                             const int64_t* __restrict__ inv_off,
                                                             const int64_t* __restrict__ inv_k,
@@ -3090,7 +3134,8 @@ __global__ __launch_bounds__(kThreads) void sparsify_kernel(int64_t D, int64_t D
                                                             double* __restrict__ norm2) {
   const int64_t i = blockIdx.x;
   double* pi = p + i * D;
-  double* xi = xs + i * Dsel;
+  double* xi = xs + i * lds;
+  for (int64_t k = Dsel + threadIdx.x; k < lds; k += kThreads) xi[k] = 0.0;
   double ss = 0;
   for (int64_t k = threadIdx.x; k < Dsel; k += kThreads) {
     const double v = col[k] >= 0 ? pi[col[k]] : 0.0;
@@ -3114,17 +3159,17 @@ __global__ __launch_bounds__(kThreads) void sparsify_kernel(int64_t D, int64_t D
   }
 }
 
-// dst[i] = S^T src[i] (rows of Dsel selected columns into rows of D
+// dst[i] = S^T src[i] (rows of selected columns, lds apart, into rows of D
 // columns, repeated selections summed in ascending selection order through
 // the inverse map inv_off/inv_k), one workgroup per row
-__global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t Dsel,
+__global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t lds,
                                                                    const int64_t* __restrict__ inv_off,
                                                                    const int64_t* __restrict__ inv_k,
                                                                    const double* __restrict__ src,
                                                                    int64_t D, double* __restrict__ dst) {
   const int64_t i = blockIdx.x;
   double* di = dst + i * D;
-  const double* si = src + i * Dsel;
+  const double* si = src + i * lds;
   for (int64_t o = threadIdx.x; o < D; o += kThreads) {
     double t = 0.0;
     for (int64_t q = inv_off[o]; q < inv_off[o + 1]; ++q) t += si[inv_k[q]];
@@ -3598,12 +3643,12 @@ void launch_power_spectrum_split(const RadialDev& rad, int S, int64_t n, const f
 
 template <class T>
 void launch_normalise(int64_t n, int64_t D, const T* p, const double* norm2, bool normalize, double* out,
-                      hipStream_t stream, const int64_t* rows) {
+                      hipStream_t stream, const int64_t* rows, int64_t ld) {
   if (n == 0 || D == 0) return;
   int64_t total = n * D;
   unsigned blocks = unsigned(std::min<int64_t>((total + 255) / 256, 65536));
-  hipLaunchKernelGGL(normalise_kernel<T>, dim3(blocks), dim3(256), 0, stream, n, D, p, norm2,
-                     int(normalize), rows, out);
+  hipLaunchKernelGGL(normalise_kernel<T>, dim3(blocks), dim3(256), 0, stream, n, D, ld > 0 ? ld : D, p,
+                     norm2, int(normalize), rows, out);
   RGPU_LAUNCH_CHECK();
 }
 
@@ -3701,35 +3746,65 @@ void launch_feature_gradient_rows(int N, int L1, int S, const PairView& pv, int6
   RGPU_LAUNCH_CHECK();
 }
 
-void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, const SelectionMap& sel, double* p, double* xs,
+void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, int64_t lds, const SelectionMap& sel, double* p, double* xs,
                      double* norm2, hipStream_t stream) {
   if (n == 0) return;
-  hipLaunchKernelGGL(sparsify_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, Dsel, sel.col,
+  hipLaunchKernelGGL(sparsify_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, Dsel, lds, sel.col,
                      sel.inv_off, sel.inv_k, p, xs, norm2);
   RGPU_LAUNCH_CHECK();
 }
 
-void launch_scatter_columns(int64_t n, int64_t Dsel, const SelectionMap& sel, const double* src, int64_t D,
+void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t D,
                             double* dst, hipStream_t stream) {
   if (n == 0) return;
-  hipLaunchKernelGGL(scatter_columns_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, Dsel, sel.inv_off,
+  hipLaunchKernelGGL(scatter_columns_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, lds, sel.inv_off,
                      sel.inv_k, src, D, dst);
   RGPU_LAUNCH_CHECK();
 }
 
-template <class T>
-void launch_backward(const RadialDev& rad, int S, const PairView& pv, const T* c, const T* p,
-                     const double* norm2, bool normalize, const double* xg, double xg_scale,
-                     const T* G, double* centre_virial, hipStream_t stream,
-                     const SoapTiles& tiles) {
+void launch_adjoint_pairs(const RadialDev& rad, int S, const PairView& pv, const double* dc,
+                          double* centre_virial, hipStream_t stream, const SoapTiles& tiles) {
   if (pv.n_centres == 0) return;
-  if (rad.use_spline)
-    launch_adjoint_t<T, false>(rad, S, pv, c, p, nullptr, nullptr, norm2, normalize, xg, xg_scale, G,
-                               centre_virial, stream, tiles);
+  const int F = rad.N * rad.L1;
+  const bool direct = !rad.use_spline;
+  const size_t fixed = ylm_table_bytes<double>(rad.L1) + align_up(sizeof(double) * size_t(S) * rad.N * rad.LL, 64);
+  auto batch = [&](int pb) { return pair_batch_bytes(pb, rad.LL, F, sizeof(double), direct, true); };
+  int PB = 8;
+  if (tiles.pb_adj > 0)
+    PB = std::min(tiles.pb_adj, 64);
   else
-    launch_adjoint_t<T, true>(rad, S, pv, c, p, nullptr, nullptr, norm2, normalize, xg, xg_scale, G,
-                              centre_virial, stream, tiles);
+    while (PB > 1 && fixed + batch(PB) > kTileAdjBudget) --PB;
+  const size_t smem = fixed + batch(PB);
+  auto go = [&](auto kern) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB, pv, dc,
+                       centre_virial);
+  };
+  if (direct)
+    go(adjoint_pairs_kernel<double, true>);
+  else
+    go(adjoint_pairs_kernel<double, false>);
+  RGPU_LAUNCH_CHECK();
 }
+
+void launch_row_dot(int64_t n, int64_t D, const double* a, const double* b, const double* norm2, double* dot,
+                    hipStream_t stream) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(row_dot_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, a, b, norm2, dot);
+  RGPU_LAUNCH_CHECK();
+}
+
+template <class To>
+void launch_gather_rows(int64_t n, int64_t D, int64_t ldd, const double* src, const int64_t* rows, To* dst,
+                        hipStream_t stream) {
+  if (n == 0 || ldd == 0) return;
+  hipLaunchKernelGGL(gather_rows_kernel<To>, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, ldd, src, rows, dst);
+  RGPU_LAUNCH_CHECK();
+}
+template void launch_gather_rows<double>(int64_t, int64_t, int64_t, const double*, const int64_t*, double*,
+                                         hipStream_t);
+template void launch_gather_rows<float>(int64_t, int64_t, int64_t, const double*, const int64_t*, float*,
+                                        hipStream_t);
 
 void launch_backward_rank1(const RadialDev& rad, int S, const PairView& pv, const double* c,
                            const double* p, const double* norm2, bool normalize, const double* Grow,
@@ -3885,9 +3960,9 @@ template void launch_power_spectrum<double>(const RadialDev&, int, int64_t, cons
 template void launch_power_spectrum<float>(const RadialDev&, int, int64_t, const float*, float*,
                                            double*, hipStream_t, const SoapTiles&);
 template void launch_normalise<double>(int64_t, int64_t, const double*, const double*, bool, double*,
-                                       hipStream_t, const int64_t*);
+                                       hipStream_t, const int64_t*, int64_t);
 template void launch_normalise<float>(int64_t, int64_t, const float*, const double*, bool, double*,
-                                      hipStream_t, const int64_t*);
+                                      hipStream_t, const int64_t*, int64_t);
 namespace {
 
 // ---------------------------------------------------------------------------
@@ -4011,9 +4086,5 @@ void launch_force_gather(const PairView& pv, const ReverseLists& rl, double* gra
                      rl.rlist, pv.pair_force, pv.centre_force, grad);
   RGPU_LAUNCH_CHECK();
 }
-
-template void launch_backward<double>(const RadialDev&, int, const PairView&, const double*,
-                                      const double*, const double*, bool, const double*, double,
-                                      const double*, double*, hipStream_t, const SoapTiles&);
 
 }  // namespace rgpu

@@ -1,0 +1,480 @@
+// Power spectrum in symmetric packed rows and its adjoint (sym_kernels.hh).
+//
+// Both products walk one angular channel per wavefront with lane = row r of
+// C_l: the power spectrum keeps C_l[r][:] in registers and the adjoint one
+// dL/dC_l[r][:], and the row C_l[c][:] of every step is the same for the
+// whole wavefront, so it is read through scalar loads and enters the FMAs as
+// a scalar operand.  No vector or LDS load feeds the FMAs except one packed
+// entry per step in the adjoint; the LDS traffic of a tiled product (two
+// operands per FMA block) bounded the kernels this replaced.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <string>
+
+#include "common.hh"
+#include "radial.hh"
+#include "packing.hh"
+#include "sym_kernels.hh"
+
+namespace rgpu {
+
+namespace {
+
+constexpr int kThreads = 256, kWaves = kThreads / 64;
+
+// constant address space: wavefront-uniform addresses become scalar loads
+typedef const __attribute__((address_space(4))) double* uniform_ptr;
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__host__ __device__ constexpr int tri_i(int r) { return r * (r + 1) / 2; }
+
+// k-th of the units 0 .. n-1 (in descending order of work) of a wavefront, -1
+// past the last: they are dealt to the nw wavefronts back and forth, which
+// evens out the work (l_max 9, one channel a unit, 4 wavefronts: 27, 25, 24,
+// 24 columns)
+__device__ __forceinline__ int wave_unit(int n, int nw, int wave, int k) {
+  const int u = nw * k + ((k & 1) ? nw - 1 - wave : wave);
+  return u < n ? u : -1;
+}
+
+// f(std::integral_constant<int, l>) for the runtime l <= LM
+template <int LM, class F>
+__device__ __forceinline__ void with_channel(int l, F&& f) {
+  if constexpr (LM >= 0) {
+    if (l == LM)
+      f(std::integral_constant<int, LM>{});
+    else
+      with_channel<LM - 1>(l, f);
+  }
+}
+
+// One workgroup of eight wavefronts per centre; a unit is half the columns of
+// a channel.  C sits in LDS for the lanes' own rows (odd row stride: no bank
+// conflicts); the loop over columns c does (2l+1) FMAs per entry, of which the
+// lanes r <= c store theirs (a run of c + 1 values).  Bound by the latency of
+// the scalar loads: eight wavefronts per copy of C put twice as many on a CU
+// as four (4096 centres, 4 species, n_max 12, l_max 9: 275 us with four).
+constexpr int kPowerWaves = 8;
+template <int LM>
+__global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int L, int64_t ld,
+                                                                     const double* __restrict__ c,
+                                                                     double* __restrict__ p,
+                                                                     double* __restrict__ norm2) {
+  const int64_t i = blockIdx.x;
+  const int LL = (L + 1) * (L + 1), LS = LL | 1, TRI = tri_i(R);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* cs = reinterpret_cast<double*>(smem_raw);
+  __shared__ double red[kPowerWaves];
+  const double* ci = c + i * int64_t(R) * LL;
+  for (int r = wave; r < R; r += kPowerWaves)
+    for (int k = lane; k < LL; k += 64) cs[r * LS + k] = ci[r * LL + k];
+  __syncthreads();
+  double ss = 0.0;
+  for (int k = 0; k * kPowerWaves < 2 * (L + 1); ++k) {
+    const int u = wave_unit(2 * (L + 1), kPowerWaves, wave, k);
+    if (u < 0) continue;
+    with_channel<LM>(L - (u >> 1), [&](auto lc) {
+      constexpr int l = decltype(lc)::value, M = 2 * l + 1;
+      const double f = 1.0 / sqrt(double(M)), f2 = f * 1.41421356237309504880;
+      double* out = p + i * ld + int64_t(l) * TRI;
+      const int half = (R + 1) / 2, c0 = (u & 1) ? half : 0, c1 = (u & 1) ? R : half;
+      for (int rb = 0; rb < c1; rb += 64) {
+        const int r = rb + lane, ro = min(r, R - 1), cb = max(rb, c0);
+        double x[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) x[m] = cs[ro * LS + l * l + m];
+        uniform_ptr y = (uniform_ptr)(ci + int64_t(cb) * LL + l * l);
+        for (int col = cb; col < c1; ++col, y += LL) {
+          double s = 0.0;
+#pragma unroll
+          for (int m = 0; m < M; ++m) s += x[m] * y[m];
+          if (r <= col) {
+            const double v = s * (r < col ? f2 : f);
+            out[tri_i(col) + r] = v;
+            ss += v * v;
+          }
+        }
+      }
+    });
+  }
+  for (int64_t o = int64_t(L + 1) * TRI + threadIdx.x; o < ld; o += 64 * kPowerWaves) p[i * ld + o] = 0.0;
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < kPowerWaves; ++w) t += red[w];
+    norm2[i] = t;
+  }
+}
+
+// dL/dC_l[r][m] = f_l sqrt 2 sum_c w(r, c) C_l[c][m], w the packed entry
+// dL/dp(r, c) (times sqrt 2 on the diagonal).  The channel's triangle of
+// dL/dp is formed in LDS, one buffer per wavefront, straight in its packed
+// order; a lane's walk along its row, tri(r) + c up to the diagonal and
+// tri(c) + r after it, is free of bank conflicts there (triangular numbers
+// run through every residue of a power of two).
+//
+// Forms of G (kForm): kDp symmetric packed rows of dL/dp, kDx full rows
+// (keys a <= b, [n1][n2][l]) of dL/dX, whose projection dL/dp = G / |p| -
+// xg p / |p|^2 is made on the way (p null: no normalisation, dL/dp = G); xg
+// null: X . G is first summed here.  A full row's entries of one channel lie
+// L+1 apart, but the workgroup's wavefronts take them channel after channel
+// from the same cached lines, which costs less than packing the rows first
+// (4689 centres, 4 species, n_max 8, l_max 6: 244 us against 183 + 139).  kGather: as
+// kDp, the entries gathered from memory (R too large for the LDS).
+//
+// Bound by the memory it streams and the latency of the scalar loads: 4096
+// centres, 4 species, n_max 12, l_max 9: 0.31 ms for 0.93 GB, where the key
+// contraction of the fused FP64 adjoint it replaced took about 1.0 ms.
+enum { kDp, kDx, kGather };
+
+template <int LM, int kForm>
+__global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, int L, int64_t ld,
+                                                                const double* __restrict__ c,
+                                                                const double* __restrict__ p,
+                                                                const double* __restrict__ norm2,
+                                                                const double* __restrict__ xg,
+                                                                const double* __restrict__ G,
+                                                                double* __restrict__ dc) {
+  const int64_t i = blockIdx.x;
+  const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), S = R / N, KB = N * N * L1;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const double rt2 = 1.41421356237309504880;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* W = reinterpret_cast<double*>(smem_raw) + wave * TRI;
+  // kDx: offsets in a full row of the entry t = (r, c) at channel 0 and of
+  // its mirror (both the same between species)
+  int2* tab = reinterpret_cast<int2*>(reinterpret_cast<double*>(smem_raw) + kWaves * TRI);
+  __shared__ double red[kWaves];
+  const double* Gi = G + i * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
+  const double* pi = p ? p + i * ld : nullptr;
+  // packed entry t of channel l of G
+  auto entry = [&](int l, int t) -> double {
+    if constexpr (kForm != kDx) {
+      return Gi[l * TRI + t];
+    } else {
+      const int2 o = tab[t];
+      const double v = Gi[o.x + l];
+      return o.x == o.y ? v : (v + Gi[o.y + l]) * 0.70710678118654752440;
+    }
+  };
+  double alpha = 1.0, beta = 0.0;
+  if constexpr (kForm == kDx) {
+    for (int col = wave; col < R; col += kWaves)
+      for (int r = lane; r <= col; r += 64) {
+        const int a = r / N, b = col / N, n1 = r - a * N, n2 = col - b * N;
+        const int k0 = (a * S - a * (a - 1) / 2 + (b - a)) * KB;
+        const int o = k0 + (n1 * N + n2) * L1;
+        tab[tri_i(col) + r] = make_int2(o, a == b ? k0 + (n2 * N + n1) * L1 : o);
+      }
+    __syncthreads();
+    if (p) {
+      const double n2 = norm2[i];
+      double x = 0.0;
+      if (xg) {
+        x = xg[i];
+      } else {
+        double d = 0.0;
+        for (int k = 0; k * kWaves <= L; ++k) {
+          const int u = wave_unit(L1, kWaves, wave, k);
+          if (u < 0) continue;
+          const double* q = pi + (L - u) * TRI;
+#pragma unroll 8
+          for (int t = lane; t < TRI; t += 64) d += q[t] * entry(L - u, t);
+        }
+        for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
+        if (lane == 0) red[wave] = d;
+        __syncthreads();
+        if (n2 > 0) x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
+      }
+      if (n2 > 0) {
+        alpha = 1.0 / sqrt(n2);
+        beta = x / n2;
+      }
+    }
+  }
+  const double* ci = c + i * int64_t(R) * LL;
+  for (int k = 0; k * kWaves <= L; ++k) {
+    const int u = wave_unit(L1, kWaves, wave, k), lk = L - u;
+    if (u < 0) continue;
+    const double* g = Gi + lk * TRI;
+    if constexpr (kForm != kGather) {
+      wave_sync();  // the previous channel is read
+      // (many loads in flight: the runs come from memory)
+      if (kForm == kDx && p) {
+        const double* q = pi + lk * TRI;
+#pragma unroll 8
+        for (int t = lane; t < TRI; t += 64) W[t] = alpha * entry(lk, t) - beta * q[t];
+      } else {
+#pragma unroll 16
+        for (int t = lane; t < TRI; t += 64) W[t] = entry(lk, t);
+      }
+      wave_sync();
+      for (int r = lane; r < R; r += 64) W[tri_i(r) + r] *= rt2;
+      wave_sync();
+    }
+    with_channel<LM>(lk, [&](auto lc) {
+      constexpr int l = decltype(lc)::value, M = 2 * l + 1;
+      const double f = rt2 / sqrt(double(M));
+      for (int rb = 0; rb < R; rb += 64) {
+        const int r = min(rb + lane, R - 1);
+        double acc[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[m] = 0.0;
+        uniform_ptr y = (uniform_ptr)(ci + l * l);
+        int a = tri_i(r);
+        for (int col = 0; col < R; ++col, y += LL) {
+          const double w = kForm == kGather ? g[a] * (col == r ? rt2 : 1.0) : W[a];
+          a += col < r ? 1 : col + 1;
+#pragma unroll
+          for (int m = 0; m < M; ++m) acc[m] += w * y[m];
+        }
+        if (rb + lane < R) {
+          const int s = r / N, n = r - s * N;
+          double* o = dc + (i * S + s) * int64_t(LL) * N + n;
+#pragma unroll
+          for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
+        }
+      }
+    });
+  }
+}
+
+// Full row <-> symmetric packed row, one workgroup per row, KC key blocks at
+// a time through LDS ([key][n1][n2][l] with an odd n1 stride): both sides move
+// along their rows (whole key blocks, runs of N packed entries), and several
+// keys per pass keep enough loads in flight.  Memory bound.
+__device__ __forceinline__ void key_table(int S, int* key_ab) {
+  for (int k = threadIdx.x; k < S * (S + 1) / 2; k += kThreads) {
+    int a, b;
+    key_pair(k, S, &a, &b);
+    key_ab[k] = (a << 8) | b;
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1, int KC, int64_t ld,
+                                                            const double* __restrict__ full,
+                                                            const int64_t* __restrict__ rows,
+                                                            double* __restrict__ out) {
+  const int64_t i = blockIdx.x;
+  const int K = S * (S + 1) / 2, NL = N * L1, KB = N * NL, NS = NL | 1, TRI = tri_i(S * N), NN = N * N;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* b = reinterpret_cast<double*>(smem_raw);
+  int* key_ab = reinterpret_cast<int*>(b + size_t(KC) * N * NS);
+  const double* src = full + (rows ? rows[i] : i) * (int64_t(K) * KB);
+  double* dst = out + i * ld;
+  key_table(S, key_ab);
+  for (int k0 = 0; k0 < K; k0 += KC) {
+    const int kc = min(KC, K - k0);
+    __syncthreads();
+#pragma unroll 4
+    for (int r = wave; r < kc * N; r += kWaves)
+      for (int o = lane; o < NL; o += 64) b[r * NS + o] = src[(int64_t(k0) * N + r) * NL + o];
+    __syncthreads();
+    for (int t = threadIdx.x; t < kc * NN; t += kThreads) {
+      const int kk = t / NN, tt = t - kk * NN, n2 = tt / N, n1 = tt - n2 * N;
+      const int sa = key_ab[k0 + kk] >> 8, sb = key_ab[k0 + kk] & 255;
+      if (sa == sb && n1 > n2) continue;
+      const bool sym = sa == sb && n1 < n2;
+      const double *bk = b + kk * N * NS, *b0 = bk + n1 * NS + n2 * L1, *b1 = bk + n2 * NS + n1 * L1;
+      int64_t o = tri_i(sb * N + n2) + sa * N + n1;
+#pragma unroll 4
+      for (int l = 0; l < L1; ++l, o += TRI)
+        dst[o] = sym ? (b0[l] + b1[l]) * 0.70710678118654752440 : b0[l];
+    }
+  }
+  for (int64_t o = int64_t(L1) * TRI + threadIdx.x; o < ld; o += kThreads) dst[o] = 0.0;
+}
+
+// dL/dp of a packed row of dL/dX in place (X = p / |p|): G / |p| - xg p /
+// |p|^2, xg null: X . G summed here.  One workgroup per row.
+__global__ __launch_bounds__(kThreads) void sym_project_kernel(int64_t ld, const double* __restrict__ p,
+                                                               const double* __restrict__ norm2,
+                                                               const double* __restrict__ xg,
+                                                               double* __restrict__ G) {
+  const int64_t i = blockIdx.x;
+  __shared__ double red[kWaves];
+  const double* q = p + i * ld;
+  double* g = G + i * ld;
+  const double n2 = norm2[i];
+  if (!(n2 > 0)) return;
+  double x;
+  if (xg) {
+    x = xg[i];
+  } else {
+    double d = 0.0;
+    for (int64_t o = threadIdx.x; o < ld; o += kThreads) d += q[o] * g[o];
+    for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d;
+    __syncthreads();
+    x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
+  }
+  const double alpha = 1.0 / sqrt(n2), beta = x / n2;
+  for (int64_t o = threadIdx.x; o < ld; o += kThreads) g[o] = alpha * g[o] - beta * q[o];
+}
+
+__global__ __launch_bounds__(kThreads) void sym_unpack_kernel(int S, int N, int L1, int KC, int64_t ld,
+                                                              const double* __restrict__ p,
+                                                              const int64_t* __restrict__ rows,
+                                                              const double* __restrict__ norm2, int normalize,
+                                                              double* __restrict__ out) {
+  const int64_t i = rows ? rows[blockIdx.x] : int64_t(blockIdx.x);
+  const int K = S * (S + 1) / 2, NL = N * L1, KB = N * NL, NS = NL | 1, TRI = tri_i(S * N), NN = N * N;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* b = reinterpret_cast<double*>(smem_raw);
+  int* key_ab = reinterpret_cast<int*>(b + size_t(KC) * N * NS);
+  const double* src = p + i * ld;
+  double* dst = out + int64_t(blockIdx.x) * (int64_t(K) * KB);
+  key_table(S, key_ab);
+  double nr = 1.0;
+  if (normalize && norm2[i] > 0) nr = sqrt(norm2[i]);
+  for (int k0 = 0; k0 < K; k0 += KC) {
+    const int kc = min(KC, K - k0);
+    __syncthreads();
+    for (int t = threadIdx.x; t < kc * NN; t += kThreads) {
+      const int kk = t / NN, tt = t - kk * NN, n2 = tt / N, n1 = tt - n2 * N;
+      const int sa = key_ab[k0 + kk] >> 8, sb = key_ab[k0 + kk] & 255;
+      if (sa == sb && n1 > n2) continue;
+      const bool sym = sa == sb && n1 < n2;
+      double *bk = b + kk * N * NS, *b0 = bk + n1 * NS + n2 * L1, *b1 = bk + n2 * NS + n1 * L1;
+      const double* q = src + tri_i(sb * N + n2) + sa * N + n1;
+#pragma unroll 4
+      for (int l = 0; l < L1; ++l, q += TRI) {
+        double v = *q;
+        if (sym) {
+          v *= 0.70710678118654752440;
+          b1[l] = v;
+        }
+        b0[l] = v;
+      }
+    }
+    __syncthreads();
+    for (int r = wave; r < kc * N; r += kWaves)
+      for (int o = lane; o < NL; o += 64) dst[(int64_t(k0) * N + r) * NL + o] = b[r * NS + o] / nr;
+  }
+}
+
+template <class K>
+void allow_lds(K kernel, size_t smem) {
+  if (smem > 160 * 1024)
+    throw InvalidArgument("hypers need " + std::to_string(smem) +
+                          " bytes of LDS per workgroup, more than the device provides");
+  if (smem > 64 * 1024)
+    RGPU_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(smem)));
+}
+
+// key blocks per pass of the row conversions (four workgroups per CU, one
+// block at least) and their LDS
+int key_blocks(int S, int N, int L1) {
+  const size_t kb = sizeof(double) * size_t(N) * ((N * L1) | 1);
+  return std::max(1, std::min(S * (S + 1) / 2, int(36 * 1024 / kb)));
+}
+size_t key_lds(int S, int N, int L1) {
+  return sizeof(double) * size_t(key_blocks(S, N, L1)) * N * ((N * L1) | 1) + sizeof(int) * size_t(S * (S + 1) / 2);
+}
+
+}  // namespace
+
+void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* p, double* norm2,
+                      hipStream_t stream) {
+  if (n == 0) return;
+  const int R = S * N;
+  const size_t smem = sizeof(double) * size_t(R) * ((L1 * L1) | 1);
+  auto go = [&](auto kern) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(64 * kPowerWaves), smem, stream, R, L1 - 1,
+                       sym_row_stride(S, N, L1), c, p, norm2);
+    RGPU_LAUNCH_CHECK();
+  };
+  // the register budget follows the largest channel the kernel is built for
+  if (L1 <= 10)
+    go(sym_power_kernel<9>);
+  else
+    go(sym_power_kernel<kMaxL1 - 1>);
+}
+
+namespace {
+
+size_t contract_lds(int R, bool full) {
+  return size_t(sym_tri(R)) * (sizeof(double) * kWaves + (full ? sizeof(int2) : 0));
+}
+constexpr size_t kContractLds = 156 * 1024;
+
+template <int kForm>
+void go_contract(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
+                 const double* xg, const double* G, double* dc, hipStream_t stream) {
+  const int R = S * N;
+  const size_t smem = kForm == kGather ? 0 : contract_lds(R, kForm == kDx);
+  auto go = [&](auto kern) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, R, N, L1 - 1, sym_row_stride(S, N, L1),
+                       c, p, norm2, xg, G, dc);
+    RGPU_LAUNCH_CHECK();
+  };
+  if (L1 <= 10)
+    go(sym_contract_kernel<9, kForm>);
+  else
+    go(sym_contract_kernel<kMaxL1 - 1, kForm>);
+}
+
+}  // namespace
+
+void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const double* G, double* dc,
+                         hipStream_t stream) {
+  if (n == 0) return;
+  if (contract_lds(S * N, false) <= kContractLds)
+    go_contract<kDp>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
+  else
+    go_contract<kGather>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
+}
+
+void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
+                              const double* xg, const double* G, DeviceBuffer<double>& work, double* dc,
+                              hipStream_t stream) {
+  if (n == 0) return;
+  if (contract_lds(S * N, true) <= kContractLds) {
+    go_contract<kDx>(S, N, L1, n, c, p, norm2, xg, G, dc, stream);
+    return;
+  }
+  const int64_t ld = sym_row_stride(S, N, L1);
+  double* g = work.reserve(size_t(n * ld));
+  launch_sym_pack(S, N, L1, n, G, nullptr, g, stream);
+  if (p) {
+    hipLaunchKernelGGL(sym_project_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, ld, p, norm2, xg, g);
+    RGPU_LAUNCH_CHECK();
+  }
+  launch_sym_contract(S, N, L1, n, c, g, dc, stream);
+}
+
+void launch_sym_pack(int S, int N, int L1, int64_t n, const double* full, const int64_t* rows, double* out,
+                     hipStream_t stream) {
+  if (n == 0) return;
+  const size_t smem = key_lds(S, N, L1);
+  allow_lds(sym_pack_kernel, smem);
+  hipLaunchKernelGGL(sym_pack_kernel, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1,
+                     key_blocks(S, N, L1), sym_row_stride(S, N, L1), full, rows, out);
+  RGPU_LAUNCH_CHECK();
+}
+
+void launch_sym_unpack(int S, int N, int L1, int64_t n, const double* p, const int64_t* rows, const double* norm2,
+                       bool normalize, double* out, hipStream_t stream) {
+  if (n == 0) return;
+  const size_t smem = key_lds(S, N, L1);
+  allow_lds(sym_unpack_kernel, smem);
+  hipLaunchKernelGGL(sym_unpack_kernel, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1,
+                     key_blocks(S, N, L1), sym_row_stride(S, N, L1), p, rows, norm2, int(normalize), out);
+  RGPU_LAUNCH_CHECK();
+}
+
+}  // namespace rgpu

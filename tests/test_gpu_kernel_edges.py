@@ -9,7 +9,8 @@ import json
 import numpy as np
 import pytest
 
-from conftest import soap_hypers
+import oracle as O
+from conftest import oracle_backward, ps_rel, soap_hypers
 from librascal_amd import _capi
 from librascal_amd.models import KRR, Kernel, SparsePoints
 from librascal_amd.representations import SphericalInvariants
@@ -84,3 +85,65 @@ def test_model_kept_across_batches():
     # a batch of another list set in between without a prediction
     rep.transform(other)
     m1.predict(rep.transform(a))
+
+
+@pytest.mark.parametrize("n_species,N,L,normalize", [
+    (1, 1, 0, True), (3, 5, 4, True), (3, 5, 4, False), (2, 3, 11, True),
+    (8, 8, 2, True), (9, 8, 2, True),    # 64 and 72 rows: one and two row blocks
+    (12, 8, 1, True), (13, 8, 1, True),  # 96 and 104 rows: triangles in LDS or gathered
+])
+def test_fp64_rows_and_channels(n_species, N, L, normalize):
+    """FP64 features, adjoint and prediction at the edges of the symmetric
+    rows: lanes per row block, channel buffers, l_max past 9, one function."""
+    el = list(range(1, n_species + 1))
+    sts = periodic_box(3 * n_species + 5, 0.06, el, d_min=1.0, seed=70 + n_species)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=normalize)
+    ctx, num = _context(hp, sts)
+    calc, batch = O.Calculator(hp), O.BatchData(sts)
+    X, _ = ctx.features()
+    Xo, _ = calc.power_spectrum(batch)
+    assert ps_rel(Xo, X, n_species, N, L) <= 1e-10
+    rng = np.random.default_rng(71)
+    G = rng.normal(size=X.shape)
+    g, s = ctx.features_backward(G)
+    g_ref, s_ref = oracle_backward(calc, batch, G)
+    # (a single normalised function is 1 everywhere: the reference is exactly
+    # zero there, and rounding of the O(1) terms that cancel is not)
+    floor = 1e-14 * np.abs(G).max()
+    assert np.abs(g - g_ref).max() <= 1e-10 * np.abs(g_ref).max() + floor
+    assert np.abs(s - s_ref).max() <= 1e-10 * np.abs(s_ref).max() + floor
+    spec, vals, w = _points(ctx, num, {z: 1 + 20 * (z % 2) for z in el}, rng)
+    ctx.set_sparse_points(2, spec, vals, w)
+    e, g, s = ctx.gap_predict()
+    e_ref, g_ref, s_ref = O.gap_predict(calc, batch, O.SparseSet(spec, vals, 2), w)
+    floor = 1e-14 * np.abs(w).sum()
+    for a, b in ((e, e_ref), (g, g_ref), (s, s_ref)):
+        assert np.abs(a - b).max() <= 1e-10 * np.abs(b).max() + floor
+    k = ctx.gap_knm("Atom")
+    assert np.abs(k - O.gap_knm(calc, batch, O.SparseSet(spec, vals, 2), "Atom")[:, np.argsort(np.argsort(
+        spec, kind="stable"))]).max() <= 1e-10 * np.abs(k).max()
+
+
+@pytest.mark.parametrize("atoms,points", [(3, 1), (40, 65), (700, 33), (1100, 330)])
+def test_fp64_product_tiles(atoms, points):
+    """The FP64 products in 16-, 32- and 64-row tiles, with remainders in
+    every dimension: energies and forces against the oracle's K_NM and against
+    the sum over halves of the model."""
+    sts = periodic_box(atoms, 0.05, (1, 8), d_min=1.0, seed=81)
+    ctx, num = _context(soap_hypers(rc=4.0, sw=0.5, sigma=0.5, N=9, L=6, spline=1e-8), sts)
+    rng = np.random.default_rng(82)
+    spec, vals, w = _points(ctx, num, {1: points, 8: points + 2}, rng)
+    ctx.set_sparse_points(3, spec, vals, w)
+    e, g, s = ctx.gap_predict()
+    k = ctx.gap_knm("Structure")
+    assert abs(k[0] @ w - e[0]) <= 1e-10 * (np.abs(k[0]) @ np.abs(w))
+    X, _ = ctx.features()
+    z = num[:, None] == spec[None, :]
+    ref = np.where(z, (X @ vals.T) ** 3, 0.0)
+    assert np.abs(ctx.gap_knm("Atom") - ref).max() <= 1e-10 * np.abs(ref).max()
+    parts = []
+    for sl in (slice(0, None, 2), slice(1, None, 2)):
+        ctx.set_sparse_points(3, spec[sl], vals[sl], w[sl])
+        parts.append(ctx.gap_predict())
+    for a, b, c in zip((e, g, s), *parts):
+        assert np.abs(a - b - c).max() <= 1e-10 * max(np.abs(b).max(), np.abs(c).max())
