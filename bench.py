@@ -269,7 +269,7 @@ EXPANSION_KERNEL = "expansion_kernel<float, 5, false, 12, 9>"
 PS_KERNEL = "power_spectrum_kernel<float, true, 12, 9>"
 ADJOINT_KERNELS = {0: ["adjoint_staged_kernel<false, 5>"], 1: ["adjoint_mfma_kernel<false, 12>"],
                    2: ["adjoint_tile_kernel<12, 9, 6, 1, 10, false, true>"],
-                   3: ["adjoint_tile_kernel<12, 9, 6, 1, 6, false, false>", "adjoint_pair_kernel<12, 9>"]}
+                   3: ["adjoint_tile_kernel<12, 9, 6, 1, 6, false, false>", "pair_force_kernel<float, 12, 64, 1>"]}
 # shader clock under this load (SQ_BUSY_CYCLES over the kernel durations)
 CLOCK_HZ = 2.0e9
 

@@ -27,7 +27,7 @@ COMMON = [
 ]
 # geometry of the neighbour list must round like separate multiply/add
 SOURCE_FLAGS = {"neighbours.hip": ["-ffp-contract=off"]}
-SOURCES = ["hypers.cc", "radial_host.cc", "neighbours.hip", "soap_kernels.hip", "sym_kernels.hip",
+SOURCES = ["hypers.cc", "radial_host.cc", "neighbours.hip", "soap_kernels.hip", "sym_kernels.hip", "pair_kernels.hip",
            "gap_kernels.hip", "gap_mfma.hip", "gap_f64.hip", "context.cc"]
 
 

@@ -20,6 +20,7 @@
 #include "hypers.hh"
 #include "neighbours.hh"
 #include "packing.hh"
+#include "pair_kernels.hh"
 #include "radial.hh"
 #include "scan.hh"
 #include "soap_kernels.hh"
@@ -924,7 +925,7 @@ void backward_device(Context& c, const float* G, double* grad, double* cvir, con
   const PairView pv = backward_view(c, &rl);
   float* work = nullptr;
   if (c.tile().adj_kind == 3)
-    work = c.adj_work.reserve(size_t(std::max<int64_t>(c.n_atoms * S * c.rd.N * c.rd.LL, 1)));
+    work = c.adj_work.reserve(size_t(c.n_atoms * S * c.rd.N * c.rd.LL + kPairSlack));
   launch_backward_split(c.rd, S, pv, c.c32.get(), c.p_hi.get(), c.p_lo.get(), c.norm2.get(), c.hp.normalize, xg,
                         xg_scale, G, cvir, c.stream, c.tile(), work);
   launch_force_gather(pv, rl, grad, c.stream);
@@ -936,13 +937,16 @@ void backward_device(Context& c, const double* G, bool full, const double* xg, d
   StageTimer t(c, RGPU_STAGE_BACKWARD);
   ReverseLists rl;
   const PairView pv = backward_view(c, &rl);
-  double* dc = c.dc64.reserve(size_t(std::max<int64_t>(c.n_atoms * S * N * c.rd.LL, 1)));
+  double* dc = c.dc64.reserve(size_t(c.n_atoms * S * N * c.rd.LL + kPairSlack));
   if (full)
     launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), c.hp.normalize ? c.p64.get() : nullptr, c.norm2.get(),
                              xg, G, c.gsym, dc, c.stream);
   else
     launch_sym_contract(S, N, L1, c.n_atoms, c.c64.get(), G, dc, c.stream);
-  launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
+  if (pair_kernels_apply(c.rd))
+    launch_pair_forces<double>(c.rd, S, pv, dc, cvir, c.stream);
+  else
+    launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
   launch_force_gather(pv, rl, grad, c.stream);
 }
 // selected columns of dL/dX (or dL/dp, rows ld apart) into the full layout
@@ -1398,7 +1402,7 @@ void autotune_t(Context& c) {
     double* cvir = cv.reserve(size_t(6 * n));
     ReverseLists rl;
     const PairView bpv = backward_view(c, &rl);
-    const size_t E = size_t(std::max<int64_t>(n * S * c.rd.N * c.rd.LL, 1));
+    const size_t E = size_t(n * S * c.rd.N * c.rd.LL + kPairSlack);
     float* work = split ? c.adj_work.reserve(E) : nullptr;
     double* dc = split ? nullptr : c.dc64.reserve(E);
     auto time_adjoint = [&](const SoapTiles& cand) {

@@ -31,6 +31,7 @@
 
 #include "soap_device.hh"
 #include "packing.hh"
+#include "pair_kernels.hh"
 #include "scan.hh"
 #include "soap_kernels.hh"
 
@@ -1971,7 +1972,7 @@ __device__ __forceinline__ void adj_tile_sweep(const float* __restrict__ g, cons
 
 // PRE: 16-byte packed values per thread of one staged chunk.  PAIRS: the
 // pair phase follows in the same workgroup (dL/dc in LDS); otherwise dL/dc
-// [S][LL][N] of centre i is written to dcg + i S LL N for adjoint_pair_kernel
+// [S][LL][N] of centre i is written to dcg + i S LL N for launch_pair_forces
 // and the workgroup needs no Y_lm table or pair batch (three per CU).
 template <int N, int L, int NR, int ROLES, int PRE, bool DIRECT, bool PAIRS>
 __global__ __launch_bounds__(kThreads, (PAIRS || ROLES > 1) ? 2 : 3) void adjoint_tile_kernel(
@@ -2330,32 +2331,13 @@ __device__ __forceinline__ void ylm_lane(int L, const float* __restrict__ yc, fl
   }
 }
 
-// ---------------------------------------------------------------------------
-// Pair phase of the mixed adjoint as a kernel of its own, after
-// adjoint_tile_kernel wrote dL/dc [S][LL][N] per centre: one workgroup per
-// centre, a group of 16 lanes per pair (16 pairs in flight).  With D[lm] =
-// sum_n dL/dc[s_j][lm][n] R_nl, the pair gradient of adjoint_pairs splits
-// over the radial channels: lane n of the group evaluates R_nl and R'_nl of
-// its channel for every l (spline) and accumulates
-//   A_n  = sum_l (R'_nl fc + R_nl fc') sum_m dc[lm][n] Y_lm,
-//   Sl_n = sum_l l R_nl sum_m dc[lm][n] Y_lm,
-//   B_n  = sum_l R_nl sum_m dc[lm][n] gY_lm   (gY: the gradient terms of Y),
-// with {Y, gY}[lm] of the pair staged once per group in LDS; the group sums
-// over n and its lane 0 forms the force in FP64 as adjoint_pairs does.  No
-// barrier between pairs (a group lives in one wavefront) and a small LDS
-// footprint keep several workgroups per CU in flight.
+// lanes per pair of expansion_group_kernel
 constexpr int kPairGroup = 16;
 
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__host__ __device__ inline size_t pair_kernel_lds(int S, int N, int L1) {
-  const int LL = L1 * L1;
-  return ylm_table_bytes<float>(L1) + align_up(sizeof(YGradTerm<float>) * 3 * LL, 64) +
-         align_up(sizeof(float) * S * LL * N, 64) + sizeof(float) * 4 * LL * (kThreads / kPairGroup);
 }
 
 // FP32 spline cell of a pair at distance d whose neighbour has species sj
@@ -2509,139 +2491,6 @@ __host__ __device__ inline size_t expansion_group_lds(int S, int N, int L1) {
   const int LL = L1 * L1, LLP = (LL + 3) & ~3;
   return ylm_table_bytes<float>(L1) + sizeof(float) * (size_t(kWaves) * (64 / kPairGroup) * LLP +
                                                        size_t(S) * N * LL);
-}
-
-template <int N, int L>
-__global__ __launch_bounds__(kThreads) void adjoint_pair_kernel(RadialDev rad, int S, PairView pv,
-                                                                const float* __restrict__ dcg,
-                                                                double* __restrict__ centre_virial) {
-  constexpr int L1 = L + 1, LL = L1 * L1, NG = kThreads / kPairGroup;
-  static_assert(N <= kPairGroup && L1 <= kPairGroup, "one lane per radial channel and per order m");
-  const int64_t i = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int gl = lane & (kPairGroup - 1), grp = tid / kPairGroup;
-  extern __shared__ __align__(64) unsigned char smem_raw[];
-  float* yc = reinterpret_cast<float*>(smem_raw);
-  YGradTerm<float>* gt = reinterpret_cast<YGradTerm<float>*>(smem_raw + ylm_table_bytes<float>(L1));
-  float* dc = reinterpret_cast<float*>(reinterpret_cast<unsigned char*>(gt) +
-                                       align_up(sizeof(YGradTerm<float>) * 3 * LL, 64));
-  f32x4* yg = reinterpret_cast<f32x4*>(reinterpret_cast<unsigned char*>(dc) +
-                                       align_up(sizeof(float) * S * LL * N, 64));
-  __shared__ double red[kWaves][9];
-  load_ylm_table<float>(rad, yc);
-  {
-    const YGradTerm<float>* src = ygrad_src<float>(rad);
-    for (int e = tid; e < 3 * LL; e += kThreads) gt[e] = src[e];
-    const int E4 = S * LL * N / 4;
-    const f32x4* d4 = reinterpret_cast<const f32x4*>(dcg + i * int64_t(S) * LL * N);
-    for (int e = tid; e < E4; e += kThreads) reinterpret_cast<f32x4*>(dc)[e] = d4[e];
-  }
-  __syncthreads();
-  const int64_t p0 = pv.centre_off[i] + 1;
-  const int np = int(pv.centre_off[i + 1] - p0);
-  f32x4* Yg = yg + grp * LL;
-  double fi[3] = {0, 0, 0}, v6[6] = {0, 0, 0, 0, 0, 0};
-  for (int q0 = 0; q0 < np; q0 += NG) {
-    const int q = q0 + grp;
-    if (q < np) {  // uniform within the group
-      const int64_t p = p0 + q;
-      const double d = pv.pair_dist[p];
-      const double vx = pv.pair_vec[3 * p], vy = pv.pair_vec[3 * p + 1], vz = pv.pair_vec[3 * p + 2];
-      const double fcd = pv.pair_fc[p], dfcd = pv.pair_dfc[p];
-      const int j = pv.pair_j[p];
-      const int sj = pv.species_of[j];
-      const SplineCell<float> cell = pair_cell(rad, d, sj);
-      float R[L1], dR[L1];
-      const int n = gl < N ? gl : N - 1;
-#pragma unroll
-      for (int l = 0; l <= L; ++l) spline_eval<float>(rad, cell, n * L1 + l, &R[l], &dR[l]);
-      const float dx = float(vx / d), dy = float(vy / d), dz = float(vz / d);
-      if (gl <= L) ylm_lane(L, yc, dx, dy, dz, gl, reinterpret_cast<float*>(Yg), 4);
-      wave_lds_sync();
-      for (int lm = gl; lm < LL; lm += kPairGroup) {
-        const YGradTerm<float>* g = gt + 3 * lm;
-        const float gx = g[0].c0 * Yg[g[0].i0].x + g[0].c1 * Yg[g[0].i1].x;
-        const float gy = g[1].c0 * Yg[g[1].i0].x + g[1].c1 * Yg[g[1].i1].x;
-        const float gz = g[2].c0 * Yg[g[2].i0].x + g[2].c1 * Yg[g[2].i1].x;
-        float* o = reinterpret_cast<float*>(Yg + lm);
-        o[1] = gx;
-        o[2] = gy;
-        o[3] = gz;
-      }
-      wave_lds_sync();
-      float A = 0.f, Sl = 0.f, Bx = 0.f, By = 0.f, Bz = 0.f;
-      if (gl < N) {
-        const float ffc = float(fcd), fdfc = float(dfcd);
-        const float* dcs = dc + sj * LL * N + gl;
-#pragma unroll
-        for (int l = 0; l <= L; ++l) {
-          float s1 = 0.f, sx = 0.f, sy = 0.f, sz = 0.f;
-#pragma unroll
-          for (int m = 0; m < 2 * l + 1; ++m) {
-            const int lm = l * l + m;
-            const float t = dcs[lm * N];
-            const f32x4 y4 = Yg[lm];
-            s1 += t * y4.x;
-            sx += t * y4.y;
-            sy += t * y4.z;
-            sz += t * y4.w;
-          }
-          A += s1 * (dR[l] * ffc + R[l] * fdfc);
-          Sl += s1 * (float(l) * R[l]);
-          Bx += sx * R[l];
-          By += sy * R[l];
-          Bz += sz * R[l];
-        }
-      }
-#pragma unroll
-      for (int off = kPairGroup / 2; off > 0; off >>= 1) {
-        A += __shfl_xor(A, off, kPairGroup);
-        Sl += __shfl_xor(Sl, off, kPairGroup);
-        Bx += __shfl_xor(Bx, off, kPairGroup);
-        By += __shfl_xor(By, off, kPairGroup);
-        Bz += __shfl_xor(Bz, off, kPairGroup);
-      }
-      if (gl == 0) {
-        const double sc = fcd / d;
-        const double gv[3] = {double(A) * vx / d + sc * double(Bx - dx * Sl),
-                              double(A) * vy / d + sc * double(By - dy * Sl),
-                              double(A) * vz / d + sc * double(Bz - dz * Sl)};
-        double* pf = pv.pair_force + 3 * p;
-        pf[0] = gv[0];
-        pf[1] = gv[1];
-        pf[2] = gv[2];
-        if (j != int(i)) {
-          fi[0] -= gv[0];
-          fi[1] -= gv[1];
-          fi[2] -= gv[2];
-        }
-        // r_ji = r_i - r_j(image) = -pair vector
-        v6[0] -= vx * gv[0];
-        v6[1] -= vy * gv[1];
-        v6[2] -= vz * gv[2];
-        v6[3] -= vy * gv[2];
-        v6[4] -= vz * gv[0];
-        v6[5] -= vx * gv[1];
-      }
-      wave_lds_sync();  // the group's {Y, gY} are read before the next pair overwrites them
-    }
-  }
-  double r[9] = {fi[0], fi[1], fi[2], v6[0], v6[1], v6[2], v6[3], v6[4], v6[5]};
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    for (int off = 32; off > 0; off >>= 1) r[k] += __shfl_down(r[k], off, 64);
-    if (lane == 0) red[wave][k] = r[k];
-  }
-  __syncthreads();
-  if (tid < 9) {
-    double t = 0;
-    for (int w = 0; w < kWaves; ++w) t += red[w][tid];
-    if (tid < 3) {
-      pv.centre_force[3 * i + tid] = t;
-    } else {
-      centre_virial[6 * i + tid - 3] = t;
-    }
-  }
 }
 
 // dL/dX of one centre per workgroup into the packed layout (packing.hh)
@@ -3280,22 +3129,15 @@ bool go_adjoint_tile(const RadialDev& rad, int S, const PairView& pv, const floa
   hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB, maxb, pv,
                      c, norm2, int(normalize), xg, xg_scale, G, centre_virial, work);
   RGPU_LAUNCH_CHECK();
-  if (!PAIRS) {
-    const size_t ps = pair_kernel_lds(S, N, L1);
-    auto pk = adjoint_pair_kernel<N, L>;
-    allow_lds(pk, ps);
-    hipLaunchKernelGGL(pk, dim3(unsigned(pv.n_centres)), dim3(kThreads), ps, stream, rad, S, pv,
-                       static_cast<const float*>(work), centre_virial);
-    RGPU_LAUNCH_CHECK();
-  }
+  if (!PAIRS) launch_pair_forces<float>(rad, S, pv, work, centre_virial, stream);
   return true;
 }
 
 // The register-tile adjoint for the (max_radial, max_angular) it is built
 // for (up to 8 species); false where it does not apply.  With a workspace
-// of n_centres S (L+1)^2 N floats and spline radial functions, the pair
-// phase runs as adjoint_pair_kernel (split); otherwise in the same
-// workgroup.
+// of n_centres S (L+1)^2 N floats (and kPairSlack more) and spline radial
+// functions, the pair phase is launch_pair_forces (split); otherwise it runs
+// in the same workgroup.
 template <int N, int L, int NR, bool DIRECT>
 bool launch_adjoint_tile_nl(const RadialDev& rad, int S, const PairView& pv, const float* c, const double* norm2,
                             bool normalize, const double* xg, double xg_scale, const float* G,

@@ -147,3 +147,45 @@ def test_fp64_product_tiles(atoms, points):
         parts.append(ctx.gap_predict())
     for a, b, c in zip((e, g, s), *parts):
         assert np.abs(a - b - c).max() <= 1e-10 * max(np.abs(b).max(), np.abs(c).max())
+
+
+def _rows_backward(ctx, G, volume):
+    """dL/dr and neg stress of one structure from its exported gradient rows."""
+    off, j, vec = ctx.neighbours()[:3]
+    f = np.einsum("pxd,pd->px", ctx.features_gradient().reshape(len(j), 3, -1),
+                  np.repeat(G, np.diff(off), axis=0))
+    g = np.zeros((len(off) - 1, 3))
+    np.add.at(g, j, f)
+    s = [-(vec[:, a] * f[:, b]).sum() / volume for a, b in ((0, 0), (1, 1), (2, 2), (1, 2), (2, 0), (0, 1))]
+    return g, np.array([s])
+
+
+@pytest.mark.parametrize("N,L", [(1, 0), (4, 4), (5, 5), (6, 6), (7, 7), (11, 9), (13, 4), (17, 9), (24, 2), (8, 10)])
+def test_pair_forces_by_wavefronts(N, L):
+    """The pair phase at the edges of its channel counts (4, 6, .. 24) and of
+    the orders side by side (l_max 4, 6, 9; past 9 the general kernel), with
+    more than 64 neighbours per centre: one structure, whose centres take four
+    wavefronts each, against the oracle, and enough copies of it that a
+    wavefront takes whole centres against the one.  More functions than 16 use
+    the DVR basis and the exported gradient rows: the overlap of so many GTOs
+    is singular to rounding, and their orthonormal basis not determined."""
+    sts = periodic_box(13, 0.08, (1, 8), d_min=1.0, seed=91)
+    hp = soap_hypers(rc=6.0, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=False)
+    if N > 16:
+        hp["radial_contribution"]["type"] = "DVR"
+    ctx, _ = _context(hp, sts)
+    X, _ = ctx.features()
+    G = np.random.default_rng(92).normal(size=X.shape)
+    g, s = ctx.features_backward(G)
+    if N > 16:
+        g_ref, s_ref = _rows_backward(ctx, G, 13 / 0.08)
+    else:
+        g_ref, s_ref = oracle_backward(O.Calculator(hp), O.BatchData(sts), G)
+    assert np.abs(g - g_ref).max() <= 1e-10 * np.abs(g_ref).max()
+    assert np.abs(s - s_ref).max() <= 1e-10 * np.abs(s_ref).max()
+    copies = 2048 // 13 + 1
+    many, _ = _context(hp, sts * copies)
+    gm, sm = many.features_backward(np.tile(G, (copies, 1)))
+    assert np.abs(gm.reshape(copies, *g.shape) - g).max() <= 1e-10 * np.abs(g).max()
+    assert np.abs(sm.reshape(copies, *s.shape) - s).max() <= 1e-10 * np.abs(s).max()
+    assert len(set(map(bytes, gm.reshape(copies, *g.shape)))) == 1
