@@ -1279,7 +1279,7 @@ void autotune_t(Context& c) {
       if (ms < best) best = ms, pick = pb;
     }
     t.pb_fwd = pick;
-    // the pair-group expansion against the per-entry one, then the
+    // the expansion by wavefronts against the per-entry one, then the
     // expansion writing c once from LDS
     {
       SoapTiles reg = t, lds = t, ent = t;
@@ -1547,7 +1547,7 @@ int rgpu_set_tiles(rgpu_context* ctx, int pairs_fwd, int keys_ps, int pairs_adj,
     if (fused > 3) throw InvalidArgument("fused must be -1, 0, 1, 2 or 3");
     t.fused = fused < 0 ? -1 : (fused == 1 ? 1 : 0);
     t.fwd_lds = fused == 2 ? 1 : 0;
-    t.fwd_group = fused == 3 ? 1 : 0;
+    t.fwd_group = fused == 3 ? 1 : (fused < 0 ? -1 : 0);
     c.have_rep = false;
     c.drop_graph();
   });
@@ -1627,7 +1627,7 @@ int rgpu_get_info(rgpu_context* ctx, int key, int64_t* value) {
       case RGPU_INFO_HALF_LIST: *value = c.tile().half_nl; break;
       case RGPU_INFO_FUSED: *value = c.tile().fused == 1; break;
       case RGPU_INFO_FWD_LDS: *value = c.tile().fwd_lds; break;
-      case RGPU_INFO_FWD_GROUP: *value = c.tile().fwd_group; break;
+      case RGPU_INFO_FWD_GROUP: *value = c.tile().fwd_group == 1; break;
       default: throw InvalidArgument("unknown info key");
     }
   });

@@ -1,4 +1,4 @@
-// Per-pair work of the adjoint, one wavefront per centre
+// Per-pair work of the expansion and of its adjoint, one wavefront per centre
 // (or a few for small batches), for spline radial functions and l_max <= 9.
 #pragma once
 
@@ -22,5 +22,10 @@ constexpr int kPairSlack = 32;
 template <class T>
 void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T* dc, double* centre_virial,
                         hipStream_t stream);
+
+// Expansion c[n][S][N][(L+1)^2] and key masks, as launch_expansion
+template <class T>
+void launch_expansion_wave(const RadialDev& rad, int S, const PairView& pv, T* c, unsigned long long* keymask,
+                           hipStream_t stream);
 
 }  // namespace rgpu

@@ -1,4 +1,5 @@
-// Pair phase of the adjoint by wavefronts (pair_kernels.hh).
+// Pair phase of the adjoint, and the expansion, by wavefronts
+// (pair_kernels.hh).
 //
 // Lanes stand for the (l, mu) of the spherical harmonics, mu = 0 .. l: a lane
 // holds dL/dc of its two orders +-mu for every radial channel of one
@@ -132,6 +133,32 @@ __device__ __forceinline__ PairRec<T> load_pair(const RadialDev& rad, const Pair
   r.wb = T(ca * dfc - (3 * a * a - 1) * fh);
   r.wc = T(b * dfc);
   r.wd = T(cb * dfc + (3 * b * b - 1) * fh);
+  return r;
+}
+
+// the same for the expansion: R fc = ra y0 + rb d0 + rc y1 + rd d1
+template <class T>
+struct PairValue {
+  T x, y, z;
+  T ra, rb, rc, rd;
+  int sp, klo;
+};
+
+template <class T>
+__device__ __forceinline__ PairValue<T> load_pair_value(const RadialDev& rad, const PairView& pv, int64_t p) {
+  PairValue<T> r;
+  const double d = pv.pair_dist[p], fc = pv.pair_fc[p];
+  r.sp = pv.species_of[pv.pair_j[p]];
+  r.x = T(pv.pair_vec[3 * p] / d);
+  r.y = T(pv.pair_vec[3 * p + 1] / d);
+  r.z = T(pv.pair_vec[3 * p + 2] / d);
+  double a, h;
+  r.klo = spline_cell_of(rad, d, r.sp, &a, &h);
+  const double b = 1 - a;
+  r.ra = T(a * fc);
+  r.rb = T(a * (a * a - 1) * fc);
+  r.rc = T(b * fc);
+  r.rd = T(b * (b * b - 1) * fc);
   return r;
 }
 
@@ -506,6 +533,143 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
   }
 }
 
+// Expansion c[i][s][n][lm] = [s == s_i][lm == 0] R0[n] / sqrt(4 pi) + sum over
+// the pairs (i, j), s_j = s, of fc R_nl Y_lm, with the layout of the pair
+// phase: a lane holds the sums of its two orders +-mu for every radial channel
+// in registers, two FMAs per channel and pair whose radial operand all lanes
+// of one l share.  (The per-entry kernel reads both operands of every FMA from
+// LDS, which bounds it; the staging of a batch bounds this one.)  One
+// wavefront per centre, several in turn: 178 -> 93 us for 264 000 pairs of
+// 8192 centres, n_max 12, l_max 9, FP32; 167 -> 72 us for 4096 centres, FP64.
+template <class T, int NT>
+__host__ __device__ inline size_t expansion_wave_lds(int L1) {
+  return sizeof(T) * (size_t(kBatch) * (((L1 * L1) + 1) / 2 * 2 + size_t(L1) * NT));
+}
+
+template <class T, int NT, int G>
+__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 5 : 4) void expansion_wave_kernel(
+    RadialDev rad, int S, PairView pv, T* __restrict__ cout, unsigned long long* __restrict__ keymask) {
+  typedef typename Vec2<T>::type V;
+  typedef T V4 __attribute__((ext_vector_type(4)));
+  constexpr int PPI = 64 / G, VN = sizeof(V) / sizeof(T);
+  const int N = rad.N, L = rad.L, L1 = rad.L1, LL = rad.LL, F = N * L1, LP = (LL + 1) / 2 * 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  T* yc = reinterpret_cast<T*>(smem_raw);
+  T* Y = yc + 4 * LL + wave * (expansion_wave_lds<T, NT>(L1) / sizeof(T));
+  T* R = Y + kBatch * LP;  // [batch][l][NT]
+  fill_ylm_table<T>(rad, yc);
+  for (int e = lane; e < kBatch * L1 * NT; e += 64) R[e] = T(0);  // surplus channels stay zero
+  __syncthreads();
+  const int un = lane & (G - 1), grp = lane / G;
+  int l = 0;
+  while ((l + 1) * (l + 2) / 2 <= un) ++l;
+  const bool unit = l <= L;
+  if (!unit) l = 0;
+  const int mu = unit ? un - l * (l + 1) / 2 : 0;
+  const int lp = l * l + l + mu, lm = l * l + l - mu;
+  const int seg = lane / L1, mo = lane - seg * L1;
+  const float inv_n = 1.0f / float(N);
+  const V4* table = Spl4<T>::table(rad);
+  const double inv_s4pi = 0.28209479177387814347;  // 1/sqrt(4 pi)
+
+  for (int64_t i = int64_t(blockIdx.x) * kWaves + wave; i < pv.n_centres; i += int64_t(gridDim.x) * kWaves) {
+    const int64_t p0 = pv.centre_off[i] + 1;  // the self pair contributes nothing here
+    const int np = int(pv.centre_off[i + 1] - p0);
+    const int si = pv.species_of[i];
+    T* ci = cout + i * int64_t(S) * N * LL;
+    unsigned long long present = 1ull << si;
+    for (int c0 = 0; c0 == 0 || c0 < np; c0 += 64) {
+      const bool act = c0 + lane < np;
+      PairValue<T> rec{};
+      rec.sp = -1;
+      if (act) rec = load_pair_value<T>(rad, pv, p0 + c0 + lane);
+      for (int s = 0; s < S; ++s) {
+        unsigned long long mine = __ballot(rec.sp == s);
+        if (c0 > 0 && !mine) continue;
+        if (mine) present |= 1ull << s;
+        T ap[NT], am[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) ap[n] = am[n] = T(0);
+        while (mine) {
+          int q[kBatch];
+          const int nb = next_batch(mine, q);
+          wave_sync();  // the previous batch is read
+          {
+            const int src = seg == 0 ? q[0] : (seg == 1 ? q[1] : (seg == 2 ? q[2] : q[3]));
+            const T x = __shfl(rec.x, src, 64), y = __shfl(rec.y, src, 64), z = __shfl(rec.z, src, 64);
+            ylm_of_order<T>(L, yc, x, y, z, mo, seg < nb, Y + seg * LP);
+          }
+          for (int e = lane; e < F; e += 64) {
+            const int el = int((float(e) + 0.5f) * inv_n), en = e - el * N;
+            V4 t[kBatch];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b)
+              t[b] = table[int64_t(lane_value(rec.klo, q[b])) * F + en * L1 + el];
+#pragma unroll
+            for (int b = 0; b < kBatch; ++b) {
+              T r = lane_value(rec.ra, q[b]) * t[b].x;
+              r += lane_value(rec.rb, q[b]) * t[b].y;
+              r += lane_value(rec.rc, q[b]) * t[b].z;
+              r += lane_value(rec.rd, q[b]) * t[b].w;
+              R[(b * L1 + el) * NT + en] = b < nb ? r : T(0);
+            }
+          }
+          wave_sync();
+          // (an empty slot's radial functions are zero; its harmonics may be
+          // stale, of an earlier pair or never written: they are not read)
+#pragma unroll 1
+          for (int b0 = 0; b0 < nb; b0 += PPI) {
+            const int b = b0 + grp;
+            const bool on = unit && b < nb;
+            const T yp = on ? Y[b * LP + lp] : T(0), ym = on ? Y[b * LP + lm] : T(0);
+            const V* r = reinterpret_cast<const V*>(R + (b * L1 + l) * NT);
+#pragma unroll
+            for (int n = 0; n < NT; n += VN) {
+              const V x = r[n / VN];
+#pragma unroll
+              for (int k = 0; k < VN; ++k) {
+                if (n + k < NT) {
+                  ap[n + k] += x[k] * yp;
+                  am[n + k] += x[k] * ym;
+                }
+              }
+            }
+          }
+        }
+        // the groups' sums; then this species' block
+        T* cs = ci + int64_t(s) * N * LL;
+        const double* centre = rad.center + (rad.sp_tab ? rad.sp_tab[si] * N : 0);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          if (n >= N) continue;
+          T vp = ap[n], vm = am[n];
+          if constexpr (G <= 32) {
+            vp += __shfl_xor(vp, 32, 64);
+            vm += __shfl_xor(vm, 32, 64);
+          }
+          if constexpr (G <= 16) {
+            vp += __shfl_xor(vp, 16, 64);
+            vm += __shfl_xor(vm, 16, 64);
+          }
+          if (unit && grp == 0) {
+            T* o = cs + n * LL;
+            if (c0 > 0) {
+              vp += o[lp];
+              vm += o[lm];
+            } else if (s == si && lp == 0) {
+              vp += T(centre[n] * inv_s4pi);
+            }
+            o[lp] = vp;
+            if (mu) o[lm] = vm;
+          }
+        }
+      }
+    }
+    if (lane == 0) keymask[i] = present;
+  }
+}
+
 template <class K>
 void allow_lds(K kernel, size_t smem) {
   if (smem > 160 * 1024)
@@ -594,6 +758,34 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
   });
 }
 
+template <class T>
+void launch_expansion_wave(const RadialDev& rad, int S, const PairView& pv, T* c, unsigned long long* keymask,
+                           hipStream_t stream) {
+  const int64_t n = pv.n_centres;
+  if (n == 0) return;
+  const int units = rad.L1 * (rad.L1 + 1) / 2;
+  with_channels(rad.N, [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    const size_t smem = sizeof(T) * size_t(4 * rad.LL) + kWaves * expansion_wave_lds<T, NT>(rad.L1);
+    const int64_t blocks =
+        std::min((n + kWaves - 1) / kWaves, int64_t(cu_count()) * (sizeof(T) == 4 ? 5 : 4));
+    auto go = [&](auto kern) {
+      allow_lds(kern, smem);
+      hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), smem, stream, rad, S, pv, c, keymask);
+      RGPU_LAUNCH_CHECK();
+    };
+    if (units <= 16)
+      go(expansion_wave_kernel<T, NT, 16>);
+    else if (units <= 32)
+      go(expansion_wave_kernel<T, NT, 32>);
+    else
+      go(expansion_wave_kernel<T, NT, 64>);
+  });
+}
+template void launch_expansion_wave<double>(const RadialDev&, int, const PairView&, double*, unsigned long long*,
+                                            hipStream_t);
+template void launch_expansion_wave<float>(const RadialDev&, int, const PairView&, float*, unsigned long long*,
+                                           hipStream_t);
 template void launch_pair_forces<double>(const RadialDev&, int, const PairView&, const double*, double*, hipStream_t);
 template void launch_pair_forces<float>(const RadialDev&, int, const PairView&, const float*, double*, hipStream_t);
 

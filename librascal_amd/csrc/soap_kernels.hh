@@ -65,7 +65,8 @@ struct SoapTiles {
   int half_nl = 0;   // expansion over the half neighbour list (1) or the full list (0)
   int fused = -1;    // power spectrum in the expansion's launch (1), separate (0), built-in (-1)
   int fwd_lds = 0;   // expansion accumulating c in LDS and writing it once (1)
-  int fwd_group = 0; // FP32 expansion on pair groups where it applies (1) or per entry (0)
+  int fwd_group = -1; // expansion by wavefronts where it applies (1), per entry (0), built-in:
+                      //   by wavefronts from 2048 centres on (-1)
 };
 
 // c[i][s][n][l*l+l+m] (finalised) and the per-centre key mask.

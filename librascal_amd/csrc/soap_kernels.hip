@@ -158,7 +158,9 @@ __device__ void ylm_wave(int L_, const T* __restrict__ yc, const T* dirs, int q0
     cos_p = x / sxy;
     sin_p = y / sxy;
   }
-  const T sin_t = sqrt(T(1) - cos_t * cos_t);
+  // (not sqrt(1 - cos_t^2), whose cancellation near the poles was most of the
+  // FP32 expansion's error: 1.3e-6 of max |c| at n_max 12, l_max 9)
+  const T sin_t = sxy;
   // cos(k phi), sin(k phi) for k = m and m+1 (Chebyshev recurrence)
   T c_m = T(1), s_m = T(0), c_m1 = cos_p, s_m1 = sin_p;
   for (int k = 1; k <= m; ++k) {
@@ -2269,228 +2271,10 @@ __global__ __launch_bounds__(kThreads, (PAIRS || ROLES > 1) ? 2 : 3) void adjoin
   }
 }
 
-// Real spherical harmonics Y_l^{+-m} (l = m..L) of one unit direction on the
-// lane of order m (0 <= m <= L), written to Y[(l*l + l +- m) * ys]: the
-// recursion of ylm_wave without the gradient (no cross-lane operations).
-__device__ __forceinline__ void ylm_lane(int L, const float* __restrict__ yc, float x, float y, float z, int m,
-                                         float* Y, int ys) {
-  const int L1 = L + 1;
-  const float* dfac = yc + 4 * L1 * L1;
-  const float* s2l1 = dfac + L1;
-  float n2 = x * x + y * y + z * z;
-  if (fabs(double(n2) - 1.0) > 1e-6) {
-    const float inv = 1.0f / sqrtf(n2);
-    x *= inv;
-    y *= inv;
-    z *= inv;
-  }
-  const float cos_t = z;
-  const float sxy = sqrtf(x * x + y * y);
-  float cos_p = 1.0f, sin_p = 0.0f;
-  if (double(sxy) >= kDblFtol) {
-    cos_p = x / sxy;
-    sin_p = y / sxy;
-  }
-  const float sin_t = sqrtf(1.0f - cos_t * cos_t);
-  float c_m = 1.0f, s_m = 0.0f, c_m1 = cos_p, s_m1 = sin_p;
-  for (int k = 1; k <= m; ++k) {
-    const float cn = 2.0f * cos_p * c_m1 - c_m;
-    const float sn = 2.0f * cos_p * s_m1 - s_m;
-    c_m = c_m1;
-    s_m = s_m1;
-    c_m1 = cn;
-    s_m1 = sn;
-  }
-  const float s2pi = 0.39894228040143267794f;
-  float diag = s2pi;
-  for (int k = 1; k <= m; ++k) diag = diag * sin_t * dfac[k];
-  const float isq2 = 0.70710678118654752440f;
-  float P1 = 0.0f, P2 = 0.0f;
-  for (int l = m; l <= L; ++l) {
-    float P;
-    if (m == l) {
-      P = diag;
-    } else if (m == l - 1) {
-      P = (l == 1) ? cos_t * 1.73205080756887729353f * s2pi : diag * cos_t * s2l1[l];
-    } else {
-      const Vec4<float>::type c4 = reinterpret_cast<const Vec4<float>::type*>(yc)[l * L1 + m];
-      float t = cos_t * P1;
-      t += c4.y * P2;
-      t *= c4.x;
-      P = t;
-    }
-    const int base = l * l + l;
-    if (m == 0) {
-      Y[base * ys] = P * isq2;
-    } else {
-      Y[(base + m) * ys] = P * c_m;
-      Y[(base - m) * ys] = P * s_m;
-    }
-    P2 = P1;
-    P1 = P;
-  }
-}
-
-// lanes per pair of expansion_group_kernel
-constexpr int kPairGroup = 16;
-
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// FP32 spline cell of a pair at distance d whose neighbour has species sj
-// (the cell search of pair_fetch, per-species tables included)
-__device__ __forceinline__ SplineCell<float> pair_cell(const RadialDev& rad, double d, int sj) {
-  int klo;
-  double xhi, h;
-  if (rad.sp_tab) {
-    const int t = rad.sp_tab[sj], last = rad.tab_n[t] - 2;
-    int k = int((d - rad.x1) * rad.tab_pu[t]) - 1;
-    k = k < 0 ? 0 : (k > last ? last : k);
-    xhi = rad.tab_grid[rad.tab_grid0[t] + k + 1];
-    h = rad.tab_h[t];
-    klo = rad.tab_cell0[t] + k;
-  } else {
-    int k = int((d - rad.x1) * rad.per_unit) - 1;
-    k = k < 0 ? 0 : (k > rad.search_size ? rad.search_size : k);
-    xhi = rad.grid[k + 1];
-    h = rad.h;
-    klo = k;
-  }
-  const double ca = (xhi - d) / h;
-  SplineCell<float> cell;
-  cell.klo = klo;
-  cell.a = float(ca);
-  cell.b = float(1 - ca);
-  cell.inv_h = rad.sp_tab ? float(1.0 / h) : float(1.0 / rad.h);
-  return cell;
-}
-
-// l of the packed index lm = l*l + l + m, for compile-time lm
-__host__ __device__ constexpr int l_of_lm_c(int lm) {
-  int l = 0;
-  while ((l + 1) * (l + 1) <= lm) ++l;
-  return l;
-}
-
-// ---------------------------------------------------------------------------
-// Expansion of the mixed path on pair groups (FP32 spline radial functions,
-// compile-time L).  One workgroup per centre; wavefront w takes the
-// neighbours of species s = w, w + 4, ... in list order, four at a time, one
-// per group of 16 lanes.  Lane n of a group evaluates f_c R_nl of its radial
-// channel for every l; the group's lanes m <= L form Y_lm of the pair
-// (ylm_lane) in LDS; every lane then adds f_c R_nl Y_lm to its registers
-// c[s][n][lm] for all lm.  The four groups' sums are added with shuffles in
-// a fixed order (so the result does not depend on timing), the species rows
-// pass through LDS and are written once, coalesced, with the centre term.
-// The same sums as expansion_kernel (calculator_spherical_expansion.hh
-// :2139-2300), accumulated in another order.
-template <int L>
-__global__ __launch_bounds__(kThreads) void expansion_group_kernel(RadialDev rad, int S, PairView pv,
-                                                                   float* __restrict__ cout,
-                                                                   unsigned long long* __restrict__ keymask) {
-  constexpr int L1 = L + 1, LL = L1 * L1, LLP = (LL + 3) & ~3;
-  constexpr int G = 64 / kPairGroup;  // groups per wavefront
-  const int N = rad.N;
-  const int64_t i = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int gl = lane & (kPairGroup - 1), grp = lane / kPairGroup;
-  extern __shared__ __align__(64) unsigned char smem_raw[];
-  float* yc = reinterpret_cast<float*>(smem_raw);
-  float* yg = reinterpret_cast<float*>(smem_raw + ylm_table_bytes<float>(L1));  // [waves][G][LLP]
-  float* cl = yg + kWaves * G * LLP;                                           // [S][N][LL]
-  __shared__ unsigned long long kmask;
-  const int si = pv.species_of[i];
-  load_ylm_table<float>(rad, yc);
-  if (tid == 0) kmask = 1ull << si;
-  __syncthreads();
-  const int64_t p0 = pv.centre_off[i] + 1;  // the self pair contributes the centre term only
-  const int np = int(pv.centre_off[i + 1] - p0);
-  float* Yg = yg + (wave * G + grp) * LLP;
-  const int n = gl < N ? gl : N - 1;
-  for (int s = wave; s < S; s += kWaves) {
-    float acc[LL];
-#pragma unroll
-    for (int lm = 0; lm < LL; ++lm) acc[lm] = 0.f;
-    bool any = false;
-    for (int b = 0; b < np; b += 64) {
-      const int t = b + lane;
-      const bool mine = t < np && pv.species_of[pv.pair_j[p0 + t]] == s;
-      unsigned long long m = __ballot(mine);
-      any = any || m != 0;
-      while (m) {
-        // the next G pairs of this species, one per group
-        int my = -1;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          if (m) {
-            const int bit = __ffsll((long long)m) - 1;
-            if (g == grp) my = bit;
-            m &= m - 1;
-          }
-        }
-        if (my >= 0) {
-          const int64_t p = p0 + b + my;
-          const double d = pv.pair_dist[p];
-          const double fcd = pv.pair_fc[p];
-          const SplineCell<float> cell = pair_cell(rad, d, s);
-          float R[L1];
-          const float fc = float(fcd);
-#pragma unroll
-          for (int l = 0; l <= L; ++l) {
-            float v;
-            spline_eval<float>(rad, cell, n * L1 + l, &v, nullptr);
-            R[l] = v * fc;
-          }
-          if (gl <= L)
-            ylm_lane(L, yc, float(pv.pair_vec[3 * p] / d), float(pv.pair_vec[3 * p + 1] / d),
-                     float(pv.pair_vec[3 * p + 2] / d), gl, Yg, 1);
-          wave_lds_sync();
-#pragma unroll
-          for (int q = 0; q < LLP / 4; ++q) {
-            const f32x4 y4 = *reinterpret_cast<const f32x4*>(Yg + 4 * q);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-              if (4 * q + u < LL) acc[4 * q + u] += R[l_of_lm_c(4 * q + u)] * y4[u];
-          }
-          wave_lds_sync();  // Y is read before the group's next pair overwrites it
-        }
-      }
-    }
-    // the groups' partial sums, (g0 + g1) + (g2 + g3)
-#pragma unroll
-    for (int lm = 0; lm < LL; ++lm) {
-      acc[lm] += __shfl_xor(acc[lm], kPairGroup, 64);
-      acc[lm] += __shfl_xor(acc[lm], 2 * kPairGroup, 64);
-    }
-    if (grp == 0 && gl < N) {
-      float* row = cl + (s * N + gl) * LL;
-#pragma unroll
-      for (int lm = 0; lm < LL; ++lm) row[lm] = acc[lm];
-    }
-    if (lane == 0 && any) atomicOr(&kmask, 1ull << s);
-  }
-  __syncthreads();
-  const int E = S * N * LL;
-  const double inv_s4pi = 0.28209479177387814347;  // 1/sqrt(4 pi)
-  const double* centre = rad.center + (rad.sp_tab ? rad.sp_tab[si] * N : 0);
-  float* ci = cout + i * int64_t(E);
-  for (int e = tid; e < E; e += kThreads) {
-    float v = cl[e];
-    const int row = e / LL;
-    if (row / N == si && e - row * LL == 0) v += float(centre[row - si * N] * inv_s4pi);
-    ci[e] = v;
-  }
-  if (tid == 0) keymask[i] = kmask;
-}
-
-__host__ __device__ inline size_t expansion_group_lds(int S, int N, int L1) {
-  const int LL = L1 * L1, LLP = (LL + 3) & ~3;
-  return ylm_table_bytes<float>(L1) + sizeof(float) * (size_t(kWaves) * (64 / kPairGroup) * LLP +
-                                                       size_t(S) * N * LL);
 }
 
 // dL/dX of one centre per workgroup into the packed layout (packing.hh)
@@ -3288,36 +3072,24 @@ void launch_adjoint_t(const RadialDev& rad, int S, const PairView& pv, const T* 
 
 }  // namespace
 
-// The pair-group expansion for the max_angular it is built for (FP32 spline
-// radial functions, max_radial <= 16, at least 3 species: with fewer, most
-// of its wavefronts would idle); false where it does not apply.
-template <class T>
-bool launch_expansion_group(const RadialDev& rad, int S, const PairView& pv, T* c,
-                            unsigned long long* keymask, hipStream_t stream, const SoapTiles& tiles) {
-  if constexpr (sizeof(T) != 4) {
-    return false;
-  } else {
-    if (!tiles.fwd_group || !rad.use_spline || rad.N > kPairGroup || S < 3) return false;
-    auto go = [&](auto kern) {
-      const size_t smem = expansion_group_lds(S, rad.N, rad.L1);
-      allow_lds(kern, smem);
-      hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, pv, c,
-                         keymask);
-      RGPU_LAUNCH_CHECK();
-      return true;
-    };
-    if (rad.L == 9) return go(expansion_group_kernel<9>);
-    if (rad.L == 6) return go(expansion_group_kernel<6>);
-    return false;
-  }
-}
+// Centres from which the expansion takes a wavefront per centre: below, too
+// few are in flight and the workgroup per centre has the shorter chain.  Per
+// entry against by wavefronts: 64 centres 13 and 19 us, 1024 centres (FP64)
+// 27 and 32 us, 1331 centres (FP32) 23 and 36 us, 4096 centres (FP64,
+// n_max 12, l_max 9) 167 and 72 us, 8192 centres (FP32) 178 and 93 us;
+// molecules of 8 atoms (n_max 8, l_max 6) FP64 46 and 48 us, FP32 (four times
+// as many) 277 and 167 us.
+constexpr int64_t kWaveExpansion = 2048;
 
 template <class T>
 void launch_expansion(const RadialDev& rad, int S, const PairView& pv, T* c,
                       unsigned long long* keymask, hipStream_t stream, const SoapTiles& tiles) {
   if (pv.n_centres == 0) return;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
-  if (launch_expansion_group<T>(rad, S, pv, c, keymask, stream, tiles)) return;
+  if ((tiles.fwd_group < 0 ? pv.n_centres >= kWaveExpansion : tiles.fwd_group == 1) && pair_kernels_apply(rad)) {
+    launch_expansion_wave<T>(rad, S, pv, c, keymask, stream);
+    return;
+  }
   const int B = rad.N * rad.LL;
   const int kpt = (B + kThreads - 1) / kThreads;
   // the benchmark shape (n_max 12, l_max 9, spline radial functions) with

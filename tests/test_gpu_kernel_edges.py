@@ -189,3 +189,30 @@ def test_pair_forces_by_wavefronts(N, L):
     assert np.abs(gm.reshape(copies, *g.shape) - g).max() <= 1e-10 * np.abs(g).max()
     assert np.abs(sm.reshape(copies, *s.shape) - s).max() <= 1e-10 * np.abs(s).max()
     assert len(set(map(bytes, gm.reshape(copies, *g.shape)))) == 1
+
+
+@pytest.mark.parametrize("N,L", [(1, 0), (4, 4), (5, 5), (7, 7), (11, 9), (13, 4), (24, 2), (8, 10)])
+def test_expansion_by_wavefronts(N, L):
+    """The expansion with a wavefront per centre (from 2048 centres on) against
+    the per-entry kernel on one of its copies: centres with more than 64
+    neighbours, an isolated atom, a species without neighbours, edges of the
+    channel counts and orders; FP64 to rounding, FP32 as between the kernels
+    elsewhere."""
+    sts = periodic_box(12, 0.08, (1, 8), d_min=1.0, seed=93)
+    sts = sts + [dict(sts[0], positions=np.zeros((1, 3)), numbers=np.array([6], np.int32),
+                      cell=100 * np.eye(3))]
+    hp = soap_hypers(rc=6.0, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8)
+    if N > 16:
+        hp["radial_contribution"]["type"] = "DVR"
+    copies = 2048 // 13 + 1
+    one, _ = _context(hp, sts)
+    many, _ = _context(hp, sts * copies)
+    for prec, tol in ((_capi.FP64, 1e-13), (_capi.MIXED, 1e-6)):
+        one.set_precision(prec)
+        many.set_precision(prec)
+        one.compute()
+        many.compute()
+        c, km = one.expansion()
+        cm, kmm = many.expansion()
+        assert np.array_equal(kmm.reshape(copies, -1), np.tile(km, (copies, 1)))
+        assert np.abs(cm.reshape(copies, *c.shape) - c).max() <= tol * np.abs(c).max()
