@@ -133,7 +133,6 @@ struct Context {
   std::vector<int64_t> sp_off;    // per species index s: [sp_off[s], sp_off[s+1])
   bool have_weights = false;
   DeviceBuffer<double> T64, alpha;  // T64 [M][ldx64()]: rows as the FP64 features'
-  DeviceBuffer<double> T64f;        // full layout [M][D] (K_NM gradient rows)
   DeviceBuffer<float> T32;
   MixedSparse mixed_sparse;
 
@@ -142,7 +141,8 @@ struct Context {
   DeviceBuffer<int> d_rows;
 
   // scratch
-  DeviceBuffer<double> e_centre, grad, cvir, tmp64, out64, knm_grad, knm_scale;
+  DeviceBuffer<double> e_centre, grad, cvir, tmp64, out64, knm_grad, knm_pair, knm_centre, knm_virial;
+  DeviceBuffer<int64_t> d_sp_order;
   DeviceBuffer<double> e_part;  // energy GEMM partials per column tile and centre
   PinnedBuffer<double> out_stage;  // page-locked staging of a prediction's outputs
   DeviceBuffer<double> d_inv_vol;  // [n_struct] 1 / cell volume
@@ -930,6 +930,14 @@ void backward_device(Context& c, const float* G, double* grad, double* cvir, con
                         xg_scale, G, cvir, c.stream, c.tile(), work);
   launch_force_gather(pv, rl, grad, c.stream);
 }
+// FP64 pair phase of the adjoint from dL/dc
+void launch_pair_phase(Context& c, const PairView& pv, const double* dc, double* cvir) {
+  const int S = int(c.species.size());
+  if (pair_kernels_apply(c.rd))
+    launch_pair_forces<double>(c.rd, S, pv, dc, cvir, c.stream);
+  else
+    launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
+}
 // FP64: G in symmetric packed rows of dL/dp, or (full) dL/dX in the full
 // layout, xg = X_i . dL/dX_i (null: summed here)
 void backward_device(Context& c, const double* G, bool full, const double* xg, double* grad, double* cvir) {
@@ -943,10 +951,7 @@ void backward_device(Context& c, const double* G, bool full, const double* xg, d
                              xg, G, c.gsym, dc, c.stream);
   else
     launch_sym_contract(S, N, L1, c.n_atoms, c.c64.get(), G, dc, c.stream);
-  if (pair_kernels_apply(c.rd))
-    launch_pair_forces<double>(c.rd, S, pv, dc, cvir, c.stream);
-  else
-    launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
+  launch_pair_phase(c, pv, dc, cvir);
   launch_force_gather(pv, rl, grad, c.stream);
 }
 // selected columns of dL/dX (or dL/dp, rows ld apart) into the full layout
@@ -2019,12 +2024,11 @@ int rgpu_set_sparse_points(rgpu_context* ctx, int zeta, int64_t n_sparse, const 
     // the values as given, then every layout the kernels read from them in
     // sorted row order
     const int64_t ldx = c.ldx64(), n1 = std::max<int64_t>(n_sparse, 1);
-    DeviceBuffer<double> raw;
-    DeviceBuffer<int64_t> d_order;
+    DeviceBuffer<double> raw, full;
     double* dr = raw.reserve(size_t(n1 * D));
-    int64_t* dord = d_order.reserve(size_t(n1));
+    int64_t* dord = c.d_sp_order.reserve(size_t(n1));
     double* dT = c.T64.reserve(size_t(n1 * ldx));
-    double* dTf = c.T64f.reserve(size_t(n1 * D));
+    double* dTf = full.reserve(size_t(n1 * D));
     float* dT32 = c.T32.reserve(size_t(n1 * D));
     if (n_sparse > 0) {
       RGPU_HIP(hipMemcpyAsync(dr, values, sizeof(double) * size_t(n_sparse * D), hipMemcpyHostToDevice, c.stream));
@@ -2132,10 +2136,12 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
     require_unmasked(c);
     ensure_rep(c);
     const int S = int(c.species.size());
-    const int64_t n = c.n_atoms, M = c.M, D = c.D(), ns = c.n_struct;
+    const int64_t n = c.n_atoms, M = c.M, ns = c.n_struct;
     const int64_t rows = 3 * n + (neg_stress ? 6 * ns : 0);
     double* o = c.knm_grad.reserve(size_t(std::max<int64_t>(rows * M, 1)));
     if (rows * M == 0) return;
+    // (points of species outside the batch have zero columns)
+    if (c.sp_off[S] < M) RGPU_HIP(hipMemsetAsync(o, 0, sizeof(double) * rows * M, c.stream));
     // d[i][m] = X_i . T_m for the centre's species (the K_NM of zeta 1)
     double* d = c.tmp64.reserve(size_t(std::max<int64_t>(n * M, 1)));
     RGPU_HIP(hipMemsetAsync(d, 0, sizeof(double) * n * M, c.stream));
@@ -2145,37 +2151,56 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
       blks.back().zeta = 1;
     }
     run_gap_f64_rows(blks.data(), S, d, M, c.stream);
-    const double* pf = full_invariants(c);
-    double* gs = c.knm_scale.reserve(size_t(std::max<int64_t>(n, 1)));
-    double* gd = c.grad.reserve(size_t(std::max<int64_t>(3 * n, 1)));
-    double* cv = c.cvir.reserve(size_t(std::max<int64_t>(6 * n, 1)));
-    double* st = c.out64.reserve(size_t(6 * std::max<int64_t>(ns, 1)));
-    // a sparsified row enters the adjoint scattered into the full layout
-    double* grow = c.sparsified() ? c.gfull.reserve(size_t(c.D_full())) : nullptr;
-    ReverseLists rl;
-    const PairView bpv = backward_view(c, &rl);
+    // the sparse points in symmetric packed rows (a selection's scattered first)
+    const int N = c.rd.N, L1 = c.rd.L1;
+    const int64_t lds = sym_row_stride(S, N, L1), E = int64_t(S) * N * c.rd.LL;
+    const double* T = c.T64.get();
+    if (c.sparsified()) {
+      double* gf = c.gfull.reserve(size_t(M * c.D_full()));
+      double* gs = c.gsym.reserve(size_t(M * lds));
+      launch_scatter_columns(M, c.ldx64(), c.selection(), T, c.D_full(), gf, c.stream);
+      launch_sym_pack(S, N, L1, M, gf, nullptr, gs, c.stream);
+      T = gs;
+    }
     // column m (species-sorted): dL/dX_i = zeta d_im^(zeta-1) T_m for the
     // centres of m's species, through the adjoint; rows written in the
-    // caller's sparse-point order
-    for (int s = 0; s < S; ++s)
-      for (int64_t m = c.sp_off[s]; m < c.sp_off[s + 1]; ++m) {
-        launch_knm_gradient_scale(n, d + m, M, c.d_species_of.get(), s, c.zeta, gs, c.stream);
-        const double* row = c.T64f.get() + m * D;
-        if (grow) {
-          launch_scatter_columns(1, D, c.selection(), row, c.D_full(), grow, c.stream);
-          row = grow;
+    // caller's sparse-point order.  As many columns at a time as fit the
+    // workspace: one by one, each of four launches over one species' centres
+    // left the chip mostly idle (300 columns of 983 centres: 18.2 ms of
+    // kernels).
+    constexpr int64_t kWorkspace = int64_t(256) << 20;
+    ReverseLists rl;
+    PairView bpv = backward_view(c, &rl);
+    bpv.set_pairs = c.pl.cap_pairs;
+    bpv.set_centres = n;
+    for (int s = 0; s < S; ++s) {
+      const int64_t ni = c.row_off[s + 1] - c.row_off[s], ms = c.sp_off[s + 1] - c.sp_off[s];
+      if (ms == 0) continue;
+      const int64_t per_set = int64_t(sizeof(double)) * (ni * E + 3 * bpv.set_pairs + 9 * n);
+      const int64_t Q = std::max<int64_t>(1, std::min({ms, kWorkspace / std::max<int64_t>(per_set, 1), int64_t(65535)}));
+      double* dc = c.dc64.reserve(size_t(Q * ni * E + kPairSlack));
+      bpv.pair_force = c.knm_pair.reserve(size_t(std::max<int64_t>(3 * Q * bpv.set_pairs, 1)));
+      bpv.centre_force = c.knm_centre.reserve(size_t(3 * Q * n));
+      double* cv = c.knm_virial.reserve(size_t(6 * Q * n));
+      bpv.ids = c.d_rows.get() + c.row_off[s];
+      bpv.n_ids = ni;
+      // (pairs of the other species' centres)
+      RGPU_HIP(hipMemsetAsync(bpv.pair_force, 0, sizeof(double) * 3 * Q * bpv.set_pairs, c.stream));
+      for (int64_t m0 = c.sp_off[s]; m0 < c.sp_off[s + 1]; m0 += Q) {
+        const int64_t q = std::min(Q, c.sp_off[s + 1] - m0);
+        const int64_t* cols = c.d_sp_order.get() + m0;
+        if (ni > 0) {
+          bpv.n_centres = q * ni;
+          const SymSets sets{bpv.ids, ni, d + m0, M, c.zeta};
+          launch_sym_contract_sets(S, N, L1, q, sets, c.c64.get(), c.hp.normalize ? c.p64.get() : nullptr,
+                                   c.norm2.get(), T + m0 * lds, dc, c.stream);
+          launch_pair_phase(c, bpv, dc, cv);
         }
-        launch_backward_rank1(c.rd, S, bpv, c.c64.get(), pf, c.norm2.get(),
-                              c.hp.normalize, row, gs, cv, c.stream, c.tile());
-        launch_force_gather(bpv, rl, gd, c.stream);
-        const int64_t col = c.sp_order[size_t(m)];
-        launch_strided_copy(gd, 3 * n, o + col, M, c.stream);
-        if (neg_stress) {
-          RGPU_HIP(hipMemsetAsync(st, 0, sizeof(double) * 6 * ns, c.stream));
-          launch_segment_sum(cv, 6, c.d_atom_off.get(), int(ns), st, c.stream, c.d_inv_vol.get());
-          launch_strided_copy(st, 6 * ns, o + 3 * n * M + col, M, c.stream);
-        }
+        launch_knm_force_gather(bpv, rl, s, q, cols, M, o, c.stream);
+        if (neg_stress)
+          launch_knm_stress(bpv, s, q, cv, c.d_atom_off.get(), ns, c.d_inv_vol.get(), cols, M, o + 3 * n * M, c.stream);
       }
+    }
     RGPU_HIP(hipMemcpyAsync(out, o, sizeof(double) * rows * M, hipMemcpyDefault, c.stream));
     RGPU_HIP(hipStreamSynchronize(c.stream));
   });

@@ -376,11 +376,13 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
   constexpr int per = kWaves / W;
   const int w = W > 1 ? wave % W : 0;
   for (int64_t i0 = int64_t(blockIdx.x) * per; i0 < pv.n_centres; i0 += int64_t(gridDim.x) * per) {
-    const int64_t i = i0 + wave / W;
-    if (W == 1 && i >= pv.n_centres) break;
+    const int64_t v = i0 + wave / W;
+    if (W == 1 && v >= pv.n_centres) break;
+    const PairEntry entry = pair_entry(pv, v);
+    const int64_t i = entry.centre;
     const int64_t p0 = pv.centre_off[i] + 1;  // the self pair contributes nothing
     const int np = int(pv.centre_off[i + 1] - p0);
-    const T* dci = dcg + i * int64_t(S) * LL * N;
+    const T* dci = dcg + v * int64_t(S) * LL * N;
     const V4* table = Spl4<T>::table(rad);
     for (int c0 = 0; c0 < np; c0 += 64 * W) {
       const int k = c0 + lane * W + w;
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
         const double Q = double(res[4 * lane]) / pv.pair_dist[p];
         const double g[3] = {Q * vx + double(res[4 * lane + 1]), Q * vy + double(res[4 * lane + 2]),
                              Q * vz + double(res[4 * lane + 3])};
-        double* pf = pv.pair_force + 3 * p;
+        double* pf = pv.pair_force + 3 * (entry.set * pv.set_pairs + p);
         pf[0] = g[0];
         pf[1] = g[1];
         pf[2] = g[2];
@@ -522,10 +524,11 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
       double t = 0;
 #pragma unroll
       for (int k = 0; k < W; ++k) t += red[wave + k][lane];
+      const int64_t o = entry.set * pv.set_centres + i;
       if (lane < 3)
-        pv.centre_force[3 * i + lane] = t;
+        pv.centre_force[3 * o + lane] = t;
       else
-        centre_virial[6 * i + lane - 3] = t;
+        centre_virial[6 * o + lane - 3] = t;
     }
     if constexpr (W > 1) __syncthreads();
     if (lane < 9) red[wave][lane] = 0.0;

@@ -26,7 +26,23 @@ struct PairView {
   // (periodic images of the centre itself left out) [n_centres][3]
   double* pair_force = nullptr;
   double* centre_force = nullptr;
+  // Pair phase of the adjoint for several dL/dc of the same batch: n_centres
+  // entries, entry v the centre ids[v % n_ids] of set v / n_ids.  dL/dc is
+  // [entry], the outputs are [set][set_pairs][3] and [set][set_centres][.].
+  // (ids null: one set of all centres.)
+  const int* ids = nullptr;
+  int64_t n_ids = 1, set_pairs = 0, set_centres = 0;
 };
+
+// entry v of the pair phase: its set and its centre
+struct PairEntry {
+  int64_t set, centre;
+};
+__device__ __forceinline__ PairEntry pair_entry(const PairView& pv, int64_t v) {
+  if (!pv.ids) return {0, v};
+  const int64_t q = v / pv.n_ids;
+  return {q, int64_t(pv.ids[v - q * pv.n_ids])};
+}
 
 // Reverse pair lists for the deterministic force sum: for atom j, the pairs
 // p (self pairs left out) whose neighbour is j, in no particular order:
@@ -178,14 +194,6 @@ template <class To>
 void launch_gather_rows(int64_t n, int64_t D, int64_t ldd, const double* src, const int64_t* rows, To* dst,
                         hipStream_t stream);
 
-// FP64 adjoint (full layout) for a rank-one dL/dX: G_i = Gscale[i] * Grow
-// (Grow [D], one sparse point's features; centres with a zero scale are
-// skipped and get a zero virial).  Used for the K_NM gradient rows.
-void launch_backward_rank1(const RadialDev& rad, int S, const PairView& pv, const double* c,
-                           const double* p, const double* norm2, bool normalize, const double* Grow,
-                           const double* Gscale, double* centre_virial,
-                           hipStream_t stream, const SoapTiles& tiles = SoapTiles());
-
 // Pack dL/dX [n][D] (full layout, FP64) into the packed layout of the mixed
 // path, rows of packed_row_stride() columns (FP32): diagonal-key entries
 // (G[n1][n2] + G[n2][n1]) / sqrt 2
@@ -203,9 +211,16 @@ void launch_backward_split(const RadialDev& rad, int S, const PairView& pv, cons
                            const float* G, double* centre_virial, hipStream_t stream,
                            const SoapTiles& tiles = SoapTiles(), float* work = nullptr);
 
-// scale[i] = zeta d[i*ld]^(zeta-1) for the centres of species s, else 0
-void launch_knm_gradient_scale(int64_t n, const double* d, int64_t ld, const int* species_of, int s,
-                               int zeta, double* scale, hipStream_t stream);
+// K_NM gradient of several sparse points of one species (sets): from the pair
+// and centre forces of the sets (pv.pair_force zero for centres of other
+// species), out[(3 j + x) ld + cols[q]] of every atom j and set q.
+void launch_knm_force_gather(const PairView& pv, const ReverseLists& rl, int species, int64_t n_sets,
+                             const int64_t* cols, int64_t ld, double* out, hipStream_t stream);
+// out[(6 st + k) ld + cols[q]] = inv_vol[st] times the sum over the structure's
+// centres of this species of centre_virial[q][i][k]
+void launch_knm_stress(const PairView& pv, int species, int64_t n_sets, const double* centre_virial,
+                       const int64_t* atom_off, int64_t n_struct, const double* inv_vol, const int64_t* cols,
+                       int64_t ld, double* out, hipStream_t stream);
 // p[0, n) = v (a kernel: no memset node when the stream is captured)
 void launch_fill(double* p, int64_t n, double v, hipStream_t stream);
 // dst[r * ld] = src[r], r < n

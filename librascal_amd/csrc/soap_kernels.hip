@@ -987,7 +987,7 @@ __global__ void normalise_kernel(int64_t n, int64_t D, int64_t ld, const T* __re
 template <class T, bool DIRECT>
 __device__ __forceinline__ void adjoint_pairs(const RadialDev& rad, int S, int PB, const PairView& pv,
                                               const T* yc, const T* dc, unsigned char* region,
-                                              int64_t i, double* __restrict__ centre_virial) {
+                                              int64_t i, double* __restrict__ centre_virial, int64_t set = 0) {
   const int N = rad.N, L1 = rad.L1, LL = rad.LL, F = N * L1, B = N * LL;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // lanes per pair: the largest power of two in [16, 64] that still gives
@@ -1084,7 +1084,7 @@ __device__ __forceinline__ void adjoint_pairs(const RadialDev& rad, int S, int P
                            A * vy / d + sc * double(pb.res[4 * q + 2]),
                            A * vz / d + sc * double(pb.res[4 * q + 3])};
       const int j = pb.pj[q];
-      double* pf = pv.pair_force + 3 * (p0 + q0 + q);
+      double* pf = pv.pair_force + 3 * (set * pv.set_pairs + p0 + q0 + q);
       pf[0] = g[0];
       pf[1] = g[1];
       pf[2] = g[2];
@@ -1110,14 +1110,14 @@ __device__ __forceinline__ void adjoint_pairs(const RadialDev& rad, int S, int P
     for (int k = 0; k < 9; ++k)
       for (int off = 32; off > 0; off >>= 1) r[k] += __shfl_down(r[k], off, 64);
     if (lane == 0) {
-      for (int k = 0; k < 3; ++k) pv.centre_force[3 * i + k] = r[k];
-      for (int k = 0; k < 6; ++k) centre_virial[6 * i + k] = r[3 + k];
+      for (int k = 0; k < 3; ++k) pv.centre_force[3 * (set * pv.set_centres + i) + k] = r[k];
+      for (int k = 0; k < 6; ++k) centre_virial[6 * (set * pv.set_centres + i) + k] = r[3 + k];
     }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Fused adjoint.  Given G = dL/dX (X = p/|p| the exported features):
+// Adjoint.  Given G = dL/dX (X = p/|p| the exported features):
 //  1. dL/dp = G/|p| - (X.G) p/|p|^2 (the transpose of the normalisation
 //     derivative, calculator_spherical_invariants.hh:588-652); X.G is either
 //     passed per centre (for the GAP energy X.G = zeta E_i, the energy being
@@ -1134,178 +1134,22 @@ __device__ __forceinline__ void adjoint_pairs(const RadialDev& rad, int S, int P
 //     the pairs naming it, in ascending pair order (no atomics: the forces
 //     are the same on every run); the virial sum r_ji (x) g is reduced per
 //     centre (sparse_kernel_predict.hh:354-364).
-constexpr int kAdjPre = 8;  // key-block elements per thread held for the prefetch
 
-template <class T, bool DIRECT>
-__global__ __launch_bounds__(kThreads) void adjoint_kernel(
-    RadialDev rad, int S, int PB, int c_in_lds, PairView pv, const T* __restrict__ c,
-    const T* __restrict__ p, const double* __restrict__ norm2, int normalize,
-    const double* __restrict__ xg, double xg_scale, const T* __restrict__ G,
-    const T* __restrict__ Grow, const double* __restrict__ Gscale,
-    double* __restrict__ centre_virial) {
-  typedef typename Vec4<T>::type V4;
-  const int64_t i = blockIdx.x;
-  // rank-one dL/dX (Grow != null): G_i = Gscale[i] Grow; a centre with a
-  // zero scale contributes nothing
-  if (Grow && Gscale[i] == 0.0) {
-    if (threadIdx.x < 6) centre_virial[6 * i + threadIdx.x] = 0.0;
-    if (threadIdx.x < 3) pv.centre_force[3 * i + threadIdx.x] = 0.0;
-    const int64_t q0 = 3 * (pv.centre_off[i] + 1), q1 = 3 * pv.centre_off[i + 1];
-    for (int64_t q = q0 + threadIdx.x; q < q1; q += kThreads) pv.pair_force[q] = 0.0;
-    return;
-  }
-  const int N = rad.N, L1 = rad.L1, LL = rad.LL, B = N * LL, E = S * B;
-  const int N4 = (N + 3) & ~3;
-  const int K = S * (S + 1) / 2;
-  const int KB = N * N * L1;
-  const int64_t D = int64_t(K) * KB;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  extern __shared__ __align__(64) unsigned char smem_raw[];
-  T* yc = reinterpret_cast<T*>(smem_raw);
-  T* dc = reinterpret_cast<T*>(smem_raw + ylm_table_bytes<T>(L1));  // dL/dc [S][LL][N]
-  unsigned char* region = reinterpret_cast<unsigned char*>(dc) + align_up(sizeof(T) * E, 64);
-  load_ylm_table<T>(rad, yc);
-  const T* cs;
-  T* gA;
-  if (c_in_lds) {
-    T* cl = reinterpret_cast<T*>(region);
-    for (int e = tid; e < E; e += kThreads) cl[e] = c[i * int64_t(E) + e];
-    cs = cl;
-    gA = reinterpret_cast<T*>(region + align_up(sizeof(T) * E, 64));
-  } else {
-    cs = c + i * int64_t(E);
-    gA = reinterpret_cast<T*>(region);
-  }
-  // gA[l][x][y] = g[y][x][l], gB[l][x][y] = g[x][y][l]; the l planes LS
-  // apart, two values more than a plane, so that the transposing stores of
-  // consecutive l (one per thread) fall in different LDS banks
-  const int LS = N * N4 + 2;
-  T* gB = gA + L1 * LS;
-  __shared__ double red[kWaves][9];
-  __shared__ double sh_ab[2];
-
-  const T* Gi = Grow ? nullptr : G + i * D;
-  const T gs = Grow ? T(Gscale[i]) : T(1);
-  auto gval = [&](int64_t o) -> T { return Grow ? gs * Grow[o] : Gi[o]; };
-  auto pval = [&](int64_t o) -> T { return p[i * D + o]; };
-  double alpha = 1.0, beta = 0.0;
-  if (normalize) {
-    const double n2 = norm2[i];
-    double dotxg = 0;
-    if (xg) {
-      dotxg = xg_scale * xg[i];
-    } else {
-      double dot = 0;
-      for (int64_t o = tid; o < D; o += kThreads) dot += double(pval(o)) * double(gval(o));
-      for (int off = 32; off > 0; off >>= 1) dot += __shfl_down(dot, off, 64);
-      if (lane == 0) red[wave][0] = dot;
-      __syncthreads();
-      if (tid == 0) {
-        double t = 0;
-        for (int w = 0; w < kWaves; ++w) t += red[w][0];
-        sh_ab[0] = t;
-      }
-      __syncthreads();
-      dotxg = n2 > 0 ? sh_ab[0] / sqrt(n2) : 0.0;
-    }
-    if (n2 > 0) {
-      alpha = 1.0 / sqrt(n2);
-      beta = dotxg / n2;
-    }
-  }
-  const T ta = T(alpha), tb = T(beta);
-  for (int e = tid; e < E; e += kThreads) dc[e] = T(0);
-  for (int e = tid; e < 2 * L1 * LS; e += kThreads) gA[e] = T(0);  // zero pads
-
-  // key blocks: element o = (x*N + y)*L1 + l; thread holds o = tid + 256 r
-  const FastDiv fNL1 = fast_div(N * L1), fL1 = fast_div(L1), fLL = fast_div(LL);
-  const bool prefetch = KB <= kAdjPre * kThreads;
-  T pre[kAdjPre];
-  auto fetch = [&](int key) {
-    if (!prefetch) return;
-    const int64_t pk = int64_t(key) * KB;
-#pragma unroll
-    for (int r = 0; r < kAdjPre; ++r) {
-      const int o = tid + kThreads * r;
-      pre[r] = o < KB ? ta * gval(pk + o) - tb * pval(pk + o) : T(0);
-    }
-  };
-  fetch(0);
-  __syncthreads();
-  const int units_a = (N4 / 4) * LL;
-  for (int key = 0; key < K; ++key) {
-    int a, b;
-    key_species(key, S, &a, &b);
-    if (prefetch) {
-#pragma unroll
-      for (int r = 0; r < kAdjPre; ++r) {
-        const int o = tid + kThreads * r;
-        if (o < KB) {
-          const int x = o / fNL1, rr = o - x * N * L1, y = rr / fL1, l = rr - y * L1;
-          gA[l * LS + y * N4 + x] = pre[r];
-          gB[l * LS + x * N4 + y] = pre[r];
-        }
-      }
-    } else {
-      const int64_t pk = int64_t(key) * KB;
-      for (int o = tid; o < KB; o += kThreads) {
-        const T g = ta * gval(pk + o) - tb * pval(pk + o);
-        const int x = o / fNL1, rr = o - x * N * L1, y = rr / fL1, l = rr - y * L1;
-        gA[l * LS + y * N4 + x] = g;
-        gB[l * LS + x * N4 + y] = g;
-      }
-    }
-    __syncthreads();
-    if (a == b) {
-      // symmetrise: gA[l][x][y] = g[y][x] + g[x][y]
-      for (int e = tid; e < L1 * LS; e += kThreads) gA[e] += gB[e];
-      __syncthreads();
-    }
-    if (key + 1 < K) fetch(key + 1);
-    const T w = (a < b) ? T(1.41421356237309504880) : T(1);
-    const int units = units_a * (a < b ? 2 : 1);
-    for (int u = tid; u < units; u += kThreads) {
-      const bool side_b = u >= units_a;
-      const int uu = side_b ? u - units_a : u;
-      const int nt = uu / fLL, lm = uu - nt * LL;
-      const int l = l_of_lm(lm);
-      const T* gt = (side_b ? gB : gA) + l * LS + 4 * nt;
-      const T* cx = cs + (side_b ? a : b) * B + lm;
-      V4 s4 = {T(0), T(0), T(0), T(0)};
-      for (int x = 0; x < N; ++x) {
-        const T cv = cx[x * LL];
-        const V4 g4 = *reinterpret_cast<const V4*>(gt + x * N4);
-        s4 += g4 * cv;
-      }
-      const T f = w / sqrt(T(2 * l + 1));
-      T* out = dc + (side_b ? b : a) * B + lm * N;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int n = 4 * nt + v;
-        if (n < N) out[n] += f * s4[v];
-      }
-    }
-    __syncthreads();
-  }
-
-  // per-pair contraction; the batch reuses the region after dL/dc
-  adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, dc, region, i, centre_virial);
-}
-
-// Pair phase alone, dL/dc [S][LL][N] of each centre from memory (dcg).
+// Pair phase alone, dL/dc [S][LL][N] of each entry (pair_entry) from memory
+// (dcg).
 template <class T, bool DIRECT>
 __global__ __launch_bounds__(kThreads) void adjoint_pairs_kernel(RadialDev rad, int S, int PB, PairView pv,
                                                                  const T* __restrict__ dcg,
                                                                  double* __restrict__ centre_virial) {
-  const int64_t i = blockIdx.x;
+  const PairEntry e0 = pair_entry(pv, blockIdx.x);
   const int E = S * rad.N * rad.LL;
   extern __shared__ __align__(64) unsigned char smem_raw[];
   T* yc = reinterpret_cast<T*>(smem_raw);
   T* dc = reinterpret_cast<T*>(smem_raw + ylm_table_bytes<T>(rad.L1));
   unsigned char* region = reinterpret_cast<unsigned char*>(dc) + align_up(sizeof(T) * E, 64);
   load_ylm_table<T>(rad, yc);
-  for (int e = threadIdx.x; e < E; e += kThreads) dc[e] = dcg[i * int64_t(E) + e];
-  adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, dc, region, i, centre_virial);
+  for (int e = threadIdx.x; e < E; e += kThreads) dc[e] = dcg[blockIdx.x * int64_t(E) + e];
+  adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, dc, region, e0.centre, centre_virial, e0.set);
 }
 
 // dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values
@@ -1339,7 +1183,7 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(int64_t D, int64_
 // Adjoint of the mixed path: dL/dX (G) and p in the packed layout (p as its
 // BF16 operand planes), the dL/dp blocks staged in LDS in the full layout
 // KCH key blocks at a time beside the expansion coefficients.  Same
-// mathematics as adjoint_kernel; the dL/dc contraction keeps its outputs in
+// mathematics as above; the dL/dc contraction keeps its outputs in
 // registers across the key blocks instead of one LDS update per key:
 //  1. g = alpha G - beta p of keys [k0, k0 + KCH) in the layout
 //     [key][x][y][l]; a diagonal key is unpacked symmetrised, g + g^T
@@ -2954,120 +2798,96 @@ bool launch_adjoint_tile(const RadialDev& rad, int S, const PairView& pv, const 
   return false;
 }
 
-template <class T, bool DIRECT>
-void launch_adjoint_t(const RadialDev& rad, int S, const PairView& pv, const T* c, const T* p,
-                      const unsigned short* p_hi, const unsigned short* p_lo,
-                      const double* norm2, bool normalize, const double* xg, double xg_scale,
-                      const T* G, double* centre_virial, hipStream_t stream,
-                      const SoapTiles& tiles, const T* Grow = nullptr,
-                      const double* Gscale = nullptr, float* work = nullptr) {
+template <bool DIRECT>
+void launch_adjoint_f32(const RadialDev& rad, int S, const PairView& pv, const float* c,
+                        const unsigned short* p_hi, const unsigned short* p_lo, const double* norm2, bool normalize,
+                        const double* xg, double xg_scale, const float* G, double* centre_virial, hipStream_t stream,
+                        const SoapTiles& tiles, float* work) {
+  typedef float T;
   const int N = rad.N, L1 = rad.L1, LL = rad.LL, F = N * L1, E = S * N * LL;
   const size_t yt = ylm_table_bytes<T>(L1);
   const size_t blk = align_up(sizeof(T) * size_t(E), 64);
-  if constexpr (sizeof(T) == 4) {
-    const int K = S * (S + 1) / 2;
-    if ((tiles.adj_kind == 2 || tiles.adj_kind == 3) && Grow == nullptr &&
-        launch_adjoint_tile<DIRECT>(rad, S, pv, c, norm2, normalize, xg, xg_scale, G, centre_virial,
-                                    tiles.adj_kind == 3 ? work : nullptr, stream, tiles))
-      return;
-    // matrix-core adjoint: packed dL/dX staged KCH key blocks at a time,
-    // the invariants not read
-    int T_col = 0;
-    for (int l = 0; l <= rad.L; ++l) T_col += (2 * l + 16) >> 4;
-    const int maxt = (S * T_col + kWaves - 1) / kWaves;
-    if (tiles.adj_kind == 1 && N <= 16 && maxt <= 16 && Grow == nullptr) {
-      const size_t cbytes = align_up(sizeof(float) * size_t(S) * N * ((LL + 15) / 32 * 32 + 16), 64);
-      size_t mbytes = 0;
-      for (int l = 0; l <= rad.L; ++l) {
-        const size_t w = 16 * ((2 * l + 16) >> 4);
-        mbytes += sizeof(float) * w * w;
-      }
-      // packed G of a chunk of keys (the largest chunk: diagonal keys are
-      // the smaller blocks)
-      const size_t kbytes = sizeof(float) * size_t(L1) * N * (4 * ((N + 1) / 4) + 2);
-      int KCH = tiles.keys_adj > 0 ? std::min(tiles.keys_adj, K) : K;
-      // (A fragments of rows N..15 read past the last staged block)
-      const size_t slack = sizeof(float) * 16 * (4 * ((N + 1) / 4) + 2);
-      auto region_of = [&](int kch, int pb) {
-        return std::max({align_up(kch * kbytes + slack, 64), align_up(mbytes, 64),
-                         pair_batch_bytes(pb, LL, F, sizeof(T), DIRECT, true)});
-      };
-      int PB = tiles.pb_adj > 0 ? std::min(tiles.pb_adj, 64) : 16;
-      if (tiles.keys_adj <= 0)
-        while (KCH > 1 && yt + cbytes + region_of(KCH, 1) > kResidentBudget) --KCH;
-      if (tiles.pb_adj <= 0)
-        while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) >
-                             std::max(align_up(KCH * kbytes, 64), align_up(mbytes, 64)))
-          --PB;
-      const size_t smem = yt + cbytes + region_of(KCH, PB);
-      auto go = [&](auto kern) {
-        allow_lds(kern, smem);
-        hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB,
-                           KCH, pv, c, norm2, int(normalize), xg, xg_scale, G, centre_virial);
-      };
-      if (maxt <= 4)
-        go(adjoint_mfma_kernel<DIRECT, 4>);
-      else if (maxt <= 8)
-        go(adjoint_mfma_kernel<DIRECT, 8>);
-      else if (maxt <= 12)
-        go(adjoint_mfma_kernel<DIRECT, 12>);
-      else
-        go(adjoint_mfma_kernel<DIRECT, 16>);
-      RGPU_LAUNCH_CHECK();
-      return;
+  const int K = S * (S + 1) / 2;
+  if ((tiles.adj_kind == 2 || tiles.adj_kind == 3) &&
+      launch_adjoint_tile<DIRECT>(rad, S, pv, c, norm2, normalize, xg, xg_scale, G, centre_virial,
+                                  tiles.adj_kind == 3 ? work : nullptr, stream, tiles))
+    return;
+  // matrix-core adjoint: packed dL/dX staged KCH key blocks at a time,
+  // the invariants not read
+  int T_col = 0;
+  for (int l = 0; l <= rad.L; ++l) T_col += (2 * l + 16) >> 4;
+  const int maxt = (S * T_col + kWaves - 1) / kWaves;
+  if (tiles.adj_kind == 1 && N <= 16 && maxt <= 16) {
+    const size_t cbytes = align_up(sizeof(float) * size_t(S) * N * ((LL + 15) / 32 * 32 + 16), 64);
+    size_t mbytes = 0;
+    for (int l = 0; l <= rad.L; ++l) {
+      const size_t w = 16 * ((2 * l + 16) >> 4);
+      mbytes += sizeof(float) * w * w;
     }
-    // mixed path: packed dL/dX and BF16 planes of p, staged in LDS KCH key
-    // blocks at a time beside c
-    if (!p_hi || !p_lo) throw InvalidArgument("the FP32 adjoint takes the split invariants");
-    const size_t kbytes = sizeof(T) * size_t(N) * N * L1;
-    const int upt = (S * ((N + 3) / 4) * LL + kThreads - 1) / kThreads;
-    if (upt > 8) throw InvalidArgument("max_radial x (max_angular+1)^2 too large for the FP32 adjoint");
+    // packed G of a chunk of keys (the largest chunk: diagonal keys are
+    // the smaller blocks)
+    const size_t kbytes = sizeof(float) * size_t(L1) * N * (4 * ((N + 1) / 4) + 2);
     int KCH = tiles.keys_adj > 0 ? std::min(tiles.keys_adj, K) : K;
-    if (tiles.keys_adj <= 0)
-      while (KCH > 1 && yt + blk + align_up(KCH * kbytes, 64) > kResidentBudget) --KCH;
-    const size_t dbytes = align_up(KCH * kbytes, 64);
+    // (A fragments of rows N..15 read past the last staged block)
+    const size_t slack = sizeof(float) * 16 * (4 * ((N + 1) / 4) + 2);
+    auto region_of = [&](int kch, int pb) {
+      return std::max({align_up(kch * kbytes + slack, 64), align_up(mbytes, 64),
+                       pair_batch_bytes(pb, LL, F, sizeof(T), DIRECT, true)});
+    };
     int PB = tiles.pb_adj > 0 ? std::min(tiles.pb_adj, 64) : 16;
+    if (tiles.keys_adj <= 0)
+      while (KCH > 1 && yt + cbytes + region_of(KCH, 1) > kResidentBudget) --KCH;
     if (tiles.pb_adj <= 0)
-      while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) > dbytes) --PB;
-    const size_t smem = yt + blk + std::max(dbytes, pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true));
+      while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) >
+                           std::max(align_up(KCH * kbytes, 64), align_up(mbytes, 64)))
+        --PB;
+    const size_t smem = yt + cbytes + region_of(KCH, PB);
     auto go = [&](auto kern) {
       allow_lds(kern, smem);
-      hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB, KCH,
-                         pv, c, p_hi, p_lo, norm2, int(normalize), xg, xg_scale, G, centre_virial);
+      hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB,
+                         KCH, pv, c, norm2, int(normalize), xg, xg_scale, G, centre_virial);
     };
-    if (upt <= 2)
-      go(adjoint_staged_kernel<DIRECT, 2>);
-    else if (upt <= 3)
-      go(adjoint_staged_kernel<DIRECT, 3>);
-    else if (upt <= 4)
-      go(adjoint_staged_kernel<DIRECT, 4>);
-    else if (upt <= 5)
-      go(adjoint_staged_kernel<DIRECT, 5>);
+    if (maxt <= 4)
+      go(adjoint_mfma_kernel<DIRECT, 4>);
+    else if (maxt <= 8)
+      go(adjoint_mfma_kernel<DIRECT, 8>);
+    else if (maxt <= 12)
+      go(adjoint_mfma_kernel<DIRECT, 12>);
     else
-      go(adjoint_staged_kernel<DIRECT, 8>);
+      go(adjoint_mfma_kernel<DIRECT, 16>);
     RGPU_LAUNCH_CHECK();
-  } else {
-    (void)p_hi;
-    (void)p_lo;
-    const int N4 = (N + 3) & ~3;
-    const size_t gbytes = sizeof(T) * 2 * size_t(L1) * (N * N4 + 2);  // two l-plane sets, LS apart
-    const int c_in_lds = yt + blk + blk + gbytes <= kAdjBudget ? 1 : 0;
-    const size_t region = (c_in_lds ? blk : 0) + gbytes;
-    const size_t fixed = yt + blk;
-    const size_t batch_room = std::max(region, kAdjBudget > fixed ? kAdjBudget - fixed : size_t(0));
-    int PB = 8;
-    if (tiles.pb_adj > 0)
-      PB = std::min(tiles.pb_adj, 64);
-    else
-      while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) > batch_room) --PB;
-    const size_t smem = fixed + std::max(region, pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true));
-    auto kern = adjoint_kernel<T, DIRECT>;
-    allow_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB,
-                       c_in_lds, pv, c, p, norm2, int(normalize), xg, xg_scale, G, Grow, Gscale,
-                       centre_virial);
-    RGPU_LAUNCH_CHECK();
+    return;
   }
+  // mixed path: packed dL/dX and BF16 planes of p, staged in LDS KCH key
+  // blocks at a time beside c
+  if (!p_hi || !p_lo) throw InvalidArgument("the FP32 adjoint takes the split invariants");
+  const size_t kbytes = sizeof(T) * size_t(N) * N * L1;
+  const int upt = (S * ((N + 3) / 4) * LL + kThreads - 1) / kThreads;
+  if (upt > 8) throw InvalidArgument("max_radial x (max_angular+1)^2 too large for the FP32 adjoint");
+  int KCH = tiles.keys_adj > 0 ? std::min(tiles.keys_adj, K) : K;
+  if (tiles.keys_adj <= 0)
+    while (KCH > 1 && yt + blk + align_up(KCH * kbytes, 64) > kResidentBudget) --KCH;
+  const size_t dbytes = align_up(KCH * kbytes, 64);
+  int PB = tiles.pb_adj > 0 ? std::min(tiles.pb_adj, 64) : 16;
+  if (tiles.pb_adj <= 0)
+    while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) > dbytes) --PB;
+  const size_t smem = yt + blk + std::max(dbytes, pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true));
+  auto go = [&](auto kern) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB, KCH,
+                       pv, c, p_hi, p_lo, norm2, int(normalize), xg, xg_scale, G, centre_virial);
+  };
+  if (upt <= 2)
+    go(adjoint_staged_kernel<DIRECT, 2>);
+  else if (upt <= 3)
+    go(adjoint_staged_kernel<DIRECT, 3>);
+  else if (upt <= 4)
+    go(adjoint_staged_kernel<DIRECT, 4>);
+  else if (upt <= 5)
+    go(adjoint_staged_kernel<DIRECT, 5>);
+  else
+    go(adjoint_staged_kernel<DIRECT, 8>);
+  RGPU_LAUNCH_CHECK();
 }
 
 }  // namespace
@@ -3420,19 +3240,6 @@ template void launch_gather_rows<double>(int64_t, int64_t, int64_t, const double
 template void launch_gather_rows<float>(int64_t, int64_t, int64_t, const double*, const int64_t*, float*,
                                         hipStream_t);
 
-void launch_backward_rank1(const RadialDev& rad, int S, const PairView& pv, const double* c,
-                           const double* p, const double* norm2, bool normalize, const double* Grow,
-                           const double* Gscale, double* centre_virial,
-                           hipStream_t stream, const SoapTiles& tiles) {
-  if (pv.n_centres == 0) return;
-  if (rad.use_spline)
-    launch_adjoint_t<double, false>(rad, S, pv, c, p, nullptr, nullptr, norm2, normalize, nullptr, 1.0,
-                                    nullptr, centre_virial, stream, tiles, Grow, Gscale);
-  else
-    launch_adjoint_t<double, true>(rad, S, pv, c, p, nullptr, nullptr, norm2, normalize, nullptr, 1.0,
-                                   nullptr, centre_virial, stream, tiles, Grow, Gscale);
-}
-
 void launch_backward_split(const RadialDev& rad, int S, const PairView& pv, const float* c,
                            const unsigned short* p_hi, const unsigned short* p_lo,
                            const double* norm2, bool normalize, const double* xg, double xg_scale,
@@ -3440,11 +3247,11 @@ void launch_backward_split(const RadialDev& rad, int S, const PairView& pv, cons
                            const SoapTiles& tiles, float* work) {
   if (pv.n_centres == 0) return;
   if (rad.use_spline)
-    launch_adjoint_t<float, false>(rad, S, pv, c, nullptr, p_hi, p_lo, norm2, normalize, xg, xg_scale,
-                                   G, centre_virial, stream, tiles, nullptr, nullptr, work);
+    launch_adjoint_f32<false>(rad, S, pv, c, p_hi, p_lo, norm2, normalize, xg, xg_scale, G, centre_virial, stream,
+                              tiles, work);
   else
-    launch_adjoint_t<float, true>(rad, S, pv, c, nullptr, p_hi, p_lo, norm2, normalize, xg, xg_scale,
-                                  G, centre_virial, stream, tiles, nullptr, nullptr, work);
+    launch_adjoint_f32<true>(rad, S, pv, c, p_hi, p_lo, norm2, normalize, xg, xg_scale, G, centre_virial, stream,
+                             tiles, work);
 }
 
 void launch_pack_gradient(int S, int N, int L1, int64_t n, const double* G, float* Gp,
@@ -3454,32 +3261,10 @@ void launch_pack_gradient(int S, int N, int L1, int64_t n, const double* G, floa
   RGPU_LAUNCH_CHECK();
 }
 
-__global__ void knm_gradient_scale_kernel(int64_t n, const double* __restrict__ d, int64_t ld,
-                                          const int* __restrict__ species_of, int s, int zeta,
-                                          double* __restrict__ scale) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double v = 0.0;
-  if (species_of[i] == s) {
-    const double x = d[i * ld];
-    v = double(zeta);
-    for (int k = 1; k < zeta; ++k) v *= x;
-  }
-  scale[i] = v;
-}
-
 __global__ void strided_copy_kernel(const double* __restrict__ src, int64_t n, double* __restrict__ dst,
                                     int64_t ld) {
   const int64_t r = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (r < n) dst[r * ld] = src[r];
-}
-
-void launch_knm_gradient_scale(int64_t n, const double* d, int64_t ld, const int* species_of, int s,
-                               int zeta, double* scale, hipStream_t stream) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(knm_gradient_scale_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, stream, n,
-                     d, ld, species_of, s, zeta, scale);
-  RGPU_LAUNCH_CHECK();
 }
 
 void launch_strided_copy(const double* src, int64_t n, double* dst, int64_t ld, hipStream_t stream) {
@@ -3676,6 +3461,102 @@ __global__ __launch_bounds__(256) void force_gather_kernel(int64_t n, const int6
   }
 }
 
+// K_NM gradient columns of several sparse points of one species at a time: a
+// wavefront per atom keeps the rank order of its list (as above) and takes the
+// sets in turn.
+__global__ __launch_bounds__(256) void knm_force_gather_kernel(PairView pv, ReverseLists rl, int species, int64_t sets,
+                                                               const int64_t* __restrict__ cols, int64_t ld,
+                                                               double* __restrict__ out) {
+  __shared__ int64_t lst[4][kGatherCap], ord[4][kGatherCap];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t j = int64_t(blockIdx.x) * 4 + w;
+  if (j >= pv.set_centres) return;  // whole wavefronts; no workgroup barrier follows
+  const int64_t b = rl.roff[j];
+  const int m = int(rl.roff[j + 1] - b);
+  const bool ranked = m <= kGatherCap, own = pv.species_of[j] == species;
+  if (ranked) {
+    for (int k = lane; k < m; k += 64) lst[w][k] = rl.rlist[b + k];
+    wave_lds_sync();
+    for (int k = lane; k < m; k += 64) {
+      const int64_t v = lst[w][k];
+      int r = 0;
+      for (int q = 0; q < m; ++q) r += lst[w][q] < v ? 1 : 0;
+      ord[w][r] = v;
+    }
+    wave_lds_sync();
+  }
+  // (the sets of one atom over gridDim.y wavefronts)
+  for (int64_t set = blockIdx.y; set < sets; set += gridDim.y) {
+    const double* pf = pv.pair_force + 3 * set * pv.set_pairs;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    if (ranked) {
+      for (int k = lane; k < m; k += 64) {
+        const double* f = pf + 3 * ord[w][k];
+        s0 += f[0];
+        s1 += f[1];
+        s2 += f[2];
+      }
+    } else {
+      int64_t prev = -1;
+      for (int k = 0; k < m; ++k) {
+        long long best = LLONG_MAX;
+        for (int q = lane; q < m; q += 64) {
+          const long long v = rl.rlist[b + q];
+          if (v > prev && v < best) best = v;
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+          const long long o = __shfl_xor(best, off, 64);
+          best = o < best ? o : best;
+        }
+        prev = best;
+        if (lane == (k & 63)) {
+          const double* f = pf + 3 * best;
+          s0 += f[0];
+          s1 += f[1];
+          s2 += f[2];
+        }
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      s0 += __shfl_xor(s0, off, 64);
+      s1 += __shfl_xor(s1, off, 64);
+      s2 += __shfl_xor(s2, off, 64);
+    }
+    if (lane < 3) {
+      const double f = lane == 0 ? s0 : (lane == 1 ? s1 : s2);
+      const double own_force = own ? pv.centre_force[3 * (set * pv.set_centres + j) + lane] : 0.0;
+      out[(3 * j + lane) * ld + cols[set]] = own_force + f;
+    }
+  }
+}
+
+// one workgroup per structure and set
+__global__ __launch_bounds__(kThreads) void knm_stress_kernel(PairView pv, int species,
+                                                              const double* __restrict__ centre_virial,
+                                                              const int64_t* __restrict__ atom_off,
+                                                              const double* __restrict__ inv_vol,
+                                                              const int64_t* __restrict__ cols, int64_t ld,
+                                                              double* __restrict__ out) {
+  const int64_t st = blockIdx.x, set = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ double red[kWaves][6];
+  double v[6] = {0, 0, 0, 0, 0, 0};
+  for (int64_t i = atom_off[st] + threadIdx.x; i < atom_off[st + 1]; i += kThreads) {
+    if (pv.species_of[i] != species) continue;
+    for (int k = 0; k < 6; ++k) v[k] += centre_virial[6 * (set * pv.set_centres + i) + k];
+  }
+  for (int k = 0; k < 6; ++k) {
+    for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+    if (lane == 0) red[wave][k] = v[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 6) {
+    double t = 0;
+    for (int w = 0; w < kWaves; ++w) t += red[w][threadIdx.x];
+    out[(6 * st + threadIdx.x) * ld + cols[set]] = t * inv_vol[st];
+  }
+}
+
 }  // namespace
 
 void launch_reverse_pairs(const PairView& pv, const ReverseLists& rl, DeviceBuffer<int64_t>& scan_scratch,
@@ -3698,6 +3579,26 @@ void launch_force_gather(const PairView& pv, const ReverseLists& rl, double* gra
   if (n == 0) return;
   hipLaunchKernelGGL(force_gather_kernel, dim3(unsigned((n + 3) / 4)), dim3(256), 0, stream, n, rl.roff,
                      rl.rlist, pv.pair_force, pv.centre_force, grad);
+  RGPU_LAUNCH_CHECK();
+}
+
+void launch_knm_force_gather(const PairView& pv, const ReverseLists& rl, int species, int64_t n_sets,
+                             const int64_t* cols, int64_t ld, double* out, hipStream_t stream) {
+  if (pv.set_centres == 0 || n_sets == 0) return;
+  // wavefronts enough to fill the chip, each with the ranks of its list
+  const int64_t split = std::min<int64_t>(n_sets, std::max<int64_t>(1, 8192 / pv.set_centres));
+  hipLaunchKernelGGL(knm_force_gather_kernel, dim3(unsigned((pv.set_centres + 3) / 4), unsigned(split)), dim3(256), 0,
+                     stream, pv, rl, species, n_sets, cols, ld, out);
+  RGPU_LAUNCH_CHECK();
+}
+
+void launch_knm_stress(const PairView& pv, int species, int64_t n_sets, const double* centre_virial,
+                       const int64_t* atom_off, int64_t n_struct, const double* inv_vol, const int64_t* cols,
+                       int64_t ld, double* out, hipStream_t stream) {
+  if (n_struct == 0 || n_sets == 0) return;
+  if (n_sets > 65535) throw InvalidArgument("too many sets in one launch");
+  hipLaunchKernelGGL(knm_stress_kernel, dim3(unsigned(n_struct), unsigned(n_sets)), dim3(kThreads), 0, stream, pv,
+                     species, centre_virial, atom_off, inv_vol, cols, ld, out);
   RGPU_LAUNCH_CHECK();
 }
 

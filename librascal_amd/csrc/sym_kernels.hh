@@ -37,6 +37,18 @@ void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* 
 // packed rows
 void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const double* G, double* dc,
                          hipStream_t stream);
+// dL/dc [n_sets][n_ids] of the kernel derivatives of sparse points T (symmetric
+// packed rows, one per set) at the centres ids: dL/dX_i = zeta d^(zeta - 1) T_q
+// with d = X_i . T_q = dot[i ld_dot + q], X = p / |p| (p null: X = p)
+struct SymSets {
+  const int* ids = nullptr;
+  int64_t n_ids = 1;
+  const double* dot = nullptr;
+  int64_t ld_dot = 0;
+  int zeta = 1;
+};
+void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
+                              const double* p, const double* norm2, const double* T, double* dc, hipStream_t stream);
 // The same from dL/dX in full rows [n][K N^2 (L+1)] (keys a <= b): X = p / |p|
 // with p in symmetric packed rows and xg[i] = X . dL/dX (null: summed here),
 // or X = p (p null).  work: packed rows where they are needed

@@ -129,12 +129,14 @@ __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int 
 // L+1 apart, but the workgroup's wavefronts take them channel after channel
 // from the same cached lines, which costs less than packing the rows first
 // (4689 centres, 4 species, n_max 8, l_max 6: 244 us against 183 + 139).  kGather: as
-// kDp, the entries gathered from memory (R too large for the LDS).
+// kDp, the entries gathered from memory (R too large for the LDS).  kRank,
+// kRankGather: dL/dX of centre ids[v % n_ids] the sparse point of set
+// v / n_ids times zeta d^(zeta - 1).
 //
 // Bound by the memory it streams and the latency of the scalar loads: 4096
 // centres, 4 species, n_max 12, l_max 9: 0.31 ms for 0.93 GB, where the key
 // contraction of the fused FP64 adjoint it replaced took about 1.0 ms.
-enum { kDp, kDx, kGather };
+enum { kDp, kDx, kGather, kRank, kRankGather };
 
 template <int LM, int kForm>
 __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, int L, int64_t ld,
@@ -143,8 +145,10 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
                                                                 const double* __restrict__ norm2,
                                                                 const double* __restrict__ xg,
                                                                 const double* __restrict__ G,
-                                                                double* __restrict__ dc) {
-  const int64_t i = blockIdx.x;
+                                                                SymSets sets, double* __restrict__ dc) {
+  constexpr bool rank = kForm == kRank || kForm == kRankGather, gather = kForm == kGather || kForm == kRankGather;
+  const int64_t v = blockIdx.x, set = rank ? v / sets.n_ids : 0;
+  const int64_t i = rank ? int64_t(sets.ids[v - set * sets.n_ids]) : v;
   const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), S = R / N, KB = N * N * L1;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double rt2 = 1.41421356237309504880;
@@ -154,7 +158,7 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
   // its mirror (both the same between species)
   int2* tab = reinterpret_cast<int2*>(reinterpret_cast<double*>(smem_raw) + kWaves * TRI);
   __shared__ double red[kWaves];
-  const double* Gi = G + i * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
+  const double* Gi = G + (rank ? set : i) * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
   const double* pi = p ? p + i * ld : nullptr;
   // packed entry t of channel l of G
   auto entry = [&](int l, int t) -> double {
@@ -201,21 +205,35 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
       }
     }
   }
+  if constexpr (rank) {
+    // dL/dX = zeta d^(zeta - 1) T, d = X . T
+    const double d = sets.dot[i * sets.ld_dot + set];
+    double a = double(sets.zeta);
+    for (int k = 1; k < sets.zeta; ++k) a *= d;
+    alpha = a;
+    if (p) {
+      const double n2 = norm2[i];
+      if (n2 > 0) {
+        alpha = a / sqrt(n2);
+        beta = a * d / n2;
+      }
+    }
+  }
   const double* ci = c + i * int64_t(R) * LL;
   for (int k = 0; k * kWaves <= L; ++k) {
     const int u = wave_unit(L1, kWaves, wave, k), lk = L - u;
     if (u < 0) continue;
     const double* g = Gi + lk * TRI;
-    if constexpr (kForm != kGather) {
+    if constexpr (!gather) {
       wave_sync();  // the previous channel is read
       // (many loads in flight: the runs come from memory)
-      if (kForm == kDx && p) {
+      if ((kForm == kDx || kForm == kRank) && p) {
         const double* q = pi + lk * TRI;
 #pragma unroll 8
         for (int t = lane; t < TRI; t += 64) W[t] = alpha * entry(lk, t) - beta * q[t];
       } else {
 #pragma unroll 16
-        for (int t = lane; t < TRI; t += 64) W[t] = entry(lk, t);
+        for (int t = lane; t < TRI; t += 64) W[t] = rank ? alpha * entry(lk, t) : entry(lk, t);
       }
       wave_sync();
       for (int r = lane; r < R; r += 64) W[tri_i(r) + r] *= rt2;
@@ -232,14 +250,21 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
         uniform_ptr y = (uniform_ptr)(ci + l * l);
         int a = tri_i(r);
         for (int col = 0; col < R; ++col, y += LL) {
-          const double w = kForm == kGather ? g[a] * (col == r ? rt2 : 1.0) : W[a];
+          double w;
+          if constexpr (gather) {
+            w = g[a];
+            if constexpr (rank) w = alpha * w - (p ? beta * pi[lk * TRI + a] : 0.0);
+            w *= col == r ? rt2 : 1.0;
+          } else {
+            w = W[a];
+          }
           a += col < r ? 1 : col + 1;
 #pragma unroll
           for (int m = 0; m < M; ++m) acc[m] += w * y[m];
         }
         if (rb + lane < R) {
           const int s = r / N, n = r - s * N;
-          double* o = dc + (i * S + s) * int64_t(LL) * N + n;
+          double* o = dc + (v * S + s) * int64_t(LL) * N + n;
 #pragma unroll
           for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
         }
@@ -413,13 +438,13 @@ constexpr size_t kContractLds = 156 * 1024;
 
 template <int kForm>
 void go_contract(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
-                 const double* xg, const double* G, double* dc, hipStream_t stream) {
+                 const double* xg, const double* G, double* dc, hipStream_t stream, const SymSets& sets = SymSets()) {
   const int R = S * N;
-  const size_t smem = kForm == kGather ? 0 : contract_lds(R, kForm == kDx);
+  const size_t smem = kForm == kGather || kForm == kRankGather ? 0 : contract_lds(R, kForm == kDx);
   auto go = [&](auto kern) {
     allow_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, R, N, L1 - 1, sym_row_stride(S, N, L1),
-                       c, p, norm2, xg, G, dc);
+                       c, p, norm2, xg, G, sets, dc);
     RGPU_LAUNCH_CHECK();
   };
   if (L1 <= 10)
@@ -437,6 +462,16 @@ void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const
     go_contract<kDp>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
   else
     go_contract<kGather>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
+}
+
+void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
+                              const double* p, const double* norm2, const double* T, double* dc, hipStream_t stream) {
+  const int64_t n = n_sets * sets.n_ids;
+  if (n == 0) return;
+  if (contract_lds(S * N, false) <= kContractLds)
+    go_contract<kRank>(S, N, L1, n, c, p, norm2, nullptr, T, dc, stream, sets);
+  else
+    go_contract<kRankGather>(S, N, L1, n, c, p, norm2, nullptr, T, dc, stream, sets);
 }
 
 void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,

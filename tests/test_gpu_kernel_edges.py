@@ -216,3 +216,33 @@ def test_expansion_by_wavefronts(N, L):
         cm, kmm = many.expansion()
         assert np.array_equal(kmm.reshape(copies, -1), np.tile(km, (copies, 1)))
         assert np.abs(cm.reshape(copies, *c.shape) - c).max() <= tol * np.abs(c).max()
+
+
+@pytest.mark.parametrize("species,atoms,N,L,spline,normalize,zeta,points", [
+    ((1, 8), 40, 8, 6, 1e-8, True, 2, {1: 3, 8: 2, 9: 1}),
+    ((1, 8), 33, 5, 4, None, True, 3, {1: 2, 8: 3}),
+    ((1, 8), 30, 4, 10, 1e-8, False, 1, {1: 2, 8: 1}),
+    ((1, 8), 31, 6, 3, 1e-8, True, 2, {8: 4}),
+    (tuple(range(1, 14)), 52, 8, 1, 1e-8, True, 2, {1: 2, 7: 1}),
+    ((6,), 1500, 12, 9, 1e-8, True, 2, {6: 40}),
+])
+def test_knm_gradient_columns(species, atoms, N, L, spline, normalize, zeta, points):
+    """K_NM gradient columns, formed several sparse points at a time, against
+    the adjoint of each column's own dL/dX: columns of one species and of
+    several, of a species outside the batch and of one without points, several
+    workspaces full, triangles past the LDS, the general pair kernel."""
+    sts = periodic_box(atoms, 0.05, species, d_min=1.0, seed=95)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=spline, normalize=normalize)
+    ctx, num = _context(hp, sts)
+    rng = np.random.default_rng(96)
+    spec, vals, w = _points(ctx, num, {z: m for z, m in points.items() if z in species}, rng)
+    if 9 in points and 9 not in species:
+        spec, vals, w = np.append(spec, 9).astype(np.int32), np.vstack([vals, vals[:1]]), np.append(w, 1.0)
+    ctx.set_sparse_points(zeta, spec, vals, w)
+    X, _ = ctx.features()
+    out = ctx.gap_knm_gradient(True)
+    for m in range(0, len(spec), max(1, len(spec) // 6)):
+        scale = np.where(num == spec[m], zeta * (X @ vals[m]) ** (zeta - 1), 0.0)
+        g, s = ctx.features_backward(scale[:, None] * vals[m])
+        ref = np.concatenate([g.ravel(), s.ravel()])
+        assert np.abs(out[:, m] - ref).max() <= 1e-10 * max(np.abs(out).max(), np.abs(ref).max())
