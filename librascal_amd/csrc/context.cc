@@ -1887,16 +1887,19 @@ int rgpu_get_features(rgpu_context* ctx, double* features, double* inv_norms) {
     const int64_t D = c.D(), nc = c.n_centres;
     const int64_t* rows = c.masked ? c.d_centre_idx.get() : nullptr;
     if (features && nc) {
-      double* o = c.out64.reserve(size_t(nc * D));
+      // (a caller's device rows are written in place)
+      const bool in_place = is_own_device_memory(features);
+      double* o = in_place ? features : c.out64.reserve(size_t(nc * D));
       if (c.precision == RGPU_FP64 && c.sparsified())
         launch_normalise<double>(nc, D, c.ps64.get(), c.norm2.get(), c.hp.normalize, o, c.stream, rows, c.ldx64());
       else if (c.precision == RGPU_FP64)
         launch_sym_unpack(int(c.species.size()), c.rd.N, c.rd.L1, nc, c.p64.get(), rows, c.norm2.get(),
                           c.hp.normalize, o, c.stream);
       else
-        launch_normalise<float>(nc, D, ensure_p32(c), c.norm2.get(), c.hp.normalize, o, c.stream,
-                                rows);
-      RGPU_HIP(hipMemcpyAsync(features, o, sizeof(double) * nc * D, hipMemcpyDefault, c.stream));
+        launch_power_spectrum_export(c.rd, int(c.species.size()), nc, c.c32.get(), c.norm2.get(), c.hp.normalize,
+                                     rows, o, c.stream, c.tile());
+      if (!in_place)
+        RGPU_HIP(hipMemcpyAsync(features, o, sizeof(double) * nc * D, hipMemcpyDefault, c.stream));
     }
     if (inv_norms && nc) {
       std::vector<double> h(static_cast<size_t>(c.n_atoms)), o(static_cast<size_t>(nc));

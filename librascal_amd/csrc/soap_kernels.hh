@@ -139,6 +139,12 @@ void launch_power_spectrum_split(const RadialDev& rad, int S, int64_t n_centres,
                                  unsigned short* p_hi, unsigned short* p_lo, double* norm2,
                                  hipStream_t stream, const SoapTiles& tiles = SoapTiles());
 
+// Rows rows[r] (rows null: r) of the same, normalised by norm2 when
+// normalising, as FP64 feature rows x for export.
+void launch_power_spectrum_export(const RadialDev& rad, int S, int64_t n, const float* c, const double* norm2,
+                                  bool normalize, const int64_t* rows, double* x, hipStream_t stream,
+                                  const SoapTiles& tiles = SoapTiles());
+
 // Normalised copy X = p / |p| (or X = p), FP64 output for export: n rows,
 // row r from row rows[r] of p (rows null: row r), p's rows ld values apart
 // (0: D).

@@ -629,13 +629,13 @@ __device__ void ps_tables(int N, int S, int* key_ab, int* tri) {
 // The power spectrum of centre i from its expansion rows in LDS (cs: S N
 // rows of LS = (L+1)^2 | 1 values, then three zero rows; key_ab and tri
 // filled), in KC-key passes over the stage buffer; writes the FP64/FP32
-// rows or the BF16 operand planes and norm2[i].  Every thread calls; ends
-// after a barrier.
-template <class T, bool SPLIT, int NC = -1, int LC = -1>
+// rows or the BF16 operand planes and norm2[i] (EXPORT: the row times scale to
+// x, in FP64, instead).  Every thread calls; ends after a barrier.
+template <class T, bool SPLIT, int NC = -1, int LC = -1, bool EXPORT = false>
 __device__ __forceinline__ void ps_body(int N_, int L_, int S, int KC, int64_t Dq, int64_t i, const T* cs, T* stage,
                         const int* key_ab, const int* tri, T* __restrict__ p,
                         unsigned short* __restrict__ p_hi, unsigned short* __restrict__ p_lo,
-                        double* __restrict__ norm2) {
+                        double* __restrict__ norm2, double* __restrict__ x = nullptr, double scale = 1.0) {
   // NC, LC: N and L fixed at compile time (the LDS offsets of a tile's rows
   // and stage entries become immediates), or -1 for the runtime values
   const int N = NC >= 0 ? NC : N_, L = LC >= 0 ? LC : L_;
@@ -779,6 +779,9 @@ __device__ __forceinline__ void ps_body(int N_, int L_, int S, int KC, int64_t D
           p_lo[ob + o] = __builtin_bit_cast(unsigned short, (__bf16)(float(v) - (float)h));
         }
       }
+    } else if constexpr (EXPORT) {
+      double* xk = x + int64_t(k0) * KB;
+      for (int o = threadIdx.x; o < kc * KB; o += kThreads) xk[o] = double(stage[o]) * scale;
     } else {
       const int64_t ob = pbase + int64_t(k0) * KB;
       for (int o = threadIdx.x; o < kc * KB; o += kThreads) {
@@ -797,6 +800,7 @@ __device__ __forceinline__ void ps_body(int N_, int L_, int S, int KC, int64_t D
       p_lo[i * Dq + o] = 0;
     }
   }
+  if (EXPORT) return;
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
@@ -838,6 +842,42 @@ __global__ __launch_bounds__(kThreads) void power_spectrum_kernel(int N_, int L_
   ps_tables<SPLIT>(N, S, key_ab, tri);
   __syncthreads();
   ps_body<T, SPLIT, NC, LC>(N, L, S, KC, Dq, i, cs, stage, key_ab, tri, p, p_hi, p_lo, norm2);
+}
+
+// The FP32 power spectrum of centre rows[r] (rows null: r) as row r of the
+// exported features: formed again from the expansion and written normalised
+// (norm2 of the operand planes' pass) straight to the caller's FP64 rows.
+// Memory bound: 413 us for 37724 centres of 4 species, n_max 8, l_max 6
+// (1.35 GB written); through FP32 rows, a normalising pass and a copy the same
+// took 1640 us.
+template <class T>
+__global__ __launch_bounds__(kThreads) void power_spectrum_export_kernel(int N, int L, int S, int KC,
+                                                                         const T* __restrict__ c,
+                                                                         const double* __restrict__ norm2,
+                                                                         int normalize,
+                                                                         const int64_t* __restrict__ rows,
+                                                                         double* __restrict__ x) {
+  const int64_t i = rows ? rows[blockIdx.x] : int64_t(blockIdx.x);
+  const int L1 = L + 1, LL = L1 * L1, B = N * LL, LS = LL | 1;
+  const int K = S * (S + 1) / 2, KB = N * N * L1;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  T* cs = reinterpret_cast<T*>(smem_raw);  // as in power_spectrum_kernel
+  T* stage = cs + align_up(size_t(S * N + 3) * LS, 4);
+  int* key_ab = reinterpret_cast<int*>(stage + KC * KB);
+  int* tri = key_ab + K;
+  const T* ci = c + i * int64_t(S) * B;
+  const FastDiv fLL = fast_div(LL);
+  for (int e = threadIdx.x; e < S * B; e += kThreads) {
+    const int row = e / fLL;
+    cs[row * LS + (e - row * LL)] = ci[e];
+  }
+  for (int e = threadIdx.x; e < 3 * LS; e += kThreads) cs[S * N * LS + e] = T(0);
+  ps_tables<false>(N, S, key_ab, tri);
+  __syncthreads();
+  const double n2 = norm2[i];
+  ps_body<T, false, -1, -1, true>(N, L, S, KC, 0, i, cs, stage, key_ab, tri, nullptr, nullptr, nullptr, nullptr,
+                                  x + int64_t(blockIdx.x) * (int64_t(K) * KB),
+                                  normalize && n2 > 0 ? 1.0 / sqrt(n2) : 1.0);
 }
 
 // ---------------------------------------------------------------------------
@@ -2937,19 +2977,26 @@ void launch_expansion(const RadialDev& rad, int S, const PairView& pv, T* c,
     throw InvalidArgument("max_radial x (max_angular+1)^2 too large (> 7168)");
 }
 
+// LDS of the power spectrum and the keys it stages per pass
+template <class T>
+size_t power_spectrum_lds(const RadialDev& rad, int S, const SoapTiles& tiles, int* keys) {
+  const int K = S * (S + 1) / 2;
+  const size_t cbytes = sizeof(T) * align_up((size_t(S) * rad.N + 3) * (rad.LL | 1), 4);
+  const size_t kb = sizeof(T) * size_t(rad.N) * rad.N * rad.L1;
+  int KC = cbytes + kb < kPsBudget ? int((kPsBudget - cbytes) / kb) : 1;
+  if (tiles.kc > 0) KC = tiles.kc;
+  *keys = KC = std::max(1, std::min(KC, K));
+  return cbytes + size_t(KC) * kb + sizeof(int) * size_t(K + rad.N * (rad.N + 1) / 2);
+}
+
 template <class T>
 void launch_power_spectrum_impl(const RadialDev& rad, int S, int64_t n, const T* c, T* p,
                                 unsigned short* p_hi, unsigned short* p_lo, double* norm2,
                                 hipStream_t stream, const SoapTiles& tiles) {
   if (n == 0) return;
-  const int K = S * (S + 1) / 2;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
-  const size_t cbytes = sizeof(T) * align_up((size_t(S) * rad.N + 3) * (rad.LL | 1), 4);
-  const size_t kb = sizeof(T) * size_t(rad.N) * rad.N * rad.L1;
-  int KC = cbytes + kb < kPsBudget ? int((kPsBudget - cbytes) / kb) : 1;
-  if (tiles.kc > 0) KC = tiles.kc;
-  KC = std::max(1, std::min(KC, K));
-  const size_t smem = cbytes + size_t(KC) * kb + sizeof(int) * size_t(K + rad.N * (rad.N + 1) / 2);
+  int KC = 0;
+  const size_t smem = power_spectrum_lds<T>(rad, S, tiles, &KC);
   // the benchmark shape (n_max 12, l_max 9) with its sizes fixed at compile time
   constexpr bool kFixedShape = true;
   if (p_hi && kFixedShape && rad.N == 12 && rad.L == 9) {
@@ -3073,6 +3120,20 @@ void launch_power_spectrum_split(const RadialDev& rad, int S, int64_t n, const f
                                  unsigned short* p_hi, unsigned short* p_lo, double* norm2,
                                  hipStream_t stream, const SoapTiles& tiles) {
   launch_power_spectrum_impl<float>(rad, S, n, c, nullptr, p_hi, p_lo, norm2, stream, tiles);
+}
+
+void launch_power_spectrum_export(const RadialDev& rad, int S, int64_t n, const float* c, const double* norm2,
+                                  bool normalize, const int64_t* rows, double* x, hipStream_t stream,
+                                  const SoapTiles& tiles) {
+  if (n == 0) return;
+  if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
+  int KC = 0;
+  const size_t smem = power_spectrum_lds<float>(rad, S, tiles, &KC);
+  auto kern = power_spectrum_export_kernel<float>;
+  allow_lds(kern, smem);
+  hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, rad.N, rad.L, S, KC, c, norm2,
+                     int(normalize), rows, x);
+  RGPU_LAUNCH_CHECK();
 }
 
 template <class T>

@@ -8,6 +8,7 @@ import json
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from conftest import oracle_backward, ps_rel, soap_hypers
@@ -246,3 +247,30 @@ def test_knm_gradient_columns(species, atoms, N, L, spline, normalize, zeta, poi
         g, s = ctx.features_backward(scale[:, None] * vals[m])
         ref = np.concatenate([g.ravel(), s.ravel()])
         assert np.abs(out[:, m] - ref).max() <= 1e-10 * max(np.abs(out).max(), np.abs(ref).max())
+
+
+@pytest.mark.parametrize("prec", [_capi.FP64, _capi.MIXED])
+@pytest.mark.parametrize("n_species,N,L,normalize", [(1, 3, 0, True), (3, 5, 4, False), (4, 12, 9, True)])
+def test_features_into_device_rows(prec, n_species, N, L, normalize):
+    """Features written straight into a caller's device rows, with and without
+    a centre mask, against the host copy: the same values; mixed rows within FP32 rounding of the FP64 ones."""
+    sts = periodic_box(41, 0.05, tuple(range(1, n_species + 1)), d_min=1.0, seed=97)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=normalize)
+    off, pos, num, cells, pbc = pack(sts)
+    mask = np.random.default_rng(98).random(len(num)) < 0.4
+    full = None
+    for m in (None, mask):
+        ctx = _capi.Context(json.dumps(hp))
+        ctx.set_structures(off, pos, num, cells, pbc, sorted(set(num.tolist())), centre_mask=m)
+        X64, _ = ctx.features()
+        ctx.set_precision(prec)
+        X, _ = ctx.features()
+        rows = torch.full(X.shape, 7.0, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        ctx.features(out=rows)
+        assert np.array_equal(rows.cpu().numpy(), X)
+        assert np.abs(X - X64).max() <= (0 if prec == _capi.FP64 else 1e-5) * np.abs(X64).max()
+        if m is None:
+            full = X
+        else:
+            assert np.abs(X - full[mask]).max() <= 1e-6 * np.abs(full).max()
