@@ -2695,9 +2695,12 @@ __global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t lds,
 }
 
 // LDS per workgroup: the forward and the power spectrum stay small enough
-// for several workgroups per CU; the adjoint may use more.
+// for several workgroups per CU; the adjoint may use more.  The power
+// spectrum's 32 KB put five on a CU; more keys per pass in 48 KB, three: 8192
+// centres of 4 species (n_max 12, l_max 9) 339 us, with 40 KB 300, 32 KB 287,
+// 24 KB 297 us; 3 species 163, 133, 121, 132 us.
 constexpr size_t kFwdBudget = 32 * 1024;
-constexpr size_t kPsBudget = 48 * 1024;
+constexpr size_t kPsBudget = 32 * 1024;
 constexpr size_t kAdjBudget = 64 * 1024;
 constexpr size_t kResidentBudget = 52 * 1024;  // three workgroups per CU
 
