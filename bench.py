@@ -263,9 +263,9 @@ TRAFFIC_FILE = "profiles/hbm_traffic_periodic_box_8192.md"
 SQ_FILE = "profiles/sq_counters_periodic_box_8192.md"
 # kernels of the headline step (the packed layout always takes the
 # direct-to-LDS GEMMs; the adjoint kernel is the autotuner's choice)
-GEMM_KERNEL = "bf16x3_gemm_dma<0, 128, 2>"
-FORCE_GEMM_KERNEL = "bf16x3_gemm_dma<1, 128, 2>"
-EXPANSION_KERNEL = "expansion_kernel<float, 5, false, 12, 9>"
+GEMM_KERNEL = "bf16x3_gemm_dma<0, 128, 128>"
+FORCE_GEMM_KERNEL = "bf16x3_gemm_dma<1, 128, 128>"
+EXPANSION_KERNEL = "expansion_wave_kernel<float, 12, 64>"
 PS_KERNEL = "power_spectrum_kernel<float, true, 12, 9>"
 ADJOINT_KERNELS = {0: ["adjoint_staged_kernel<false, 5>"], 1: ["adjoint_mfma_kernel<false, 12>"],
                    2: ["adjoint_tile_kernel<12, 9, 6, 1, 10, false, true>"],

@@ -53,4 +53,7 @@ struct NLGeom {
   int64_t ext0;         // first extended (atom or ghost) slot
 };
 
+// compute units of the current device
+int device_cu_count();
+
 }  // namespace rgpu

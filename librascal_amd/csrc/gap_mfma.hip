@@ -12,7 +12,8 @@
 // lo.hi) accumulated in FP32.
 //
 // Tiling: 256 threads (4 wavefronts, 2 x 2), block tile 128 x 128, K step 32;
-// each wavefront owns 64 x 64 = 2 x 2 MFMA tiles.  Two LDS stages (one
+// each wavefront owns 64 x 64 = 2 x 2 MFMA tiles (64 x 64 block tiles, one
+// MFMA tile a wavefront, where there are few).  Two LDS stages (one
 // barrier per K step), the next K step's global loads issued before the
 // MFMAs of the current one.  Every operand row is 16-byte aligned and every
 // K a multiple of 32: the packed feature rows are padded to that, and so are
@@ -41,6 +42,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
 constexpr int BM = 128, BN = 128, BK = 32, NT = 256;
+constexpr int kMinBN = 64;  // of the smaller tiles
 constexpr int kMaxProblems = 16;
 constexpr int kGroupM = 8;  // row panels per tile group
 
@@ -97,27 +99,27 @@ __device__ __forceinline__ T pow_int(T v, int n) {
   return r;
 }
 
-// Epilogue of a TBM x 128 block tile whose wavefronts form (TBM / 64) x 2
-// and own 64 x 64 = 2 x 2 MFMA tiles each; esum: LDS [2][TBM]
-template <int EPI, int TBM>
+// Epilogue of a TBM x TBN block tile whose wavefronts form 2 x 2 and own
+// WI x WJ MFMA tiles each; esum: LDS [2][TBM]
+template <int EPI, int TBM, int TBN, int WI, int WJ>
 __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Problem& P, int64_t r0,
-                                              int64_t c0, f32x16 (&acc)[2][2], double (*esum)[TBM]) {
+                                              int64_t c0, f32x16 (&acc)[WI][WJ], double (*esum)[TBM]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   // epilogue; element e = 4*g + q of a 32x32 tile sits at
   // row 8*g + 4*(lane/32) + q, column lane%32
   const int half = lane >> 5, fr = lane & 31;
   if (EPI == 0) {
-    double rowsum[2][16];
+    double rowsum[WI][16];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) rowsum[i][e] = 0.0;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < WI; ++i) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int rl = wm * 64 + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
+        const int rl = wm * 32 * WI + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
         const int64_t r = r0 + rl;
         if (r >= P.M) continue;
         const int centre = P.c_rows[r];
@@ -127,8 +129,8 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
           inv = n2 > 0 ? 1.0 / sqrt(n2) : 1.0;
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int64_t c = c0 + wn * 64 + j * 32 + fr;
+        for (int j = 0; j < WJ; ++j) {
+          const int64_t c = c0 + wn * 32 * WJ + j * 32 + fr;
           if (c >= P.N) {
             if (P.wth && c < P.ldw) P.wth[r * P.ldw + c] = P.wtl[r * P.ldw + c] = 0;
             continue;
@@ -148,7 +150,7 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
     }
     // reduce over the 32 columns held by the lanes of each half
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         double v = rowsum[i][e];
@@ -157,38 +159,43 @@ __device__ __forceinline__ void gemm_epilogue(const ProblemSet& ps, const Proble
       }
     if (fr == 0) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < WI; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          esum[wn][wm * 64 + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3)] = rowsum[i][e];
+          esum[wn][wm * 32 * WI + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3)] = rowsum[i][e];
     }
     __syncthreads();
     if (P.epart && tid < TBM) {
       const int64_t r = r0 + tid;
-      if (r < P.M) P.epart[(c0 / BN) * P.ldp + P.c_rows[r]] = esum[0][tid] + esum[1][tid];
+      if (r < P.M) P.epart[(c0 / TBN) * P.ldp + P.c_rows[r]] = esum[0][tid] + esum[1][tid];
     }
   } else {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < WI; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int64_t r = r0 + wm * 64 + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
+        const int64_t r = r0 + wm * 32 * WI + i * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
         if (r >= P.M) continue;
         float* g = P.G + int64_t(P.c_rows[r]) * P.ldg;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int64_t c = c0 + wn * 64 + j * 32 + fr;
+        for (int j = 0; j < WJ; ++j) {
+          const int64_t c = c0 + wn * 32 * WJ + j * 32 + fr;
           if (c < P.N) g[c] = acc[i][j][e];
         }
       }
   }
 }
 
-// s_waitcnt vmcnt(N), the other counters left alone (gfx9 encoding)
+// s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding)
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));
+}
+// (__syncthreads would wait for every load in flight)
+__device__ __forceinline__ void bare_barrier() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 // Direct-to-LDS variant (global_load_lds_dwordx4: the loads write LDS
@@ -205,21 +212,24 @@ __device__ __forceinline__ int dma_frag_slot(int rb, int c, int l) {
   return (2 * rb + ((l >> 4) & 1)) * 64 + 4 * r + ((2 * c + (l >> 5)) ^ dma_swz(r));
 }
 
-template <int TBM, int NS>
+// LDS stages; three and four were no faster with either tile
+constexpr int NS = 2;
+
+template <int TBM, int TBN>
 struct DmaLds {
   bf16x8 A[NS][2][TBM / 16 * 64];  // [stage][hi, lo][slot]
-  bf16x8 B[NS][2][BN / 16 * 64];
+  bf16x8 B[NS][2][TBN / 16 * 64];
   double esum[2][TBM];
 };
 
-// TBM x 128 block tile, TBM / 32 wavefronts, NS LDS stages with NS - 1 K
-// steps in flight; K % 32 == 0 and 16-byte aligned rows
-template <int EPI, int TBM, int NS>
+// TBM x TBN block tile of four wavefronts, NS LDS stages with NS - 1 K steps
+// in flight; K % 32 == 0 and 16-byte aligned rows
+template <int EPI, int TBM, int TBN>
 __device__ __forceinline__ void gemm_tile_dma(const ProblemSet& ps, const Problem& P, int64_t r0,
-                                              int64_t c0, DmaLds<TBM, NS>& sm) {
-  constexpr int W = TBM / 32;
-  constexpr int GA = TBM / 16 / W, GB = BN / 16 / W;  // groups per plane and wavefront
-  static_assert(GA * W * 16 == TBM && GB * W * 16 == BN, "group partition");
+                                              int64_t c0, DmaLds<TBM, TBN>& sm) {
+  constexpr int W = NT / 64, WI = TBM / 64, WJ = TBN / 64;  // MFMA tiles of a wavefront
+  constexpr int GA = TBM / 16 / W, GB = TBN / 16 / W;  // groups per plane and wavefront
+  static_assert(GA * W * 16 == TBM && GB * W * 16 == TBN, "group partition");
   constexpr int PER = 2 * (GA + GB);  // load instructions per wavefront and K step
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -260,34 +270,34 @@ __device__ __forceinline__ void gemm_tile_dma(const ProblemSet& ps, const Proble
     }
   };
 
-  f32x16 acc[2][2];
+  f32x16 acc[WI][WJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < WJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
   auto compute = [&](int s) {
 #pragma unroll
     for (int c = 0; c < BK / 16; ++c) {
-      bf16x8 ah[2], al[2], bh[2], bl[2];
+      bf16x8 ah[WI], al[WI], bh[WJ], bl[WJ];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int f = dma_frag_slot(wm * 2 + i, c, lane);
+      for (int i = 0; i < WI; ++i) {
+        const int f = dma_frag_slot(wm * WI + i, c, lane);
         ah[i] = sm.A[s][0][f];
         al[i] = sm.A[s][1][f];
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int f = dma_frag_slot(wn * 2 + j, c, lane);
+      for (int j = 0; j < WJ; ++j) {
+        const int f = dma_frag_slot(wn * WJ + j, c, lane);
         bh[j] = sm.B[s][0][f];
         bl[j] = sm.B[s][1][f];
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < WI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < WJ; ++j) {
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bh[j], acc[i][j], 0, 0, 0);
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[i], bl[j], acc[i][j], 0, 0, 0);
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[i], bh[j], acc[i][j], 0, 0, 0);
@@ -304,7 +314,7 @@ __device__ __forceinline__ void gemm_tile_dma(const ProblemSet& ps, const Proble
     // orders the previous step's fragment reads before the refill of its
     // stage
     wait_vmcnt<(NS - 2) * PER>();
-    __syncthreads();
+    bare_barrier();
     issue(s_fill, kt + NS - 1);
     compute(s_read);
     s_read = s_read + 1 == NS ? 0 : s_read + 1;
@@ -312,7 +322,7 @@ __device__ __forceinline__ void gemm_tile_dma(const ProblemSet& ps, const Proble
   }
   // no load may still write this workgroup's LDS when it exits
   wait_vmcnt<0>();
-  gemm_epilogue<EPI, TBM>(ps, P, r0, c0, acc, sm.esum);
+  gemm_epilogue<EPI, TBM, TBN, WI, WJ>(ps, P, r0, c0, acc, sm.esum);
 }
 
 // problem index and tile (row, column) of linear block bid.  Workgroups
@@ -341,14 +351,14 @@ __device__ __forceinline__ bool tile_of(const ProblemSet& ps, int* pi_out, int64
 }
 
 // EPI 0: GAP kernel epilogue, 1: store rows of G
-template <int EPI, int TBM, int NS>
-__global__ __launch_bounds__(TBM * 2, 512 / (TBM * 2)) void bf16x3_gemm_dma(ProblemSet ps) {
+template <int EPI, int TBM, int TBN>
+__global__ __launch_bounds__(NT, 2) void bf16x3_gemm_dma(ProblemSet ps) {
   int pi;
   int64_t tm, tn;
   if (!tile_of(ps, &pi, &tm, &tn)) return;
   const Problem& P = ps.p[pi];
-  __shared__ __align__(16) DmaLds<TBM, NS> sm;
-  gemm_tile_dma<EPI, TBM, NS>(ps, P, tm * TBM, tn * BN, sm);
+  __shared__ __align__(16) DmaLds<TBM, TBN> sm;
+  gemm_tile_dma<EPI, TBM, TBN>(ps, P, tm * TBM, tn * TBN, sm);
 }
 
 // Packed BF16 planes of the sparse points in both orientations: 32 points x
@@ -395,14 +405,14 @@ __global__ __launch_bounds__(NT) void split_sparse_kernel(const double* __restri
   }
 }
 
-// tile counts and first tiles of the set's problems for block rows bm
-int64_t layout_tiles(ProblemSet& ps, int bm) {
+// tile counts and first tiles of the set's problems for bm x bn tiles
+int64_t layout_tiles(ProblemSet& ps, int bm, int bn) {
   int64_t tiles = 0;
   for (int i = 0; i < ps.n; ++i) {
     Problem& P = ps.p[i];
     P.tile0 = tiles;
     P.tiles_m = int((P.M + bm - 1) / bm);
-    P.tiles_n = int((P.N + BN - 1) / BN);
+    P.tiles_n = int((P.N + bn - 1) / bn);
     tiles += int64_t(P.tiles_m) * P.tiles_n;
   }
   return tiles;
@@ -410,22 +420,31 @@ int64_t layout_tiles(ProblemSet& ps, int bm) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// columns per tile of the set's launch
 template <int EPI>
-void launch_set(ProblemSet& ps, hipStream_t stream) {
-  if (ps.n == 0) return;
+int launch_set(ProblemSet& ps, hipStream_t stream) {
+  if (ps.n == 0) return BN;
   for (int i = 0; i < ps.n; ++i) {
     const Problem& P = ps.p[i];
     if (P.K % BK != 0 || P.lda % 8 != 0 || P.ldb % 8 != 0 || !aligned16(P.Ahi) || !aligned16(P.Alo) ||
         !aligned16(P.Bhi) || !aligned16(P.Blo))
       throw InvalidArgument("internal: unaligned operands of the mixed GAP product");
   }
-  ps.total_tiles = layout_tiles(ps, BM);
-  if (ps.total_tiles == 0) return;
-  const unsigned grid = unsigned((ps.total_tiles + 7) / 8 * 8);  // whole rounds over the 8 XCDs
-  // 128 x 128 tiles; two stages of direct-to-LDS loads measured faster than
-  // three (with 256-row tiles)
-  hipLaunchKernelGGL((bf16x3_gemm_dma<EPI, BM, 2>), dim3(grid), dim3(NT), 0, stream, ps);
-  RGPU_LAUNCH_CHECK();
+  auto go = [&](auto kern, int bm, int bn) {
+    ps.total_tiles = layout_tiles(ps, bm, bn);
+    if (ps.total_tiles == 0) return bn;
+    const unsigned grid = unsigned((ps.total_tiles + 7) / 8 * 8);  // whole rounds over the 8 XCDs
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), 0, stream, ps);
+    RGPU_LAUNCH_CHECK();
+    return bn;
+  };
+  // Under three quarters of a 128 x 128 tile per CU, 64 x 64 tiles: a tile
+  // alone on its CU takes the same time however few there are (96 tiles, 60 K
+  // steps: 78 us, 48 us in small ones; 168 tiles, 208 K steps: 255 and
+  // 194 us), while with the chip full their extra operand traffic shows (512
+  // tiles, 363 K steps: 602 and 1035 us).
+  if (4 * layout_tiles(ps, BM, BN) <= 3 * int64_t(device_cu_count())) return go(bf16x3_gemm_dma<EPI, 64, 64>, 64, 64);
+  return go(bf16x3_gemm_dma<EPI, BM, BN>, BM, BN);
 }
 
 }  // namespace
@@ -493,7 +512,7 @@ void prepare_mixed_sparse(MixedSparse& ms, const double* T, int64_t M, int S, in
 
 int64_t gap_mixed_wt_stride(int64_t n_cols) { return (n_cols + BK - 1) / BK * BK; }
 
-int gap_mixed_energy_tiles(int64_t n_cols) { return int((n_cols + BN - 1) / BN); }
+int gap_mixed_energy_tiles(int64_t n_cols) { return int((n_cols + kMinBN - 1) / kMinBN); }
 
 void run_gap_mixed_kernel(const GapBlock<float>* blks, int n_blocks, const MixedSparse& ms,
                           SplitPlanes xs, double* energy, double* part, int64_t ld, const SplitPlanes* wts,
@@ -529,9 +548,10 @@ void run_gap_mixed_kernel(const GapBlock<float>* blks, int n_blocks, const Mixed
       ps.zeta = blk.zeta;
       et.rows[et.n] = blk.row_idx;
       et.m[et.n] = blk.n_rows;
-      et.tiles[et.n++] = gap_mixed_energy_tiles(blk.n_cols);
+      et.n++;
     }
-    launch_set<0>(ps, stream);
+    const int bn = launch_set<0>(ps, stream);
+    for (int i = 0; i < et.n; ++i) et.tiles[i] = int((ps.p[i].N + bn - 1) / bn);
     if (energy) launch_energy_tiles(et, part, ld, energy, stream);
   }
 }

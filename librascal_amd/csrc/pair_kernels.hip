@@ -706,23 +706,6 @@ void with_channels(int N, F&& f) {
 
 bool pair_kernels_apply(const RadialDev& rad) { return rad.use_spline && rad.L <= kMaxPairL && rad.N <= kMaxN; }
 
-namespace {
-
-int cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  RGPU_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= 64) throw RuntimeError("device index out of range");
-  if (!cached[dev]) {
-    int v = 0;
-    RGPU_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
-    cached[dev] = v;
-  }
-  return cached[dev];
-}
-
-}  // namespace
-
 template <class T>
 void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T* dc, double* centre_virial,
                         hipStream_t stream) {
@@ -743,7 +726,7 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
       RGPU_LAUNCH_CHECK();
     };
     // as many workgroups as are resident (registers: 4 FP32, 3 FP64 per CU)
-    const int64_t resident = int64_t(cu_count()) * (sizeof(T) == 4 ? 4 : 3);
+    const int64_t resident = int64_t(device_cu_count()) * (sizeof(T) == 4 ? 4 : 3);
     auto by_units = [&](auto w) {
       constexpr int W = decltype(w)::value;
       const int64_t blocks = W > 1 ? n : std::min((n + kWaves - 1) / kWaves, resident);
@@ -771,7 +754,7 @@ void launch_expansion_wave(const RadialDev& rad, int S, const PairView& pv, T* c
     constexpr int NT = decltype(nt)::value;
     const size_t smem = sizeof(T) * size_t(4 * rad.LL) + kWaves * expansion_wave_lds<T, NT>(rad.L1);
     const int64_t blocks =
-        std::min((n + kWaves - 1) / kWaves, int64_t(cu_count()) * (sizeof(T) == 4 ? 5 : 4));
+        std::min((n + kWaves - 1) / kWaves, int64_t(device_cu_count()) * (sizeof(T) == 4 ? 5 : 4));
     auto go = [&](auto kern) {
       allow_lds(kern, smem);
       hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), smem, stream, rad, S, pv, c, keymask);

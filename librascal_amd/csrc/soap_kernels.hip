@@ -3026,19 +3026,6 @@ void launch_power_spectrum_impl(const RadialDev& rad, int S, int64_t n, const T*
   RGPU_LAUNCH_CHECK();
 }
 
-int device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  RGPU_HIP(hipGetDevice(&dev));
-  if (dev < 0 || dev >= 64) throw RuntimeError("device index out of range");
-  if (!cached[dev]) {
-    int v = 0;
-    RGPU_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
-    cached[dev] = v;
-  }
-  return cached[dev];
-}
-
 template <class T, int KPT, bool DIRECT, bool SPLIT, bool PS>
 void launch_fused_t(const RadialDev& rad, int S, const PairView& pv, T* c, unsigned long long* keymask,
                     T* p, unsigned short* p_hi, unsigned short* p_lo, double* norm2, hipStream_t stream,
@@ -3664,6 +3651,19 @@ void launch_knm_stress(const PairView& pv, int species, int64_t n_sets, const do
   hipLaunchKernelGGL(knm_stress_kernel, dim3(unsigned(n_struct), unsigned(n_sets)), dim3(kThreads), 0, stream, pv,
                      species, centre_virial, atom_off, inv_vol, cols, ld, out);
   RGPU_LAUNCH_CHECK();
+}
+
+int device_cu_count() {
+  static int cached[64] = {0};
+  int dev = 0;
+  RGPU_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= 64) throw RuntimeError("device index out of range");
+  if (!cached[dev]) {
+    int v = 0;
+    RGPU_HIP(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev));
+    cached[dev] = v;
+  }
+  return cached[dev];
 }
 
 }  // namespace rgpu

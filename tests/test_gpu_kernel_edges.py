@@ -274,3 +274,24 @@ def test_features_into_device_rows(prec, n_species, N, L, normalize):
             full = X
         else:
             assert np.abs(X - full[mask]).max() <= 1e-6 * np.abs(full).max()
+
+
+@pytest.mark.parametrize("atoms,points", [(66, 65), (520, 300), (2900, 1030)])
+def test_mixed_product_tiles(atoms, points):
+    """The mixed products in 64 x 64 tiles and, from three quarters of a
+    128 x 128 tile per CU on, in those, with remainders of both: energies and
+    forces against the FP64 path, and the energy against the K_NM of the same
+    context."""
+    sts = periodic_box(atoms, 0.05, (1, 8), d_min=1.0, seed=101)
+    ctx, num = _context(soap_hypers(rc=4.0, sw=0.5, sigma=0.5, N=9, L=6, spline=1e-8), sts)
+    rng = np.random.default_rng(102)
+    counts = {z: min(points, int((num == z).sum())) for z in (1, 8)}
+    spec, vals, w = _points(ctx, num, counts, rng)
+    ctx.set_sparse_points(2, spec, vals, w)
+    e, g, s = ctx.gap_predict()
+    ctx.set_precision(_capi.MIXED)
+    em, gm, sm = ctx.gap_predict()
+    k = ctx.gap_knm("Structure")
+    assert abs(em[0] - k[0] @ w) <= 1e-4 * (np.abs(k[0]) @ np.abs(w))
+    assert abs(em[0] - e[0]) <= 1e-4 * (np.abs(k[0]) @ np.abs(w))
+    assert np.sqrt(np.mean((gm - g) ** 2)) <= 1e-4 * np.sqrt(np.mean(g ** 2))
