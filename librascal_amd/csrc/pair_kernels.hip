@@ -378,10 +378,11 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
   for (int64_t i0 = int64_t(blockIdx.x) * per; i0 < pv.n_centres; i0 += int64_t(gridDim.x) * per) {
     const int64_t v = i0 + wave / W;
     if (W == 1 && v >= pv.n_centres) break;
-    const PairEntry entry = pair_entry(pv, v);
+    const bool live = v < pv.n_centres;  // (W > 1: every wavefront reaches the barriers)
+    const PairEntry entry = pair_entry(pv, live ? v : pv.n_centres - 1);
     const int64_t i = entry.centre;
     const int64_t p0 = pv.centre_off[i] + 1;  // the self pair contributes nothing
-    const int np = int(pv.centre_off[i + 1] - p0);
+    const int np = live ? int(pv.centre_off[i + 1] - p0) : 0;
     const T* dci = dcg + v * int64_t(S) * LL * N;
     const V4* table = Spl4<T>::table(rad);
     for (int c0 = 0; c0 < np; c0 += 64 * W) {
@@ -520,7 +521,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
       __syncthreads();
     else
       wave_sync();
-    if (w == 0 && lane < 9) {
+    if (w == 0 && live && lane < 9) {
       double t = 0;
 #pragma unroll
       for (int k = 0; k < W; ++k) t += red[wave + k][lane];
@@ -712,11 +713,11 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
   const int64_t n = pv.n_centres;
   if (n == 0) return;
   const int units = rad.L1 * (rad.L1 + 1) / 2;
-  // One wavefront per centre once there are about as many as are resident;
-  // below that its serial chain over the pairs shows, and four share a
-  // centre's (FP64, four against one: 64 centres 17 against 31 us, 1024
-  // centres 57 against 52 us, 4096 centres 318 against 166 us).
-  const bool wide = n < 1024;
+  // As many wavefronts per centre as keep the chip filled: fewer centres share
+  // a centre's pairs, whose serial chain shows (one, two, four wavefronts:
+  // 64 centres 31, 23, 18 us; 1024 centres 52, 42, 57; 1331 centres in FP32
+  // 47, 38, 51; 4096 centres 167, 220, 319 us).
+  const int wide = n < 512 ? 4 : (n < 2048 ? 2 : 1);
   with_channels(rad.N, [&](auto nt) {
     constexpr int NT = decltype(nt)::value;
     const size_t smem = sizeof(T) * size_t(4 * rad.LL) + kWaves * force_wave_lds<T, NT>(rad.L1);
@@ -729,7 +730,7 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
     const int64_t resident = int64_t(device_cu_count()) * (sizeof(T) == 4 ? 4 : 3);
     auto by_units = [&](auto w) {
       constexpr int W = decltype(w)::value;
-      const int64_t blocks = W > 1 ? n : std::min((n + kWaves - 1) / kWaves, resident);
+      const int64_t blocks = W > 1 ? (n * W + kWaves - 1) / kWaves : std::min((n + kWaves - 1) / kWaves, resident);
       if (units <= 16)
         go(pair_force_kernel<T, NT, 16, W>, blocks);
       else if (units <= 32)
@@ -737,8 +738,10 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
       else
         go(pair_force_kernel<T, NT, 64, W>, blocks);
     };
-    if (wide)
-      by_units(std::integral_constant<int, kWaves>{});
+    if (wide == 4)
+      by_units(std::integral_constant<int, 4>{});
+    else if (wide == 2)
+      by_units(std::integral_constant<int, 2>{});
     else
       by_units(std::integral_constant<int, 1>{});
   });

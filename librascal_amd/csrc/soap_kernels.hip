@@ -1235,13 +1235,14 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(int64_t D, int64_
 //     for a > b, w_ab = sqrt 2 for a != b); after the last chunk written
 //     over c;
 //  3. the pair phase, its batches over the g region.
-// UPT = units per thread (ceil(S * ceil(N/4) * LL / 256)).
-template <bool DIRECT, int UPT>
+// UPT = units per thread (ceil(S * ceil(N/4) * LL / 256)).  Without PAIRS
+// dL/dc [S][LL][N] goes to dcg + i S LL N for launch_pair_forces.
+template <bool DIRECT, int UPT, bool PAIRS>
 __global__ __launch_bounds__(kThreads) void adjoint_staged_kernel(
     RadialDev rad, int S, int PB, int KCH, PairView pv, const float* __restrict__ c,
     const unsigned short* __restrict__ p_hi, const unsigned short* __restrict__ p_lo,
     const double* __restrict__ norm2, int normalize, const double* __restrict__ xg, double xg_scale,
-    const float* __restrict__ G, double* __restrict__ centre_virial) {
+    const float* __restrict__ G, double* __restrict__ centre_virial, float* __restrict__ dcg) {
   typedef float T;
   typedef typename Vec4<T>::type V4;
   const int64_t i = blockIdx.x;
@@ -1253,13 +1254,13 @@ __global__ __launch_bounds__(kThreads) void adjoint_staged_kernel(
   extern __shared__ __align__(64) unsigned char smem_raw[];
   T* yc = reinterpret_cast<T*>(smem_raw);
   // c [S][N][LL], then dL/dc [S][LL][N]
-  T* cd = reinterpret_cast<T*>(smem_raw + ylm_table_bytes<T>(L1));
+  T* cd = reinterpret_cast<T*>(smem_raw + (PAIRS ? ylm_table_bytes<T>(L1) : 0));
   unsigned char* region = reinterpret_cast<unsigned char*>(cd) + align_up(sizeof(T) * E, 64);
   T* gl = reinterpret_cast<T*>(region);
   __shared__ double red[kWaves];
   __shared__ double sh_ab[2];
   __shared__ int tri[kMaxN * (kMaxN + 1) / 2];  // n1 << 8 | n2 of the packed diagonal pairs
-  load_ylm_table<T>(rad, yc);
+  if constexpr (PAIRS) load_ylm_table<T>(rad, yc);
   for (int e = tid; e < E; e += kThreads) cd[e] = c[i * int64_t(E) + e];
   for (int t = tid; t < N * (N + 1) / 2; t += kThreads) {
     int n1, n2;
@@ -1400,7 +1401,8 @@ __global__ __launch_bounds__(kThreads) void adjoint_staged_kernel(
       }
     }
   }
-  __syncthreads();  // every unit has read c
+  if constexpr (PAIRS) __syncthreads();  // every unit has read c
+  T* dc = PAIRS ? cd : dcg + i * int64_t(E);
 #pragma unroll
   for (int k = 0; k < UPT; ++k) {
     const int u = tid + kThreads * k;
@@ -1410,13 +1412,14 @@ __global__ __launch_bounds__(kThreads) void adjoint_staged_kernel(
       const T f = T(1) / sqrt(T(2 * l_of_lm(lm) + 1));
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (n0 + v < N) cd[a * B + lm * N + n0 + v] = f * acc[k][v];
+        if (n0 + v < N) dc[a * B + lm * N + n0 + v] = f * acc[k][v];
     }
   }
-  __syncthreads();
-
-  // 3. pairs; the batches reuse the g region
-  adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, cd, region, i, centre_virial);
+  if constexpr (PAIRS) {
+    __syncthreads();
+    // 3. pairs; the batches reuse the g region
+    adjoint_pairs<T, DIRECT>(rad, S, PB, pv, yc, cd, region, i, centre_virial);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2902,35 +2905,51 @@ void launch_adjoint_f32(const RadialDev& rad, int S, const PairView& pv, const f
     return;
   }
   // mixed path: packed dL/dX and BF16 planes of p, staged in LDS KCH key
-  // blocks at a time beside c
+  // blocks at a time beside c; the pair phase by wavefronts where it applies
+  // (1331 centres, 2 species, n_max 10, l_max 8: 94 us in one kernel, 20 + 38
+  // us in two)
   if (!p_hi || !p_lo) throw InvalidArgument("the FP32 adjoint takes the split invariants");
   const size_t kbytes = sizeof(T) * size_t(N) * N * L1;
   const int upt = (S * ((N + 3) / 4) * LL + kThreads - 1) / kThreads;
   if (upt > 8) throw InvalidArgument("max_radial x (max_angular+1)^2 too large for the FP32 adjoint");
+  const bool pairs = DIRECT || !work || !pair_kernels_apply(rad);
+  const size_t fixed = (pairs ? yt : 0) + blk;
   int KCH = tiles.keys_adj > 0 ? std::min(tiles.keys_adj, K) : K;
   if (tiles.keys_adj <= 0)
-    while (KCH > 1 && yt + blk + align_up(KCH * kbytes, 64) > kResidentBudget) --KCH;
+    while (KCH > 1 && fixed + align_up(KCH * kbytes, 64) > kResidentBudget) --KCH;
   const size_t dbytes = align_up(KCH * kbytes, 64);
   int PB = tiles.pb_adj > 0 ? std::min(tiles.pb_adj, 64) : 16;
   if (tiles.pb_adj <= 0)
     while (PB > 1 && pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true) > dbytes) --PB;
-  const size_t smem = yt + blk + std::max(dbytes, pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true));
+  const size_t smem =
+      fixed + (pairs ? std::max(dbytes, pair_batch_bytes(PB, LL, F, sizeof(T), DIRECT, true)) : dbytes);
   auto go = [&](auto kern) {
     allow_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(unsigned(pv.n_centres)), dim3(kThreads), smem, stream, rad, S, PB, KCH,
-                       pv, c, p_hi, p_lo, norm2, int(normalize), xg, xg_scale, G, centre_virial);
+                       pv, c, p_hi, p_lo, norm2, int(normalize), xg, xg_scale, G, centre_virial, work);
+    RGPU_LAUNCH_CHECK();
   };
-  if (upt <= 2)
-    go(adjoint_staged_kernel<DIRECT, 2>);
-  else if (upt <= 3)
-    go(adjoint_staged_kernel<DIRECT, 3>);
-  else if (upt <= 4)
-    go(adjoint_staged_kernel<DIRECT, 4>);
-  else if (upt <= 5)
-    go(adjoint_staged_kernel<DIRECT, 5>);
-  else
-    go(adjoint_staged_kernel<DIRECT, 8>);
-  RGPU_LAUNCH_CHECK();
+  auto by_units = [&](auto with_pairs) {
+    constexpr bool P = decltype(with_pairs)::value;
+    if (upt <= 2)
+      go(adjoint_staged_kernel<DIRECT, 2, P>);
+    else if (upt <= 3)
+      go(adjoint_staged_kernel<DIRECT, 3, P>);
+    else if (upt <= 4)
+      go(adjoint_staged_kernel<DIRECT, 4, P>);
+    else if (upt <= 5)
+      go(adjoint_staged_kernel<DIRECT, 5, P>);
+    else
+      go(adjoint_staged_kernel<DIRECT, 8, P>);
+  };
+  if constexpr (!DIRECT) {
+    if (!pairs) {
+      by_units(std::false_type{});
+      launch_pair_forces<float>(rad, S, pv, work, centre_virial, stream);
+      return;
+    }
+  }
+  by_units(std::true_type{});
 }
 
 }  // namespace

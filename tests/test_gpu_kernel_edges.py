@@ -166,8 +166,8 @@ def test_pair_forces_by_wavefronts(N, L):
     """The pair phase at the edges of its channel counts (4, 6, .. 24) and of
     the orders side by side (l_max 4, 6, 9; past 9 the general kernel), with
     more than 64 neighbours per centre: one structure, whose centres take four
-    wavefronts each, against the oracle, and enough copies of it that a
-    wavefront takes whole centres against the one.  More functions than 16 use
+    wavefronts each, against the oracle, and enough copies of it that centres
+    take two or one against the one.  More functions than 16 use
     the DVR basis and the exported gradient rows: the overlap of so many GTOs
     is singular to rounding, and their orthonormal basis not determined."""
     sts = periodic_box(13, 0.08, (1, 8), d_min=1.0, seed=91)
@@ -184,12 +184,18 @@ def test_pair_forces_by_wavefronts(N, L):
         g_ref, s_ref = oracle_backward(O.Calculator(hp), O.BatchData(sts), G)
     assert np.abs(g - g_ref).max() <= 1e-10 * np.abs(g_ref).max()
     assert np.abs(s - s_ref).max() <= 1e-10 * np.abs(s_ref).max()
-    copies = 2048 // 13 + 1
-    many, _ = _context(hp, sts * copies)
-    gm, sm = many.features_backward(np.tile(G, (copies, 1)))
-    assert np.abs(gm.reshape(copies, *g.shape) - g).max() <= 1e-10 * np.abs(g).max()
-    assert np.abs(sm.reshape(copies, *s.shape) - s).max() <= 1e-10 * np.abs(s).max()
-    assert len(set(map(bytes, gm.reshape(copies, *g.shape)))) == 1
+    for copies in (512 // 13 + 2, 2048 // 13 + 1):
+        many, _ = _context(hp, sts * copies)
+        gm, sm = many.features_backward(np.tile(G, (copies, 1)))
+        assert np.abs(gm.reshape(copies, *g.shape) - g).max() <= 1e-10 * np.abs(g).max()
+        assert np.abs(sm.reshape(copies, *s.shape) - s).max() <= 1e-10 * np.abs(s).max()
+        assert len(set(map(bytes, gm.reshape(copies, *g.shape)))) == 1
+    if L < 10 and N < 17:
+        # the mixed path's key contraction before the same phase
+        ctx.set_precision(_capi.MIXED)
+        gm, _ = ctx.features_backward(G)
+        assert np.sqrt(np.mean((gm - g) ** 2)) <= 1e-4 * np.sqrt(np.mean(g ** 2))
+
 
 
 @pytest.mark.parametrize("N,L", [(1, 0), (4, 4), (5, 5), (7, 7), (11, 9), (13, 4), (24, 2), (8, 10)])
