@@ -141,7 +141,7 @@ struct Context {
   DeviceBuffer<int> d_rows;
 
   // scratch
-  DeviceBuffer<double> e_centre, grad, cvir, tmp64, out64, knm_grad, knm_pair, knm_centre, knm_virial;
+  DeviceBuffer<double> e_centre, grad, cvir, tmp64, out64, knm_grad, knm_pair, knm_centre, knm_virial, knm_dp;
   DeviceBuffer<int64_t> d_sp_order;
   DeviceBuffer<double> e_part;  // energy GEMM partials per column tile and centre
   PinnedBuffer<double> out_stage;  // page-locked staging of a prediction's outputs
@@ -2165,6 +2165,13 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
       launch_sym_pack(S, N, L1, M, gf, nullptr, gs, c.stream);
       T = gs;
     }
+    // the part of dL/dc along p, which the normalisation projects out
+    const double* dp = nullptr;
+    if (c.hp.normalize) {
+      double* e = c.knm_dp.reserve(size_t(n * E));
+      launch_sym_contract(S, N, L1, n, c.c64.get(), c.p64.get(), e, c.stream);
+      dp = e;
+    }
     // column m (species-sorted): dL/dX_i = zeta d_im^(zeta-1) T_m for the
     // centres of m's species, through the adjoint; rows written in the
     // caller's sparse-point order.  As many columns at a time as fit the
@@ -2195,8 +2202,7 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
         if (ni > 0) {
           bpv.n_centres = q * ni;
           const SymSets sets{bpv.ids, ni, d + m0, M, c.zeta};
-          launch_sym_contract_sets(S, N, L1, q, sets, c.c64.get(), c.hp.normalize ? c.p64.get() : nullptr,
-                                   c.norm2.get(), T + m0 * lds, dc, c.stream);
+          launch_sym_contract_sets(S, N, L1, q, sets, c.c64.get(), c.norm2.get(), dp, T + m0 * lds, dc, c.stream);
           launch_pair_phase(c, bpv, dc, cv);
         }
         launch_knm_force_gather(bpv, rl, s, q, cols, M, o, c.stream);

@@ -39,7 +39,8 @@ void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const
                          hipStream_t stream);
 // dL/dc [n_sets][n_ids] of the kernel derivatives of sparse points T (symmetric
 // packed rows, one per set) at the centres ids: dL/dX_i = zeta d^(zeta - 1) T_q
-// with d = X_i . T_q = dot[i ld_dot + q], X = p / |p| (p null: X = p)
+// with d = X_i . T_q = dot[i ld_dot + q], X = p / |p|; E: dL/dc of dL/dp = p for
+// every centre of the batch (launch_sym_contract; null: X = p)
 struct SymSets {
   const int* ids = nullptr;
   int64_t n_ids = 1;
@@ -48,7 +49,7 @@ struct SymSets {
   int zeta = 1;
 };
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
-                              const double* p, const double* norm2, const double* T, double* dc, hipStream_t stream);
+                              const double* norm2, const double* E, const double* T, double* dc, hipStream_t stream);
 // The same from dL/dX in full rows [n][K N^2 (L+1)] (keys a <= b): X = p / |p|
 // with p in symmetric packed rows and xg[i] = X . dL/dX (null: summed here),
 // or X = p (p null).  work: packed rows where they are needed

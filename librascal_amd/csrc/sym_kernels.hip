@@ -129,14 +129,12 @@ __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int 
 // L+1 apart, but the workgroup's wavefronts take them channel after channel
 // from the same cached lines, which costs less than packing the rows first
 // (4689 centres, 4 species, n_max 8, l_max 6: 244 us against 183 + 139).  kGather: as
-// kDp, the entries gathered from memory (R too large for the LDS).  kRank,
-// kRankGather: dL/dX of centre ids[v % n_ids] the sparse point of set
-// v / n_ids times zeta d^(zeta - 1).
+// kDp, the entries gathered from memory (R too large for the LDS).
 //
 // Bound by the memory it streams and the latency of the scalar loads: 4096
 // centres, 4 species, n_max 12, l_max 9: 0.31 ms for 0.93 GB, where the key
 // contraction of the fused FP64 adjoint it replaced took about 1.0 ms.
-enum { kDp, kDx, kGather, kRank, kRankGather };
+enum { kDp, kDx, kGather };
 
 template <int LM, int kForm>
 __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, int L, int64_t ld,
@@ -145,10 +143,8 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
                                                                 const double* __restrict__ norm2,
                                                                 const double* __restrict__ xg,
                                                                 const double* __restrict__ G,
-                                                                SymSets sets, double* __restrict__ dc) {
-  constexpr bool rank = kForm == kRank || kForm == kRankGather, gather = kForm == kGather || kForm == kRankGather;
-  const int64_t v = blockIdx.x, set = rank ? v / sets.n_ids : 0;
-  const int64_t i = rank ? int64_t(sets.ids[v - set * sets.n_ids]) : v;
+                                                                double* __restrict__ dc) {
+  const int64_t i = blockIdx.x;
   const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), S = R / N, KB = N * N * L1;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double rt2 = 1.41421356237309504880;
@@ -158,7 +154,7 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
   // its mirror (both the same between species)
   int2* tab = reinterpret_cast<int2*>(reinterpret_cast<double*>(smem_raw) + kWaves * TRI);
   __shared__ double red[kWaves];
-  const double* Gi = G + (rank ? set : i) * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
+  const double* Gi = G + i * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
   const double* pi = p ? p + i * ld : nullptr;
   // packed entry t of channel l of G
   auto entry = [&](int l, int t) -> double {
@@ -205,35 +201,21 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
       }
     }
   }
-  if constexpr (rank) {
-    // dL/dX = zeta d^(zeta - 1) T, d = X . T
-    const double d = sets.dot[i * sets.ld_dot + set];
-    double a = double(sets.zeta);
-    for (int k = 1; k < sets.zeta; ++k) a *= d;
-    alpha = a;
-    if (p) {
-      const double n2 = norm2[i];
-      if (n2 > 0) {
-        alpha = a / sqrt(n2);
-        beta = a * d / n2;
-      }
-    }
-  }
   const double* ci = c + i * int64_t(R) * LL;
   for (int k = 0; k * kWaves <= L; ++k) {
     const int u = wave_unit(L1, kWaves, wave, k), lk = L - u;
     if (u < 0) continue;
     const double* g = Gi + lk * TRI;
-    if constexpr (!gather) {
+    if constexpr (kForm != kGather) {
       wave_sync();  // the previous channel is read
       // (many loads in flight: the runs come from memory)
-      if ((kForm == kDx || kForm == kRank) && p) {
+      if (kForm == kDx && p) {
         const double* q = pi + lk * TRI;
 #pragma unroll 8
         for (int t = lane; t < TRI; t += 64) W[t] = alpha * entry(lk, t) - beta * q[t];
       } else {
 #pragma unroll 16
-        for (int t = lane; t < TRI; t += 64) W[t] = rank ? alpha * entry(lk, t) : entry(lk, t);
+        for (int t = lane; t < TRI; t += 64) W[t] = entry(lk, t);
       }
       wave_sync();
       for (int r = lane; r < R; r += 64) W[tri_i(r) + r] *= rt2;
@@ -250,26 +232,125 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
         uniform_ptr y = (uniform_ptr)(ci + l * l);
         int a = tri_i(r);
         for (int col = 0; col < R; ++col, y += LL) {
-          double w;
-          if constexpr (gather) {
-            w = g[a];
-            if constexpr (rank) w = alpha * w - (p ? beta * pi[lk * TRI + a] : 0.0);
-            w *= col == r ? rt2 : 1.0;
-          } else {
-            w = W[a];
-          }
+          const double w = kForm == kGather ? g[a] * (col == r ? rt2 : 1.0) : W[a];
           a += col < r ? 1 : col + 1;
 #pragma unroll
           for (int m = 0; m < M; ++m) acc[m] += w * y[m];
         }
         if (rb + lane < R) {
           const int s = r / N, n = r - s * N;
-          double* o = dc + (v * S + s) * int64_t(LL) * N + n;
+          double* o = dc + (i * S + s) * int64_t(LL) * N + n;
 #pragma unroll
           for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
         }
       }
     });
+  }
+}
+
+// dL/dc of several sparse points (sets) at kSetCentres centres of their
+// species, one workgroup for a set: with W the symmetric matrix of a packed
+// channel, dL/dC_l = alpha f W(T) C_l - beta f W(p) C_l, whose second product
+// E does not depend on the set and comes from memory.  The columns of C_l of
+// all the centres side by side make the first a matrix product without
+// padding (16x16x4: a lane holds A[lane % 16][lane / 16], B[lane / 16][lane % 16]
+// and the rows lane / 16 + 4 e of column lane % 16 of the result); T's channel is
+// staged once in LDS (from memory where it is too large).  Forming alpha T -
+// beta p for each centre and set read both rows for every one of them and
+// took 1.18 ms for 300 sets of 983 centres in three species (n_max 8, l_max
+// 6); this takes 0.89 ms, bound by the gathered 8-byte loads of c and E and
+// the stores (W as a full matrix in LDS, with fewer index operations: 0.98).
+constexpr int kSetCentres = 16;
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <bool LDS>
+__global__ __launch_bounds__(kThreads) void sym_contract_sets_kernel(int R, int N, int L, int64_t ld, SymSets sets,
+                                                                     const double* __restrict__ c,
+                                                                     const double* __restrict__ norm2,
+                                                                     const double* __restrict__ E,
+                                                                     const double* __restrict__ T,
+                                                                     double* __restrict__ dc) {
+  const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), S = R / N;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = lane >> 4, x = lane & 15;
+  const int64_t set = blockIdx.y, i0 = int64_t(blockIdx.x) * kSetCentres;
+  const int nc = int(min(int64_t(kSetCentres), sets.n_ids - i0));
+  const double rt2 = 1.41421356237309504880;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* W = reinterpret_cast<double*>(smem_raw);
+  __shared__ double al[kSetCentres], be[kSetCentres];
+  __shared__ int centre[kSetCentres];
+  if (threadIdx.x < kSetCentres) {
+    // dL/dX = zeta d^(zeta - 1) T, d = X . T (a centre past the end: unused)
+    const int i = sets.ids[i0 + min(int(threadIdx.x), nc - 1)];
+    const double d = sets.dot[i * sets.ld_dot + set];
+    double a = double(sets.zeta), b = 0.0;
+    for (int k = 1; k < sets.zeta; ++k) a *= d;
+    if (E) {
+      const double n2 = norm2[i];
+      if (n2 > 0) {
+        b = a * d / n2;
+        a /= sqrt(n2);
+      }
+    }
+    centre[threadIdx.x] = i;
+    al[threadIdx.x] = a;
+    be[threadIdx.x] = b;
+  }
+  const double* Ts = T + set * ld;
+  const int B = S * LL * N;
+  double* dcs = dc + (set * sets.n_ids + i0) * B;
+  const float inv_n = 1.0f / float(N);
+  for (int l = 0; l <= L; ++l) {
+    const int M = 2 * l + 1, cols = nc * M;
+    const double f = rt2 / sqrt(double(M));
+    const double* g = Ts + l * TRI;
+    if constexpr (LDS) {
+      __syncthreads();  // the previous channel is read
+#pragma unroll 4
+      for (int t = threadIdx.x; t < TRI; t += kThreads) W[t] = g[t];
+      __syncthreads();
+      for (int r = threadIdx.x; r < R; r += kThreads) W[tri_i(r) + r] *= rt2;
+    }
+    __syncthreads();
+    const float inv_m = 1.0f / float(M);
+    auto centre_of = [&](int col) { return int((float(col) + 0.5f) * inv_m); };
+    for (int c0 = 16 * wave; c0 < cols; c0 += 16 * kWaves) {
+      const int col = min(c0 + x, cols - 1), ic = centre_of(col);
+      const double* cp = c + int64_t(centre[ic] * R) * LL + l * l + (col - ic * M);
+      // this lane's four columns of the result
+      const double* ee[4];
+      double* oo[4];
+      double av[4], bv[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int oc = min(c0 + q + 4 * e, cols - 1), io = centre_of(oc), o = (l * l + (oc - io * M)) * N;
+        ee[e] = E + (E ? int64_t(centre[io]) * B + o : 0);
+        oo[e] = dcs + int64_t(io) * B + o;
+        av[e] = al[io] * f;
+        bv[e] = be[io];
+      }
+      for (int rb = 0; rb < R; rb += 16) {
+        const int r = min(rb + x, R - 1), tr = tri_i(r);
+        const int s = int((float(r) + 0.5f) * inv_n), sn = s * LL * N + (r - s * N);
+        double ev[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ev[e] = E ? ee[e][sn] : 0.0;
+        f64x4 acc = {0, 0, 0, 0};
+        // (rows past R: a zero operand)
+#pragma unroll 6
+        for (int k0 = 0; k0 < R; k0 += 4) {
+          const int k = min(k0 + q, R - 1), t = k <= r ? tr + k : tri_i(k) + r;
+          const double w = LDS ? W[t] : g[t] * (k == r ? rt2 : 1.0);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + q < R ? cp[k * LL] : 0.0, k0 + q < R ? w : 0.0, acc, 0, 0, 0);
+        }
+        if (rb + x < R) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c0 + q + 4 * e < cols) oo[e][sn] = av[e] * acc[e] - bv[e] * ev[e];
+        }
+      }
+    }
   }
 }
 
@@ -438,13 +519,13 @@ constexpr size_t kContractLds = 156 * 1024;
 
 template <int kForm>
 void go_contract(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
-                 const double* xg, const double* G, double* dc, hipStream_t stream, const SymSets& sets = SymSets()) {
+                 const double* xg, const double* G, double* dc, hipStream_t stream) {
   const int R = S * N;
-  const size_t smem = kForm == kGather || kForm == kRankGather ? 0 : contract_lds(R, kForm == kDx);
+  const size_t smem = kForm == kGather ? 0 : contract_lds(R, kForm == kDx);
   auto go = [&](auto kern) {
     allow_lds(kern, smem);
     hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, R, N, L1 - 1, sym_row_stride(S, N, L1),
-                       c, p, norm2, xg, G, sets, dc);
+                       c, p, norm2, xg, G, dc);
     RGPU_LAUNCH_CHECK();
   };
   if (L1 <= 10)
@@ -465,13 +546,22 @@ void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const
 }
 
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
-                              const double* p, const double* norm2, const double* T, double* dc, hipStream_t stream) {
-  const int64_t n = n_sets * sets.n_ids;
-  if (n == 0) return;
-  if (contract_lds(S * N, false) <= kContractLds)
-    go_contract<kRank>(S, N, L1, n, c, p, norm2, nullptr, T, dc, stream, sets);
+                              const double* norm2, const double* E, const double* T, double* dc,
+                              hipStream_t stream) {
+  if (n_sets == 0 || sets.n_ids == 0) return;
+  if (n_sets > 65535) throw InvalidArgument("too many sets in one launch");
+  const int R = S * N;
+  const size_t smem = sizeof(double) * size_t(sym_tri(R));
+  auto go = [&](auto kern, size_t smem) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned((sets.n_ids + kSetCentres - 1) / kSetCentres), unsigned(n_sets)),
+                       dim3(kThreads), smem, stream, R, N, L1 - 1, sym_row_stride(S, N, L1), sets, c, norm2, E, T, dc);
+    RGPU_LAUNCH_CHECK();
+  };
+  if (smem <= kContractLds)
+    go(sym_contract_sets_kernel<true>, smem);
   else
-    go_contract<kRankGather>(S, N, L1, n, c, p, norm2, nullptr, T, dc, stream, sets);
+    go(sym_contract_sets_kernel<false>, 0);
 }
 
 void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
