@@ -43,6 +43,15 @@ __device__ __forceinline__ int wave_unit(int n, int nw, int wave, int k) {
   return u < n ? u : -1;
 }
 
+// the keys a <= b, a << 8 | b
+__device__ __forceinline__ void key_table(int S, int* key_ab) {
+  for (int k = threadIdx.x; k < S * (S + 1) / 2; k += kThreads) {
+    int a, b;
+    key_pair(k, S, &a, &b);
+    key_ab[k] = (a << 8) | b;
+  }
+}
+
 // f(std::integral_constant<int, l>) for the runtime l <= LM
 template <int LM, class F>
 __device__ __forceinline__ void with_channel(int l, F&& f) {
@@ -113,6 +122,39 @@ __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int 
     for (int w = 0; w < kPowerWaves; ++w) t += red[w];
     norm2[i] = t;
   }
+}
+
+// One channel of the product below: dc (dL/dc of the centre) rows lm of
+// channel l from the packed triangle w, in LDS with its diagonal times sqrt 2, or (kMemory)
+// in memory as it is.
+template <int LM, bool kMemory>
+__device__ __forceinline__ void contract_channel(int ll, int R, int N, int LL, int lane, const double* w,
+                                                 const double* ci, double* __restrict__ dc) {
+  const double rt2 = 1.41421356237309504880;
+  with_channel<LM>(ll, [&](auto lc) {
+    constexpr int l = decltype(lc)::value, M = 2 * l + 1;
+    const double f = rt2 / sqrt(double(M));
+    for (int rb = 0; rb < R; rb += 64) {
+      const int r = min(rb + lane, R - 1);
+      double acc[M];
+#pragma unroll
+      for (int m = 0; m < M; ++m) acc[m] = 0.0;
+      uniform_ptr y = (uniform_ptr)(ci + l * l);
+      int a = tri_i(r);
+      for (int col = 0; col < R; ++col, y += LL) {
+        const double v = kMemory ? w[a] * (col == r ? rt2 : 1.0) : w[a];
+        a += col < r ? 1 : col + 1;
+#pragma unroll
+        for (int m = 0; m < M; ++m) acc[m] += v * y[m];
+      }
+      if (rb + lane < R) {
+        const int s = r / N, n = r - s * N;
+        double* o = dc + int64_t(s) * LL * N + n;
+#pragma unroll
+        for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
+      }
+    }
+  });
 }
 
 // dL/dC_l[r][m] = f_l sqrt 2 sum_c w(r, c) C_l[c][m], w the packed entry
@@ -221,30 +263,105 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
       for (int r = lane; r < R; r += 64) W[tri_i(r) + r] *= rt2;
       wave_sync();
     }
-    with_channel<LM>(lk, [&](auto lc) {
-      constexpr int l = decltype(lc)::value, M = 2 * l + 1;
-      const double f = rt2 / sqrt(double(M));
-      for (int rb = 0; rb < R; rb += 64) {
-        const int r = min(rb + lane, R - 1);
-        double acc[M];
+    contract_channel<LM, kForm == kGather>(lk, R, N, LL, lane, kForm == kGather ? g : W, ci,
+                                           dc + i * int64_t(R) * LL);
+  }
+}
+
+// The same from full rows of dL/dX, the whole packed row formed in LDS first
+// (channels LT apart): the full row is read once along itself, where taking
+// the entries channel by channel (kDx) touches a cache line per entry.  2000
+// centres: 98 -> 71 us (4 species, n_max 8, l_max 6), 178 -> 83 us (3
+// species, n_max 10, l_max 8); bound by the chain of its phases.
+__host__ __device__ inline int full_stride(int R) { return tri_i(R) | 1; }
+
+template <int LM>
+__global__ __launch_bounds__(kThreads) void sym_contract_full_kernel(int R, int N, int L, int64_t ld,
+                                                                     const double* __restrict__ c,
+                                                                     const double* __restrict__ p,
+                                                                     const double* __restrict__ norm2,
+                                                                     const double* __restrict__ xg,
+                                                                     const double* __restrict__ G,
+                                                                     double* __restrict__ dc) {
+  const int64_t i = blockIdx.x;
+  const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), LT = full_stride(R), S = R / N, NL = N * L1, KB = N * NL;
+  const int K = S * (S + 1) / 2;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const double rt2 = 1.41421356237309504880;
+  extern __shared__ __align__(64) unsigned char smem_raw[];
+  double* W = reinterpret_cast<double*>(smem_raw);
+  int* key_ab = reinterpret_cast<int*>(W + L1 * LT);
+  __shared__ double red[kWaves];
+  key_table(S, key_ab);
+  __syncthreads();
+  const double* Gi = G + i * int64_t(K) * KB;
+  const float inv_kb = 1.0f / float(KB), inv_nl = 1.0f / float(NL), inv_l = 1.0f / float(L1);
+  // (several loads in flight, then the mirrors of the diagonal keys' entries)
+  constexpr int U = 8;
+  for (int e0 = threadIdx.x; e0 < K * KB; e0 += U * kThreads) {
+    double v[U], w[U];
+    int to[U];
 #pragma unroll
-        for (int m = 0; m < M; ++m) acc[m] = 0.0;
-        uniform_ptr y = (uniform_ptr)(ci + l * l);
-        int a = tri_i(r);
-        for (int col = 0; col < R; ++col, y += LL) {
-          const double w = kForm == kGather ? g[a] * (col == r ? rt2 : 1.0) : W[a];
-          a += col < r ? 1 : col + 1;
+    for (int u = 0; u < U; ++u) v[u] = Gi[min(e0 + u * kThreads, K * KB - 1)];
 #pragma unroll
-          for (int m = 0; m < M; ++m) acc[m] += w * y[m];
-        }
-        if (rb + lane < R) {
-          const int s = r / N, n = r - s * N;
-          double* o = dc + (i * S + s) * int64_t(LL) * N + n;
-#pragma unroll
-          for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
-        }
+    for (int u = 0; u < U; ++u) {
+      const int e = min(e0 + u * kThreads, K * KB - 1);
+      int k = int((float(e) + 0.5f) * inv_kb);
+      k -= k * KB > e ? 1 : 0;
+      k += (k + 1) * KB <= e ? 1 : 0;
+      const int o = e - k * KB, n1 = int((float(o) + 0.5f) * inv_nl), o1 = o - n1 * NL;
+      const int n2 = int((float(o1) + 0.5f) * inv_l), l = o1 - n2 * L1;
+      const int a = key_ab[k] >> 8, b = key_ab[k] & 255;
+      to[u] = a == b && n1 > n2 ? -1 : l * LT + tri_i(b * N + n2) + a * N + n1;
+      if (a == b && n1 < n2) {
+        w[u] = Gi[k * KB + n2 * NL + n1 * L1 + l];
+        v[u] *= 0.70710678118654752440;
+      } else {
+        w[u] = 0.0;
       }
-    });
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (to[u] >= 0) W[to[u]] = v[u] + 0.70710678118654752440 * w[u];
+  }
+  __syncthreads();
+  if (p) {
+    const double n2 = norm2[i];
+    const double* pi = p + i * ld;
+    const float inv_t = 1.0f / float(TRI);
+    auto channel_of = [&](int t) { return int((float(t) + 0.5f) * inv_t); };
+    double x = 0.0;
+    if (xg) {
+      x = xg[i];
+    } else {
+      double d = 0.0;
+#pragma unroll 8
+      for (int t = threadIdx.x; t < L1 * TRI; t += kThreads) d += pi[t] * W[t + channel_of(t) * (LT - TRI)];
+      for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
+      if (lane == 0) red[wave] = d;
+      __syncthreads();
+      if (n2 > 0) x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
+    }
+    if (n2 > 0) {
+      const double alpha = 1.0 / sqrt(n2), beta = x / n2;
+#pragma unroll 8
+      for (int t = threadIdx.x; t < L1 * TRI; t += kThreads) {
+        double* w = W + t + channel_of(t) * (LT - TRI);
+        *w = alpha * *w - beta * pi[t];
+      }
+    }
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < L1 * R; e += kThreads) {
+    const int l = e / R, r = e - l * R;
+    W[l * LT + tri_i(r) + r] *= rt2;
+  }
+  __syncthreads();
+  for (int k = 0; k * kWaves <= L; ++k) {
+    const int u = wave_unit(L1, kWaves, wave, k);
+    if (u >= 0)
+      contract_channel<LM, false>(L - u, R, N, LL, lane, W + (L - u) * LT, c + i * int64_t(R) * LL,
+                                  dc + i * int64_t(R) * LL);
   }
 }
 
@@ -358,14 +475,6 @@ __global__ __launch_bounds__(kThreads) void sym_contract_sets_kernel(int R, int 
 // a time through LDS ([key][n1][n2][l] with an odd n1 stride): both sides move
 // along their rows (whole key blocks, runs of N packed entries), and several
 // keys per pass keep enough loads in flight.  Memory bound.
-__device__ __forceinline__ void key_table(int S, int* key_ab) {
-  for (int k = threadIdx.x; k < S * (S + 1) / 2; k += kThreads) {
-    int a, b;
-    key_pair(k, S, &a, &b);
-    key_ab[k] = (a << 8) | b;
-  }
-}
-
 __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1, int KC, int64_t ld,
                                                             const double* __restrict__ full,
                                                             const int64_t* __restrict__ rows,
@@ -516,6 +625,10 @@ size_t contract_lds(int R, bool full) {
   return size_t(sym_tri(R)) * (sizeof(double) * kWaves + (full ? sizeof(int2) : 0));
 }
 constexpr size_t kContractLds = 156 * 1024;
+// sym_contract_full_kernel: three workgroups per CU at least (with 2 species,
+// n_max 12, l_max 9 it took 73 us against 107 by channels, 3 species 176
+// against 254, but 4 species, one workgroup, 552 against 476; 2000 centres)
+constexpr size_t kFullLds = 54 * 1024;
 
 template <int kForm>
 void go_contract(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
@@ -568,6 +681,21 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
                               const double* xg, const double* G, DeviceBuffer<double>& work, double* dc,
                               hipStream_t stream) {
   if (n == 0) return;
+  const int R = S * N;
+  const size_t whole = sizeof(double) * size_t(L1) * full_stride(R) + sizeof(int) * size_t(S) * (S + 1) / 2;
+  if (whole <= kFullLds) {
+    auto go = [&](auto kern) {
+      allow_lds(kern, whole);
+      hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), whole, stream, R, N, L1 - 1,
+                         sym_row_stride(S, N, L1), c, p, norm2, xg, G, dc);
+      RGPU_LAUNCH_CHECK();
+    };
+    if (L1 <= 10)
+      go(sym_contract_full_kernel<9>);
+    else
+      go(sym_contract_full_kernel<kMaxL1 - 1>);
+    return;
+  }
   if (contract_lds(S * N, true) <= kContractLds) {
     go_contract<kDx>(S, N, L1, n, c, p, norm2, xg, G, dc, stream);
     return;
