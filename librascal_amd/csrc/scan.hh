@@ -84,53 +84,55 @@ __global__ static __launch_bounds__(kScanThreads) void scan_small_kernel(
   if (threadIdx.x == 0) *total = carry_sh;
 }
 
-// Whole scan in one workgroup of 1024 threads (8 items each per chunk,
-// running carry between chunks), out[n] = total; for short arrays, where
-// one launch beats three.
-constexpr int kScan1Threads = 1024;
+// Whole scan in one launch, out[n] = total: every workgroup sums all that
+// comes before its tile itself (coalesced, from the L2) and then scans its
+// tile, so none waits for another; for arrays short enough that this costs
+// less than two more launches.  One workgroup that went over the whole array,
+// each thread with 8 consecutive items, took 12.6 us for 4689 items and 35 us
+// for 37724; this takes 4.3 and 7.2 us.
+constexpr int kScan1Threads = 1024, kScan1Items = 2, kScan1Tile = kScan1Threads * kScan1Items;
+constexpr int64_t kScan1Max = 65536;
 template <class In>
 __global__ __launch_bounds__(kScan1Threads) void scan_single_kernel(const In* __restrict__ in,
                                                                     int64_t* __restrict__ out,
                                                                     int64_t n) {
-  __shared__ int64_t wsum[kScan1Threads / 64];
-  __shared__ int64_t carry_sh;
+  __shared__ int64_t wpre[kScan1Threads / 64], wsum[kScan1Threads / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (threadIdx.x == 0) carry_sh = 0;
-  __syncthreads();
-  for (int64_t c0 = 0; c0 < n; c0 += int64_t(kScan1Threads) * kScanItems) {
-    const int64_t base = c0 + int64_t(threadIdx.x) * kScanItems;
-    int64_t v[kScanItems];
-    int64_t tsum = 0;
-    for (int k = 0; k < kScanItems; ++k) {
-      v[k] = base + k < n ? int64_t(in[base + k]) : 0;
-      tsum += v[k];
-    }
-    int64_t incl = tsum;
-    for (int off = 1; off < 64; off <<= 1) {
-      const int64_t o = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += o;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    int64_t run = carry_sh;
-    for (int w = 0; w < wave; ++w) run += wsum[w];
-    const int64_t last = run + incl;  // inclusive end of this thread
-    run += incl - tsum;
-    for (int k = 0; k < kScanItems; ++k) {
-      if (base + k < n) out[base + k] = run;
-      run += v[k];
-    }
-    __syncthreads();
-    if (threadIdx.x == kScan1Threads - 1) carry_sh = last;
-    __syncthreads();
+  const int64_t t0 = int64_t(blockIdx.x) * kScan1Tile, base = t0 + int64_t(threadIdx.x) * kScan1Items;
+  int64_t v[kScan1Items], tsum = 0, pre = 0;
+#pragma unroll
+  for (int k = 0; k < kScan1Items; ++k) {
+    v[k] = base + k < n ? int64_t(in[base + k]) : 0;
+    tsum += v[k];
   }
-  if (threadIdx.x == 0) out[n] = carry_sh;
+#pragma unroll 8
+  for (int64_t e = threadIdx.x; e < t0; e += kScan1Threads) pre += int64_t(in[e]);
+  for (int off = 32; off > 0; off >>= 1) pre += __shfl_xor(pre, off, 64);
+  int64_t incl = tsum;
+  for (int off = 1; off < 64; off <<= 1) {
+    const int64_t o = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += o;
+  }
+  if (lane == 63) {
+    wpre[wave] = pre;
+    wsum[wave] = incl;
+  }
+  __syncthreads();
+  int64_t run = incl - tsum;
+  for (int w = 0; w < kScan1Threads / 64; ++w) run += wpre[w] + (w < wave ? wsum[w] : 0);
+#pragma unroll
+  for (int k = 0; k < kScan1Items; ++k) {
+    if (base + k < n) out[base + k] = run;
+    run += v[k];
+  }
+  // (its items past the end are zero)
+  if (t0 + kScan1Tile >= n && threadIdx.x == kScan1Threads - 1) out[n] = run;
 }
 
 // scratch that exclusive_scan_device(n) uses (reserved ahead of a graph
 // capture, so that nothing is allocated inside it)
 inline void exclusive_scan_reserve(int64_t n, DeviceBuffer<int64_t>& scratch) {
-  if (n > 8 * int64_t(kScan1Threads) * kScanItems) scratch.reserve(size_t(2 * ((n + kScanTile - 1) / kScanTile)));
+  if (n > kScan1Max) scratch.reserve(size_t(2 * ((n + kScanTile - 1) / kScanTile)));
 }
 
 // out[i] = sum_{k<i} in[k] for i < n and out[n] = total, all on the device
@@ -142,8 +144,9 @@ void exclusive_scan_device(const In* in, int64_t* out, int64_t n, hipStream_t st
     RGPU_HIP(hipMemsetAsync(out, 0, sizeof(int64_t), stream));
     return;
   }
-  if (n <= 8 * int64_t(kScan1Threads) * kScanItems) {
-    hipLaunchKernelGGL(scan_single_kernel<In>, dim3(1), dim3(kScan1Threads), 0, stream, in, out, n);
+  if (n <= kScan1Max) {
+    hipLaunchKernelGGL(scan_single_kernel<In>, dim3(unsigned((n + kScan1Tile - 1) / kScan1Tile)),
+                       dim3(kScan1Threads), 0, stream, in, out, n);
     RGPU_LAUNCH_CHECK();
     return;
   }

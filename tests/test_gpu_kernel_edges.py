@@ -301,3 +301,20 @@ def test_mixed_product_tiles(atoms, points):
     assert abs(em[0] - k[0] @ w) <= 1e-4 * (np.abs(k[0]) @ np.abs(w))
     assert abs(em[0] - e[0]) <= 1e-4 * (np.abs(k[0]) @ np.abs(w))
     assert np.sqrt(np.mean((gm - g) ** 2)) <= 1e-4 * np.sqrt(np.mean(g ** 2))
+
+
+@pytest.mark.parametrize("pairs", [1, 1024, 1025, 32768, 32769])
+def test_offsets_at_scan_tiles(pairs):
+    """Neighbour lists of isolated pairs of atoms: offsets at one, two and
+    many tiles of the one-launch prefix sum and past its largest length."""
+    n = 2 * pairs
+    pos = np.zeros((n, 3))
+    pos[1::2, 0] = 1.0
+    ctx = _capi.Context(json.dumps(soap_hypers(rc=2.0, sw=0.5, sigma=0.5, N=1, L=0, spline=1e-8)))
+    ctx.set_structures(np.arange(0, n + 1, 2), pos, np.ones(n, np.int32),
+                       np.tile((10 * np.eye(3)).ravel(), (pairs, 1)), np.zeros((pairs, 3), np.int32), [1])
+    off, j, vec = ctx.neighbours()
+    assert np.array_equal(off, 2 * np.arange(n + 1))
+    assert np.array_equal(j[0::2], np.arange(n)) and np.array_equal(j[1::2], np.arange(n) ^ 1)
+    c, _ = ctx.expansion()
+    assert np.all(c == c[0])
