@@ -243,8 +243,8 @@ int rgpu_gap_predict(rgpu_context* ctx, double* energy, double* gradient, double
  * energy GEMM's per-column-tile partial sums live in a static device array
  * of 2^23 doubles (64 MiB per device), so a batch of n centres is accepted
  * when ceil(n/32)*32 + n*T <= 2^23, T being the column tiles of the widest
- * species block (ceil(M_s/128) mixed, ceil(M_s/64) FP64; larger batches
- * are rejected with an error), and every context buffer must already be
+ * species block (ceil(M_s/128) mixed, ceil(M_s/64) FP64 and, where n*T is
+ * at most 2^22, mixed; larger batches are rejected with an error), and every context buffer must already be
  * sized for the batch
  * (one rgpu_gap_predict on it first; otherwise an error, nothing allocated).
  * The call is stream-ordered (no synchronisation): the energies are ready

@@ -1062,12 +1062,15 @@ void emit_outputs(Context& c, const double* e_centre, double* energy, double* gr
 // T (the partial row sums it keeps per centre)
 template <class T>
 int energy_tiles(const Context& c) {
+  const int S = int(c.sp_off.size()) - 1;
   int t = 0;
-  for (size_t s = 0; s + 1 < c.sp_off.size(); ++s) {
-    const int64_t m = c.sp_off[s + 1] - c.sp_off[s];
-    t = std::max(t, std::is_same<T, float>::value ? gap_mixed_energy_tiles(m) : gap_f64_energy_tiles(m));
+  std::array<int64_t, kMaxSpecies> rows{}, cols{};
+  for (int s = 0; s < S; ++s) {
+    rows[size_t(s)] = c.row_off[s + 1] - c.row_off[s];
+    cols[size_t(s)] = c.sp_off[s + 1] - c.sp_off[s];
+    t = std::max(t, gap_f64_energy_tiles(cols[size_t(s)]));
   }
-  return t;
+  return std::is_same<T, float>::value ? gap_mixed_energy_tiles(rows.data(), cols.data(), S, c.n_atoms) : t;
 }
 
 template <class T>
@@ -1079,7 +1082,6 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
   if (want_grad) require_unmasked(c);
   double* ec = c.e_centre.reserve(size_t(std::max<int64_t>(n, 1)));
   double* part = c.e_part.reserve(size_t(std::max<int64_t>(n * energy_tiles<T>(c), 1)));
-  RGPU_HIP(hipMemsetAsync(ec, 0, sizeof(double) * n, c.stream));
   const T* X = nullptr;
   if constexpr (std::is_same<T, double>::value) X = invariants_of<double>(c);
   std::vector<GapBlock<T>> blks;
@@ -1095,9 +1097,10 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
                                                                     : gap_f64_k_stride(blks.back().n_cols));
     if (blks.back().n_rows > 0 && blks.back().n_cols == 0) rows_without_points = true;
   }
+  // (the products write the energies and G of every species with sparse points)
+  if (rows_without_points) RGPU_HIP(hipMemsetAsync(ec, 0, sizeof(double) * n, c.stream));
   T* G = nullptr;
   if (want_grad) {
-    // the force product writes every row of a species with sparse points
     G = Gbuf<T>(c).reserve(size_t(std::max<int64_t>(n * D, 1)));
     if (rows_without_points) RGPU_HIP(hipMemsetAsync(G, 0, sizeof(T) * n * D, c.stream));
   }

@@ -11,9 +11,10 @@ namespace rgpu {
 // and W~ rows hold zeros from their last column up to this stride
 int64_t gap_f64_k_stride(int64_t k);
 
-// K GEMM + epilogue for all species blocks (grouped): energy per centre (+=;
-// summed over the column tiles through part, [gap_f64_energy_tiles(n_cols)
-// of the widest block] x [ld >= n_centres] doubles, see EnergyTiles) and
+// K GEMM + epilogue for all species blocks (grouped): energy per centre (of
+// the blocks with sparse points; summed over the column tiles through part,
+// [gap_f64_energy_tiles(n_cols) of the widest block] x [ld >= n_centres]
+// doubles, see EnergyTiles) and
 // wts[b] [n_rows][gap_f64_k_stride(n_cols)] (wts may be null)
 int gap_f64_energy_tiles(int64_t n_cols);
 void run_gap_f64_kernel(const GapBlock<double>* blks, int n_blocks, double* energy, double* part, int64_t ld,

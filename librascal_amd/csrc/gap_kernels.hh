@@ -38,7 +38,7 @@ void launch_rows_segment_sum(const double* in, int64_t w, const int64_t* seg_off
 
 // Per-centre energies without atomics: a GEMM's energy epilogue stores the
 // partial row sum of its column tile t at part[t * ld + centre], and
-// launch_energy_tiles adds the sum over the tiles, taken in tile order, to
+// launch_energy_tiles writes the sum over the tiles, taken in tile order, to
 // energy[centre] (the same value on every run).  One entry per species
 // block: its centres and its number of column tiles.
 struct EnergyTiles {

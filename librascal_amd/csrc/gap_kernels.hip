@@ -104,8 +104,9 @@ __global__ void energy_tiles_kernel(EnergyTiles et, const double* __restrict__ p
   if (pi >= et.n) return;
   const int c = et.rows[pi][r];
   double s = 0.0;
+#pragma unroll 8
   for (int t = 0; t < et.tiles[pi]; ++t) s += part[int64_t(t) * ld + c];
-  energy[c] += s;
+  energy[c] = s;
 }
 
 // out[s][m] = sum of in[a][m] over the rows a of segment s, in row order

@@ -43,12 +43,12 @@ int64_t gap_mixed_wt_stride(int64_t n_cols);
 // K tile GEMM + epilogue for all species blocks in grouped launches.  The
 // features are given split: X = xs.hi + xs.lo, [n_centres][D] (rows gathered
 // through the blocks' row_idx, un-normalised, scaled by 1/|p| in the
-// epilogue).  Outputs: energy (per centre, +=; summed over the column
-// tiles through part, [gap_mixed_energy_tiles(n_cols) of the widest block]
-// x [ld >= n_centres] doubles, see EnergyTiles) and the weighted kernel
-// gradient W~ of each block, split, [n_rows][gap_mixed_wt_stride(n_cols)]
-// (wts may be null).
-int gap_mixed_energy_tiles(int64_t n_cols);
+// epilogue).  Outputs: energy (of the blocks with sparse points, per centre;
+// summed over the column tiles through part, [gap_mixed_energy_tiles of the
+// blocks' row and column counts] x [ld >= n_centres] doubles, see EnergyTiles)
+// and the weighted kernel gradient W~ of each block, split,
+// [n_rows][gap_mixed_wt_stride(n_cols)] (wts may be null).
+int gap_mixed_energy_tiles(const int64_t* rows, const int64_t* cols, int n_blocks, int64_t ld);
 void run_gap_mixed_kernel(const GapBlock<float>* blks, int n_blocks, const MixedSparse& ms,
                           SplitPlanes xs, double* energy, double* part, int64_t ld, const SplitPlanes* wts,
                           hipStream_t stream);

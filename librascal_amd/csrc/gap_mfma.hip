@@ -420,6 +420,18 @@ int64_t layout_tiles(ProblemSet& ps, int bm, int bn) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Under three quarters of a 128 x 128 tile per CU, 64 x 64 tiles: a tile
+// alone on its CU takes the same time however few there are (96 tiles, 60 K
+// steps: 78 us, 48 us in small ones; 168 tiles, 208 K steps: 255 and 194 us),
+// while with the chip full their extra operand traffic shows (512 tiles, 363 K
+// steps: 602 and 1035 us).  They double the partial sums of the energies
+// (rows x column tiles), which stay under 2^22 so that no batch outgrows a
+// scratch array for it.
+bool small_tiles(int64_t tiles, int64_t rows, int64_t cols) {
+  return 4 * tiles <= 3 * int64_t(device_cu_count()) &&
+         rows * ((cols + kMinBN - 1) / kMinBN) <= int64_t(1) << 22;
+}
+
 // columns per tile of the set's launch
 template <int EPI>
 int launch_set(ProblemSet& ps, hipStream_t stream) {
@@ -438,12 +450,11 @@ int launch_set(ProblemSet& ps, hipStream_t stream) {
     RGPU_LAUNCH_CHECK();
     return bn;
   };
-  // Under three quarters of a 128 x 128 tile per CU, 64 x 64 tiles: a tile
-  // alone on its CU takes the same time however few there are (96 tiles, 60 K
-  // steps: 78 us, 48 us in small ones; 168 tiles, 208 K steps: 255 and
-  // 194 us), while with the chip full their extra operand traffic shows (512
-  // tiles, 363 K steps: 602 and 1035 us).
-  if (4 * layout_tiles(ps, BM, BN) <= 3 * int64_t(device_cu_count())) return go(bf16x3_gemm_dma<EPI, 64, 64>, 64, 64);
+  const int64_t tiles = layout_tiles(ps, BM, BN);
+  int64_t cols = 0;
+  for (int i = 0; i < ps.n; ++i) cols = std::max(cols, ps.p[i].N);
+  if (EPI == 0 ? small_tiles(tiles, ps.p[0].ldp, cols) : small_tiles(tiles, 0, 0))
+    return go(bf16x3_gemm_dma<EPI, 64, 64>, 64, 64);
   return go(bf16x3_gemm_dma<EPI, BM, BN>, BM, BN);
 }
 
@@ -512,7 +523,20 @@ void prepare_mixed_sparse(MixedSparse& ms, const double* T, int64_t M, int S, in
 
 int64_t gap_mixed_wt_stride(int64_t n_cols) { return (n_cols + BK - 1) / BK * BK; }
 
-int gap_mixed_energy_tiles(int64_t n_cols) { return int((n_cols + kMinBN - 1) / kMinBN); }
+int gap_mixed_energy_tiles(const int64_t* rows, const int64_t* cols, int n_blocks, int64_t ld) {
+  int64_t t = 0;
+  for (int b0 = 0; b0 < n_blocks; b0 += kMaxProblems) {
+    int64_t tiles = 0, widest = 0;
+    for (int b = b0; b < std::min(n_blocks, b0 + kMaxProblems); ++b) {
+      if (rows[b] == 0 || cols[b] == 0) continue;
+      tiles += (rows[b] + BM - 1) / BM * ((cols[b] + BN - 1) / BN);
+      widest = std::max(widest, cols[b]);
+    }
+    const int bn = small_tiles(tiles, ld, widest) ? kMinBN : BN;
+    t = std::max(t, (widest + bn - 1) / bn);
+  }
+  return int(t);
+}
 
 void run_gap_mixed_kernel(const GapBlock<float>* blks, int n_blocks, const MixedSparse& ms,
                           SplitPlanes xs, double* energy, double* part, int64_t ld, const SplitPlanes* wts,
