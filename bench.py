@@ -267,7 +267,7 @@ GEMM_KERNEL = "bf16x3_gemm_dma<0, 128, 128>"
 FORCE_GEMM_KERNEL = "bf16x3_gemm_dma<1, 128, 128>"
 EXPANSION_KERNEL = "expansion_wave_kernel<float, 12, 64>"
 PS_KERNEL = "power_spectrum_kernel<float, true, 12, 9>"
-ADJOINT_KERNELS = {0: ["adjoint_staged_kernel<false, 5>"], 1: ["adjoint_mfma_kernel<false, 12>"],
+ADJOINT_KERNELS = {0: ["adjoint_staged_kernel<false, 5, true>"], 1: ["adjoint_mfma_kernel<false, 12>"],
                    2: ["adjoint_tile_kernel<12, 9, 6, 1, 10, false, true>"],
                    3: ["adjoint_tile_kernel<12, 9, 6, 1, 6, false, false>", "pair_force_kernel<float, 12, 64, 1>"]}
 # shader clock under this load (SQ_BUSY_CYCLES over the kernel durations)
