@@ -1,12 +1,13 @@
 // Power spectrum in symmetric packed rows and its adjoint (sym_kernels.hh).
 //
-// Both products walk one angular channel per wavefront with lane = row r of
-// C_l: the power spectrum keeps C_l[r][:] in registers and the adjoint one
-// dL/dC_l[r][:], and the row C_l[c][:] of every step is the same for the
-// whole wavefront, so it is read through scalar loads and enters the FMAs as
-// a scalar operand.  No vector or LDS load feeds the FMAs except one packed
-// entry per step in the adjoint; the LDS traffic of a tiled product (two
-// operands per FMA block) bounded the kernels this replaced.
+// The power spectrum multiplies tiles of C_l's rows on the FP64 matrix cores,
+// both operands read from LDS in the same layout.  The adjoint walks one
+// angular channel per wavefront with lane = row r of C_l, dL/dC_l[r][:] in
+// registers; the row C_l[c][:] of every step is the same for the whole
+// wavefront, so it is read through scalar loads and enters the FMAs as a
+// scalar operand, beside one packed entry per step from LDS.  (A matrix-core
+// form of that one took 354 us where this takes 318: its operands come
+// through the packed triangle, and it leaves fewer wavefronts in flight.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,6 +34,8 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 __host__ __device__ constexpr int tri_i(int r) { return r * (r + 1) / 2; }
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 // k-th of the units 0 .. n-1 (in descending order of work) of a wavefront, -1
 // past the last: they are dealt to the nw wavefronts back and forth, which
@@ -63,14 +66,17 @@ __device__ __forceinline__ void with_channel(int l, F&& f) {
   }
 }
 
-// One workgroup of eight wavefronts per centre; a unit is half the columns of
-// a channel.  C sits in LDS for the lanes' own rows (odd row stride: no bank
-// conflicts); the loop over columns c does (2l+1) FMAs per entry, of which the
-// lanes r <= c store theirs (a run of c + 1 values).  Bound by the latency of
-// the scalar loads: eight wavefronts per copy of C put twice as many on a CU
-// as four (4096 centres, 4 species, n_max 12, l_max 9: 275 us with four).
+// One workgroup of eight wavefronts per centre, C in LDS (odd row stride: no
+// bank conflicts); a unit is a 16 x 16 tile (rows of C_l against rows of C_l, on
+// and above the diagonal) of one channel on the matrix cores (16x16x4: a lane
+// holds A[lane % 16][lane / 16], B[lane / 16][lane % 16] and the rows lane / 16 + 4 e
+// of column lane % 16 of the result), the lanes of a column run along the
+// packed entries of c.  Memory bound for many centres: 4096 centres of 4
+// species, n_max 12, l_max 9 223 -> 132 us (0.54 GB), 4689 of n_max 8, l_max 6
+// 70 -> 44 us, 1024 of 2 species, n_max 10, l_max 8 18.8 -> 14.5 us, against a
+// lane per row and FMAs with the other row as a scalar operand, whose loads'
+// latency bound it.
 constexpr int kPowerWaves = 8;
-template <int LM>
 __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int L, int64_t ld,
                                                                      const double* __restrict__ c,
                                                                      double* __restrict__ p,
@@ -86,32 +92,31 @@ __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int 
     for (int k = lane; k < LL; k += 64) cs[r * LS + k] = ci[r * LL + k];
   __syncthreads();
   double ss = 0.0;
-  for (int k = 0; k * kPowerWaves < 2 * (L + 1); ++k) {
-    const int u = wave_unit(2 * (L + 1), kPowerWaves, wave, k);
-    if (u < 0) continue;
-    with_channel<LM>(L - (u >> 1), [&](auto lc) {
-      constexpr int l = decltype(lc)::value, M = 2 * l + 1;
-      const double f = 1.0 / sqrt(double(M)), f2 = f * 1.41421356237309504880;
-      double* out = p + i * ld + int64_t(l) * TRI;
-      const int half = (R + 1) / 2, c0 = (u & 1) ? half : 0, c1 = (u & 1) ? R : half;
-      for (int rb = 0; rb < c1; rb += 64) {
-        const int r = rb + lane, ro = min(r, R - 1), cb = max(rb, c0);
-        double x[M];
+  const int q = lane >> 4, x = lane & 15, RT = (R + 15) / 16, pairs = RT * (RT + 1) / 2;
+  for (int k = wave; k < (L + 1) * pairs; k += kPowerWaves) {
+    const int l = L - k / pairs, u = k - (L - l) * pairs, M = 2 * l + 1;
+    const double f = 1.0 / sqrt(double(M)), f2 = f * 1.41421356237309504880;
+    double* out = p + i * ld + int64_t(l) * TRI;
+    int ct = 0;
+    while (tri_i(ct + 1) <= u) ++ct;
+    const int rt = u - tri_i(ct);
+    const double* a = cs + min(16 * ct + x, R - 1) * LS + l * l + q;
+    const double* b = cs + min(16 * rt + x, R - 1) * LS + l * l + q;
+    f64x4 acc = {0, 0, 0, 0};
+    for (int m = 0; m < M; m += 4) {
+      const bool in = m + q < M;
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? a[m] : 0.0, in ? b[m] : 0.0, acc, 0, 0, 0);
+    }
+    const int row = 16 * rt + x;
 #pragma unroll
-        for (int m = 0; m < M; ++m) x[m] = cs[ro * LS + l * l + m];
-        uniform_ptr y = (uniform_ptr)(ci + int64_t(cb) * LL + l * l);
-        for (int col = cb; col < c1; ++col, y += LL) {
-          double s = 0.0;
-#pragma unroll
-          for (int m = 0; m < M; ++m) s += x[m] * y[m];
-          if (r <= col) {
-            const double v = s * (r < col ? f2 : f);
-            out[tri_i(col) + r] = v;
-            ss += v * v;
-          }
-        }
+    for (int e = 0; e < 4; ++e) {
+      const int col = 16 * ct + q + 4 * e;
+      if (row <= col && col < R) {
+        const double v = acc[e] * (row < col ? f2 : f);
+        out[tri_i(col) + row] = v;
+        ss += v * v;
       }
-    });
+    }
   }
   for (int64_t o = int64_t(L + 1) * TRI + threadIdx.x; o < ld; o += 64 * kPowerWaves) p[i * ld + o] = 0.0;
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
@@ -378,7 +383,6 @@ __global__ __launch_bounds__(kThreads) void sym_contract_full_kernel(int R, int 
 // 6); this takes 0.89 ms, bound by the gathered 8-byte loads of c and E and
 // the stores (W as a full matrix in LDS, with fewer index operations: 0.98).
 constexpr int kSetCentres = 16;
-typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 template <bool LDS>
 __global__ __launch_bounds__(kThreads) void sym_contract_sets_kernel(int R, int N, int L, int64_t ld, SymSets sets,
@@ -606,17 +610,10 @@ void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* 
   if (n == 0) return;
   const int R = S * N;
   const size_t smem = sizeof(double) * size_t(R) * ((L1 * L1) | 1);
-  auto go = [&](auto kern) {
-    allow_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(64 * kPowerWaves), smem, stream, R, L1 - 1,
-                       sym_row_stride(S, N, L1), c, p, norm2);
-    RGPU_LAUNCH_CHECK();
-  };
-  // the register budget follows the largest channel the kernel is built for
-  if (L1 <= 10)
-    go(sym_power_kernel<9>);
-  else
-    go(sym_power_kernel<kMaxL1 - 1>);
+  allow_lds(sym_power_kernel, smem);
+  hipLaunchKernelGGL(sym_power_kernel, dim3(unsigned(n)), dim3(64 * kPowerWaves), smem, stream, R, L1 - 1,
+                     sym_row_stride(S, N, L1), c, p, norm2);
+  RGPU_LAUNCH_CHECK();
 }
 
 namespace {
