@@ -1087,7 +1087,7 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
   std::vector<GapBlock<T>> blks;
   std::vector<int64_t> wt_off;
   int64_t wt_total = 0;
-  bool rows_without_points = false;
+  int64_t n_written = 0;  // centres of the species with sparse points
   for (int s = 0; s < S; ++s) {
     blks.push_back(gap_block<T>(c, s, X, sparse_values<T>(c)));
     blks.back().D = D;
@@ -1095,14 +1095,16 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     // (rows padded to whole K steps of the force product)
     wt_total += blks.back().n_rows * (std::is_same<T, float>::value ? gap_mixed_wt_stride(blks.back().n_cols)
                                                                     : gap_f64_k_stride(blks.back().n_cols));
-    if (blks.back().n_rows > 0 && blks.back().n_cols == 0) rows_without_points = true;
+    if (blks.back().n_cols > 0) n_written += blks.back().n_rows;
   }
-  // (the products write the energies and G of every species with sparse points)
-  if (rows_without_points) RGPU_HIP(hipMemsetAsync(ec, 0, sizeof(double) * n, c.stream));
+  // The products write the energies and G of these centres only; the energies
+  // of the others (atoms that the mask leaves out among them) are summed over
+  // the structures too.
+  if (n_written < n) RGPU_HIP(hipMemsetAsync(ec, 0, sizeof(double) * n, c.stream));
   T* G = nullptr;
   if (want_grad) {
     G = Gbuf<T>(c).reserve(size_t(std::max<int64_t>(n * D, 1)));
-    if (rows_without_points) RGPU_HIP(hipMemsetAsync(G, 0, sizeof(T) * n * D, c.stream));
+    if (n_written < n) RGPU_HIP(hipMemsetAsync(G, 0, sizeof(T) * n * D, c.stream));
   }
   if constexpr (std::is_same<T, float>::value) {
     std::vector<SplitPlanes> wts(static_cast<size_t>(S));

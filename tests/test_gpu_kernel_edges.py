@@ -318,3 +318,26 @@ def test_offsets_at_scan_tiles(pairs):
     assert np.array_equal(j[0::2], np.arange(n)) and np.array_equal(j[1::2], np.arange(n) ^ 1)
     c, _ = ctx.expansion()
     assert np.all(c == c[0])
+
+
+@pytest.mark.parametrize("prec,tol", [(_capi.FP64, 1e-10), (_capi.MIXED, 1e-4)])
+def test_masked_energies_after_other_predictions(prec, tol):
+    """Energies of masked batches on a context that has predicted others
+    before, with sparse points for every species: the atoms that the mask
+    leaves out contribute nothing, whatever their energies were."""
+    sts = periodic_box(60, 0.05, (1, 8), d_min=1.0, seed=12) + periodic_box(37, 0.05, (1, 8), d_min=1.0, seed=13)
+    ctx, num = _context(soap_hypers(rc=4.0, sw=0.5, sigma=0.5, N=6, L=4, spline=1e-8), sts)
+    off, pos, _, cells, pbc = pack(sts)
+    rng = np.random.default_rng(11)
+    spec, vals, _ = _points(ctx, num, {1: 7, 8: 9}, rng)
+    w = rng.uniform(0.5, 1.5, len(spec))
+    ctx.set_precision(prec)
+    ctx.set_sparse_points(2, spec, vals, w)
+    e_atom = ctx.gap_knm("Atom") @ w
+    for mask in (rng.random(len(num)) < 0.5, num == 8, np.zeros(len(num), bool), np.arange(len(num)) < 60):
+        ctx.set_structures(off, pos, num, cells, pbc, [1, 8])
+        ctx.gap_predict()
+        ctx.set_structures(off, pos, num, cells, pbc, [1, 8], centre_mask=mask)
+        e = ctx.gap_predict(gradient=False, neg_stress=False)[0]
+        ref = np.add.reduceat(np.where(mask, e_atom, 0.0), off[:-1])
+        assert np.abs(e - ref).max() <= tol * np.abs(e_atom).sum()
