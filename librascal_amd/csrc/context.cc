@@ -133,6 +133,12 @@ struct Context {
   std::vector<int64_t> sp_off;    // per species index s: [sp_off[s], sp_off[s+1])
   bool have_weights = false;
   DeviceBuffer<double> T64, alpha;  // T64 [M][ldx64()]: rows as the FP64 features'
+  // Full rows of the sparse points, gap_f64_k_stride(D()) apart, for K_MM:
+  // held only when a diagonal key's block of some point is not symmetric, since
+  // two such points' product is not that of their symmetric packed rows.
+  DeviceBuffer<double> T_full;
+  DeviceBuffer<int> d_asymmetric;
+  bool asymmetric = false;
   DeviceBuffer<float> T32;
   MixedSparse mixed_sparse;
 
@@ -2038,17 +2044,30 @@ int rgpu_set_sparse_points(rgpu_context* ctx, int zeta, int64_t n_sparse, const 
     double* dT = c.T64.reserve(size_t(n1 * ldx));
     double* dTf = full.reserve(size_t(n1 * D));
     float* dT32 = c.T32.reserve(size_t(n1 * D));
+    int asymmetric = 0;
     if (n_sparse > 0) {
       RGPU_HIP(hipMemcpyAsync(dr, values, sizeof(double) * size_t(n_sparse * D), hipMemcpyHostToDevice, c.stream));
       RGPU_HIP(hipMemcpyAsync(dord, order.data(), sizeof(int64_t) * size_t(n_sparse), hipMemcpyHostToDevice,
                               c.stream));
       launch_gather_rows<double>(n_sparse, D, D, dr, dord, dTf, c.stream);
       launch_gather_rows<float>(n_sparse, D, D, dr, dord, dT32, c.stream);
-      if (c.sparsified())
+      if (c.sparsified()) {
         launch_gather_rows<double>(n_sparse, D, ldx, dr, dord, dT, c.stream);
-      else
-        launch_sym_pack(S, c.rd.N, c.rd.L1, n_sparse, dr, dord, dT, c.stream);
+      } else {
+        int* da = c.d_asymmetric.reserve(1);
+        RGPU_HIP(hipMemsetAsync(da, 0, sizeof(int), c.stream));
+        launch_sym_pack(S, c.rd.N, c.rd.L1, n_sparse, dr, dord, dT, c.stream, da);
+        RGPU_HIP(hipMemcpyAsync(&asymmetric, da, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+      }
       RGPU_HIP(hipStreamSynchronize(c.stream));
+    }
+    c.asymmetric = asymmetric != 0;
+    if (c.asymmetric) {
+      const int64_t ldf = gap_f64_k_stride(D);
+      launch_gather_rows<double>(n_sparse, D, ldf, dr, dord, c.T_full.reserve(size_t(n_sparse * ldf)), c.stream);
+      RGPU_HIP(hipStreamSynchronize(c.stream));
+    } else {
+      c.T_full.release();
     }
     double* da = c.alpha.reserve(a.size());
     RGPU_HIP(hipMemcpy(da, a.data(), sizeof(double) * a.size(), hipMemcpyHostToDevice));
@@ -2115,9 +2134,9 @@ int rgpu_gap_kmm(rgpu_context* ctx, double* kmm) {
       b.n_rows = b.n_cols = m1 - m0;
       b.row_idx = rows + m0;
       b.col0 = m0;
-      b.X = b.Tm = c.T64.get();
+      b.X = b.Tm = c.asymmetric ? c.T_full.get() : c.T64.get();
       b.zeta = c.zeta;
-      b.D = c.ldx64();
+      b.D = c.asymmetric ? gap_f64_k_stride(c.D()) : c.ldx64();
       blks.push_back(b);
       m0 = m1;
     }

@@ -59,9 +59,11 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
 
 // Full rows [.][K N^2 (L+1)] to symmetric packed rows and back.  Packing row
 // r from full row rows[r] (rows null: row r); unpacking row r of out from
-// packed row rows[r], divided by its norm when normalising.
+// packed row rows[r], divided by its norm when normalising.  asymmetric (may
+// be null): set to 1 when a diagonal key's block of a full row is not symmetric
+// (such a row is not recovered from its packed one).
 void launch_sym_pack(int S, int N, int L1, int64_t n, const double* full, const int64_t* rows, double* out,
-                     hipStream_t stream);
+                     hipStream_t stream, int* asymmetric = nullptr);
 void launch_sym_unpack(int S, int N, int L1, int64_t n, const double* p, const int64_t* rows, const double* norm2,
                        bool normalize, double* out, hipStream_t stream);
 

@@ -479,11 +479,16 @@ __global__ __launch_bounds__(kThreads) void sym_contract_sets_kernel(int R, int 
 // a time through LDS ([key][n1][n2][l] with an odd n1 stride): both sides move
 // along their rows (whole key blocks, runs of N packed entries), and several
 // keys per pass keep enough loads in flight.  Memory bound.
+// CHECK: *asymmetric = 1 when a diagonal key's block of some row is not
+// symmetric (every writer stores the same value).
+template <bool CHECK>
 __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1, int KC, int64_t ld,
                                                             const double* __restrict__ full,
                                                             const int64_t* __restrict__ rows,
-                                                            double* __restrict__ out) {
+                                                            double* __restrict__ out,
+                                                            int* __restrict__ asymmetric) {
   const int64_t i = blockIdx.x;
+  bool differ = false;
   const int K = S * (S + 1) / 2, NL = N * L1, KB = N * NL, NS = NL | 1, TRI = tri_i(S * N), NN = N * N;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   extern __shared__ __align__(64) unsigned char smem_raw[];
@@ -507,10 +512,13 @@ __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1
       const double *bk = b + kk * N * NS, *b0 = bk + n1 * NS + n2 * L1, *b1 = bk + n2 * NS + n1 * L1;
       int64_t o = tri_i(sb * N + n2) + sa * N + n1;
 #pragma unroll 4
-      for (int l = 0; l < L1; ++l, o += TRI)
+      for (int l = 0; l < L1; ++l, o += TRI) {
         dst[o] = sym ? (b0[l] + b1[l]) * 0.70710678118654752440 : b0[l];
+        if (CHECK && sym) differ |= b0[l] != b1[l];
+      }
     }
   }
+  if (CHECK && differ) *asymmetric = 1;
   for (int64_t o = int64_t(L1) * TRI + threadIdx.x; o < ld; o += kThreads) dst[o] = 0.0;
 }
 
@@ -708,13 +716,19 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
 }
 
 void launch_sym_pack(int S, int N, int L1, int64_t n, const double* full, const int64_t* rows, double* out,
-                     hipStream_t stream) {
+                     hipStream_t stream, int* asymmetric) {
   if (n == 0) return;
   const size_t smem = key_lds(S, N, L1);
-  allow_lds(sym_pack_kernel, smem);
-  hipLaunchKernelGGL(sym_pack_kernel, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1,
-                     key_blocks(S, N, L1), sym_row_stride(S, N, L1), full, rows, out);
-  RGPU_LAUNCH_CHECK();
+  auto go = [&](auto kern) {
+    allow_lds(kern, smem);
+    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1, key_blocks(S, N, L1),
+                       sym_row_stride(S, N, L1), full, rows, out, asymmetric);
+    RGPU_LAUNCH_CHECK();
+  };
+  if (asymmetric)
+    go(sym_pack_kernel<true>);
+  else
+    go(sym_pack_kernel<false>);
 }
 
 void launch_sym_unpack(int S, int N, int L1, int64_t n, const double* p, const int64_t* rows, const double* norm2,

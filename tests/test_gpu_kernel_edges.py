@@ -341,3 +341,30 @@ def test_masked_energies_after_other_predictions(prec, tol):
         e = ctx.gap_predict(gradient=False, neg_stress=False)[0]
         ref = np.add.reduceat(np.where(mask, e_atom, 0.0), off[:-1])
         assert np.abs(e - ref).max() <= tol * np.abs(e_atom).sum()
+
+
+@pytest.mark.parametrize("zeta,N,L,M,where", [
+    (1, 4, 2, 2, "all"), (2, 5, 4, 33, "all"), (1, 8, 6, 70, "one entry"), (3, 6, 3, 65, "all"), (1, 1, 3, 4, "all"),
+])
+def test_kmm_of_points_that_are_not_symmetric(zeta, N, L, M, where):
+    """K_MM of sparse points whose diagonal keys' blocks are not symmetric
+    (random points, or one entry of one point), of symmetric ones after them
+    and of the first again, with a species outside the batch, against the
+    oracle."""
+    sts = periodic_box(30, 0.05, (1, 8), d_min=1.0, seed=111)
+    ctx, num = _context(soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8), sts)
+    X, _ = ctx.features()
+    rng = np.random.default_rng(112)
+    spec = np.concatenate([[1, 8, 9], rng.choice([1, 8, 9], M)]).astype(np.int32)
+    symmetric = X[rng.choice(len(X), len(spec))]
+    points = symmetric.copy()
+    if where == "all":
+        points = rng.normal(size=points.shape)
+    else:
+        points[2, 1 * (L + 1)] += 0.5  # key (1, 1), n1 = 0, n2 = 1, l = 0
+    for vals in (points, symmetric, points):
+        ctx.set_sparse_points(zeta, spec, vals, np.ones(len(spec)))
+        ss = O.SparseSet(spec, vals, zeta)
+        ref = np.zeros((len(spec), len(spec)))
+        ref[np.ix_(ss.order, ss.order)] = O.gap_kmm(ss)
+        assert np.abs(ctx.gap_kmm() - ref).max() <= 1e-10 * np.abs(ref).max()
