@@ -537,6 +537,14 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
   }
 }
 
+// Row stride of the expansion's radial functions in LDS: whole vectors, so that
+// every row is aligned for the vector reads and the last one's end inside.
+template <class T, int NT>
+__host__ __device__ constexpr int expansion_row() {
+  constexpr int VN = sizeof(typename Vec2<T>::type) / sizeof(T);
+  return (NT + VN - 1) / VN * VN;
+}
+
 // Expansion c[i][s][n][lm] = [s == s_i][lm == 0] R0[n] / sqrt(4 pi) + sum over
 // the pairs (i, j), s_j = s, of fc R_nl Y_lm, with the layout of the pair
 // phase: a lane holds the sums of its two orders +-mu for every radial channel
@@ -547,7 +555,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_k
 // 8192 centres, n_max 12, l_max 9, FP32; 167 -> 72 us for 4096 centres, FP64.
 template <class T, int NT>
 __host__ __device__ inline size_t expansion_wave_lds(int L1) {
-  return sizeof(T) * (size_t(kBatch) * (((L1 * L1) + 1) / 2 * 2 + size_t(L1) * NT));
+  return sizeof(T) * (size_t(kBatch) * (((L1 * L1) + 1) / 2 * 2 + size_t(L1) * expansion_row<T, NT>()));
 }
 
 template <class T, int NT, int G>
@@ -555,15 +563,16 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 5 : 4) void expansion_wa
     RadialDev rad, int S, PairView pv, T* __restrict__ cout, unsigned long long* __restrict__ keymask) {
   typedef typename Vec2<T>::type V;
   typedef T V4 __attribute__((ext_vector_type(4)));
-  constexpr int PPI = 64 / G, VN = sizeof(V) / sizeof(T);
+  constexpr int PPI = 64 / G, VN = sizeof(V) / sizeof(T), NR = expansion_row<T, NT>();
+  static_assert(NR % VN == 0 && NR >= NT, "rows are read as vectors");
   const int N = rad.N, L = rad.L, L1 = rad.L1, LL = rad.LL, F = N * L1, LP = (LL + 1) / 2 * 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   extern __shared__ __align__(64) unsigned char smem_raw[];
   T* yc = reinterpret_cast<T*>(smem_raw);
   T* Y = yc + 4 * LL + wave * (expansion_wave_lds<T, NT>(L1) / sizeof(T));
-  T* R = Y + kBatch * LP;  // [batch][l][NT]
+  T* R = Y + kBatch * LP;  // [batch][l][NR]
   fill_ylm_table<T>(rad, yc);
-  for (int e = lane; e < kBatch * L1 * NT; e += 64) R[e] = T(0);  // surplus channels stay zero
+  for (int e = lane; e < kBatch * L1 * NR; e += 64) R[e] = T(0);  // surplus channels stay zero
   __syncthreads();
   const int un = lane & (G - 1), grp = lane / G;
   int l = 0;
@@ -616,7 +625,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 5 : 4) void expansion_wa
               r += lane_value(rec.rb, q[b]) * t[b].y;
               r += lane_value(rec.rc, q[b]) * t[b].z;
               r += lane_value(rec.rd, q[b]) * t[b].w;
-              R[(b * L1 + el) * NT + en] = b < nb ? r : T(0);
+              R[(b * L1 + el) * NR + en] = b < nb ? r : T(0);
             }
           }
           wave_sync();
@@ -627,7 +636,7 @@ __global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 5 : 4) void expansion_wa
             const int b = b0 + grp;
             const bool on = unit && b < nb;
             const T yp = on ? Y[b * LP + lp] : T(0), ym = on ? Y[b * LP + lm] : T(0);
-            const V* r = reinterpret_cast<const V*>(R + (b * L1 + l) * NT);
+            const V* r = reinterpret_cast<const V*>(R + (b * L1 + l) * NR);
 #pragma unroll
             for (int n = 0; n < NT; n += VN) {
               const V x = r[n / VN];

@@ -368,3 +368,24 @@ def test_kmm_of_points_that_are_not_symmetric(zeta, N, L, M, where):
         ref = np.zeros((len(spec), len(spec)))
         ref[np.ix_(ss.order, ss.order)] = O.gap_kmm(ss)
         assert np.abs(ctx.gap_kmm() - ref).max() <= 1e-10 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("N,L", [(5, 3), (6, 6), (9, 2), (10, 8)])
+def test_expansion_by_wavefronts_of_odd_pairs_of_channels(N, L):
+    """The expansion by wavefronts built for 6 and 10 channels, whose rows are
+    not whole 16-byte vectors in FP32, against the per-entry kernel; the bounds
+    of the test of the other channel counts."""
+    sts = periodic_box(12, 0.08, (1, 8), d_min=1.0, seed=121)
+    hp = soap_hypers(rc=6.0, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8)
+    copies = 2048 // 12 + 1
+    one, _ = _context(hp, sts)
+    many, _ = _context(hp, sts * copies)
+    for prec, tol in ((_capi.FP64, 1e-13), (_capi.MIXED, 1e-6)):
+        one.set_precision(prec)
+        many.set_precision(prec)
+        one.compute()
+        many.compute()
+        c, km = one.expansion()
+        cm, kmm = many.expansion()
+        assert np.array_equal(kmm.reshape(copies, -1), np.tile(km, (copies, 1)))
+        assert np.abs(cm.reshape(copies, *c.shape) - c).max() <= tol * np.abs(c).max()
