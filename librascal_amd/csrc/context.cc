@@ -2091,24 +2091,18 @@ int rgpu_gram_f64(int64_t rows, int64_t cols, const double* A, double* out) {
       if (cols > 0) std::fill(out, out + nc, 0.0);
       return;
     }
-    DeviceBuffer<double> dA, dAt, dC;
+    DeviceBuffer<double> dA, dAp, dAt, dC;
     DeviceBuffer<int> dI;
     std::vector<int> iota(static_cast<size_t>(cols));
     for (int64_t k = 0; k < cols; ++k) iota[size_t(k)] = int(k);
-    const int64_t lda = (cols + 1) / 2 * 2;  // 16-byte rows
-    double* a = dA.reserve(size_t(rows) * size_t(lda));
+    double* a = dA.reserve(size_t(rows) * size_t(cols));
+    double* ap = cols % 2 ? dAp.reserve(size_t(rows) * size_t(cols + 1)) : nullptr;
     double* at = dAt.reserve(size_t(cols) * size_t(gap_f64_k_stride(rows)));
     double* cm = dC.reserve(nc);
     int* io = dI.reserve(iota.size());
-    if (lda == cols) {
-      RGPU_HIP(hipMemcpy(a, A, sizeof(double) * size_t(rows) * size_t(cols), hipMemcpyHostToDevice));
-    } else {
-      RGPU_HIP(hipMemset(a, 0, sizeof(double) * size_t(rows) * size_t(lda)));
-      RGPU_HIP(hipMemcpy2D(a, sizeof(double) * size_t(lda), A, sizeof(double) * size_t(cols),
-                           sizeof(double) * size_t(cols), size_t(rows), hipMemcpyHostToDevice));
-    }
+    RGPU_HIP(hipMemcpy(a, A, sizeof(double) * size_t(rows) * size_t(cols), hipMemcpyHostToDevice));
     RGPU_HIP(hipMemcpy(io, iota.data(), sizeof(int) * iota.size(), hipMemcpyHostToDevice));
-    run_gram_f64(rows, cols, a, lda, at, io, cm, nullptr);
+    run_gram_f64(rows, cols, a, ap, at, io, cm, nullptr);
     RGPU_HIP(hipMemcpy(out, cm, sizeof(double) * nc, hipMemcpyDeviceToHost));
   });
 }

@@ -29,9 +29,10 @@ void run_gap_f64_rows(const GapBlock<double>* blks, int n_blocks, double* out, i
 void run_gap_f64_force(const GapBlock<double>* blks, int n_blocks, double* const* wts, const double* xg,
                        double xg_scale, double* G, hipStream_t stream);
 
-// C (n x n) = A^T A for A [rows][lda >= n], lda even (device pointers; At:
-// room for n x gap_f64_k_stride(rows) doubles, iota: 0 .. n-1 as ints)
-void run_gram_f64(int64_t rows, int64_t n, const double* A, int64_t lda, double* At, const int* iota, double* C,
+// C (n x n) = A^T A for A [rows][n] (device pointers; Ap: room for rows x (n +
+// 1) doubles when n is odd, else not used; At: room for n x
+// gap_f64_k_stride(rows) doubles; iota: 0 .. n-1 as ints)
+void run_gram_f64(int64_t rows, int64_t n, const double* A, double* Ap, double* At, const int* iota, double* C,
                   hipStream_t stream);
 
 }  // namespace rgpu

@@ -389,3 +389,13 @@ def test_expansion_by_wavefronts_of_odd_pairs_of_channels(N, L):
         cm, kmm = many.expansion()
         assert np.array_equal(kmm.reshape(copies, -1), np.tile(km, (copies, 1)))
         assert np.abs(cm.reshape(copies, *c.shape) - c).max() <= tol * np.abs(c).max()
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (15, 1), (16, 63), (17, 64), (33, 65), (47, 3), (1001, 333)])
+def test_gram_of_odd_and_even_columns(shape):
+    """A^T A where the rows of A are padded to an even length (an odd number of
+    columns) and where they are not, at the edges of the 64-wide tiles and of
+    the K steps of 16."""
+    A = np.random.default_rng(shape[0]).normal(size=shape)
+    ref = A.T @ A
+    assert np.abs(_capi.gram_f64(A) - ref).max() <= 1e-12 * np.abs(ref).max()
