@@ -1479,10 +1479,11 @@ void autotune_t(Context& c) {
       t.adj_kind = bestv.adj_kind;
     }
     // pairs per batch of the pair phase in the adjoint's workgroup (0: the
-    // most that fit; adj_kind 3 has a kernel of its own for it)
+    // most that fit).  The pair phase by wavefronts, FP64's where it applies
+    // and adj_kind 3's, takes no partition.
     best = 1e30f;
     pick = 0;
-    if (!split || t.adj_kind != 3)
+    if (split ? t.adj_kind != 3 : !pair_kernels_apply(c.rd))
       for (int pb : {0, 2, 4, 6, 8, 12, 16, 24, 32}) {
         SoapTiles cand = t;
         cand.pb_adj = pb;

@@ -399,3 +399,19 @@ def test_gram_of_odd_and_even_columns(shape):
     A = np.random.default_rng(shape[0]).normal(size=shape)
     ref = A.T @ A
     assert np.abs(_capi.gram_f64(A) - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("spline,L", [(1e-8, 3), (1e-8, 10), (None, 3)])
+def test_autotuned_fp64_pair_phase(spline, L):
+    """The FP64 autotuner chooses pairs per batch for the general pair phase
+    only: the one by wavefronts takes none, and the set reports none."""
+    sts = periodic_box(60, 0.05, (1, 8), d_min=1.0, seed=131)
+    ctx, _ = _context(soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=5, L=L, spline=spline), sts)
+    X, _ = ctx.features()
+    G = np.random.default_rng(132).normal(size=X.shape)
+    g, s = ctx.features_backward(G)
+    tiles = ctx.autotune()
+    assert tiles["pairs_adj"] in ((0,) if spline and L <= 9 else (0, 2, 4, 6, 8, 12, 16, 24, 32))
+    gt, st = ctx.features_backward(G)
+    assert np.abs(gt - g).max() <= 1e-12 * np.abs(g).max()
+    assert np.abs(st - s).max() <= 1e-12 * np.abs(s).max()
