@@ -78,10 +78,10 @@ struct Context {
   // coefficient_subselection: full-layout column of each selected
   // coefficient (-1 for a species pair outside the batch's species list)
   std::vector<int64_t> sel_col;
-  DeviceBuffer<int64_t> d_sel_col, d_sel_inv_off, d_sel_inv_k;  // selection and its inverse
+  DeviceBuffer<int64_t> d_sel_col, d_sel_packed, d_sel_inv_off, d_sel_inv_k;  // selection and its inverse
   SelectionMap selection() const {
     SelectionMap m;
-    m.col = d_sel_col.get();
+    m.packed = d_sel_packed.get();
     m.inv_off = d_sel_inv_off.get();
     m.inv_k = d_sel_inv_k.get();
     return m;
@@ -90,9 +90,12 @@ struct Context {
   // representation
   bool have_rep = false;
   // FP64 invariants as symmetric packed rows (sym_kernels.hh), and in the
-  // full layout where something needs that (sparsified: S^T ps64)
+  // full layout where something needs that
   DeviceBuffer<double> c64, p64, pfull;
-  DeviceBuffer<double> ps64;         // selected invariants [n_atoms][ldx64()] (un-normalised)
+  // sparsified: the selected invariants [n_atoms][ldx64()] (un-normalised), and
+  // S^T of them in the full layout and packed, formed when an adjoint asks
+  DeviceBuffer<double> ps64, sel_full, sel_packed;
+  bool sel_valid = false;
   DeviceBuffer<double> gfull, gsym;  // dL/dX scattered into the full layout, and packed
   DeviceBuffer<double> dc64, xdot;   // dL/dc of the FP64 adjoint, X . dL/dX
   DeviceBuffer<double> dcp, dcs;     // stored expansion derivatives (gradient export)
@@ -676,19 +679,19 @@ void compute_rep(Context& c) {
   // FP64 keeps the invariants in FP64 (symmetric packed rows); the mixed
   // path stores them as the BF16 hi/lo operand planes of the matrix-core GEMMs
   double* pp = nullptr;
-  double* pf = nullptr;  // the full layout of the fused launch and of a selection
+  double* pf = nullptr;  // the full layout of the fused launch
   if (ps && !split) {
     pp = c.p64.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
-    if (c.sparsified() || c.tile().fused == 1) pf = c.pfull.reserve(size_t(std::max<int64_t>(n * D, 1)));
+    if (c.tile().fused == 1) pf = c.pfull.reserve(size_t(std::max<int64_t>(n * D, 1)));
   }
   const int64_t Dp = c.Dp();
   unsigned short* ph = ps && split ? c.p_hi.reserve(size_t(std::max<int64_t>(n * Dp, 1))) : nullptr;
   unsigned short* pl = ps && split ? c.p_lo.reserve(size_t(std::max<int64_t>(n * Dp, 1))) : nullptr;
   double* n2 = ps ? c.norm2.reserve(size_t(std::max<int64_t>(n, 1))) : nullptr;
-  // sparsified: the selected coefficients and their norms (p keeps S^T xs)
+  // sparsified: the selected coefficients and their norms
   double* xs = split || !c.sparsified() ? nullptr
                                         : c.ps64.reserve(size_t(std::max<int64_t>(n * c.ldx64(), 1)));
-  c.p32_valid = false;
+  c.p32_valid = c.sel_valid = false;
   const int64_t* n_pairs_dev = c.pl.centre_off.get() + n;
   // the half list's buffers are sized for the full list, before any capture
   HalfList hl{};
@@ -731,13 +734,13 @@ void compute_rep(Context& c) {
     if constexpr (split) {
       if (!fused) launch_power_spectrum_split(c.rd, S, n, cc, ph, pl, n2, c.stream, c.tile());
     } else {
-      if (!fused) launch_sym_power(S, c.rd.N, c.rd.L1, n, cc, pp, n2, c.stream);
-      if (xs) {
-        if (!fused) launch_sym_unpack(S, c.rd.N, c.rd.L1, n, pp, nullptr, nullptr, false, pf, c.stream);
-        launch_sparsify(n, D, c.D(), c.ldx64(), c.selection(), pf, xs, n2, c.stream);
-      }
-      if (fused || xs)
+      if (fused)
         launch_sym_pack(S, c.rd.N, c.rd.L1, n, pf, nullptr, pp, c.stream);
+      else
+        launch_sym_power(S, c.rd.N, c.rd.L1, n, cc, pp, n2, c.stream);
+      if (xs)
+        launch_select_invariants(n, sym_row_stride(S, c.rd.N, c.rd.L1), c.D(), c.ldx64(), c.selection(), pp, xs, n2,
+                                 c.stream);
     }
   };
   std::array<uintptr_t, 30> sig{};
@@ -749,7 +752,7 @@ void compute_rep(Context& c) {
         uintptr_t(pl), uintptr_t(n2), uintptr_t(c.pl.centre_off.get()),
         uintptr_t(c.pl.pair_j.get()), uintptr_t(c.pl.pair_vec.get()), uintptr_t(c.pl.pair_dist.get()),
         uintptr_t(c.d_species_of.get()), uintptr_t(c.tile().pb_fwd), uintptr_t(c.tile().kc),
-        uintptr_t(c.d_sel_col.get()), uintptr_t(c.tile().half_nl), uintptr_t(hl.src),
+        uintptr_t(c.d_sel_packed.get()), uintptr_t(c.tile().half_nl), uintptr_t(hl.src),
         uintptr_t(hl.rows), uintptr_t(c.tile().fused), uintptr_t(c.tile().fwd_lds),
         uintptr_t(c.tile().fwd_group), uintptr_t(c.d_sel_inv_off.get()), uintptr_t(c.d_sel_inv_k.get()),
         uintptr_t(pf)};
@@ -936,6 +939,23 @@ void backward_device(Context& c, const float* G, double* grad, double* cvir, con
                         xg_scale, G, cvir, c.stream, c.tile(), work);
   launch_force_gather(pv, rl, grad, c.stream);
 }
+// S^T xs of a selection, in the full layout and packed
+void ensure_selected_rows(Context& c) {
+  if (c.sel_valid) return;
+  const int S = int(c.species.size());
+  const int64_t n = c.n_atoms, D = c.D_full();
+  double* f = c.sel_full.reserve(size_t(std::max<int64_t>(n * D, 1)));
+  double* s = c.sel_packed.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
+  launch_scatter_columns(n, c.ldx64(), c.selection(), c.ps64.get(), D, f, c.stream);
+  launch_sym_pack(S, c.rd.N, c.rd.L1, n, f, nullptr, s, c.stream);
+  c.sel_valid = true;
+}
+// the un-normalised FP64 features (a selection's scattered) in packed rows
+const double* packed_features(Context& c) {
+  if (!c.sparsified()) return c.p64.get();
+  ensure_selected_rows(c);
+  return c.sel_packed.get();
+}
 // FP64 pair phase of the adjoint from dL/dc
 void launch_pair_phase(Context& c, const PairView& pv, const double* dc, double* cvir) {
   const int S = int(c.species.size());
@@ -953,8 +973,8 @@ void backward_device(Context& c, const double* G, bool full, const double* xg, d
   const PairView pv = backward_view(c, &rl);
   double* dc = c.dc64.reserve(size_t(c.n_atoms * S * N * c.rd.LL + kPairSlack));
   if (full)
-    launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), c.hp.normalize ? c.p64.get() : nullptr, c.norm2.get(),
-                             xg, G, c.gsym, dc, c.stream);
+    launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), c.hp.normalize ? packed_features(c) : nullptr,
+                             c.norm2.get(), xg, G, c.gsym, dc, c.stream);
   else
     launch_sym_contract(S, N, L1, c.n_atoms, c.c64.get(), G, dc, c.stream);
   launch_pair_phase(c, pv, dc, cvir);
@@ -966,9 +986,8 @@ const double* scatter_selected(Context& c, const double* G, int64_t ld) {
   launch_scatter_columns(c.n_atoms, ld, c.selection(), G, c.D_full(), gf, c.stream);
   return gf;
 }
-// the FP64 invariants in the full layout (a selection keeps them: S^T xs)
+// the FP64 invariants in the full layout
 const double* full_invariants(Context& c) {
-  if (c.sparsified()) return c.pfull.get();
   double* pf = c.pfull.reserve(size_t(std::max<int64_t>(c.n_atoms * c.D_full(), 1)));
   launch_sym_unpack(int(c.species.size()), c.rd.N, c.rd.L1, c.n_atoms, c.p64.get(), nullptr, nullptr, false, pf,
                     c.stream);
@@ -1703,7 +1722,8 @@ int rgpu_set_structures(rgpu_context* ctx, int n_struct, const int64_t* atom_off
     }
     // coefficient_subselection: full-layout column of each selected
     // coefficient over this species list
-    std::vector<int64_t> scol;
+    // and its entry of a symmetric packed row (SelectionMap)
+    std::vector<int64_t> scol, spacked;
     if (c.hp.kind == SoapHypers::kPowerSpectrum && c.hp.sparsified) {
       const int N = c.hp.max_radial, L1 = c.hp.max_angular + 1, S = int(sp.size());
       for (size_t k = 0; k < c.hp.sel_a.size(); ++k) {
@@ -1711,12 +1731,17 @@ int rgpu_set_structures(rgpu_context* ctx, int n_struct, const int64_t* atom_off
         auto ib = std::lower_bound(sp.begin(), sp.end(), c.hp.sel_b[k]);
         if (ia == sp.end() || *ia != c.hp.sel_a[k] || ib == sp.end() || *ib != c.hp.sel_b[k]) {
           scol.push_back(-1);
+          spacked.push_back(-1);
           continue;
         }
         const int a = int(ia - sp.begin()), b = int(ib - sp.begin());
         const int64_t key = int64_t(a) * S - int64_t(a) * (a - 1) / 2 + (b - a);
         scol.push_back((key * N * N + int64_t(c.hp.sel_n1[k]) * N + c.hp.sel_n2[k]) * L1 +
                        c.hp.sel_l[k]);
+        const int r0 = a * N + c.hp.sel_n1[k], r1 = b * N + c.hp.sel_n2[k];
+        const int64_t lo = std::min(r0, r1), hi = std::max(r0, r1);
+        spacked.push_back(2 * (c.hp.sel_l[k] * sym_tri(int64_t(S) * N) + sym_tri(hi) + lo) +
+                          (a == b && r0 != r1 ? 1 : 0));
       }
     }
     // RadialDimReduction: the spline table of each batch species (a species
@@ -1756,6 +1781,8 @@ int rgpu_set_structures(rgpu_context* ctx, int n_struct, const int64_t* atom_off
       int64_t* dsc = c.d_sel_col.reserve(scol.size());
       RGPU_HIP(hipMemcpyAsync(dsc, scol.data(), sizeof(int64_t) * scol.size(), hipMemcpyHostToDevice,
                               c.stream));
+      int64_t* dsp = c.d_sel_packed.reserve(spacked.size());
+      RGPU_HIP(hipMemcpyAsync(dsp, spacked.data(), sizeof(int64_t) * spacked.size(), hipMemcpyHostToDevice, c.stream));
       // inverse: the selections naming each full-layout column, ascending
       const int64_t Df = c.D_full();
       std::vector<int64_t> inv_off(size_t(Df + 1), 0), inv_k;
@@ -1985,7 +2012,8 @@ int rgpu_features_backward(rgpu_context* ctx, const double* dL_dX, double* dL_dr
         g64 = scatter_selected(c, g64, D);
         if (c.hp.normalize) {
           double* d = c.xdot.reserve(size_t(std::max<int64_t>(n, 1)));
-          launch_row_dot(n, c.D_full(), c.pfull.get(), g64, c.norm2.get(), d, c.stream);
+          ensure_selected_rows(c);
+          launch_row_dot(n, c.D_full(), c.sel_full.get(), g64, c.norm2.get(), d, c.stream);
           dot = d;
         }
       }
@@ -2188,7 +2216,7 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
     const double* dp = nullptr;
     if (c.hp.normalize) {
       double* e = c.knm_dp.reserve(size_t(n * E));
-      launch_sym_contract(S, N, L1, n, c.c64.get(), c.p64.get(), e, c.stream);
+      launch_sym_contract(S, N, L1, n, c.c64.get(), packed_features(c), e, c.stream);
       dp = e;
     }
     // column m (species-sorted): dL/dX_i = zeta d_im^(zeta-1) T_m for the

@@ -167,19 +167,20 @@ void launch_feature_gradient_rows(int N, int L1, int S, const PairView& pv, int6
                                   const double* c, const double* p_rows, const double* norm2,
                                   bool normalize, const double* dcp, const double* dcs, int64_t Dout,
                                   const int64_t* col, double* out, hipStream_t stream);
-// coefficient_subselection as device arrays: col[k] (Dsel; -1 for a
-// coefficient outside the layout) and its inverse, the selections k naming
-// full-layout column o in ascending order at inv_k[inv_off[o] ..
-// inv_off[o+1])
+// coefficient_subselection as device arrays: packed[k] (Dsel; -1 for a
+// coefficient outside the layout), twice the entry of a symmetric packed row
+// (sym_kernels.hh) that holds coefficient k, plus 1 where the entry is sqrt 2
+// times it; and the selections k naming full-layout column o in ascending
+// order at inv_k[inv_off[o] .. inv_off[o+1])
 struct SelectionMap {
-  const int64_t* col = nullptr;
+  const int64_t* packed = nullptr;
   const int64_t* inv_off = nullptr;
   const int64_t* inv_k = nullptr;
 };
-// xs[i][k] = p[i][col[k]] (rows lds apart, zero pad), norm2[i] = |xs_i|^2,
-// then p[i] = S^T xs_i (the selected coefficients, zero elsewhere)
-void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, int64_t lds, const SelectionMap& sel, double* p, double* xs,
-                     double* norm2, hipStream_t stream);
+// xs[i] = the selected coefficients (rows lds apart, zero pad) of the symmetric
+// packed rows p (ld apart), norm2[i] = |xs_i|^2
+void launch_select_invariants(int64_t n, int64_t ld, int64_t Dsel, int64_t lds, const SelectionMap& sel,
+                              const double* p, double* xs, double* norm2, hipStream_t stream);
 // dst[i][:D] = S^T src[i][:Dsel], src rows lds apart (repeated selections summed in ascending
 // selection order)
 void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t D,

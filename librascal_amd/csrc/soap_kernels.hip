@@ -2640,42 +2640,32 @@ __global__ __launch_bounds__(kThreads) void feature_gradient_rows_kernel(
     }
 }
 
-// Sparsified invariants (coefficient_subselection): xs[i][k] = p[i][col[k]]
-// (0 for col[k] < 0) and norm2[i] = |xs_i|^2; then row i of p becomes S^T xs_i
-// for the selection matrix S (the selected coefficients, summed over
-// repeated selections, zero elsewhere): with it and |xs_i| the adjoint's
-// normalisation term is the one of the selected features.
-__global__ __launch_bounds__(kThreads) void sparsify_kernel(int64_t D, int64_t Dsel, int64_t lds,
-                                                            const int64_t* __restrict__ col,
-                                                            const int64_t* __restrict__ inv_off,
-                                                            const int64_t* __restrict__ inv_k,
-                                                            double* __restrict__ p,
-                                                            double* __restrict__ xs,
-                                                            double* __restrict__ norm2) {
+// Sparsified invariants (coefficient_subselection): xs[i][k] = p[i] at the
+// packed entry of the selected coefficient (0 where there is none) and norm2[i]
+// = |xs_i|^2, one workgroup per row
+__global__ __launch_bounds__(kThreads) void select_invariants_kernel(int64_t ld, int64_t Dsel, int64_t lds,
+                                                                     const int64_t* __restrict__ packed,
+                                                                     const double* __restrict__ p,
+                                                                     double* __restrict__ xs,
+                                                                     double* __restrict__ norm2) {
   const int64_t i = blockIdx.x;
-  double* pi = p + i * D;
+  const double* pi = p + i * ld;
   double* xi = xs + i * lds;
-  for (int64_t k = Dsel + threadIdx.x; k < lds; k += kThreads) xi[k] = 0.0;
   double ss = 0;
-  for (int64_t k = threadIdx.x; k < Dsel; k += kThreads) {
-    const double v = col[k] >= 0 ? pi[col[k]] : 0.0;
+  for (int64_t k = threadIdx.x; k < lds; k += kThreads) {
+    const int64_t e = k < Dsel ? packed[k] : -1;
+    const double v = e < 0 ? 0.0 : pi[e >> 1] * (e & 1 ? 0.70710678118654752440 : 1.0);
     xi[k] = v;
     ss += v * v;
   }
   __shared__ double red[kWaves];
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_down(ss, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();  // also: every selected value has been read and xi written
+  __syncthreads();
   if (threadIdx.x == 0) {
     double t = 0;
     for (int w = 0; w < kWaves; ++w) t += red[w];
     norm2[i] = t;
-  }
-  // column o takes the selections naming it, in ascending selection order
-  for (int64_t o = threadIdx.x; o < D; o += kThreads) {
-    double t = 0.0;
-    for (int64_t q = inv_off[o]; q < inv_off[o + 1]; ++q) t += xi[inv_k[q]];
-    pi[o] = t;
   }
 }
 
@@ -3250,11 +3240,11 @@ void launch_feature_gradient_rows(int N, int L1, int S, const PairView& pv, int6
   RGPU_LAUNCH_CHECK();
 }
 
-void launch_sparsify(int64_t n, int64_t D, int64_t Dsel, int64_t lds, const SelectionMap& sel, double* p, double* xs,
-                     double* norm2, hipStream_t stream) {
+void launch_select_invariants(int64_t n, int64_t ld, int64_t Dsel, int64_t lds, const SelectionMap& sel,
+                              const double* p, double* xs, double* norm2, hipStream_t stream) {
   if (n == 0) return;
-  hipLaunchKernelGGL(sparsify_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, Dsel, lds, sel.col,
-                     sel.inv_off, sel.inv_k, p, xs, norm2);
+  hipLaunchKernelGGL(select_invariants_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, ld, Dsel, lds,
+                     sel.packed, p, xs, norm2);
   RGPU_LAUNCH_CHECK();
 }
 

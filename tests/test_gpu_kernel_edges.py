@@ -415,3 +415,64 @@ def test_autotuned_fp64_pair_phase(spline, L):
     gt, st = ctx.features_backward(G)
     assert np.abs(gt - g).max() <= 1e-12 * np.abs(g).max()
     assert np.abs(st - s).max() <= 1e-12 * np.abs(s).max()
+
+
+def _selection(S, N, L, seed, k=25, repeats=True):
+    """k selected coefficients of species pairs a <= b, either order of the
+    radial channels, and one of a species outside the batch: the hypers and the
+    dense columns of all but that last one."""
+    rng = np.random.default_rng(seed)
+    a = rng.integers(1, S + 1, k)
+    b = np.maximum(a, rng.integers(1, S + 1, k))
+    rows = np.stack([a, b, rng.integers(0, N, k), rng.integers(0, N, k), rng.integers(0, L + 1, k)], axis=1)
+    if not repeats:
+        rows = rng.permutation(np.unique(rows, axis=0))
+    a, b, n1, n2, l = rows.T
+    key = (a - 1) * S - (a - 1) * (a - 2) // 2 + (b - a)
+    sub = {q: v.tolist() + [e] for q, v, e in zip(("a", "b", "n1", "n2", "l"), rows.T, (1, 99, 0, 0, 0))}
+    return sub, ((key * N + n1) * N + n2) * (L + 1) + l
+
+
+@pytest.mark.parametrize("S,N,L,normalize", [(1, 2, 0, True), (2, 5, 3, True), (3, 4, 2, False), (2, 16, 4, True)])
+def test_selected_invariants_from_packed_rows(S, N, L, normalize):
+    """coefficient_subselection taken from the packed rows: the features, their
+    adjoint (several times on one representation, and on the next positions
+    through a graph replay) and K_NM gradient against the dense layout.
+    (Repeated coefficients without normalisation.)"""
+    sts = periodic_box(9 * S + 2, 0.05, tuple(range(1, S + 1)), d_min=1.0, seed=141)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=False)
+    if N > 13:
+        hp["radial_contribution"]["type"] = "DVR"
+    rng = np.random.default_rng(142)
+    sub, col = _selection(S, N, L, 143, repeats=not normalize)
+    raw, num = _context(hp, sts)
+    sel, _ = _context(dict(hp, normalize=normalize, coefficient_subselection=sub), sts)
+    sel.enable_graphs()
+    pos = pack(sts)[1]
+    for step in range(2):
+        for c in (raw, sel):
+            c.update_positions(pos * (1 - 0.02 * step))
+            c.compute()
+        P, _ = raw.features()
+        p = np.hstack([P[:, col], np.zeros((len(num), 1))])
+        norm = np.linalg.norm(p, axis=1, keepdims=True) if normalize else np.ones((len(num), 1))
+        X, _ = sel.features()
+        assert np.abs(X - p / norm).max() <= 1e-12 * np.abs(p / norm).max()
+
+        def backward(G):
+            # dL/dp of the selection, summed into the dense columns
+            g = (G - X * (X * G).sum(1, keepdims=True)) / norm if normalize else G
+            dense = np.zeros(P.shape)
+            np.add.at(dense.T, col, g[:, :-1].T)
+            return raw.features_backward(dense)
+
+        for _ in range(2):
+            G = rng.normal(size=X.shape)
+            for x, y in zip(backward(G), sel.features_backward(G)):
+                assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max()
+        T = X[:3] + 0.01
+        sel.set_sparse_points(2, num[:3], T, np.ones(3))
+        out = sel.gap_knm_gradient()
+        ref = np.stack([backward(np.where(num == num[m], 2 * (X @ T[m]), 0.0)[:, None] * T[m])[0].ravel()
+                        for m in range(3)], axis=1)
+        assert np.abs(out - ref).max() <= 1e-10 * np.abs(ref).max()
