@@ -93,8 +93,8 @@ struct Context {
   // full layout where something needs that
   DeviceBuffer<double> c64, p64, pfull;
   // sparsified: the selected invariants [n_atoms][ldx64()] (un-normalised), and
-  // S^T of them in the full layout and packed, formed when an adjoint asks
-  DeviceBuffer<double> ps64, sel_full, sel_packed;
+  // S^T of them in packed rows, formed when an adjoint asks
+  DeviceBuffer<double> ps64, sel_packed;
   bool sel_valid = false;
   DeviceBuffer<double> gfull, gsym;  // dL/dX scattered into the full layout, and packed
   DeviceBuffer<double> dc64, xdot;   // dL/dc of the FP64 adjoint, X . dL/dX
@@ -939,21 +939,18 @@ void backward_device(Context& c, const float* G, double* grad, double* cvir, con
                         xg_scale, G, cvir, c.stream, c.tile(), work);
   launch_force_gather(pv, rl, grad, c.stream);
 }
-// S^T xs of a selection, in the full layout and packed
-void ensure_selected_rows(Context& c) {
-  if (c.sel_valid) return;
-  const int S = int(c.species.size());
-  const int64_t n = c.n_atoms, D = c.D_full();
-  double* f = c.sel_full.reserve(size_t(std::max<int64_t>(n * D, 1)));
-  double* s = c.sel_packed.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
-  launch_scatter_columns(n, c.ldx64(), c.selection(), c.ps64.get(), D, f, c.stream);
-  launch_sym_pack(S, c.rd.N, c.rd.L1, n, f, nullptr, s, c.stream);
-  c.sel_valid = true;
-}
-// the un-normalised FP64 features (a selection's scattered) in packed rows
+// the un-normalised FP64 features in packed rows (a selection's: S^T xs)
 const double* packed_features(Context& c) {
   if (!c.sparsified()) return c.p64.get();
-  ensure_selected_rows(c);
+  if (!c.sel_valid) {
+    const int S = int(c.species.size());
+    const int64_t n = c.n_atoms, D = c.D_full();
+    double* f = c.pfull.reserve(size_t(std::max<int64_t>(n * D, 1)));
+    double* s = c.sel_packed.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
+    launch_scatter_columns(n, c.ldx64(), c.selection(), c.ps64.get(), D, f, c.stream);
+    launch_sym_pack(S, c.rd.N, c.rd.L1, n, f, nullptr, s, c.stream);
+    c.sel_valid = true;
+  }
   return c.sel_packed.get();
 }
 // FP64 pair phase of the adjoint from dL/dc
@@ -2009,13 +2006,14 @@ int rgpu_features_backward(rgpu_context* ctx, const double* dL_dX, double* dL_dr
     if (c.precision == RGPU_FP64) {
       const double* dot = nullptr;
       if (c.sparsified()) {
-        g64 = scatter_selected(c, g64, D);
+        // (X . dL/dX over the selection itself: a coefficient selected twice
+        // enters both factors of a product of the spread-out rows twice)
         if (c.hp.normalize) {
           double* d = c.xdot.reserve(size_t(std::max<int64_t>(n, 1)));
-          ensure_selected_rows(c);
-          launch_row_dot(n, c.D_full(), c.sel_full.get(), g64, c.norm2.get(), d, c.stream);
+          launch_row_dot(n, D, c.ps64.get(), c.ldx64(), g64, D, c.norm2.get(), d, c.stream);
           dot = d;
         }
+        g64 = scatter_selected(c, g64, D);
       }
       backward_device(c, g64, true, dot, gd, cv);
     } else {

@@ -193,9 +193,10 @@ void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, con
 // dL/dr_j, Voigt xx,yy,zz,yz,xz,xy, not divided by the volume).
 void launch_adjoint_pairs(const RadialDev& rad, int S, const PairView& pv, const double* dc,
                           double* centre_virial, hipStream_t stream, const SoapTiles& tiles = SoapTiles());
-// dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values
-void launch_row_dot(int64_t n, int64_t D, const double* a, const double* b, const double* norm2, double* dot,
-                    hipStream_t stream);
+// dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values, lda
+// and ldb apart
+void launch_row_dot(int64_t n, int64_t D, const double* a, int64_t lda, const double* b, int64_t ldb,
+                    const double* norm2, double* dot, hipStream_t stream);
 // dst row r (ldd values, zero past D) = src row rows[r] (D values)
 template <class To>
 void launch_gather_rows(int64_t n, int64_t D, int64_t ldd, const double* src, const int64_t* rows, To* dst,

@@ -1193,14 +1193,14 @@ __global__ __launch_bounds__(kThreads) void adjoint_pairs_kernel(RadialDev rad, 
 }
 
 // dot[i] = a_i . b_i / sqrt(norm2[i]) (0 for a zero norm), rows of D values
-__global__ __launch_bounds__(kThreads) void row_dot_kernel(int64_t D, const double* __restrict__ a,
-                                                           const double* __restrict__ b,
+__global__ __launch_bounds__(kThreads) void row_dot_kernel(int64_t D, const double* __restrict__ a, int64_t lda,
+                                                           const double* __restrict__ b, int64_t ldb,
                                                            const double* __restrict__ norm2,
                                                            double* __restrict__ dot) {
   const int64_t i = blockIdx.x;
   __shared__ double red[kWaves];
   double d = 0;
-  for (int64_t o = threadIdx.x; o < D; o += kThreads) d += a[i * D + o] * b[i * D + o];
+  for (int64_t o = threadIdx.x; o < D; o += kThreads) d += a[i * lda + o] * b[i * ldb + o];
   for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d;
   __syncthreads();
@@ -3281,10 +3281,10 @@ void launch_adjoint_pairs(const RadialDev& rad, int S, const PairView& pv, const
   RGPU_LAUNCH_CHECK();
 }
 
-void launch_row_dot(int64_t n, int64_t D, const double* a, const double* b, const double* norm2, double* dot,
-                    hipStream_t stream) {
+void launch_row_dot(int64_t n, int64_t D, const double* a, int64_t lda, const double* b, int64_t ldb,
+                    const double* norm2, double* dot, hipStream_t stream) {
   if (n == 0) return;
-  hipLaunchKernelGGL(row_dot_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, a, b, norm2, dot);
+  hipLaunchKernelGGL(row_dot_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, D, a, lda, b, ldb, norm2, dot);
   RGPU_LAUNCH_CHECK();
 }
 

@@ -476,3 +476,28 @@ def test_selected_invariants_from_packed_rows(S, N, L, normalize):
         ref = np.stack([backward(np.where(num == num[m], 2 * (X @ T[m]), 0.0)[:, None] * T[m])[0].ravel()
                         for m in range(3)], axis=1)
         assert np.abs(out - ref).max() <= 1e-10 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("S,N,L", [(1, 1, 0), (2, 3, 2)])
+def test_adjoint_of_repeated_selections(S, N, L):
+    """Normalised features whose selection repeats coefficients: the adjoint
+    against the dense layout's (repeated entries of dL/dX add up; the
+    normalisation's part is over the selection's own entries)."""
+    sts = periodic_box(9 * S + 2, 0.05, tuple(range(1, S + 1)), d_min=1.0, seed=151)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=False)
+    sub, col = _selection(S, N, L, 152, k=60)
+    raw, num = _context(hp, sts)
+    sel, _ = _context(dict(hp, normalize=True, coefficient_subselection=sub), sts)
+    P, _ = raw.features()
+    p = np.hstack([P[:, col], np.zeros((len(num), 1))])
+    norm = np.linalg.norm(p, axis=1, keepdims=True)
+    X, _ = sel.features()
+    assert np.abs(X - p / norm).max() <= 1e-12
+    G = np.random.default_rng(153).normal(size=X.shape)
+    g = (G - X * (X * G).sum(1, keepdims=True)) / norm
+    dense, scale = np.zeros(P.shape), np.zeros(P.shape)
+    np.add.at(dense.T, col, g[:, :-1].T)
+    np.add.at(scale.T, col, (np.abs(G) / norm)[:, :-1].T)
+    # (a single function's reference is zero but for rounding)
+    for x, y, s in zip(raw.features_backward(dense), sel.features_backward(G), raw.features_backward(scale)):
+        assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max() + 1e-13 * np.abs(s).max()
