@@ -2691,9 +2691,15 @@ __global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t lds,
 // for several workgroups per CU; the adjoint may use more.  The power
 // spectrum's 32 KB put five on a CU; more keys per pass in 48 KB, three: 8192
 // centres of 4 species (n_max 12, l_max 9) 339 us, with 40 KB 300, 32 KB 287,
-// 24 KB 297 us; 3 species 163, 133, 121, 132 us.
+// 24 KB 297 us; 3 species 163, 133, 121, 132 us.  Where that is more than 8
+// passes (many species), each a chain with two barriers, their number counts
+// for more: up to 48 KB there.  Expansion and power spectrum in 32 KB and so:
+// 1725 centres of 10 species (n_max 6, l_max 12) 751 -> 353 us, 16 of 6
+// (n_max 12, l_max 9) 99 -> 71 us and 2500 of them 286 -> 239 us, 434 of 10
+// (n_max 12, l_max 6) 150 -> 118 us.
 constexpr size_t kFwdBudget = 32 * 1024;
-constexpr size_t kPsBudget = 32 * 1024;
+constexpr size_t kPsBudget = 32 * 1024, kPsBudgetMany = 48 * 1024;
+constexpr int kPsPasses = 8;
 constexpr size_t kAdjBudget = 64 * 1024;
 constexpr size_t kResidentBudget = 52 * 1024;  // three workgroups per CU
 
@@ -2995,7 +3001,9 @@ size_t power_spectrum_lds(const RadialDev& rad, int S, const SoapTiles& tiles, i
   const int K = S * (S + 1) / 2;
   const size_t cbytes = sizeof(T) * align_up((size_t(S) * rad.N + 3) * (rad.LL | 1), 4);
   const size_t kb = sizeof(T) * size_t(rad.N) * rad.N * rad.L1;
-  int KC = cbytes + kb < kPsBudget ? int((kPsBudget - cbytes) / kb) : 1;
+  auto keys_in = [&](size_t budget) { return cbytes + kb < budget ? int((budget - cbytes) / kb) : 1; };
+  int KC = keys_in(kPsBudget);
+  if (KC * kPsPasses < K) KC = std::max(KC, std::min(keys_in(kPsBudgetMany), (K + kPsPasses - 1) / kPsPasses));
   if (tiles.kc > 0) KC = tiles.kc;
   *keys = KC = std::max(1, std::min(KC, K));
   return cbytes + size_t(KC) * kb + sizeof(int) * size_t(K + rad.N * (rad.N + 1) / 2);

@@ -501,3 +501,16 @@ def test_adjoint_of_repeated_selections(S, N, L):
     # (a single function's reference is zero but for rounding)
     for x, y, s in zip(raw.features_backward(dense), sel.features_backward(G), raw.features_backward(scale)):
         assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max() + 1e-13 * np.abs(s).max()
+
+
+@pytest.mark.parametrize("S,N,L", [(6, 12, 9), (10, 6, 12), (8, 8, 8), (13, 2, 3)])
+def test_mixed_power_spectrum_of_many_species(S, N, L):
+    """Key blocks per pass of the mixed power spectrum on both sides of its
+    rule (few large passes, many small ones, all keys in one): the features
+    within FP32 rounding of the FP64 ones."""
+    sts = periodic_box(3 * S + 1, 0.05, tuple(range(1, S + 1)), d_min=1.0, seed=161)
+    ctx, _ = _context(soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8), sts)
+    X, _ = ctx.features()
+    ctx.set_precision(_capi.MIXED)
+    Xm, _ = ctx.features()
+    assert np.abs(Xm - X).max() <= 1e-5 * np.abs(X).max()
