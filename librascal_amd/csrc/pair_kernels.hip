@@ -313,6 +313,20 @@ __device__ __forceinline__ T group_sums(T v0, T v1, T v2, T v3, int lane) {
   }
 }
 
+// Wavefronts per SIMD that the registers are shared out for.  Past 16 channels
+// (FP64: past 12) a lane's channels spilled at the usual number (24 channels
+// in FP64: 80 to 105 registers): 4520 centres of 3 species, n_max 20, l_max 2,
+// FP64 expansion with the features 199 -> 156 us; the adjoint of 700 centres,
+// n_max 24, l_max 2, 109 -> 95 us.
+template <class T, int NT>
+__host__ __device__ constexpr int force_waves() {
+  return sizeof(T) == 4 ? (NT <= 16 ? 4 : 3) : (NT <= 12 ? 3 : 2);
+}
+template <class T, int NT>
+__host__ __device__ constexpr int expansion_waves() {
+  return sizeof(T) == 4 ? (NT <= 16 ? 5 : 4) : (NT <= 12 ? 4 : (NT <= 16 ? 3 : 2));
+}
+
 // per-wavefront LDS of the pair phase
 template <class T, int NT>
 __host__ __device__ inline size_t force_wave_lds(int L1) {
@@ -322,7 +336,7 @@ __host__ __device__ inline size_t force_wave_lds(int L1) {
 // NT: radial channels rounded up (the surplus ones zero); G: lanes per pair;
 // W: wavefronts per centre
 template <class T, int NT, int G, int W>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 4 : 3) void pair_force_kernel(RadialDev rad, int S, PairView pv,
+__global__ __launch_bounds__(kThreads, (force_waves<T, NT>())) void pair_force_kernel(RadialDev rad, int S, PairView pv,
                                                               const T* __restrict__ dcg,
                                                               double* __restrict__ centre_virial) {
   typedef typename Vec2<T>::type V;
@@ -559,7 +573,7 @@ __host__ __device__ inline size_t expansion_wave_lds(int L1) {
 }
 
 template <class T, int NT, int G>
-__global__ __launch_bounds__(kThreads, sizeof(T) == 4 ? 5 : 4) void expansion_wave_kernel(
+__global__ __launch_bounds__(kThreads, (expansion_waves<T, NT>())) void expansion_wave_kernel(
     RadialDev rad, int S, PairView pv, T* __restrict__ cout, unsigned long long* __restrict__ keymask) {
   typedef typename Vec2<T>::type V;
   typedef T V4 __attribute__((ext_vector_type(4)));
@@ -735,8 +749,8 @@ void launch_pair_forces(const RadialDev& rad, int S, const PairView& pv, const T
       hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), smem, stream, rad, S, pv, dc, centre_virial);
       RGPU_LAUNCH_CHECK();
     };
-    // as many workgroups as are resident (registers: 4 FP32, 3 FP64 per CU)
-    const int64_t resident = int64_t(device_cu_count()) * (sizeof(T) == 4 ? 4 : 3);
+    // as many workgroups as are resident (by the registers)
+    const int64_t resident = int64_t(device_cu_count()) * force_waves<T, NT>();
     auto by_units = [&](auto w) {
       constexpr int W = decltype(w)::value;
       const int64_t blocks = W > 1 ? (n * W + kWaves - 1) / kWaves : std::min((n + kWaves - 1) / kWaves, resident);
@@ -766,7 +780,7 @@ void launch_expansion_wave(const RadialDev& rad, int S, const PairView& pv, T* c
     constexpr int NT = decltype(nt)::value;
     const size_t smem = sizeof(T) * size_t(4 * rad.LL) + kWaves * expansion_wave_lds<T, NT>(rad.L1);
     const int64_t blocks =
-        std::min((n + kWaves - 1) / kWaves, int64_t(device_cu_count()) * (sizeof(T) == 4 ? 5 : 4));
+        std::min((n + kWaves - 1) / kWaves, int64_t(device_cu_count()) * expansion_waves<T, NT>());
     auto go = [&](auto kern) {
       allow_lds(kern, smem);
       hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(kThreads), smem, stream, rad, S, pv, c, keymask);
