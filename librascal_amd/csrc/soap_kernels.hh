@@ -82,7 +82,7 @@ struct SoapTiles {
   int fused = -1;    // power spectrum in the expansion's launch (1), separate (0), built-in (-1)
   int fwd_lds = 0;   // expansion accumulating c in LDS and writing it once (1)
   int fwd_group = -1; // expansion by wavefronts where it applies (1), per entry (0), built-in:
-                      //   by wavefronts from 2048 centres on (-1)
+                      //   by wavefronts for large batches (-1)
 };
 
 // c[i][s][n][l*l+l+m] (finalised) and the per-centre key mask.

@@ -2956,15 +2956,27 @@ void launch_adjoint_f32(const RadialDev& rad, int S, const PairView& pv, const f
 // 27 and 32 us, 1331 centres (FP32) 23 and 36 us, 4096 centres (FP64,
 // n_max 12, l_max 9) 167 and 72 us, 8192 centres (FP32) 178 and 93 us;
 // molecules of 8 atoms (n_max 8, l_max 6) FP64 46 and 48 us, FP32 (four times
-// as many) 277 and 167 us.
-constexpr int64_t kWaveExpansion = 2048;
+// as many) 277 and 167 us.  The fewer orders, the fewer lanes hold sums and the
+// more of the time goes into writing every species' block (with the neighbour
+// list of about 20 neighbours a centre, 2 species, per entry against by
+// wavefronts: l_max 7, n_max 12 2100 centres FP64 56 and 60, FP32 47 and 48 us,
+// 4500 88 and 88, 70 and 58; l_max 4, n_max 8 2100 39 and 41, 36 and 37, 12000
+// 108 and 98, 92 and 70; l_max 2, n_max 20 12000 105 and 161, 88 and 96; and 4
+// species, n_max 12, l_max 0 12000 92 and 117, 80 and 81), so with fewer it
+// starts later, and below l_max 6 only in FP32 and with up to 16 channels.
+template <class T>
+bool wave_expansion_pays(const RadialDev& rad, int64_t n) {
+  if (rad.L >= 9) return n >= 2048;
+  if (rad.L >= 6) return n >= 4096;
+  return sizeof(T) == 4 && rad.N <= 16 && n >= 8192;
+}
 
 template <class T>
 void launch_expansion(const RadialDev& rad, int S, const PairView& pv, T* c,
                       unsigned long long* keymask, hipStream_t stream, const SoapTiles& tiles) {
   if (pv.n_centres == 0) return;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
-  if ((tiles.fwd_group < 0 ? pv.n_centres >= kWaveExpansion : tiles.fwd_group == 1) && pair_kernels_apply(rad)) {
+  if ((tiles.fwd_group < 0 ? wave_expansion_pays<T>(rad, pv.n_centres) : tiles.fwd_group == 1) && pair_kernels_apply(rad)) {
     launch_expansion_wave<T>(rad, S, pv, c, keymask, stream);
     return;
   }

@@ -514,3 +514,46 @@ def test_mixed_power_spectrum_of_many_species(S, N, L):
     ctx.set_precision(_capi.MIXED)
     Xm, _ = ctx.features()
     assert np.abs(Xm - X).max() <= 1e-5 * np.abs(X).max()
+
+
+@pytest.mark.parametrize("N,L", [(1, 0), (4, 4), (6, 6), (7, 7), (9, 2), (10, 8), (11, 9), (13, 4), (24, 2), (20, 7)])
+def test_expansion_set_to_wavefronts(N, L):
+    """The expansion by wavefronts where it is asked for, at every channel
+    count it is built for, against the per-entry kernel on the same batch:
+    centres with more than 64 neighbours, an isolated atom, a species without
+    neighbours."""
+    sts = periodic_box(12, 0.08, (1, 8), d_min=1.0, seed=171)
+    sts = sts + [dict(sts[0], positions=np.zeros((1, 3)), numbers=np.array([6], np.int32), cell=100 * np.eye(3))]
+    hp = soap_hypers(rc=6.0, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8)
+    if N > 16:
+        hp["radial_contribution"]["type"] = "DVR"
+    ctx, _ = _context(hp, sts * 3)
+    for prec, tol in ((_capi.FP64, 1e-13), (_capi.MIXED, 1e-6)):
+        ctx.set_precision(prec)
+        ctx.set_tiles(fused=0)
+        c, km = ctx.expansion()
+        ctx.set_tiles(fused=3)
+        cw, kmw = ctx.expansion()
+        assert np.array_equal(km, kmw)
+        assert np.abs(cw - c).max() <= tol * np.abs(c).max()
+
+
+@pytest.mark.parametrize("n,N,L", [(2047, 3, 9), (2048, 3, 9), (4095, 4, 6), (4096, 4, 6), (8191, 2, 1), (8192, 2, 1)])
+def test_expansion_kernel_by_number_of_centres(n, N, L):
+    """Both sides of the centre counts at which the built-in expansion goes by
+    wavefronts: the same coefficients as with either kernel set."""
+    pos = np.zeros((n, 3))
+    pos[1::2, 0] = 1.0
+    pos[0::4, 1] = 0.3
+    pos = pos + np.array([5.0, 5.0, 5.0])
+    off = np.append(np.arange(0, n, 2), n)
+    ctx = _capi.Context(json.dumps(soap_hypers(rc=2.0, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8)))
+    ctx.set_structures(off, pos, np.ones(n, np.int32), np.tile((20 * np.eye(3)).ravel(), (len(off) - 1, 1)),
+                       np.zeros((len(off) - 1, 3), np.int32), [1])
+    for prec, tol in ((_capi.FP64, 1e-13), (_capi.MIXED, 1e-6)):
+        ctx.set_precision(prec)
+        c, _ = ctx.expansion()
+        for fused in (0, 3):
+            ctx.set_tiles(fused=fused)
+            assert np.abs(ctx.expansion()[0] - c).max() <= tol * np.abs(c).max()
+        ctx.set_tiles()
