@@ -129,153 +129,146 @@ __global__ __launch_bounds__(64 * kPowerWaves) void sym_power_kernel(int R, int 
   }
 }
 
-// One channel of the product below: dc (dL/dc of the centre) rows lm of
-// channel l from the packed triangle w, in LDS with its diagonal times sqrt 2, or (kMemory)
-// in memory as it is.
-template <int LM, bool kMemory>
-__device__ __forceinline__ void contract_channel(int ll, int R, int N, int LL, int lane, const double* w,
+// Rows [r0, r0 + 64) (a lane each) and orders of group grp of GM of one channel
+// of the product below: dc (dL/dc of the centre) rows lm of channel l from the
+// packed triangle w, with its diagonal times sqrt 2 in LDS, or (kMemory) as it is
+// in memory, alpha w - beta p (p may be null).
+template <int LM, int GM, bool kMemory>
+__device__ __forceinline__ void contract_channel(int ll, int r0, int grp, int R, int N, int LL, int lane,
+                                                 const double* w, const double* p, double alpha, double beta,
                                                  const double* ci, double* __restrict__ dc) {
   const double rt2 = 1.41421356237309504880;
   with_channel<LM>(ll, [&](auto lc) {
-    constexpr int l = decltype(lc)::value, M = 2 * l + 1;
+    constexpr int l = decltype(lc)::value, M = 2 * l + 1, CNT = (M + GM - 1) / GM;
+    const int m_own = grp * CNT;
+    if (m_own >= M) return;
+    // (the last group may overlap the one before; it stores its own orders)
+    const int m0 = GM == 1 ? 0 : min(m_own, M - CNT);
     const double f = rt2 / sqrt(double(M));
-    for (int rb = 0; rb < R; rb += 64) {
-      const int r = min(rb + lane, R - 1);
-      double acc[M];
+    const int r = min(r0 + lane, R - 1);
+    double acc[CNT];
 #pragma unroll
-      for (int m = 0; m < M; ++m) acc[m] = 0.0;
-      uniform_ptr y = (uniform_ptr)(ci + l * l);
-      int a = tri_i(r);
-      for (int col = 0; col < R; ++col, y += LL) {
-        const double v = kMemory ? w[a] * (col == r ? rt2 : 1.0) : w[a];
-        a += col < r ? 1 : col + 1;
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[m] += v * y[m];
+    for (int m = 0; m < CNT; ++m) acc[m] = 0.0;
+    uniform_ptr y = (uniform_ptr)(ci + l * l + m0);
+    int a = tri_i(r);
+    // (columns whose scalar loads are in flight together, by the registers)
+    constexpr int U = CNT <= 4 ? 8 : (CNT <= 9 ? 4 : (CNT <= 19 ? 2 : 1));
+#pragma unroll U
+    for (int col = 0; col < R; ++col, y += LL) {
+      double v;
+      if constexpr (kMemory) {
+        v = p ? alpha * w[a] - beta * p[a] : w[a];
+        v *= col == r ? rt2 : 1.0;
+      } else {
+        v = w[a];
       }
-      if (rb + lane < R) {
-        const int s = r / N, n = r - s * N;
-        double* o = dc + int64_t(s) * LL * N + n;
+      a += col < r ? 1 : col + 1;
 #pragma unroll
-        for (int m = 0; m < M; ++m) o[(l * l + m) * N] = f * acc[m];
-      }
+      for (int m = 0; m < CNT; ++m) acc[m] += v * y[m];
+    }
+    if (r0 + lane < R) {
+      const int s = r / N, n = r - s * N;
+      double* o = dc + int64_t(s) * LL * N + n;
+#pragma unroll
+      for (int m = 0; m < CNT; ++m)
+        if (GM == 1 || m0 + m >= m_own) o[(l * l + m0 + m) * N] = f * acc[m];
     }
   });
 }
 
 // dL/dC_l[r][m] = f_l sqrt 2 sum_c w(r, c) C_l[c][m], w the packed entry
 // dL/dp(r, c) (times sqrt 2 on the diagonal).  The channel's triangle of
-// dL/dp is formed in LDS, one buffer per wavefront, straight in its packed
-// order; a lane's walk along its row, tri(r) + c up to the diagonal and
-// tri(c) + r after it, is free of bank conflicts there (triangular numbers
-// run through every residue of a power of two).
+// dL/dp is formed in LDS, straight in its packed order; a lane's walk along its
+// row, tri(r) + c up to the diagonal and tri(c) + r after it, is free of bank
+// conflicts there (triangular numbers run through every residue of a power of
+// two).
 //
-// Forms of G (kForm): kDp symmetric packed rows of dL/dp, kDx full rows
-// (keys a <= b, [n1][n2][l]) of dL/dX, whose projection dL/dp = G / |p| -
-// xg p / |p|^2 is made on the way (p null: no normalisation, dL/dp = G); xg
-// null: X . G is first summed here.  A full row's entries of one channel lie
-// L+1 apart, but the workgroup's wavefronts take them channel after channel
-// from the same cached lines, which costs less than packing the rows first
-// (4689 centres, 4 species, n_max 8, l_max 6: 244 us against 183 + 139).  kGather: as
-// kDp, the entries gathered from memory (R too large for the LDS).
+// With p the packed rows G hold dL/dX of X = p / |p| and dL/dp = G / |p| - x p /
+// |p|^2 is made on the way, x = xg[i], or (xg null) the n_dot values of the
+// centre's products p . G that packing left in dot, over |p|.
 //
-// Bound by the memory it streams and the latency of the scalar loads: 4096
-// centres, 4 species, n_max 12, l_max 9: 0.31 ms for 0.93 GB, where the key
-// contraction of the fused FP64 adjoint it replaced took about 1.0 ms.
-enum { kDp, kDx, kGather };
+// kShare: kOwn a triangle for each wavefront, which takes whole channels;
+// kShared one for the workgroup, whose wavefronts take blocks of 64 rows and
+// GM groups of the orders; kNone the entries gathered from memory (the triangle
+// too large for the LDS).
+//
+// Bound by the memory it streams and the latency of the scalar loads, which the
+// unrolled columns take together: 4096 centres, 4 species, n_max 12, l_max 9:
+// 0.25 ms for 0.93 GB (0.32 one column at a time), where the key contraction
+// of the fused FP64 adjoint it replaced took about 1.0 ms.
+enum { kOwn, kShared, kNone };
 
-template <int LM, int kForm>
+template <int LM, int kShare, int GM, bool kProject>
 __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, int L, int64_t ld,
                                                                 const double* __restrict__ c,
                                                                 const double* __restrict__ p,
                                                                 const double* __restrict__ norm2,
                                                                 const double* __restrict__ xg,
+                                                                const double* __restrict__ dot, int n_dot,
                                                                 const double* __restrict__ G,
                                                                 double* __restrict__ dc) {
   const int64_t i = blockIdx.x;
-  const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R), S = R / N, KB = N * N * L1;
+  const int L1 = L + 1, LL = L1 * L1, TRI = tri_i(R);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const double rt2 = 1.41421356237309504880;
   extern __shared__ __align__(64) unsigned char smem_raw[];
-  double* W = reinterpret_cast<double*>(smem_raw) + wave * TRI;
-  // kDx: offsets in a full row of the entry t = (r, c) at channel 0 and of
-  // its mirror (both the same between species)
-  int2* tab = reinterpret_cast<int2*>(reinterpret_cast<double*>(smem_raw) + kWaves * TRI);
-  __shared__ double red[kWaves];
-  const double* Gi = G + i * (kForm == kDx ? int64_t(S) * (S + 1) / 2 * KB : ld);
-  const double* pi = p ? p + i * ld : nullptr;
-  // packed entry t of channel l of G
-  auto entry = [&](int l, int t) -> double {
-    if constexpr (kForm != kDx) {
-      return Gi[l * TRI + t];
-    } else {
-      const int2 o = tab[t];
-      const double v = Gi[o.x + l];
-      return o.x == o.y ? v : (v + Gi[o.y + l]) * 0.70710678118654752440;
-    }
-  };
+  double* W = reinterpret_cast<double*>(smem_raw) + (kShare == kOwn ? wave * TRI : 0);
+  const double* Gi = G + i * ld;
+  const double* pi = kProject ? p + i * ld : nullptr;
   double alpha = 1.0, beta = 0.0;
-  if constexpr (kForm == kDx) {
-    for (int col = wave; col < R; col += kWaves)
-      for (int r = lane; r <= col; r += 64) {
-        const int a = r / N, b = col / N, n1 = r - a * N, n2 = col - b * N;
-        const int k0 = (a * S - a * (a - 1) / 2 + (b - a)) * KB;
-        const int o = k0 + (n1 * N + n2) * L1;
-        tab[tri_i(col) + r] = make_int2(o, a == b ? k0 + (n2 * N + n1) * L1 : o);
-      }
-    __syncthreads();
-    if (p) {
-      const double n2 = norm2[i];
+  if constexpr (kProject) {
+    const double n2 = norm2[i];
+    if (n2 > 0) {
       double x = 0.0;
       if (xg) {
         x = xg[i];
       } else {
-        double d = 0.0;
-        for (int k = 0; k * kWaves <= L; ++k) {
-          const int u = wave_unit(L1, kWaves, wave, k);
-          if (u < 0) continue;
-          const double* q = pi + (L - u) * TRI;
-#pragma unroll 8
-          for (int t = lane; t < TRI; t += 64) d += q[t] * entry(L - u, t);
-        }
-        for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
-        if (lane == 0) red[wave] = d;
-        __syncthreads();
-        if (n2 > 0) x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
+        for (int k = 0; k < n_dot; ++k) x += dot[i * n_dot + k];
+        x /= sqrt(n2);
       }
-      if (n2 > 0) {
-        alpha = 1.0 / sqrt(n2);
-        beta = x / n2;
-      }
+      alpha = 1.0 / sqrt(n2);
+      beta = x / n2;
     }
   }
   const double* ci = c + i * int64_t(R) * LL;
-  for (int k = 0; k * kWaves <= L; ++k) {
-    const int u = wave_unit(L1, kWaves, wave, k), lk = L - u;
-    if (u < 0) continue;
-    const double* g = Gi + lk * TRI;
-    if constexpr (kForm != kGather) {
+  double* di = dc + i * int64_t(R) * LL;
+  if constexpr (kShare == kOwn) {
+    for (int k = 0; k * kWaves <= L; ++k) {
+      const int u = wave_unit(L1, kWaves, wave, k), lk = L - u;
+      if (u < 0) continue;
+      const double *g = Gi + lk * TRI, *q = kProject ? pi + lk * TRI : nullptr;
       wave_sync();  // the previous channel is read
       // (many loads in flight: the runs come from memory)
-      if (kForm == kDx && p) {
-        const double* q = pi + lk * TRI;
-#pragma unroll 8
-        for (int t = lane; t < TRI; t += 64) W[t] = alpha * entry(lk, t) - beta * q[t];
-      } else {
 #pragma unroll 16
-        for (int t = lane; t < TRI; t += 64) W[t] = entry(lk, t);
-      }
+      for (int t = lane; t < TRI; t += 64) W[t] = kProject ? alpha * g[t] - beta * q[t] : g[t];
       wave_sync();
       for (int r = lane; r < R; r += 64) W[tri_i(r) + r] *= rt2;
       wave_sync();
+      for (int rb = 0; rb < R; rb += 64)
+        contract_channel<LM, 1, false>(lk, rb, 0, R, N, LL, lane, W, nullptr, 1.0, 0.0, ci, di);
     }
-    contract_channel<LM, kForm == kGather>(lk, R, N, LL, lane, kForm == kGather ? g : W, ci,
-                                           dc + i * int64_t(R) * LL);
+  } else {
+    const int RB = (R + 63) / 64;
+    for (int l = L - int(blockIdx.y); l >= 0; l -= int(gridDim.y)) {
+      const double *g = Gi + l * TRI, *q = kProject ? pi + l * TRI : nullptr;
+      if constexpr (kShare == kShared) {
+        __syncthreads();  // the previous channel is read
+#pragma unroll 8
+        for (int t = threadIdx.x; t < TRI; t += kThreads) W[t] = kProject ? alpha * g[t] - beta * q[t] : g[t];
+        __syncthreads();
+        for (int r = threadIdx.x; r < R; r += kThreads) W[tri_i(r) + r] *= rt2;
+        __syncthreads();
+      }
+      for (int u = wave; u < RB * GM; u += kWaves)
+        contract_channel<LM, GM, kShare == kNone>(l, (u / GM) * 64, u % GM, R, N, LL, lane, kShare == kNone ? g : W, q,
+                                                  alpha, beta, ci, di);
+    }
   }
 }
 
 // The same from full rows of dL/dX, the whole packed row formed in LDS first
 // (channels LT apart): the full row is read once along itself, where taking
-// the entries channel by channel (kDx) touches a cache line per entry.  2000
+// the entries channel by channel touches a cache line per entry.  2000
 // centres: 98 -> 71 us (4 species, n_max 8, l_max 6), 178 -> 83 us (3
 // species, n_max 10, l_max 8); bound by the chain of its phases.
 __host__ __device__ inline int full_stride(int R) { return tri_i(R) | 1; }
@@ -364,9 +357,10 @@ __global__ __launch_bounds__(kThreads) void sym_contract_full_kernel(int R, int 
   __syncthreads();
   for (int k = 0; k * kWaves <= L; ++k) {
     const int u = wave_unit(L1, kWaves, wave, k);
-    if (u >= 0)
-      contract_channel<LM, false>(L - u, R, N, LL, lane, W + (L - u) * LT, c + i * int64_t(R) * LL,
-                                  dc + i * int64_t(R) * LL);
+    if (u < 0) continue;
+    for (int rb = 0; rb < R; rb += 64)
+      contract_channel<LM, 1, false>(L - u, rb, 0, R, N, LL, lane, W + (L - u) * LT, nullptr, 1.0, 0.0,
+                                     c + i * int64_t(R) * LL, dc + i * int64_t(R) * LL);
   }
 }
 
@@ -475,20 +469,24 @@ __global__ __launch_bounds__(kThreads) void sym_contract_sets_kernel(int R, int 
   }
 }
 
-// Full row <-> symmetric packed row, one workgroup per row, KC key blocks at
-// a time through LDS ([key][n1][n2][l] with an odd n1 stride): both sides move
-// along their rows (whole key blocks, runs of N packed entries), and several
-// keys per pass keep enough loads in flight.  Memory bound.
-// CHECK: *asymmetric = 1 when a diagonal key's block of some row is not
-// symmetric (every writer stores the same value).
-template <bool CHECK>
+// Full row <-> symmetric packed row, KC key blocks at a time through LDS
+// ([key][n1][n2][l] with an odd n1 stride): both sides move along their rows
+// (whole key blocks, runs of N packed entries), and several keys per pass keep
+// enough loads in flight.  The passes of a row go to gridDim.y workgroups, more
+// than one where there are few rows.  Memory bound.
+// kExtra: kCheck *flag = 1 when a diagonal key's block of some row is not
+// symmetric (every writer stores the same value); kDot dot[i gridDim.y + y] =
+// this workgroup's part of p . G.
+enum { kPlain, kCheck, kDot };
+template <int kExtra>
 __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1, int KC, int64_t ld,
                                                             const double* __restrict__ full,
                                                             const int64_t* __restrict__ rows,
-                                                            double* __restrict__ out,
-                                                            int* __restrict__ asymmetric) {
+                                                            double* __restrict__ out, int* __restrict__ flag,
+                                                            const double* __restrict__ p, double* __restrict__ dot) {
   const int64_t i = blockIdx.x;
   bool differ = false;
+  double sum = 0.0;
   const int K = S * (S + 1) / 2, NL = N * L1, KB = N * NL, NS = NL | 1, TRI = tri_i(S * N), NN = N * N;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   extern __shared__ __align__(64) unsigned char smem_raw[];
@@ -496,13 +494,17 @@ __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1
   int* key_ab = reinterpret_cast<int*>(b + size_t(KC) * N * NS);
   const double* src = full + (rows ? rows[i] : i) * (int64_t(K) * KB);
   double* dst = out + i * ld;
+  const double* pi = kExtra == kDot ? p + i * ld : nullptr;
+  const float inv_nl = 1.0f / float(NL);
   key_table(S, key_ab);
-  for (int k0 = 0; k0 < K; k0 += KC) {
+  for (int k0 = int(blockIdx.y) * KC; k0 < K; k0 += int(gridDim.y) * KC) {
     const int kc = min(KC, K - k0);
     __syncthreads();
-#pragma unroll 4
-    for (int r = wave; r < kc * N; r += kWaves)
-      for (int o = lane; o < NL; o += 64) b[r * NS + o] = src[(int64_t(k0) * N + r) * NL + o];
+#pragma unroll 8
+    for (int e = threadIdx.x; e < kc * KB; e += kThreads) {
+      const int r = int((float(e) + 0.5f) * inv_nl);
+      b[r * (NS - NL) + e] = src[int64_t(k0) * KB + e];
+    }
     __syncthreads();
     for (int t = threadIdx.x; t < kc * NN; t += kThreads) {
       const int kk = t / NN, tt = t - kk * NN, n2 = tt / N, n1 = tt - n2 * N;
@@ -513,40 +515,23 @@ __global__ __launch_bounds__(kThreads) void sym_pack_kernel(int S, int N, int L1
       int64_t o = tri_i(sb * N + n2) + sa * N + n1;
 #pragma unroll 4
       for (int l = 0; l < L1; ++l, o += TRI) {
-        dst[o] = sym ? (b0[l] + b1[l]) * 0.70710678118654752440 : b0[l];
-        if (CHECK && sym) differ |= b0[l] != b1[l];
+        const double v = sym ? (b0[l] + b1[l]) * 0.70710678118654752440 : b0[l];
+        dst[o] = v;
+        if (kExtra == kCheck && sym) differ |= b0[l] != b1[l];
+        if (kExtra == kDot) sum += v * pi[o];
       }
     }
   }
-  if (CHECK && differ) *asymmetric = 1;
-  for (int64_t o = int64_t(L1) * TRI + threadIdx.x; o < ld; o += kThreads) dst[o] = 0.0;
-}
-
-// dL/dp of a packed row of dL/dX in place (X = p / |p|): G / |p| - xg p /
-// |p|^2, xg null: X . G summed here.  One workgroup per row.
-__global__ __launch_bounds__(kThreads) void sym_project_kernel(int64_t ld, const double* __restrict__ p,
-                                                               const double* __restrict__ norm2,
-                                                               const double* __restrict__ xg,
-                                                               double* __restrict__ G) {
-  const int64_t i = blockIdx.x;
-  __shared__ double red[kWaves];
-  const double* q = p + i * ld;
-  double* g = G + i * ld;
-  const double n2 = norm2[i];
-  if (!(n2 > 0)) return;
-  double x;
-  if (xg) {
-    x = xg[i];
-  } else {
-    double d = 0.0;
-    for (int64_t o = threadIdx.x; o < ld; o += kThreads) d += q[o] * g[o];
-    for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = d;
+  if (blockIdx.y == 0)
+    for (int64_t o = int64_t(L1) * TRI + threadIdx.x; o < ld; o += kThreads) dst[o] = 0.0;
+  if (kExtra == kCheck && differ) *flag = 1;
+  if constexpr (kExtra == kDot) {
+    __shared__ double red[kWaves];
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
+    if (lane == 0) red[wave] = sum;
     __syncthreads();
-    x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
+    if (threadIdx.x == 0) dot[i * gridDim.y + blockIdx.y] = (red[0] + red[1]) + (red[2] + red[3]);
   }
-  const double alpha = 1.0 / sqrt(n2), beta = x / n2;
-  for (int64_t o = threadIdx.x; o < ld; o += kThreads) g[o] = alpha * g[o] - beta * q[o];
 }
 
 __global__ __launch_bounds__(kThreads) void sym_unpack_kernel(int S, int N, int L1, int KC, int64_t ld,
@@ -556,16 +541,16 @@ __global__ __launch_bounds__(kThreads) void sym_unpack_kernel(int S, int N, int 
                                                               double* __restrict__ out) {
   const int64_t i = rows ? rows[blockIdx.x] : int64_t(blockIdx.x);
   const int K = S * (S + 1) / 2, NL = N * L1, KB = N * NL, NS = NL | 1, TRI = tri_i(S * N), NN = N * N;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   extern __shared__ __align__(64) unsigned char smem_raw[];
   double* b = reinterpret_cast<double*>(smem_raw);
   int* key_ab = reinterpret_cast<int*>(b + size_t(KC) * N * NS);
   const double* src = p + i * ld;
   double* dst = out + int64_t(blockIdx.x) * (int64_t(K) * KB);
+  const float inv_nl = 1.0f / float(NL);
   key_table(S, key_ab);
   double nr = 1.0;
   if (normalize && norm2[i] > 0) nr = sqrt(norm2[i]);
-  for (int k0 = 0; k0 < K; k0 += KC) {
+  for (int k0 = int(blockIdx.y) * KC; k0 < K; k0 += int(gridDim.y) * KC) {
     const int kc = min(KC, K - k0);
     __syncthreads();
     for (int t = threadIdx.x; t < kc * NN; t += kThreads) {
@@ -586,8 +571,11 @@ __global__ __launch_bounds__(kThreads) void sym_unpack_kernel(int S, int N, int 
       }
     }
     __syncthreads();
-    for (int r = wave; r < kc * N; r += kWaves)
-      for (int o = lane; o < NL; o += 64) dst[(int64_t(k0) * N + r) * NL + o] = b[r * NS + o] / nr;
+#pragma unroll 4
+    for (int e = threadIdx.x; e < kc * KB; e += kThreads) {
+      const int r = int((float(e) + 0.5f) * inv_nl);
+      dst[int64_t(k0) * KB + e] = b[r * (NS - NL) + e] / nr;
+    }
   }
 }
 
@@ -626,30 +614,64 @@ void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* 
 
 namespace {
 
-size_t contract_lds(int R, bool full) {
-  return size_t(sym_tri(R)) * (sizeof(double) * kWaves + (full ? sizeof(int2) : 0));
-}
 constexpr size_t kContractLds = 156 * 1024;
 // sym_contract_full_kernel: three workgroups per CU at least (with 2 species,
 // n_max 12, l_max 9 it took 73 us against 107 by channels, 3 species 176
 // against 254, but 4 species, one workgroup, 552 against 476; 2000 centres)
 constexpr size_t kFullLds = 54 * 1024;
+// A triangle for each wavefront while two workgroups per CU have them (R <= 65),
+// else one for the workgroup, four times as many of which fit.  Adjoint of a
+// prediction, own against shared: 64 rows (8 species, n_max 8, l_max 4) 76 and
+// 85 us, 52 rows (4, 13, 8) 235 and 321; 72 rows (6, 12, 9) 383 and 265, 90 rows
+// (10, 9, 4) 353 and 248 (1000 to 2000 centres).
+constexpr size_t kOwnLds = 68 * 1024;
 
-template <int kForm>
+// workgroups that share a row's passes in the row conversions: one but where
+// there are too few rows to fill the chip
+unsigned row_split(int S, int N, int L1, int64_t n) {
+  const int kc = key_blocks(S, N, L1), passes = (S * (S + 1) / 2 + kc - 1) / kc;
+  return unsigned(std::max<int64_t>(1, std::min<int64_t>(passes, 1024 / n)));
+}
+
+template <int kExtra>
+void go_pack(int S, int N, int L1, int64_t n, unsigned split, const double* full, const int64_t* rows, double* out,
+             int* flag, const double* p, double* dot, hipStream_t stream) {
+  const size_t smem = key_lds(S, N, L1);
+  allow_lds(sym_pack_kernel<kExtra>, smem);
+  hipLaunchKernelGGL(sym_pack_kernel<kExtra>, dim3(unsigned(n), split), dim3(kThreads), smem, stream, S, N, L1,
+                     key_blocks(S, N, L1), sym_row_stride(S, N, L1), full, rows, out, flag, p, dot);
+  RGPU_LAUNCH_CHECK();
+}
+
+template <bool kProject>
 void go_contract(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
-                 const double* xg, const double* G, double* dc, hipStream_t stream) {
+                 const double* xg, const double* dot, int n_dot, const double* G, double* dc, hipStream_t stream) {
   const int R = S * N;
-  const size_t smem = kForm == kGather ? 0 : contract_lds(R, kForm == kDx);
-  auto go = [&](auto kern) {
+  const size_t tri = sizeof(double) * size_t(sym_tri(R));
+  auto go = [&](auto kern, size_t smem, unsigned split) {
     allow_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, R, N, L1 - 1, sym_row_stride(S, N, L1),
-                       c, p, norm2, xg, G, dc);
+    hipLaunchKernelGGL(kern, dim3(unsigned(n), split), dim3(kThreads), smem, stream, R, N, L1 - 1,
+                       sym_row_stride(S, N, L1), c, p, norm2, xg, dot, n_dot, G, dc);
     RGPU_LAUNCH_CHECK();
   };
+  auto by_form = [&](auto lm) {
+    constexpr int LM = decltype(lm)::value;
+    // (channels over more workgroups where there are few centres)
+    const unsigned split = unsigned(std::max<int64_t>(1, std::min<int64_t>(L1, 1024 / n)));
+    const int rb = (R + 63) / 64;
+    if (kWaves * tri <= kOwnLds)
+      go(sym_contract_kernel<LM, kOwn, 1, kProject>, kWaves * tri, 1);
+    else if (tri > kContractLds)
+      go(sym_contract_kernel<LM, kNone, 2, kProject>, 0, split);
+    else if (rb == 1 || rb == 3)
+      go(sym_contract_kernel<LM, kShared, 4, kProject>, tri, split);
+    else
+      go(sym_contract_kernel<LM, kShared, 2, kProject>, tri, split);
+  };
   if (L1 <= 10)
-    go(sym_contract_kernel<9, kForm>);
+    by_form(std::integral_constant<int, 9>{});
   else
-    go(sym_contract_kernel<kMaxL1 - 1, kForm>);
+    by_form(std::integral_constant<int, kMaxL1 - 1>{});
 }
 
 }  // namespace
@@ -657,10 +679,7 @@ void go_contract(int S, int N, int L1, int64_t n, const double* c, const double*
 void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const double* G, double* dc,
                          hipStream_t stream) {
   if (n == 0) return;
-  if (contract_lds(S * N, false) <= kContractLds)
-    go_contract<kDp>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
-  else
-    go_contract<kGather>(S, N, L1, n, c, nullptr, nullptr, nullptr, G, dc, stream);
+  go_contract<false>(S, N, L1, n, c, nullptr, nullptr, nullptr, nullptr, 0, G, dc, stream);
 }
 
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
@@ -701,34 +720,30 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
       go(sym_contract_full_kernel<kMaxL1 - 1>);
     return;
   }
-  if (contract_lds(S * N, true) <= kContractLds) {
-    go_contract<kDx>(S, N, L1, n, c, p, norm2, xg, G, dc, stream);
-    return;
-  }
+  // Packed first, with p . G where that is needed.  (A form that took the full
+  // row's entries channel by channel, L+1 values apart, touched every cache line
+  // L+1 times.)
   const int64_t ld = sym_row_stride(S, N, L1);
-  double* g = work.reserve(size_t(n * ld));
-  launch_sym_pack(S, N, L1, n, G, nullptr, g, stream);
-  if (p) {
-    hipLaunchKernelGGL(sym_project_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, ld, p, norm2, xg, g);
-    RGPU_LAUNCH_CHECK();
-  }
-  launch_sym_contract(S, N, L1, n, c, g, dc, stream);
+  const unsigned split = row_split(S, N, L1, n);
+  double* g = work.reserve(size_t(n * ld + n * split));
+  if (p && !xg)
+    go_pack<kDot>(S, N, L1, n, split, G, nullptr, g, nullptr, p, g + n * ld, stream);
+  else
+    go_pack<kPlain>(S, N, L1, n, split, G, nullptr, g, nullptr, nullptr, nullptr, stream);
+  if (p)
+    go_contract<true>(S, N, L1, n, c, p, norm2, xg, g + n * ld, int(split), g, dc, stream);
+  else
+    go_contract<false>(S, N, L1, n, c, nullptr, nullptr, nullptr, nullptr, 0, g, dc, stream);
 }
 
 void launch_sym_pack(int S, int N, int L1, int64_t n, const double* full, const int64_t* rows, double* out,
                      hipStream_t stream, int* asymmetric) {
   if (n == 0) return;
-  const size_t smem = key_lds(S, N, L1);
-  auto go = [&](auto kern) {
-    allow_lds(kern, smem);
-    hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1, key_blocks(S, N, L1),
-                       sym_row_stride(S, N, L1), full, rows, out, asymmetric);
-    RGPU_LAUNCH_CHECK();
-  };
+  const unsigned split = row_split(S, N, L1, n);
   if (asymmetric)
-    go(sym_pack_kernel<true>);
+    go_pack<kCheck>(S, N, L1, n, split, full, rows, out, asymmetric, nullptr, nullptr, stream);
   else
-    go(sym_pack_kernel<false>);
+    go_pack<kPlain>(S, N, L1, n, split, full, rows, out, nullptr, nullptr, nullptr, stream);
 }
 
 void launch_sym_unpack(int S, int N, int L1, int64_t n, const double* p, const int64_t* rows, const double* norm2,
@@ -736,7 +751,7 @@ void launch_sym_unpack(int S, int N, int L1, int64_t n, const double* p, const i
   if (n == 0) return;
   const size_t smem = key_lds(S, N, L1);
   allow_lds(sym_unpack_kernel, smem);
-  hipLaunchKernelGGL(sym_unpack_kernel, dim3(unsigned(n)), dim3(kThreads), smem, stream, S, N, L1,
+  hipLaunchKernelGGL(sym_unpack_kernel, dim3(unsigned(n), row_split(S, N, L1, n)), dim3(kThreads), smem, stream, S, N, L1,
                      key_blocks(S, N, L1), sym_row_stride(S, N, L1), p, rows, norm2, int(normalize), out);
   RGPU_LAUNCH_CHECK();
 }

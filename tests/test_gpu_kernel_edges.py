@@ -557,3 +557,41 @@ def test_expansion_kernel_by_number_of_centres(n, N, L):
             ctx.set_tiles(fused=fused)
             assert np.abs(ctx.expansion()[0] - c).max() <= tol * np.abs(c).max()
         ctx.set_tiles()
+
+
+@pytest.mark.parametrize("S,N,L,normalize", [
+    (5, 13, 1, True), (6, 11, 3, True), (3, 23, 10, False),  # 65, 66, 69 rows: own triangles, one shared by two row blocks
+    (13, 10, 2, True), (12, 16, 1, True),                    # 130 and 192 rows: three row blocks
+    (13, 16, 1, True), (13, 16, 0, False),                   # 208: entries from memory
+    (2, 20, 12, True), (4, 12, 9, True),                     # rows past those formed whole in LDS, own triangles
+])
+def test_fp64_adjoint_of_wide_rows(S, N, L, normalize):
+    """The FP64 adjoint from full rows at the edges of its forms (rows formed
+    whole in LDS, a triangle per wavefront or per workgroup, entries from
+    memory; the passes and channels of a row over several workgroups, for few
+    centres, or one) and the prediction's on the same triangles."""
+    sts = periodic_box(2 * S + 3, 0.06, tuple(range(1, S + 1)), d_min=1.0, seed=181)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8, normalize=normalize)
+    if N > 13:
+        hp["radial_contribution"]["type"] = "DVR"
+    ctx, num = _context(hp, sts)
+    X, _ = ctx.features()
+    rng = np.random.default_rng(182)
+    G = rng.normal(size=X.shape)
+    g, s = ctx.features_backward(G)
+    ref = (oracle_backward(O.Calculator(hp), O.BatchData(sts), G) if N <= 13 else
+           _rows_backward(ctx, G, (2 * S + 3) / 0.06))
+    for x, y in zip((g, s), ref):
+        assert np.abs(x - y).max() <= 1e-10 * np.abs(y).max()
+    copies = 1024 // len(num) + 2
+    many, _ = _context(hp, sts * copies)
+    gm, sm = many.features_backward(np.tile(G, (copies, 1)))
+    assert np.abs(gm.reshape(copies, *g.shape) - g).max() <= 1e-10 * np.abs(g).max()
+    assert np.abs(sm.reshape(copies, *s.shape) - s).max() <= 1e-10 * np.abs(s).max()
+    # a linear kernel's prediction is the adjoint of one dL/dX
+    T = X[:4] + 0.1 * rng.normal(size=(4, X.shape[1]))
+    w = rng.normal(size=4)
+    ctx.set_sparse_points(1, num[:4], T, w)
+    dX = (num[:, None] == num[None, :4]) @ (w[:, None] * T)
+    for x, y in zip(ctx.gap_predict()[1:], ctx.features_backward(dX)):
+        assert np.abs(x - y).max() <= 1e-10 * np.abs(y).max()
