@@ -2759,6 +2759,7 @@ void launch_expansion_k(const RadialDev& rad, int S, const PairView& pv, T* c,
 // dynamic LDS of the register-tile adjoint: two workgroups per CU with the
 // pair phase in the same workgroup, three without it
 constexpr size_t kTileAdjBudget = 77 * 1024;
+constexpr size_t kMaxLds = 156 * 1024;
 constexpr size_t kTileSplitBudget = 52 * 1024;
 
 template <int N, int L, int NR, int ROLES, int PRE, bool DIRECT, bool PAIRS>
@@ -3287,7 +3288,15 @@ void launch_adjoint_pairs(const RadialDev& rad, int S, const PairView& pv, const
   if (tiles.pb_adj > 0)
     PB = std::min(tiles.pb_adj, 64);
   else
-    while (PB > 1 && fixed + batch(PB) > kTileAdjBudget) --PB;
+    // Two workgroups per CU, but with four pairs at least: the work of a batch is
+    // spread over its pairs.  2000 centres of 2 species, n_max 20, l_max 12 without
+    // splines take 2.70 ms pair by pair in 79 KB and 1.42 ms by eight in 147 KB,
+    // with splines 1.10 and 0.72; 1000 of 4, n_max 12, l_max 9 0.51 ms by six in 76
+    // KB and 0.61 by eight in 85 KB.
+    for (const size_t budget : {kTileAdjBudget, kMaxLds}) {
+      for (PB = 8; PB > 1 && fixed + batch(PB) > budget;) --PB;
+      if (PB >= 4) break;
+    }
   const size_t smem = fixed + batch(PB);
   auto go = [&](auto kern) {
     allow_lds(kern, smem);

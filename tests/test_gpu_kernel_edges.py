@@ -595,3 +595,23 @@ def test_fp64_adjoint_of_wide_rows(S, N, L, normalize):
     dX = (num[:, None] == num[None, :4]) @ (w[:, None] * T)
     for x, y in zip(ctx.gap_predict()[1:], ctx.features_backward(dX)):
         assert np.abs(x - y).max() <= 1e-10 * np.abs(y).max()
+
+
+@pytest.mark.parametrize("S,N,L,spline", [(2, 20, 12, None), (2, 20, 12, 1e-8), (4, 12, 9, None), (10, 8, 10, 1e-8)])
+def test_general_pair_phase_of_large_rows(S, N, L, spline):
+    """The general pair phase of the FP64 adjoint where two workgroups per CU
+    hold four pairs and more, and where one takes the whole LDS: against one
+    pair at a time, and against the exported gradient rows."""
+    sts = periodic_box(2 * S + 3, 0.06, tuple(range(1, S + 1)), d_min=1.0, seed=191)
+    hp = soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=spline, normalize=False)
+    if N > 13:
+        hp["radial_contribution"]["type"] = "DVR"
+    ctx, _ = _context(hp, sts)
+    X, _ = ctx.features()
+    G = np.random.default_rng(192).normal(size=X.shape)
+    got = ctx.features_backward(G)
+    for x, y in zip(got, _rows_backward(ctx, G, (2 * S + 3) / 0.06)):
+        assert np.abs(x - y).max() <= 1e-10 * np.abs(y).max()
+    ctx.set_tiles(pairs_adj=1)
+    for x, y in zip(got, ctx.features_backward(G)):
+        assert np.abs(x - y).max() <= 1e-12 * np.abs(y).max()
