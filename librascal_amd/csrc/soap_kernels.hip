@@ -2696,10 +2696,12 @@ __global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t lds,
 // for more: up to 48 KB there.  Expansion and power spectrum in 32 KB and so:
 // 1725 centres of 10 species (n_max 6, l_max 12) 751 -> 353 us, 16 of 6
 // (n_max 12, l_max 9) 99 -> 71 us and 2500 of them 286 -> 239 us, 434 of 10
-// (n_max 12, l_max 6) 150 -> 118 us.
+// (n_max 12, l_max 6) 150 -> 118 us.  So do few centres (two per CU), which leave
+// the room unused: 100 of 10 species (n_max 12, l_max 6) 137 -> 105 us.
 constexpr size_t kFwdBudget = 32 * 1024;
 constexpr size_t kPsBudget = 32 * 1024, kPsBudgetMany = 48 * 1024;
 constexpr int kPsPasses = 8;
+constexpr int64_t kPsFew = 512;
 constexpr size_t kAdjBudget = 64 * 1024;
 constexpr size_t kResidentBudget = 52 * 1024;  // three workgroups per CU
 
@@ -3010,13 +3012,16 @@ void launch_expansion(const RadialDev& rad, int S, const PairView& pv, T* c,
 
 // LDS of the power spectrum and the keys it stages per pass
 template <class T>
-size_t power_spectrum_lds(const RadialDev& rad, int S, const SoapTiles& tiles, int* keys) {
+size_t power_spectrum_lds(const RadialDev& rad, int S, int64_t n, const SoapTiles& tiles, int* keys) {
   const int K = S * (S + 1) / 2;
   const size_t cbytes = sizeof(T) * align_up((size_t(S) * rad.N + 3) * (rad.LL | 1), 4);
   const size_t kb = sizeof(T) * size_t(rad.N) * rad.N * rad.L1;
   auto keys_in = [&](size_t budget) { return cbytes + kb < budget ? int((budget - cbytes) / kb) : 1; };
   int KC = keys_in(kPsBudget);
-  if (KC * kPsPasses < K) KC = std::max(KC, std::min(keys_in(kPsBudgetMany), (K + kPsPasses - 1) / kPsPasses));
+  if (n <= kPsFew)
+    KC = keys_in(kPsBudgetMany);
+  else if (KC * kPsPasses < K)
+    KC = std::max(KC, std::min(keys_in(kPsBudgetMany), (K + kPsPasses - 1) / kPsPasses));
   if (tiles.kc > 0) KC = tiles.kc;
   *keys = KC = std::max(1, std::min(KC, K));
   return cbytes + size_t(KC) * kb + sizeof(int) * size_t(K + rad.N * (rad.N + 1) / 2);
@@ -3029,7 +3034,7 @@ void launch_power_spectrum_impl(const RadialDev& rad, int S, int64_t n, const T*
   if (n == 0) return;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
   int KC = 0;
-  const size_t smem = power_spectrum_lds<T>(rad, S, tiles, &KC);
+  const size_t smem = power_spectrum_lds<T>(rad, S, n, tiles, &KC);
   // the benchmark shape (n_max 12, l_max 9) with its sizes fixed at compile time
   constexpr bool kFixedShape = true;
   if (p_hi && kFixedShape && rad.N == 12 && rad.L == 9) {
@@ -3148,7 +3153,7 @@ void launch_power_spectrum_export(const RadialDev& rad, int S, int64_t n, const 
   if (n == 0) return;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
   int KC = 0;
-  const size_t smem = power_spectrum_lds<float>(rad, S, tiles, &KC);
+  const size_t smem = power_spectrum_lds<float>(rad, S, n, tiles, &KC);
   auto kern = power_spectrum_export_kernel<float>;
   allow_lds(kern, smem);
   hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), smem, stream, rad.N, rad.L, S, KC, c, norm2,
