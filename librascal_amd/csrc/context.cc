@@ -140,7 +140,7 @@ struct Context {
   // held only when a diagonal key's block of some point is not symmetric, since
   // two such points' product is not that of their symmetric packed rows.
   DeviceBuffer<double> T_full;
-  DeviceBuffer<int> d_asymmetric;
+  PinnedBuffer<int> asymmetric_flag;
   bool asymmetric = false;
   DeviceBuffer<float> T32;
   MixedSparse mixed_sparse;
@@ -2071,24 +2071,21 @@ int rgpu_set_sparse_points(rgpu_context* ctx, int zeta, int64_t n_sparse, const 
     double* dT = c.T64.reserve(size_t(n1 * ldx));
     double* dTf = full.reserve(size_t(n1 * D));
     float* dT32 = c.T32.reserve(size_t(n1 * D));
-    int asymmetric = 0;
+    int* flag = c.asymmetric_flag.reserve(1);  // (written by the packing kernel)
+    *flag = 0;
     if (n_sparse > 0) {
       RGPU_HIP(hipMemcpyAsync(dr, values, sizeof(double) * size_t(n_sparse * D), hipMemcpyHostToDevice, c.stream));
       RGPU_HIP(hipMemcpyAsync(dord, order.data(), sizeof(int64_t) * size_t(n_sparse), hipMemcpyHostToDevice,
                               c.stream));
       launch_gather_rows<double>(n_sparse, D, D, dr, dord, dTf, c.stream);
       launch_gather_rows<float>(n_sparse, D, D, dr, dord, dT32, c.stream);
-      if (c.sparsified()) {
+      if (c.sparsified())
         launch_gather_rows<double>(n_sparse, D, ldx, dr, dord, dT, c.stream);
-      } else {
-        int* da = c.d_asymmetric.reserve(1);
-        RGPU_HIP(hipMemsetAsync(da, 0, sizeof(int), c.stream));
-        launch_sym_pack(S, c.rd.N, c.rd.L1, n_sparse, dr, dord, dT, c.stream, da);
-        RGPU_HIP(hipMemcpyAsync(&asymmetric, da, sizeof(int), hipMemcpyDeviceToHost, c.stream));
-      }
+      else
+        launch_sym_pack(S, c.rd.N, c.rd.L1, n_sparse, dr, dord, dT, c.stream, c.asymmetric_flag.device());
       RGPU_HIP(hipStreamSynchronize(c.stream));
     }
-    c.asymmetric = asymmetric != 0;
+    c.asymmetric = *flag != 0;
     if (c.asymmetric) {
       const int64_t ldf = gap_f64_k_stride(D);
       launch_gather_rows<double>(n_sparse, D, ldf, dr, dord, c.T_full.reserve(size_t(n_sparse * ldf)), c.stream);
