@@ -1000,7 +1000,7 @@ const float* ensure_p32(Context& c) {
     float* p = c.p32.reserve(size_t(std::max<int64_t>(n * c.D(), 1)));
     double* n2 = c.tmp_norm2.reserve(size_t(std::max<int64_t>(n, 1)));
     if (n > 0)
-      launch_power_spectrum<float>(c.rd, int(c.species.size()), n, c.c32.get(), p, n2, c.stream,
+      launch_power_spectrum(c.rd, int(c.species.size()), n, c.c32.get(), p, n2, c.stream,
                                    c.tile());
     c.p32_valid = true;
   }

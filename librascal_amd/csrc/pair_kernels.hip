@@ -89,29 +89,6 @@ struct PairRec {
   int sp, klo;
 };
 
-// Spline cell of a pair at distance d whose neighbour has species sp (the
-// cell search of the reference's interpolator; with one table per species, on
-// the neighbour species' own grid): its number, the weight of its upper end
-// and its width
-__device__ __forceinline__ int spline_cell_of(const RadialDev& rad, double d, int sp, double* a, double* h) {
-  int k;
-  double xhi;
-  if (rad.sp_tab) {
-    const int t = rad.sp_tab[sp], last = rad.tab_n[t] - 2;
-    k = int((d - rad.x1) * rad.tab_pu[t]) - 1;
-    k = k < 0 ? 0 : (k > last ? last : k);
-    xhi = rad.tab_grid[rad.tab_grid0[t] + k + 1];
-    *h = rad.tab_h[t];
-    *a = (xhi - d) / *h;
-    return rad.tab_cell0[t] + k;
-  }
-  k = int((d - rad.x1) * rad.per_unit) - 1;
-  k = k < 0 ? 0 : (k > rad.search_size ? rad.search_size : k);
-  *h = rad.h;
-  *a = (rad.grid[k + 1] - d) / *h;
-  return k;
-}
-
 template <class T>
 __device__ __forceinline__ PairRec<T> load_pair(const RadialDev& rad, const PairView& pv, int64_t p) {
   PairRec<T> r;
@@ -120,9 +97,9 @@ __device__ __forceinline__ PairRec<T> load_pair(const RadialDev& rad, const Pair
   r.x = T(pv.pair_vec[3 * p] / d);
   r.y = T(pv.pair_vec[3 * p + 1] / d);
   r.z = T(pv.pair_vec[3 * p + 2] / d);
-  double a, h;
-  r.klo = spline_cell_of(rad, d, r.sp, &a, &h);
-  const double b = 1 - a, fr = fc / d, fh = fc / h;
+  double xhi, h;
+  r.klo = spline_cell_of(rad, d, r.sp, &xhi, &h);
+  const double a = (xhi - d) / h, b = 1 - a, fr = fc / d, fh = fc / h;
   const double ca = a * (a * a - 1), cb = b * (b * b - 1);
   r.ra = T(a * fr);
   r.rb = T(ca * fr);
@@ -152,9 +129,9 @@ __device__ __forceinline__ PairValue<T> load_pair_value(const RadialDev& rad, co
   r.x = T(pv.pair_vec[3 * p] / d);
   r.y = T(pv.pair_vec[3 * p + 1] / d);
   r.z = T(pv.pair_vec[3 * p + 2] / d);
-  double a, h;
-  r.klo = spline_cell_of(rad, d, r.sp, &a, &h);
-  const double b = 1 - a;
+  double xhi, h;
+  r.klo = spline_cell_of(rad, d, r.sp, &xhi, &h);
+  const double a = (xhi - d) / h, b = 1 - a;
   r.ra = T(a * fc);
   r.rb = T(a * (a * a - 1) * fc);
   r.rc = T(b * fc);

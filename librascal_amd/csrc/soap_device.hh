@@ -283,6 +283,27 @@ struct SplineCell {
   T a, b, inv_h;
 };
 
+// Spline cell of a pair at distance d whose neighbour has species sp (the cell
+// search of the reference's interpolator): its number, its upper end and its
+// width; with one table per species, on the neighbour species' own grid, its
+// cells numbered on from the tables before it
+__device__ __forceinline__ int spline_cell_of(const RadialDev& rad, double d, int sp, double* xhi, double* h) {
+  int k;
+  if (rad.sp_tab) {
+    const int t = rad.sp_tab[sp], last = rad.tab_n[t] - 2;
+    k = int((d - rad.x1) * rad.tab_pu[t]) - 1;
+    k = k < 0 ? 0 : (k > last ? last : k);
+    *xhi = rad.tab_grid[rad.tab_grid0[t] + k + 1];
+    *h = rad.tab_h[t];
+    return rad.tab_cell0[t] + k;
+  }
+  k = int((d - rad.x1) * rad.per_unit) - 1;
+  k = k < 0 ? 0 : (k > rad.search_size ? rad.search_size : k);
+  *xhi = rad.grid[k + 1];
+  *h = rad.h;
+  return k;
+}
+
 template <class T>
 __device__ inline SplineCell<T> spline_cell(const RadialDev& R, double r) {
   SplineCell<T> c;

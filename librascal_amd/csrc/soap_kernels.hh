@@ -127,8 +127,7 @@ void launch_expansion_ps(const RadialDev& rad, int S, const PairView& pv, T* c,
                          double* norm2, hipStream_t stream, const SoapTiles& tiles = SoapTiles());
 
 // p[i][key(a<=b)][n1*N+n2][l] UN-normalised, and norm2[i] = |p_i|^2 (FP64).
-template <class T>
-void launch_power_spectrum(const RadialDev& rad, int S, int64_t n_centres, const T* c, T* p,
+void launch_power_spectrum(const RadialDev& rad, int S, int64_t n_centres, const float* c, float* p,
                            double* norm2, hipStream_t stream, const SoapTiles& tiles = SoapTiles());
 
 // The same power spectrum in the packed layout (packing.hh) written as the

@@ -362,23 +362,7 @@ __device__ __forceinline__ void pair_fetch(const RadialDev& rad, const PairView&
     f.j = pv.pair_j[p];
     f.sp = pv.species_of[f.j];
     if (!DIRECT) {
-      // spline cell as in spline_cell(); with one table per species, on
-      // the neighbour species' own grid, its cells numbered on from the
-      // tables before it
-      if (rad.sp_tab) {
-        const int t = rad.sp_tab[f.sp], last = rad.tab_n[t] - 2;
-        int k = int((f.d - rad.x1) * rad.tab_pu[t]) - 1;
-        k = k < 0 ? 0 : (k > last ? last : k);
-        f.xhi = rad.tab_grid[rad.tab_grid0[t] + k + 1];
-        f.h = rad.tab_h[t];
-        f.klo = rad.tab_cell0[t] + k;
-      } else {
-        int k = int((f.d - rad.x1) * rad.per_unit) - 1;
-        k = k < 0 ? 0 : (k > rad.search_size ? rad.search_size : k);
-        f.xhi = rad.grid[k + 1];
-        f.h = rad.h;
-        f.klo = k;
-      }
+      f.klo = spline_cell_of(rad, f.d, f.sp, &f.xhi, &f.h);
     }
   }
 }
@@ -812,9 +796,6 @@ __device__ __forceinline__ void ps_body(int N_, int L_, int S, int KC, int64_t D
   __syncthreads();  // red and the stage may be reused
 }
 
-// out row r = row rows[r] of p (rows null: row r), divided by its norm when
-// normalising
-
 template <class T, bool SPLIT, int NC = -1, int LC = -1>
 __global__ __launch_bounds__(kThreads) void power_spectrum_kernel(int N_, int L_, int S, int KC, int64_t Dq,
                                                                   const T* __restrict__ c,
@@ -999,6 +980,8 @@ __global__ __launch_bounds__(kThreads, 4) void expansion_ps_kernel(
   }
 }
 
+// out row r = row rows[r] of p (rows null: row r; rows ld apart), divided by its
+// norm when normalising
 template <class T>
 __global__ void normalise_kernel(int64_t n, int64_t D, int64_t ld, const T* __restrict__ p,
                                  const double* __restrict__ norm2, int normalize,
@@ -3135,10 +3118,9 @@ template void launch_expansion_ps<float>(const RadialDev&, int, const PairView&,
                                          unsigned long long*, float*, unsigned short*, unsigned short*,
                                          double*, hipStream_t, const SoapTiles&);
 
-template <class T>
-void launch_power_spectrum(const RadialDev& rad, int S, int64_t n, const T* c, T* p, double* norm2,
+void launch_power_spectrum(const RadialDev& rad, int S, int64_t n, const float* c, float* p, double* norm2,
                            hipStream_t stream, const SoapTiles& tiles) {
-  launch_power_spectrum_impl<T>(rad, S, n, c, p, nullptr, nullptr, norm2, stream, tiles);
+  launch_power_spectrum_impl<float>(rad, S, n, c, p, nullptr, nullptr, norm2, stream, tiles);
 }
 
 void launch_power_spectrum_split(const RadialDev& rad, int S, int64_t n, const float* c,
@@ -3448,10 +3430,6 @@ template void launch_expansion<double>(const RadialDev&, int, const PairView&, d
                                        unsigned long long*, hipStream_t, const SoapTiles&);
 template void launch_expansion<float>(const RadialDev&, int, const PairView&, float*,
                                       unsigned long long*, hipStream_t, const SoapTiles&);
-template void launch_power_spectrum<double>(const RadialDev&, int, int64_t, const double*, double*,
-                                            double*, hipStream_t, const SoapTiles&);
-template void launch_power_spectrum<float>(const RadialDev&, int, int64_t, const float*, float*,
-                                           double*, hipStream_t, const SoapTiles&);
 template void launch_normalise<double>(int64_t, int64_t, const double*, const double*, bool, double*,
                                        hipStream_t, const int64_t*, int64_t);
 template void launch_normalise<float>(int64_t, int64_t, const float*, const double*, bool, double*,

@@ -9,7 +9,8 @@
 // a multiple of 32.  A dot product of two such rows equals the dot product of
 // the full feature rows (keys a <= b, [n1][n2][l]) when one of them is a
 // feature row; for another vector t the entries of a diagonal key are
-// (t[n1][n2] + t[n2][n1]) / sqrt 2 (n1 < n2) and t[n][n].  It is as short as
+// (t[n1][n2] + t[n2][n1]) / sqrt 2 (n1 < n2) and t[n][n]; of two such vectors
+// it is the product of their symmetric parts only.  A row is as short as
 // the key-major packed row (packing.hh), but an angular channel is one
 // contiguous run, so a wavefront can take a channel with a lane per row r and
 // every other operand wavefront-uniform.
@@ -50,9 +51,10 @@ struct SymSets {
 };
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
                               const double* norm2, const double* E, const double* T, double* dc, hipStream_t stream);
-// The same from dL/dX in full rows [n][K N^2 (L+1)] (keys a <= b): X = p / |p|
-// with p in symmetric packed rows and xg[i] = X . dL/dX (null: summed here),
-// or X = p (p null).  work: packed rows where they are needed
+// dL/dc of each centre, as launch_sym_contract, from dL/dX in full rows
+// [n][K N^2 (L+1)] (keys a <= b): X = p / |p| with p in symmetric packed rows and
+// xg[i] = X . dL/dX (null: summed here), or X = p (p null).  work: packed rows
+// where they are needed
 void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
                               const double* xg, const double* G, DeviceBuffer<double>& work, double* dc,
                               hipStream_t stream);
