@@ -615,3 +615,53 @@ def test_general_pair_phase_of_large_rows(S, N, L, spline):
     ctx.set_tiles(pairs_adj=1)
     for x, y in zip(got, ctx.features_backward(G)):
         assert np.abs(x - y).max() <= 1e-12 * np.abs(y).max()
+
+
+@pytest.mark.parametrize("species,atoms,points,N,L", [((1, 6, 7, 8), 1003, 17, 12, 9), ((6,), 2890, 2885, 3, 2)])
+def test_fp64_products_in_64_row_tiles(species, atoms, points, N, L):
+    """The FP64 products past 2048 tiles of 64 x 64, with remainders of rows,
+    columns and K steps: the force product (4 species: 184 column tiles of
+    features) and the energy and K_NM products (2885 sparse points), against
+    numpy and the adjoint of the model's dL/dX."""
+    sts = periodic_box(atoms, 0.05, species, d_min=1.0, seed=201)
+    ctx, num = _context(soap_hypers(rc=3.5, sw=0.5, sigma=0.5, N=N, L=L, spline=1e-8), sts)
+    rng = np.random.default_rng(202)
+    spec, vals, w = _points(ctx, num, {z: points for z in species}, rng)
+    ctx.set_sparse_points(2, spec, vals, w)
+    X, _ = ctx.features()
+    dot = np.where(num[:, None] == spec[None, :], X @ vals.T, 0.0)
+    assert np.abs(ctx.gap_knm("Atom") - dot ** 2).max() <= 1e-10 * np.abs(dot ** 2).max()
+    e, g, s = ctx.gap_predict()
+    assert abs(e[0] - (dot ** 2 @ w).sum()) <= 1e-10 * (np.abs(dot ** 2) @ np.abs(w)).sum()
+    gr, sr = ctx.features_backward((2 * dot * w) @ vals)
+    assert np.abs(g - gr).max() <= 1e-10 * np.abs(gr).max()
+    assert np.abs(s - sr).max() <= 1e-10 * np.abs(sr).max()
+
+
+def test_model_loaded_again_after_other_layouts():
+    """Predictions after the context's model was dropped by a batch with another
+    species list, or by a K_MM over one, equal a fresh calculator's."""
+    def calculator():
+        return SphericalInvariants(interaction_cutoff=3.5, cutoff_smooth_width=0.5, max_radial=4,
+                                   max_angular=3, gaussian_sigma_type="Constant")
+
+    frames = {sp: periodic_box(30, 0.05, sp, d_min=1.0, seed=210 + sp[-1]) for sp in ((1, 8), (1, 6))}
+
+    def model(rep, sp):
+        r = np.random.default_rng(sp[-1])
+        pts = SparsePoints.from_arrays(rep, sp, np.repeat(sp, 5), r.normal(size=(10, rep.get_num_coefficients(2))))
+        ker = Kernel(rep, name="GAP", kernel_type="Sparse", target_type="Structure", zeta=2)
+        return ker, pts, KRR(r.normal(size=10), ker, pts, {z: 0.0 for z in (1, 6, 8)})
+
+    fresh = calculator()
+    want = model(fresh, (1, 8))[2].predict_energy_forces_stress(fresh.transform(frames[(1, 8)]))
+    rep = calculator()
+    _, _, m = model(rep, (1, 8))
+    ker, pts, other = model(rep, (1, 6))
+    between = (lambda: None, lambda: rep.transform(frames[(1, 6)]),
+               lambda: other.predict(rep.transform(frames[(1, 6)])), lambda: ker(pts))
+    for do in between:
+        do()
+        got = m.predict_energy_forces_stress(rep.transform(frames[(1, 8)]))
+        for x, y in zip(got, want):
+            assert np.array_equal(x, y)
