@@ -2936,25 +2936,24 @@ void launch_adjoint_f32(const RadialDev& rad, int S, const PairView& pv, const f
 
 }  // namespace
 
-// Centres from which the expansion takes a wavefront per centre: below, too
-// few are in flight and the workgroup per centre has the shorter chain.  Per
-// entry against by wavefronts: 64 centres 13 and 19 us, 1024 centres (FP64)
-// 27 and 32 us, 1331 centres (FP32) 23 and 36 us, 4096 centres (FP64,
-// n_max 12, l_max 9) 167 and 72 us, 8192 centres (FP32) 178 and 93 us;
-// molecules of 8 atoms (n_max 8, l_max 6) FP64 46 and 48 us, FP32 (four times
-// as many) 277 and 167 us.  The fewer orders, the fewer lanes hold sums and the
-// more of the time goes into writing every species' block (with the neighbour
-// list of about 20 neighbours a centre, 2 species, per entry against by
-// wavefronts: l_max 7, n_max 12 2100 centres FP64 56 and 60, FP32 47 and 48 us,
-// 4500 88 and 88, 70 and 58; l_max 4, n_max 8 2100 39 and 41, 36 and 37, 12000
-// 108 and 98, 92 and 70; l_max 2, n_max 20 12000 105 and 161, 88 and 96; and 4
-// species, n_max 12, l_max 0 12000 92 and 117, 80 and 81), so with fewer it
-// starts later, and below l_max 6 only in FP32 and with up to 16 channels.
+// Where the expansion takes a wavefront per centre.  With few centres too few
+// are in flight and the workgroup per centre has the shorter chain (per entry
+// against by wavefronts, about 30 neighbours: l_max 8, n_max 10, 2 species, 2100
+// centres FP64 79 and 66, FP32 61 and 54 us with the neighbour list; l_max 7,
+// n_max 9 66 and 65, 54 and 54, 3000 83 and 72, 62 and 58; 4096 centres of 4
+// species, n_max 12, l_max 9 the expansion alone 167 and 72 us in FP64, 8192 178
+// and 93 in FP32; 1331 centres in FP32 23 and 36).  Every species' block of a
+// centre costs it the sums over the lanes and the stores however few orders there
+// are (12000 centres, n_max 10, l_max 2: 1 species FP64 91 and 81 us, 4 species
+// 104 and 119; n_max 12, l_max 0, 4 species 92 and 117), and many channels leave
+// few wavefronts in flight (n_max 20, l_max 2, 1 species 101 and 128; n_max 16,
+// l_max 4 126 and 128, in FP32 113 and 81; l_max 6 179 and 143).  In FP32 the sums
+// by wavefronts are also the more exact ones (4.1e-7 of max |c| against 6.6e-7), so
+// there they start at 2048 for every l_max.
 template <class T>
-bool wave_expansion_pays(const RadialDev& rad, int64_t n) {
-  if (rad.L >= 9) return n >= 2048;
-  if (rad.L >= 6) return n >= 4096;
-  return sizeof(T) == 4 && rad.N <= 16 && n >= 8192;
+bool wave_expansion_pays(const RadialDev& rad, int S, int64_t n) {
+  if (n < (rad.L >= 8 || sizeof(T) == 4 ? 2048 : 3072)) return false;
+  return rad.N <= 12 ? rad.LL >= 4 * S : rad.L >= (sizeof(T) == 4 ? 4 : 6);
 }
 
 template <class T>
@@ -2962,7 +2961,7 @@ void launch_expansion(const RadialDev& rad, int S, const PairView& pv, T* c,
                       unsigned long long* keymask, hipStream_t stream, const SoapTiles& tiles) {
   if (pv.n_centres == 0) return;
   if (S > kMaxSpecies) throw InvalidArgument("at most 64 species");
-  if ((tiles.fwd_group < 0 ? wave_expansion_pays<T>(rad, pv.n_centres) : tiles.fwd_group == 1) && pair_kernels_apply(rad)) {
+  if ((tiles.fwd_group < 0 ? wave_expansion_pays<T>(rad, S, pv.n_centres) : tiles.fwd_group == 1) && pair_kernels_apply(rad)) {
     launch_expansion_wave<T>(rad, S, pv, c, keymask, stream);
     return;
   }

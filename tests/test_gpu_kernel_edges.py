@@ -538,9 +538,9 @@ def test_expansion_set_to_wavefronts(N, L):
         assert np.abs(cw - c).max() <= tol * np.abs(c).max()
 
 
-@pytest.mark.parametrize("n,N,L", [(2047, 3, 9), (2048, 3, 9), (4095, 4, 6), (4096, 4, 6), (8191, 2, 1), (8192, 2, 1)])
+@pytest.mark.parametrize("n,N,L", [(2047, 3, 9), (2048, 3, 9), (2048, 4, 6), (3072, 4, 6), (3072, 2, 0), (3072, 13, 4)])
 def test_expansion_kernel_by_number_of_centres(n, N, L):
-    """Both sides of the centre counts at which the built-in expansion goes by
+    """Both sides of the sizes at which the built-in expansion goes by
     wavefronts: the same coefficients as with either kernel set."""
     pos = np.zeros((n, 3))
     pos[1::2, 0] = 1.0
