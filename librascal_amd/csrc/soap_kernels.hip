@@ -2686,7 +2686,11 @@ constexpr size_t kPsBudget = 32 * 1024, kPsBudgetMany = 48 * 1024;
 constexpr int kPsPasses = 8;
 constexpr int64_t kPsFew = 512;
 constexpr size_t kAdjBudget = 64 * 1024;
-constexpr size_t kResidentBudget = 52 * 1024;  // three workgroups per CU
+// three workgroups per CU: with the kernels' own 1.2 KB, 42 granules of 1280 bytes
+// each (at 52 KB some shapes took one more and two workgroups: the mixed adjoint
+// of 581 centres of 6 species, n_max 9, l_max 8 244 us,
+// 193 now)
+constexpr size_t kResidentBudget = 51 * 1024;
 
 // LDS limit per workgroup of the current device (queried once per device;
 // launches may be captured into graphs, where device queries are avoided)
