@@ -96,7 +96,7 @@ struct Context {
   // S^T of them in packed rows, formed when an adjoint asks
   DeviceBuffer<double> ps64, sel_packed;
   bool sel_valid = false;
-  DeviceBuffer<double> gfull, gsym;  // dL/dX scattered into the full layout, and packed
+  DeviceBuffer<double> gsym;         // dL/dX in packed rows
   DeviceBuffer<double> dc64, xdot;   // dL/dc of the FP64 adjoint, X . dL/dX
   DeviceBuffer<double> dcp, dcs;     // stored expansion derivatives (gradient export)
   DeviceBuffer<float> adj_work;      // dL/dc between the adjoint's two kernels (adj_kind 3)
@@ -943,12 +943,9 @@ void backward_device(Context& c, const float* G, double* grad, double* cvir, con
 const double* packed_features(Context& c) {
   if (!c.sparsified()) return c.p64.get();
   if (!c.sel_valid) {
-    const int S = int(c.species.size());
-    const int64_t n = c.n_atoms, D = c.D_full();
-    double* f = c.pfull.reserve(size_t(std::max<int64_t>(n * D, 1)));
-    double* s = c.sel_packed.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
-    launch_scatter_columns(n, c.ldx64(), c.selection(), c.ps64.get(), D, f, c.stream);
-    launch_sym_pack(S, c.rd.N, c.rd.L1, n, f, nullptr, s, c.stream);
+    const int64_t n = c.n_atoms, ld = sym_row_stride(int(c.species.size()), c.rd.N, c.rd.L1);
+    double* s = c.sel_packed.reserve(size_t(std::max<int64_t>(n * ld, 1)));
+    launch_scatter_selected(n, c.ldx64(), c.selection(), c.ps64.get(), ld, s, c.stream);
     c.sel_valid = true;
   }
   return c.sel_packed.get();
@@ -961,27 +958,32 @@ void launch_pair_phase(Context& c, const PairView& pv, const double* dc, double*
   else
     launch_adjoint_pairs(c.rd, S, pv, dc, cvir, c.stream, c.tile());
 }
-// FP64: G in symmetric packed rows of dL/dp, or (full) dL/dX in the full
-// layout, xg = X_i . dL/dX_i (null: summed here)
-void backward_device(Context& c, const double* G, bool full, const double* xg, double* grad, double* cvir) {
+// FP64: G in symmetric packed rows of dL/dp, or (kDx) of dL/dX with xg = X_i .
+// dL/dX_i, or (kFullDx) dL/dX in the full layout
+enum class GradientRows { kDp, kDx, kFullDx };
+void backward_device(Context& c, const double* G, GradientRows rows, const double* xg, double* grad, double* cvir) {
   const int S = int(c.species.size()), N = c.rd.N, L1 = c.rd.L1;
   StageTimer t(c, RGPU_STAGE_BACKWARD);
   ReverseLists rl;
   const PairView pv = backward_view(c, &rl);
   double* dc = c.dc64.reserve(size_t(c.n_atoms * S * N * c.rd.LL + kPairSlack));
-  if (full)
-    launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), c.hp.normalize ? packed_features(c) : nullptr,
-                             c.norm2.get(), xg, G, c.gsym, dc, c.stream);
+  const double* p = c.hp.normalize && rows != GradientRows::kDp ? packed_features(c) : nullptr;
+  if (rows == GradientRows::kFullDx)
+    launch_sym_contract_full(S, N, L1, c.n_atoms, c.c64.get(), p, c.norm2.get(), G, c.gsym, dc, c.stream);
+  else if (p)
+    launch_sym_contract_projected(S, N, L1, c.n_atoms, c.c64.get(), p, c.norm2.get(), xg, G, dc, c.stream);
   else
     launch_sym_contract(S, N, L1, c.n_atoms, c.c64.get(), G, dc, c.stream);
   launch_pair_phase(c, pv, dc, cvir);
   launch_force_gather(pv, rl, grad, c.stream);
 }
-// selected columns of dL/dX (or dL/dp, rows ld apart) into the full layout
-const double* scatter_selected(Context& c, const double* G, int64_t ld) {
-  double* gf = c.gfull.reserve(size_t(std::max<int64_t>(c.n_atoms * c.D_full(), 1)));
-  launch_scatter_columns(c.n_atoms, ld, c.selection(), G, c.D_full(), gf, c.stream);
-  return gf;
+// n rows of selected coefficients of dL/dX, dL/dp or sparse points (ld apart) as
+// symmetric packed rows
+const double* scatter_selected(Context& c, int64_t n, const double* G, int64_t ld) {
+  const int64_t lds = sym_row_stride(int(c.species.size()), c.rd.N, c.rd.L1);
+  double* gs = c.gsym.reserve(size_t(std::max<int64_t>(n * lds, 1)));
+  launch_scatter_selected(n, ld, c.selection(), G, lds, gs, c.stream);
+  return gs;
 }
 // the FP64 invariants in the full layout
 const double* full_invariants(Context& c) {
@@ -1167,13 +1169,9 @@ void gap_predict_t(Context& c, double* energy, double* gradient, double* neg_str
     // (the force gather writes every atom's gradient)
     // the GAP energy is homogeneous of degree zeta in X, so X_i . G_i = zeta E_i
     if constexpr (std::is_same<T, double>::value) {
-      // (dL/dp already: a selection's is scattered into the full layout and packed)
-      if (c.sparsified()) {
-        double* gs = c.gsym.reserve(size_t(std::max<int64_t>(n * sym_row_stride(S, c.rd.N, c.rd.L1), 1)));
-        launch_sym_pack(S, c.rd.N, c.rd.L1, n, scatter_selected(c, G, c.ldx64()), nullptr, gs, c.stream);
-        G = gs;
-      }
-      backward_device(c, G, false, nullptr, gd, cv);
+      // (dL/dp already, a selection's of its coefficients)
+      const double* g = c.sparsified() ? scatter_selected(c, n, G, c.ldx64()) : G;
+      backward_device(c, g, GradientRows::kDp, nullptr, gd, cv);
     } else {
       backward_device(c, G, gd, cv, ec, double(c.zeta));
     }
@@ -1780,16 +1778,16 @@ int rgpu_set_structures(rgpu_context* ctx, int n_struct, const int64_t* atom_off
                               c.stream));
       int64_t* dsp = c.d_sel_packed.reserve(spacked.size());
       RGPU_HIP(hipMemcpyAsync(dsp, spacked.data(), sizeof(int64_t) * spacked.size(), hipMemcpyHostToDevice, c.stream));
-      // inverse: the selections naming each full-layout column, ascending
-      const int64_t Df = c.D_full();
-      std::vector<int64_t> inv_off(size_t(Df + 1), 0), inv_k;
-      for (int64_t k : scol)
-        if (k >= 0) ++inv_off[size_t(k + 1)];
-      for (int64_t o = 0; o < Df; ++o) inv_off[size_t(o + 1)] += inv_off[size_t(o)];
-      inv_k.resize(size_t(std::max<int64_t>(inv_off[size_t(Df)], 1)));
+      // inverse: the selections of each packed entry, ascending
+      const int64_t ld = sym_row_stride(int(sp.size()), c.hp.max_radial, c.hp.max_angular + 1);
+      std::vector<int64_t> inv_off(size_t(ld + 1), 0), inv_k;
+      for (int64_t e : spacked)
+        if (e >= 0) ++inv_off[size_t((e >> 1) + 1)];
+      for (int64_t o = 0; o < ld; ++o) inv_off[size_t(o + 1)] += inv_off[size_t(o)];
+      inv_k.resize(size_t(std::max<int64_t>(inv_off[size_t(ld)], 1)));
       std::vector<int64_t> fill(inv_off.begin(), inv_off.end() - 1);
-      for (size_t k = 0; k < scol.size(); ++k)
-        if (scol[k] >= 0) inv_k[size_t(fill[size_t(scol[k])]++)] = int64_t(k);
+      for (size_t k = 0; k < spacked.size(); ++k)
+        if (spacked[k] >= 0) inv_k[size_t(fill[size_t(spacked[k] >> 1)]++)] = int64_t(2 * k) + (spacked[k] & 1);
       int64_t* dio = c.d_sel_inv_off.reserve(inv_off.size());
       int64_t* dik = c.d_sel_inv_k.reserve(inv_k.size());
       RGPU_HIP(hipStreamSynchronize(c.stream));  // no kernel still reads the old map
@@ -1973,7 +1971,7 @@ int rgpu_get_features_gradient(rgpu_context* ctx, double* out) {
     // un-normalised invariants of the output columns, rows D apart
     const double* sel = nullptr;
     if (c.sparsified()) {
-      double* t = c.gfull.reserve(size_t(n * D));
+      double* t = c.pfull.reserve(size_t(n * D));
       launch_normalise<double>(n, D, c.ps64.get(), nullptr, false, t, c.stream, nullptr, c.ldx64());
       sel = t;
     }
@@ -2004,18 +2002,16 @@ int rgpu_features_backward(rgpu_context* ctx, const double* dL_dX, double* dL_dr
       g64 = t;
     }
     if (c.precision == RGPU_FP64) {
-      const double* dot = nullptr;
-      if (c.sparsified()) {
+      if (!c.sparsified()) {
+        backward_device(c, g64, GradientRows::kFullDx, nullptr, gd, cv);
+      } else {
         // (X . dL/dX over the selection itself: a coefficient selected twice
         // enters both factors of a product of the spread-out rows twice)
-        if (c.hp.normalize) {
-          double* d = c.xdot.reserve(size_t(std::max<int64_t>(n, 1)));
-          launch_row_dot(n, D, c.ps64.get(), c.ldx64(), g64, D, c.norm2.get(), d, c.stream);
-          dot = d;
-        }
-        g64 = scatter_selected(c, g64, D);
+        double* dot = c.xdot.reserve(size_t(std::max<int64_t>(n, 1)));
+        if (c.hp.normalize)
+          launch_row_dot(n, D, c.ps64.get(), c.ldx64(), g64, D, c.norm2.get(), dot, c.stream);
+        backward_device(c, scatter_selected(c, n, g64, D), GradientRows::kDx, dot, gd, cv);
       }
-      backward_device(c, g64, true, dot, gd, cv);
     } else {
       // dL/dX in the packed layout of the mixed path
       float* g32 = c.G32.reserve(size_t(std::max<int64_t>(n * c.Dp(), 1)));
@@ -2200,13 +2196,7 @@ int rgpu_gap_knm_gradient(rgpu_context* ctx, int neg_stress, double* out) {
     const int N = c.rd.N, L1 = c.rd.L1;
     const int64_t lds = sym_row_stride(S, N, L1), E = int64_t(S) * N * c.rd.LL;
     const double* T = c.T64.get();
-    if (c.sparsified()) {
-      double* gf = c.gfull.reserve(size_t(M * c.D_full()));
-      double* gs = c.gsym.reserve(size_t(M * lds));
-      launch_scatter_columns(M, c.ldx64(), c.selection(), T, c.D_full(), gf, c.stream);
-      launch_sym_pack(S, N, L1, M, gf, nullptr, gs, c.stream);
-      T = gs;
-    }
+    if (c.sparsified()) T = scatter_selected(c, M, T, c.ldx64());
     // the part of dL/dc along p, which the normalisation projects out
     const double* dp = nullptr;
     if (c.hp.normalize) {

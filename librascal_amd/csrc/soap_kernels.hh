@@ -169,8 +169,8 @@ void launch_feature_gradient_rows(int N, int L1, int S, const PairView& pv, int6
 // coefficient_subselection as device arrays: packed[k] (Dsel; -1 for a
 // coefficient outside the layout), twice the entry of a symmetric packed row
 // (sym_kernels.hh) that holds coefficient k, plus 1 where the entry is sqrt 2
-// times it; and the selections k naming full-layout column o in ascending
-// order at inv_k[inv_off[o] .. inv_off[o+1])
+// times it; and, packed entry by entry, the selections k that it holds, each 2 k
+// plus that 1, in ascending order at inv_k[inv_off[e] .. inv_off[e + 1])
 struct SelectionMap {
   const int64_t* packed = nullptr;
   const int64_t* inv_off = nullptr;
@@ -180,10 +180,10 @@ struct SelectionMap {
 // packed rows p (ld apart), norm2[i] = |xs_i|^2
 void launch_select_invariants(int64_t n, int64_t ld, int64_t Dsel, int64_t lds, const SelectionMap& sel,
                               const double* p, double* xs, double* norm2, hipStream_t stream);
-// dst[i][:D] = S^T src[i][:Dsel], src rows lds apart (repeated selections summed in ascending
-// selection order)
-void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t D,
-                            double* dst, hipStream_t stream);
+// dst[i] (rows of ld values) = the symmetric packed row of S^T src[i], src rows
+// lds apart (repeated selections summed in ascending selection order)
+void launch_scatter_selected(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t ld,
+                             double* dst, hipStream_t stream);
 
 // Pair phase of the FP64 adjoint: from dL/dc [n][S][(L+1)^2][N] of each
 // centre, the pair and centre forces of dL/dr (pv.pair_force,

@@ -2652,20 +2652,23 @@ __global__ __launch_bounds__(kThreads) void select_invariants_kernel(int64_t ld,
   }
 }
 
-// dst[i] = S^T src[i] (rows of selected columns, lds apart, into rows of D
-// columns, repeated selections summed in ascending selection order through
-// the inverse map inv_off/inv_k), one workgroup per row
-__global__ __launch_bounds__(kThreads) void scatter_columns_kernel(int64_t lds,
-                                                                   const int64_t* __restrict__ inv_off,
-                                                                   const int64_t* __restrict__ inv_k,
-                                                                   const double* __restrict__ src,
-                                                                   int64_t D, double* __restrict__ dst) {
+// dst[i] = S^T src[i] as a symmetric packed row (repeated selections, and the two
+// orders of a diagonal key's channels, summed in ascending selection order through
+// the inverse map), one workgroup per row
+__global__ __launch_bounds__(kThreads) void scatter_selected_kernel(int64_t lds,
+                                                                    const int64_t* __restrict__ inv_off,
+                                                                    const int64_t* __restrict__ inv_k,
+                                                                    const double* __restrict__ src,
+                                                                    int64_t ld, double* __restrict__ dst) {
   const int64_t i = blockIdx.x;
-  double* di = dst + i * D;
+  double* di = dst + i * ld;
   const double* si = src + i * lds;
-  for (int64_t o = threadIdx.x; o < D; o += kThreads) {
+  for (int64_t o = threadIdx.x; o < ld; o += kThreads) {
     double t = 0.0;
-    for (int64_t q = inv_off[o]; q < inv_off[o + 1]; ++q) t += si[inv_k[q]];
+    for (int64_t q = inv_off[o]; q < inv_off[o + 1]; ++q) {
+      const int64_t k = inv_k[q];
+      t += si[k >> 1] * (k & 1 ? 0.70710678118654752440 : 1.0);
+    }
     di[o] = t;
   }
 }
@@ -3259,11 +3262,11 @@ void launch_select_invariants(int64_t n, int64_t ld, int64_t Dsel, int64_t lds, 
   RGPU_LAUNCH_CHECK();
 }
 
-void launch_scatter_columns(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t D,
-                            double* dst, hipStream_t stream) {
+void launch_scatter_selected(int64_t n, int64_t lds, const SelectionMap& sel, const double* src, int64_t ld,
+                             double* dst, hipStream_t stream) {
   if (n == 0) return;
-  hipLaunchKernelGGL(scatter_columns_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, lds, sel.inv_off,
-                     sel.inv_k, src, D, dst);
+  hipLaunchKernelGGL(scatter_selected_kernel, dim3(unsigned(n)), dim3(kThreads), 0, stream, lds, sel.inv_off,
+                     sel.inv_k, src, ld, dst);
   RGPU_LAUNCH_CHECK();
 }
 

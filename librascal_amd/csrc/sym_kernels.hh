@@ -38,6 +38,11 @@ void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* 
 // packed rows
 void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const double* G, double* dc,
                          hipStream_t stream);
+// the same from dL/dX, X = p / |p|, in symmetric packed rows: p likewise, xg[i] =
+// X . dL/dX
+void launch_sym_contract_projected(int S, int N, int L1, int64_t n, const double* c, const double* p,
+                                   const double* norm2, const double* xg, const double* G, double* dc,
+                                   hipStream_t stream);
 // dL/dc [n_sets][n_ids] of the kernel derivatives of sparse points T (symmetric
 // packed rows, one per set) at the centres ids: dL/dX_i = zeta d^(zeta - 1) T_q
 // with d = X_i . T_q = dot[i ld_dot + q], X = p / |p|; E: dL/dc of dL/dp = p for
@@ -52,12 +57,10 @@ struct SymSets {
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
                               const double* norm2, const double* E, const double* T, double* dc, hipStream_t stream);
 // dL/dc of each centre, as launch_sym_contract, from dL/dX in full rows
-// [n][K N^2 (L+1)] (keys a <= b): X = p / |p| with p in symmetric packed rows and
-// xg[i] = X . dL/dX (null: summed here), or X = p (p null).  work: packed rows
-// where they are needed
+// [n][K N^2 (L+1)] (keys a <= b): X = p / |p| with p in symmetric packed rows,
+// or X = p (p null).  work: packed rows where they are needed
 void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
-                              const double* xg, const double* G, DeviceBuffer<double>& work, double* dc,
-                              hipStream_t stream);
+                              const double* G, DeviceBuffer<double>& work, double* dc, hipStream_t stream);
 
 // Full rows [.][K N^2 (L+1)] to symmetric packed rows and back.  Packing row
 // r from full row rows[r] (rows null: row r); unpacking row r of out from

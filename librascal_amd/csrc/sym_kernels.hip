@@ -278,7 +278,6 @@ __global__ __launch_bounds__(kThreads) void sym_contract_full_kernel(int R, int 
                                                                      const double* __restrict__ c,
                                                                      const double* __restrict__ p,
                                                                      const double* __restrict__ norm2,
-                                                                     const double* __restrict__ xg,
                                                                      const double* __restrict__ G,
                                                                      double* __restrict__ dc) {
   const int64_t i = blockIdx.x;
@@ -328,19 +327,14 @@ __global__ __launch_bounds__(kThreads) void sym_contract_full_kernel(int R, int 
     const double* pi = p + i * ld;
     const float inv_t = 1.0f / float(TRI);
     auto channel_of = [&](int t) { return int((float(t) + 0.5f) * inv_t); };
-    double x = 0.0;
-    if (xg) {
-      x = xg[i];
-    } else {
-      double d = 0.0;
+    double d = 0.0;
 #pragma unroll 8
-      for (int t = threadIdx.x; t < L1 * TRI; t += kThreads) d += pi[t] * W[t + channel_of(t) * (LT - TRI)];
-      for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
-      if (lane == 0) red[wave] = d;
-      __syncthreads();
-      if (n2 > 0) x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
-    }
+    for (int t = threadIdx.x; t < L1 * TRI; t += kThreads) d += pi[t] * W[t + channel_of(t) * (LT - TRI)];
+    for (int off = 32; off > 0; off >>= 1) d += __shfl_down(d, off, 64);
+    if (lane == 0) red[wave] = d;
+    __syncthreads();
     if (n2 > 0) {
+      const double x = ((red[0] + red[1]) + (red[2] + red[3])) / sqrt(n2);
       const double alpha = 1.0 / sqrt(n2), beta = x / n2;
 #pragma unroll 8
       for (int t = threadIdx.x; t < L1 * TRI; t += kThreads) {
@@ -682,6 +676,13 @@ void launch_sym_contract(int S, int N, int L1, int64_t n, const double* c, const
   go_contract<false>(S, N, L1, n, c, nullptr, nullptr, nullptr, nullptr, 0, G, dc, stream);
 }
 
+void launch_sym_contract_projected(int S, int N, int L1, int64_t n, const double* c, const double* p,
+                                   const double* norm2, const double* xg, const double* G, double* dc,
+                                   hipStream_t stream) {
+  if (n == 0) return;
+  go_contract<true>(S, N, L1, n, c, p, norm2, xg, nullptr, 0, G, dc, stream);
+}
+
 void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSets& sets, const double* c,
                               const double* norm2, const double* E, const double* T, double* dc,
                               hipStream_t stream) {
@@ -706,8 +707,7 @@ void launch_sym_contract_sets(int S, int N, int L1, int64_t n_sets, const SymSet
 }
 
 void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, const double* p, const double* norm2,
-                              const double* xg, const double* G, DeviceBuffer<double>& work, double* dc,
-                              hipStream_t stream) {
+                              const double* G, DeviceBuffer<double>& work, double* dc, hipStream_t stream) {
   if (n == 0) return;
   const int R = S * N;
   const size_t whole = sizeof(double) * size_t(L1) * full_stride(R) + sizeof(int) * size_t(S) * (S + 1) / 2;
@@ -715,7 +715,7 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
     auto go = [&](auto kern) {
       allow_lds(kern, whole);
       hipLaunchKernelGGL(kern, dim3(unsigned(n)), dim3(kThreads), whole, stream, R, N, L1 - 1,
-                         sym_row_stride(S, N, L1), c, p, norm2, xg, G, dc);
+                         sym_row_stride(S, N, L1), c, p, norm2, G, dc);
       RGPU_LAUNCH_CHECK();
     };
     if (L1 <= 10)
@@ -730,14 +730,13 @@ void launch_sym_contract_full(int S, int N, int L1, int64_t n, const double* c, 
   const int64_t ld = sym_row_stride(S, N, L1);
   const unsigned split = row_split(S, N, L1, n);
   double* g = work.reserve(size_t(n * ld + n * split));
-  if (p && !xg)
+  if (p) {
     go_pack<kDot>(S, N, L1, n, split, G, nullptr, g, nullptr, p, g + n * ld, stream);
-  else
+    go_contract<true>(S, N, L1, n, c, p, norm2, nullptr, g + n * ld, int(split), g, dc, stream);
+  } else {
     go_pack<kPlain>(S, N, L1, n, split, G, nullptr, g, nullptr, nullptr, nullptr, stream);
-  if (p)
-    go_contract<true>(S, N, L1, n, c, p, norm2, xg, g + n * ld, int(split), g, dc, stream);
-  else
     go_contract<false>(S, N, L1, n, c, nullptr, nullptr, nullptr, nullptr, 0, g, dc, stream);
+  }
 }
 
 void launch_sym_pack(int S, int N, int L1, int64_t n, const double* full, const int64_t* rows, double* out,
