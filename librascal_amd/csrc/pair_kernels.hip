@@ -9,9 +9,9 @@
 // read dL/dc and the harmonics of every order from LDS, 20 bytes for 4 FMAs,
 // which bounded it; the chain from staging a batch to its sums does now, with
 // 3 (FP64) or 4 wavefronts per SIMD.  Before and after: FP32, n_max 12,
-// l_max 9, 8192 centres (264 000 pairs) 282 and 174 us; FP64, 4096 centres
-// 332 and 162 us, n_max 10, l_max 8, 1024 centres 61 and 52 us, 64 centres
-// of n_max 8, l_max 6 24 and 17 us.
+// l_max 9, 8192 centres of 27 neighbours 282 and 174 us (204 with 31 neighbours);
+// FP64, 4096 centres 332 and 162 us, n_max 10, l_max 8, 1024 centres 61 and 52
+// us, 64 centres of n_max 8, l_max 6 24 and 17 us.
 //
 // A wavefront takes its centre's pairs 64 at a time, a lane each for the pair
 // records and the final force, and works through them species by species in
@@ -542,8 +542,9 @@ __host__ __device__ constexpr int expansion_row() {
 // in registers, two FMAs per channel and pair whose radial operand all lanes
 // of one l share.  (The per-entry kernel reads both operands of every FMA from
 // LDS, which bounds it; the staging of a batch bounds this one.)  One
-// wavefront per centre, several in turn: 178 -> 93 us for 264 000 pairs of
-// 8192 centres, n_max 12, l_max 9, FP32; 167 -> 72 us for 4096 centres, FP64.
+// wavefront per centre, several in turn: 178 -> 93 us for 8192 centres
+// of 27 neighbours, n_max 12, l_max 9, FP32 (104 with 31); 167 -> 72 us for 4096
+// centres, FP64.
 template <class T, int NT>
 __host__ __device__ inline size_t expansion_wave_lds(int L1) {
   return sizeof(T) * (size_t(kBatch) * (((L1 * L1) + 1) / 2 * 2 + size_t(L1) * expansion_row<T, NT>()));

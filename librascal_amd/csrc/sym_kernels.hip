@@ -6,8 +6,9 @@
 // registers; the row C_l[c][:] of every step is the same for the whole
 // wavefront, so it is read through scalar loads and enters the FMAs as a
 // scalar operand, beside one packed entry per step from LDS.  (A matrix-core
-// form of that one took 354 us where this takes 318: its operands come
-// through the packed triangle, and it leaves fewer wavefronts in flight.)
+// form of that one took 354 us where this took 318, and takes 249 with several
+// columns in flight: its operands come through the packed triangle, and it
+// leaves fewer wavefronts in flight.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -267,10 +268,9 @@ __global__ __launch_bounds__(kThreads) void sym_contract_kernel(int R, int N, in
 }
 
 // The same from full rows of dL/dX, the whole packed row formed in LDS first
-// (channels LT apart): the full row is read once along itself, where taking
-// the entries channel by channel touches a cache line per entry.  2000
-// centres: 98 -> 71 us (4 species, n_max 8, l_max 6), 178 -> 83 us (3
-// species, n_max 10, l_max 8); bound by the chain of its phases.
+// (channels LT apart): the full row is read once along itself, and no packed row
+// goes through memory.  4689 centres of 4 species, n_max 8, l_max 6: 173 us,
+// bound by the chain of its phases.
 __host__ __device__ inline int full_stride(int R) { return tri_i(R) | 1; }
 
 template <int LM>
@@ -609,10 +609,12 @@ void launch_sym_power(int S, int N, int L1, int64_t n, const double* c, double* 
 namespace {
 
 constexpr size_t kContractLds = 156 * 1024;
-// sym_contract_full_kernel: three workgroups per CU at least (with 2 species,
-// n_max 12, l_max 9 it took 73 us against 107 by channels, 3 species 176
-// against 254, but 4 species, one workgroup, 552 against 476; 2000 centres)
-constexpr size_t kFullLds = 54 * 1024;
+// sym_contract_full_kernel: two workgroups per CU at least.  Adjoint from full
+// rows, whole in LDS against packed first: 2000 centres of 2 species, n_max 12,
+// l_max 9 (23 KB) 129 and 158 us, 3 species (52 KB) 237 and 303, 4 species, n_max
+// 10, l_max 8 (57 KB) 261 and 310, 1500 of 6, n_max 8, l_max 6 (64 KB) 147 and 225,
+// but 2000 of 4, n_max 12, l_max 9 (91 KB) 509 and 441.
+constexpr size_t kFullLds = 78 * 1024;
 // A triangle for each wavefront while two workgroups per CU have them (R <= 65),
 // else one for the workgroup, four times as many of which fit.  Adjoint of a
 // prediction, own against shared: 64 rows (8 species, n_max 8, l_max 4) 76 and

@@ -563,7 +563,8 @@ def test_expansion_kernel_by_number_of_centres(n, N, L):
     (5, 13, 1, True), (6, 11, 3, True), (3, 23, 10, False),  # 65, 66, 69 rows: own triangles, one shared by two row blocks
     (13, 10, 2, True), (12, 16, 1, True),                    # 130 and 192 rows: three row blocks
     (13, 16, 1, True), (13, 16, 0, False),                   # 208: entries from memory
-    (2, 20, 12, True), (4, 12, 9, True),                     # rows past those formed whole in LDS, own triangles
+    (4, 10, 8, True), (7, 8, 6, False),                      # 57 and 86 KB: formed whole in LDS, or packed first
+    (2, 20, 12, True), (4, 12, 9, True),                     # past those, own triangles
 ])
 def test_fp64_adjoint_of_wide_rows(S, N, L, normalize):
     """The FP64 adjoint from full rows at the edges of its forms (rows formed
